@@ -72,6 +72,12 @@ def test_dequant_bit_exact(K, cb, k, n):
     assert bad.shape[0] == 0, f"{bad.shape[0]} differing fp16 words, first at {tuple(bad[0])}"
 
 
+@pytest.mark.parametrize("K,cb,k,n", [(1, 1, 640, 896), (6, 0, 896, 640), (7, 2, 640, 896)])
+def test_dequant_bit_exact_many_blocks(K, cb, k, n):
+    """Odd block counts and ~9 draws of every 16-bit state: the decode rounds by the fp16 rounding mode."""
+    test_dequant_bit_exact(K, cb, k, n)
+
+
 def test_dequant_torch_op_matches_oracle():
     from sglang_exl3 import ops
 
