@@ -157,6 +157,23 @@ int exl3_gemm(const uint16_t* x, const int16_t* trellis, const uint16_t* suh, co
  * every call leaves the counters zero. */
 size_t exl3_gemm_workspace_size(int m, int k, int n, int K);
 
+/* Scratch bytes exl3_linear_cat needs (zero-filled before its first use, left
+ * zeroed by every call). */
+size_t exl3_linear_cat_workspace_size(int m, int k, const int* n, int count, int K);
+
+/* One to four EXL3 weights of one K and codebook over the same input rows,
+ * outputs side by side: y[m][n[0] + n[1] + ..] = [x . W_0 | x . W_1 | ..], any
+ * m >= 1, each weight with its own suh and svh.  x_dtype and y_dtype:
+ * EXL3_DTYPE_F16 or EXL3_DTYPE_BF16; bfloat16 inputs are rounded to f16, and a
+ * bfloat16 output is the f16 result rounded, as casts around exl3_gemm give
+ * it.  trellis / suh / svh / n: host arrays of `count` entries.  The kernels
+ * and row thresholds are exl3_gemm's for the width of the whole output.
+ * Replaces the linear per output shard with the casts and torch.cat around
+ * them (src/sglang_exl3/dense.py:317-371). */
+int exl3_linear_cat(const void* x, int x_dtype, const int16_t* const* trellis, const uint16_t* const* suh,
+                    const uint16_t* const* svh, const int* n, int count, void* y, int y_dtype, int m, int k, int K,
+                    int codebook, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Many-row EXL3 GEMM on MFMA with the input already rotated:
  *   out[m][n] (f32) = svh[n] * (H . (a . T)[m][128-block])[n] / sqrt(128)
  * a: f16 [M][k] = fp16(H(x (.) suh) / sqrt(128)) per 128 block; trellis
@@ -247,6 +264,18 @@ int exl3_moe_layer(const uint16_t* x, const int32_t* topk_ids, const float* topk
                    int num_experts, uint16_t* out, int tokens, int topk, int hidden, int inter,
                    int K_gate, int K_up, int K_down, int codebook, float swiglu_limit,
                    void* workspace, size_t workspace_bytes, void* stream);
+
+/* exl3_moe_layer with x and out of element type `dtype` (EXL3_DTYPE_F16 or
+ * EXL3_DTYPE_BF16): bfloat16 rows are rounded to f16 as they are read, and a
+ * bfloat16 output is the f16 result rounded, as casts around exl3_moe_layer
+ * give it.  Same workspace. */
+int exl3_moe_layer_typed(const void* x, const int32_t* topk_ids, const float* topk_weights,
+                         const int64_t* gate_trellis, const int64_t* gate_suh, const int64_t* gate_svh,
+                         const int64_t* up_trellis, const int64_t* up_suh, const int64_t* up_svh,
+                         const int64_t* down_trellis, const int64_t* down_suh, const int64_t* down_svh,
+                         int num_experts, void* out, int tokens, int topk, int hidden, int inter, int K_gate,
+                         int K_up, int K_down, int codebook, float swiglu_limit, int dtype, void* workspace,
+                         size_t workspace_bytes, void* stream);
 
 /* One-token fused MoE: out[0] = fp16( sum_e rw[e] * down_{ids[e]}(...) ) as
  * exl3_moe_layer with tokens = 1, topk = num_ids and fp16 routing weights;

@@ -36,16 +36,22 @@ __global__ void fill_f32_kernel(float* p, size_t n, float v) {
         p[i] = v;
 }
 
-__global__ void f32_to_f16_kernel(const float* src, __half* dst, size_t n2) {
+__global__ void f32_to_f16_kernel(const float* src, __half* dst, size_t n2, int y_bf16) {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n2; i += (size_t)gridDim.x * blockDim.x) {
         const float2 v = reinterpret_cast<const float2*>(src)[i];
-        reinterpret_cast<__half2*>(dst)[i] = __floats2half2_rn(v.x, v.y);
+        reinterpret_cast<uint32_t*>(dst)[i] = y_bits(__floats2half2_rn(v.x, v.y), y_bf16);
     }
 }
 
 struct FatPlan {
     int mt, splits;
 };
+
+bool mats_n256(const MatSet& s) {
+    for (int j = 0; j < s.count; ++j)
+        if (s.n[j] % FB_COLS) return false;
+    return true;
+}
 
 // Wide tiles (256 x 256, fat_big_kernel) above kFatNarrowMaxRows rows (env
 // EXL3_FAT_WIDE=0 turns them off); up to there the narrow kernel with 16-row
@@ -139,11 +145,12 @@ int wide_tail_tiles(int m, int k, int n, bool gu) {
 
 // f16out: a call with fp16 output (exl3_gemm), whose narrow k-splits use the
 // partial-tile hand-off (fat_handoff) unless EXL3_FAT_HANDOFF=0.
-FatPlan plan_fat(int M, int k, int n, bool f16out) {
+// n256: every matrix of the call is a multiple of 256 columns wide.
+FatPlan plan_fat(int M, int k, int n, bool f16out, bool n256) {
     FatPlan pl;
     const int ksteps = k / 64;
     pl.splits = 1;
-    if (fat_wide_allowed() && M > kFatNarrowMaxRows && n % FB_COLS == 0 &&
+    if (fat_wide_allowed() && M > kFatNarrowMaxRows && n256 &&
         (fat_wide_mode() == 2 || (long long)(n / FB_COLS) * ((M + FB_ROWS - 1) / FB_ROWS) >= kFatWideMinTiles)) {
         pl.mt = FAT_MT_WIDE;
         const long long base = (long long)(n / FB_COLS) * ((M + FB_ROWS - 1) / FB_ROWS);
@@ -201,6 +208,15 @@ bool fat_handoff(const FatPlan& pl, int m, int n) {
            (size_t)(n / 128) * (size_t)((m + pl.mt - 1) / pl.mt) <= kWsMaxCounters && fat_handoff_on();
 }
 
+// Plan of an fp16-output call over `mats` matrices: several matrices do not
+// take the fp32 atomics (only reached by the tuning overrides), so such a plan
+// runs unsplit.
+FatPlan plan_rows(int m, int k, int n, int mats, bool n256, bool f16out = true) {
+    FatPlan pl = plan_fat(m, k, n, f16out, n256);
+    if (mats > 1 && pl.splits > 1 && !fat_handoff(pl, m, n)) pl.splits = 1;
+    return pl;
+}
+
 // Rows from which a 16-row tile's split hand-off goes to a finish launch
 // (split_out; env EXL3_FAT_SPLIT_OUT=0: never).
 constexpr int kSplitOutMinRows = 6;
@@ -224,12 +240,18 @@ int fat_split_finish(const FatParams& p, int splits, hipStream_t st, const char*
 // rowsum: chunk sums of a's rows, [M][k/128], for a raw-entry plan (else null).
 // partials / counters: the split hand-off's partial tiles and counters
 // (fat_handoff plans with fp16 output; else null).
+// mats: several matrices side by side (n: their columns together), y_bf16:
+// out16 is bfloat16.
 int run_fat(const uint16_t* a, const int16_t* trellis, float* out32, __half* out16, const uint16_t* svh,
             const int64_t* token_idx, const uint16_t* route_w, int M, int k, int n, int K, int cb, bool zero_first,
             hipStream_t st, int tail = 0, char* tail_part = nullptr, int* tail_sync = nullptr,
-            const float* rowsum = nullptr, float* partials = nullptr, int* counters = nullptr) {
-    const FatPlan pl = plan_fat(M, k, n, out16 != nullptr);
+            const float* rowsum = nullptr, float* partials = nullptr, int* counters = nullptr,
+            const MatSet* mats = nullptr, int y_bf16 = 0) {
+    const FatPlan pl = mats ? plan_rows(M, k, n, mats->count, mats_n256(*mats), out16 != nullptr)
+                            : plan_fat(M, k, n, out16 != nullptr, n % FB_COLS == 0);
     FatParams p{};
+    if (mats && mats->count > 1) p.mats = *mats;
+    p.y_bf16 = y_bf16;
     if (partials && pl.splits > 1) {
         p.handoff = 1;
         p.partials = partials;
@@ -289,49 +311,50 @@ size_t fat_xr_bytes(int m, int k) { return fat_xr_only_bytes(m, k) + (((size_t)m
 // [counters][accumulators][xr][split partial tiles S*m*n fp32 (narrow
 // hand-off) | out fp32 m*n (wide plan with k-splits) | tail-split hand-off
 // tiles (unsplit wide launch)].
-size_t fat_gemm_scratch_bytes(int m, int k, int n) {
-    const FatPlan pl = plan_fat(m, k, n, true);
+size_t fat_gemm_scratch_bytes(int m, int k, int n, int mats, bool n256) {
+    const FatPlan pl = plan_rows(m, k, n, mats, n256);
     const bool split = pl.splits > 1;
     const size_t tail = (!split && pl.mt == FAT_MT_WIDE) ? fat_tail_bytes(wide_tail_tiles(m, k, n, false)) : 0;
     const size_t out = fat_handoff(pl, m, n) ? (size_t)pl.splits * m * n * 4 : (size_t)m * n * 4;
-    return kWsScratchOffset + fat_xr_bytes(m, k) + (split ? out : tail);
+    return kWsScratchOffset + fat_xr_bytes(m * mats, k) + (split ? out : tail);
 }
 
-int fat_gemm_rows(const uint16_t* x, const int16_t* trellis, const uint16_t* suh, const uint16_t* svh, uint16_t* y,
-                  int m, int k, int n, int K, int cb, void* ws, size_t ws_bytes, hipStream_t st) {
-    const size_t need = fat_gemm_scratch_bytes(m, k, n);
+int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_t* y, int m, int k, int n, int K,
+                  int cb, int x_bf16, int y_bf16, void* ws, size_t ws_bytes, hipStream_t st) {
+    const bool n256 = mats_n256(mats);
+    const size_t need = fat_gemm_scratch_bytes(m, k, n, mats.count, n256);
     EXL3_REQUIRE_CODE(ws && ws_bytes >= need, EXL3_ERR_WORKSPACE,
-                      "exl3_gemm: %zu workspace bytes needed for m=%d, %zu given", need, m,
-                      ws ? ws_bytes : (size_t)0);
-    EXL3_REQUIRE(aligned(x, 4) && aligned(y, 4) && aligned(suh, 4), "exl3_gemm: misaligned pointer");
+                      "%s: %zu workspace bytes needed for m=%d, %zu given", fn, need, m, ws ? ws_bytes : (size_t)0);
+    const size_t xrows = (size_t)m * mats.count;
     __half* xr = reinterpret_cast<__half*>(reinterpret_cast<char*>(ws) + kWsScratchOffset);
-    float* o32 = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + kWsScratchOffset + fat_xr_bytes(m, k));
-    const FatPlan pl = plan_fat(m, k, n, true);
+    float* o32 = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + kWsScratchOffset + fat_xr_bytes((int)xrows, k));
+    const FatPlan pl = plan_rows(m, k, n, mats.count, n256);
     float* rs = fat_raw(cb, pl.mt, false)
-                    ? reinterpret_cast<float*>(reinterpret_cast<char*>(xr) + fat_xr_only_bytes(m, k))
+                    ? reinterpret_cast<float*>(reinterpret_cast<char*>(xr) + fat_xr_only_bytes((int)xrows, k))
                     : nullptr;
-    const long long chunks = (long long)m * (k / 128);
-    rotate_rows_kernel<<<(unsigned)((chunks + 3) / 4), 256, 0, st>>>(reinterpret_cast<const __half*>(x),
-                                                                      reinterpret_cast<const __half*>(suh), xr, chunks,
-                                                                      k, rs);
-    int rc = launch_status("exl3_gemm rotate launch");
+    RotateSuh suhs{};
+    for (int j = 0; j < mats.count; ++j) suhs.suh[j] = mats.suh[j];
+    int rc = rotate_rows(reinterpret_cast<const __half*>(x), suhs, mats.count, xr, m, k, x_bf16, rs, st,
+                         "exl3_gemm rotate launch");
     if (rc) return rc;
+    const int16_t* trellis = reinterpret_cast<const int16_t*>(mats.trellis[0]);
+    const uint16_t* svh = reinterpret_cast<const uint16_t*>(mats.svh[0]);
     if (pl.splits == 1) {
         const int tail = pl.mt == FAT_MT_WIDE ? wide_tail_tiles(m, k, n, false) : 0;
         return run_fat(reinterpret_cast<const uint16_t*>(xr), trellis, nullptr, reinterpret_cast<__half*>(y), svh,
                        nullptr, nullptr, m, k, n, K, cb, false, st, tail, reinterpret_cast<char*>(o32),
-                       reinterpret_cast<int*>(ws), rs);
+                       reinterpret_cast<int*>(ws), rs, nullptr, nullptr, &mats, y_bf16);
     }
     if (fat_handoff(pl, m, n))
         return run_fat(reinterpret_cast<const uint16_t*>(xr), trellis, nullptr, reinterpret_cast<__half*>(y), svh,
                        nullptr, nullptr, m, k, n, K, cb, false, st, 0, nullptr, nullptr, rs, o32,
-                       reinterpret_cast<int*>(ws));
+                       reinterpret_cast<int*>(ws), &mats, y_bf16);
     rc = run_fat(reinterpret_cast<const uint16_t*>(xr), trellis, o32, nullptr, svh, nullptr, nullptr, m, k, n, K, cb,
-                 true, st, 0, nullptr, nullptr, rs);
+                 true, st, 0, nullptr, nullptr, rs, nullptr, nullptr, &mats);
     if (rc) return rc;
     const size_t n2 = (size_t)m * n / 2;
     f32_to_f16_kernel<<<(unsigned)((n2 + 255) / 256 < 8192 ? (n2 + 255) / 256 : 8192), 256, 0, st>>>(
-        o32, reinterpret_cast<__half*>(y), n2);
+        o32, reinterpret_cast<__half*>(y), n2, y_bf16);
     return launch_status("exl3_gemm convert launch");
 }
 
@@ -398,11 +421,8 @@ int fat_gate_up_rows(const uint16_t* x, const uint16_t* suh, const int16_t* gate
     char* w8 = reinterpret_cast<char*>(ws);
     __half* xr = reinterpret_cast<__half*>(w8 + kWsScratchOffset);
     float* rs = fat_raw(cb, pl.mt, true) ? reinterpret_cast<float*>(w8 + kWsScratchOffset + fat_xr_only_bytes(m, k)) : nullptr;
-    const long long chunks = (long long)m * (k / 128);
-    rotate_rows_kernel<<<(unsigned)((chunks + 3) / 4), 256, 0, st>>>(reinterpret_cast<const __half*>(x),
-                                                                      reinterpret_cast<const __half*>(suh), xr, chunks,
-                                                                      k, rs);
-    int rc = launch_status("exl3_gate_up_swiglu rotate launch");
+    int rc = rotate_rows(reinterpret_cast<const __half*>(x), RotateSuh{{reinterpret_cast<const __half*>(suh)}}, 1, xr, m,
+                         k, 0, rs, st, "exl3_gate_up_swiglu rotate launch");
     if (rc) return rc;
     FatParams p{};
     p.rowsum = rs;
@@ -474,5 +494,5 @@ extern "C" int exl3_fat_gemm_scatter(const uint16_t* a, const int16_t* trellis, 
 extern "C" size_t exl3_gemm_workspace_size(int m, int k, int n, int K) {
     if (m < 1 || k < 128 || n < 128) return 0;
     if (m <= gemm_gemv_rows(n)) return exl3_gemv_workspace_size(m, k, n, K, 1);
-    return fat_gemm_scratch_bytes(m, k, n);
+    return fat_gemm_scratch_bytes(m, k, n, 1, n % 256 == 0);
 }

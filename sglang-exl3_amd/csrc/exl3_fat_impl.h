@@ -122,6 +122,11 @@ struct FatParams {
     // epilogue applies kMul1Kinv * acc + kMul1Bias * (sum of the rows' x over
     // the k range), from rowsum[row][k/128] (rotate_rows_kernel's chunk sums).
     const float* rowsum;
+    // Several matrices side by side (mats.count > 1, plain mode with out16): n
+    // is the width of the whole output, `a` (and rowsum) holds the rows rotated
+    // for each matrix in turn, and a column block's matrix comes from mats.
+    MatSet mats;
+    int y_bf16;  // out16 is bfloat16 (plain modes)
 };
 
 // Sum over chunks [c0, c0 + nc) of row `row` of rowsum (one wave).
@@ -188,6 +193,18 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
     const uint32_t* trel = (p.gu && (blockIdx.x & 1)) ? p.trellis2 : p.trellis;
     const __half* svh_p = p.svh;
     const __half* dsuh = nullptr;  // grouped up pass: the down projection's suh
+    const __half* arows = p.a;
+    const float* rowsum = p.rowsum;
+    int bxm = bx, nm = p.n;  // column block and width inside the matrix
+    if (p.mats.count > 1) {
+        const MatRef r = mat_of_block(p.mats, bx);
+        trel = r.trellis;
+        svh_p = r.svh;
+        bxm = bx - r.nb0;
+        nm = r.n;
+        arows += (size_t)r.j * p.M * p.k;
+        if constexpr (RAW) rowsum += (size_t)r.j * p.M * (p.k >> 7);
+    }
     int m0 = blockIdx.y * MT;
     int rows = min(MT, p.M - m0);
     if (p.gmode) {
@@ -203,14 +220,14 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
     }
     const int tid = threadIdx.x, cw = tid >> 6, lane = tid & 63;
     const int g = lane >> 4, i = lane & 15, q = i & 7;
-    const int ntiles = p.n >> 4;
+    const int ntiles = nm >> 4;
     const int nsteps = p.ksteps;
     const int kt0 = sidx * nsteps * 4;
-    const int nt = bx * 8 + cw * 2 + (i >> 3);
+    const int nt = bxm * 8 + cw * 2 + (i >> 3);
     const EXL3_GLOBAL uint32_t* tb = gptr(trel) + ((size_t)(kt0 + g) * ntiles + nt) * (8 * K) + K * q;
     const size_t step_stride = (size_t)4 * ntiles * (8 * K);
     const int prev_addr = ((lane & ~7) | ((lane + 7) & 7)) << 2;
-    const __half2 svv = ld_h2(gptr(svh_p) + bx * 128 + 2 * lane);  // epilogue scale, requested early
+    const __half2 svv = ld_h2(gptr(svh_p) + bxm * 128 + 2 * lane);  // epilogue scale, requested early
 
     float4_t acc[RB][2];
 #pragma unroll
@@ -224,7 +241,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
     for (int d = 0; d < D; ++d)
         if (d < nsteps) load_words<K>(tb + (size_t)d * step_stride, w[d]);
 
-    const EXL3_GLOBAL __half* ag = gptr(p.a);
+    const EXL3_GLOBAL __half* ag = gptr(arows);
     for (int c0 = 0; c0 < nsteps; c0 += CH) {
         // stage the chunk's A: rows x (CH * 4) slices of 16 k, permuted
         if (c0) __syncthreads();  // every wave is done with the previous chunk
@@ -366,7 +383,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
                         L.v[t] = t < S ? coherent_load2(pv + row * 128 + (size_t)t * rs) : make_float2(0.f, 0.f);
                     L.rs = 0.f;
                     if constexpr (RAW) {
-                        const float* r = p.rowsum + (size_t)(m0 + row) * nchk;
+                        const float* r = rowsum + (size_t)(m0 + row) * nchk;
                         for (int c = lane; c < nchk; c += 64) L.rs += gptr(r)[c];
                     }
                 };
@@ -383,7 +400,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
                         vb = vb * kMul1Kinv + sx;
                     }
                     fwht128_pair_fast(va, vb, lane);
-                    st_h2(gptr(p.out16) + (size_t)(m0 + row) * p.n + c0, h2_rn((va * kHadNorm) * sva, (vb * kHadNorm) * svb));
+                    st_y2(gptr(p.out16) + (size_t)(m0 + row) * p.n + c0, h2_rn((va * kHadNorm) * sva, (vb * kHadNorm) * svb), p.y_bf16);
                 };
                 constexpr int RS = FAT_THREADS / 64;
                 RowLoads1 la, lb;
@@ -403,12 +420,12 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
                 sum_splits2<1, 4>(src, rs, S, v2);
                 float va = v2[0].x, vb = v2[0].y;
                 if constexpr (RAW) {
-                    const float sx = kMul1Bias * fat_row_sum(p.rowsum, p.k >> 7, m0 + row, 0, p.k >> 7, lane);
+                    const float sx = kMul1Bias * fat_row_sum(rowsum, p.k >> 7, m0 + row, 0, p.k >> 7, lane);
                     va = va * kMul1Kinv + sx;
                     vb = vb * kMul1Kinv + sx;
                 }
                 fwht128_pair_fast(va, vb, lane);
-                st_h2(gptr(p.out16) + (size_t)(m0 + row) * p.n + c0, h2_rn((va * kHadNorm) * sva, (vb * kHadNorm) * svb));
+                st_y2(gptr(p.out16) + (size_t)(m0 + row) * p.n + c0, h2_rn((va * kHadNorm) * sva, (vb * kHadNorm) * svb), p.y_bf16);
             }
             return;
         }
@@ -439,7 +456,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
                         L.v[j][t] = t < S ? coherent_load2((j ? pu : pg) + row * 128 + (size_t)t * rs) : make_float2(0.f, 0.f);
                 L.rs = 0.f;
                 if constexpr (RAW) {
-                    const float* r = p.rowsum + (size_t)(m0 + row) * nchk;
+                    const float* r = rowsum + (size_t)(m0 + row) * nchk;
                     for (int c = lane; c < nchk; c += 64) L.rs += gptr(r)[c];
                 }
             };
@@ -476,7 +493,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
             float2 gu2[2];
             sum_splits2<2, 4>(src, rs, S, gu2);
             float sx = 0.f;
-            if constexpr (RAW) sx = kMul1Bias * fat_row_sum(p.rowsum, p.k >> 7, m0 + row, 0, p.k >> 7, lane);
+            if constexpr (RAW) sx = kMul1Bias * fat_row_sum(rowsum, p.k >> 7, m0 + row, 0, p.k >> 7, lane);
             finish(row, gu2[0].x, gu2[0].y, gu2[1].x, gu2[1].y, sx);
         }
         return;
@@ -486,7 +503,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
         float va = ct[row * 128 + 2 * lane], vb = ct[row * 128 + 2 * lane + 1];
         if constexpr (RAW) {
             // this split's k range: chunks kt0 / 8 .. + nsteps / 2
-            const float sx = kMul1Bias * fat_row_sum(p.rowsum, p.k >> 7, m0 + row, kt0 >> 3, nsteps >> 1, lane);
+            const float sx = kMul1Bias * fat_row_sum(rowsum, p.k >> 7, m0 + row, kt0 >> 3, nsteps >> 1, lane);
             va = va * kMul1Kinv + sx;
             vb = vb * kMul1Kinv + sx;
         }
@@ -495,7 +512,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
         vb = (vb * kHadNorm) * svb;
         const int src = m0 + row;
         if (p.out16) {
-            st_h2(gptr(p.out16) + (size_t)src * p.n + c0, h2_rn(va, vb));
+            st_y2(gptr(p.out16) + (size_t)src * p.n + c0, h2_rn(va, vb), p.y_bf16);
             continue;
         }
         size_t dst = (size_t)src;
@@ -546,12 +563,21 @@ __global__ __launch_bounds__(256) void fat_split_finish_kernel(FatParams p, int 
 #pragma unroll
         for (int t = 0; t < 4; ++t) v[j][t] = t < S ? ld2(pj + (size_t)t * rs) : make_float2(0.f, 0.f);
     }
-    const __half2 sv0 = ld_h2(gptr(p.svh) + c0);
+    const __half* svh = p.svh;
+    const float* rowsum = p.rowsum;
+    int cm = c0;
+    if (!GU && p.mats.count > 1) {
+        const MatRef r = mat_of_block(p.mats, bx);
+        svh = r.svh;
+        cm = c0 - r.nb0 * 128;
+        if constexpr (RAW) rowsum += (size_t)r.j * p.M * (p.k >> 7);
+    }
+    const __half2 sv0 = ld_h2(gptr(svh) + cm);
     const __half2 sv1 = GU ? ld_h2(gptr(p.svh2) + c0) : sv0;
     float rsum = 0.f;
     if constexpr (RAW) {
         const int nchk = p.k >> 7;
-        const float* r = p.rowsum + (size_t)row * nchk;
+        const float* r = rowsum + (size_t)row * nchk;
         for (int c = lane; c < nchk; c += 64) rsum += gptr(r)[c];
     }
     float2 sm[NP];
@@ -575,8 +601,8 @@ __global__ __launch_bounds__(256) void fat_split_finish_kernel(FatParams p, int 
             vb = vb * kMul1Kinv + sx;
         }
         fwht128_pair_fast(va, vb, lane);
-        st_h2(gptr(p.out16) + (size_t)row * p.n + c0,
-              h2_rn((va * kHadNorm) * __low2float(sv0), (vb * kHadNorm) * __high2float(sv0)));
+        st_y2(gptr(p.out16) + (size_t)row * p.n + c0,
+              h2_rn((va * kHadNorm) * __low2float(sv0), (vb * kHadNorm) * __high2float(sv0)), p.y_bf16);
     }
 }
 
@@ -724,13 +750,25 @@ __global__ __launch_bounds__(FB_THREADS, 2) void fat_big_kernel(FatParams p) {
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
     const int rh = wv >> 2, cq = wv & 3;
     const int g = lane >> 4, i = lane & 15, q = i & 7;
-    const int ntiles = p.n >> 4;
+    int ntiles = p.n >> 4;
     const int nsteps = half >= 0 ? p.ksteps / 2 : p.ksteps;  // even
     const int kt0 = sidx * p.ksteps * 4 + (half > 0 ? nsteps * 4 : 0);
     // this wave decodes group rh of quarter cq: column tiles 4cq + 2rh + (i >> 3)
     // (gate/up mode: quarters 0, 1 of the gate block bx, 2, 3 of the up block bx)
-    const int nt = GU ? bx * 8 + (cq & 1) * 4 + rh * 2 + (i >> 3) : bx * (FB_COLS / 16) + cq * 4 + rh * 2 + (i >> 3);
+    int nt = GU ? bx * 8 + (cq & 1) * 4 + rh * 2 + (i >> 3) : bx * (FB_COLS / 16) + cq * 4 + rh * 2 + (i >> 3);
     const uint32_t* trel = (GU && cq >= 2) ? p.trellis2 : p.trellis;
+    const __half* arows = p.a;
+    const __half* svh_p = p.svh;
+    int svc0 = bx * FB_COLS;  // the tile's first column inside its matrix
+    if (!GU && p.mats.count > 1) {  // every matrix a multiple of FB_COLS wide
+        const MatRef r = mat_of_block(p.mats, bx * (FB_COLS / 128));
+        trel = r.trellis;
+        svh_p = r.svh;
+        arows += (size_t)r.j * p.M * p.k;
+        nt -= r.nb0 * 8;
+        svc0 -= r.nb0 * 128;
+        ntiles = r.n >> 4;
+    }
     const EXL3_GLOBAL uint32_t* tb = gptr(trel) + ((size_t)(kt0 + g) * ntiles + nt) * (8 * K) + K * q;
     const size_t step_stride = (size_t)4 * ntiles * (8 * K);
     const int prev_addr = ((lane & ~7) | ((lane + 7) & 7)) << 2;
@@ -739,7 +777,7 @@ __global__ __launch_bounds__(FB_THREADS, 2) void fat_big_kernel(FatParams p) {
     // physical chunk u & 7, which holds logical chunk (u & 7) ^ (row & 7) ^
     // ((row >> 3) & 1).  Rows past M repeat the last row (never stored).
     const EXL3_GLOBAL char* abase =
-        reinterpret_cast<const EXL3_GLOBAL char*>(gptr(p.a)) + ((size_t)m0 * p.k + (size_t)kt0 * 16) * 2;
+        reinterpret_cast<const EXL3_GLOBAL char*>(gptr(arows)) + ((size_t)m0 * p.k + (size_t)kt0 * 16) * 2;
     uint32_t aoff[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -1046,7 +1084,7 @@ __global__ __launch_bounds__(FB_THREADS, 2) void fat_big_kernel(FatParams p) {
             const float hn = fwht_x16_norm(lane);
             const int c0 = bx * FB_COLS + col;
             // svh and the outputs are only 4- (8-) byte aligned by contract
-            const EXL3_GLOBAL uint32_t* svp = reinterpret_cast<const EXL3_GLOBAL uint32_t*>(gptr(p.svh) + c0);
+            const EXL3_GLOBAL uint32_t* svp = reinterpret_cast<const EXL3_GLOBAL uint32_t*>(gptr(svh_p) + svc0 + col);
             uint32_t sw[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) sw[e] = svp[e];
@@ -1086,7 +1124,7 @@ __global__ __launch_bounds__(FB_THREADS, 2) void fat_big_kernel(FatParams p) {
             if (p.out16) {
                 __half* o = p.out16 + (size_t)src * p.n + c0;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) st_h2(gptr(o) + 2 * e, h2_rn(v[2 * e], v[2 * e + 1]));
+                for (int e = 0; e < 8; ++e) st_y2(gptr(o) + 2 * e, h2_rn(v[2 * e], v[2 * e + 1]), p.y_bf16);
                 continue;
             }
             float* o = p.out32 + (size_t)src * p.n + c0;

@@ -56,8 +56,9 @@ int gemv_launch(int K, int cb, int mb, const GemvParams& p, int experts, hipStre
     return EXL3_ERR_UNSUPPORTED;
 }
 
-int fat_gemm_rows(const uint16_t* x, const int16_t* trellis, const uint16_t* suh, const uint16_t* svh, uint16_t* y,
-                  int m, int k, int n, int K, int cb, void* ws, size_t ws_bytes, hipStream_t st);
+size_t fat_gemm_scratch_bytes(int m, int k, int n, int mats, bool n256);
+int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_t* y, int m, int k, int n, int K,
+                  int cb, int x_bf16, int y_bf16, void* ws, size_t ws_bytes, hipStream_t st);
 
 // Rows up to which exl3_gemm runs the GEMV kernels; above, the input is
 // rotated once and the MFMA GEMM runs (env EXL3_GEMM_GEMV_ROWS, at most 64).
@@ -241,9 +242,17 @@ int run_gemv(const char* fn, GemvParams p, int K, int codebook, int experts, voi
     if (pl.sk) {
         GemvSkParams q{};
         q.x = p.x;
-        q.trellis = p.trellis;
-        q.suh = p.suh;
-        q.svh = p.svh;
+        if (p.mats.count > 1) {
+            q.mats = p.mats;
+        } else {
+            q.mats.count = 1;
+            q.mats.n[0] = p.n;
+            q.mats.trellis[0] = p.trellis;
+            q.mats.suh[0] = p.suh;
+            q.mats.svh[0] = p.svh;
+        }
+        q.x_bf16 = p.x_bf16;
+        q.y_bf16 = p.y_bf16;
         q.y = p.y;
         q.acc = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(ws) + kWsAccOffset);
         q.m = p.m;
@@ -272,9 +281,9 @@ int run_gemv(const char* fn, GemvParams p, int K, int codebook, int experts, voi
     if (gemv_pre_rotates(pl, p.m, experts) && !p.gu) {
         __half* xr = reinterpret_cast<__half*>(reinterpret_cast<char*>(ws) + kWsScratchOffset +
                                                gemv_partials_bytes(pl, p.m, p.n, experts));
-        const long long chunks = (long long)p.m * (p.k / 128);
-        rotate_rows_kernel<<<(unsigned)((chunks + 3) / 4), 256, 0, st>>>(p.x, p.suh, xr, chunks, p.k);
-        const int rc = launch_status("exl3 gemv rotate launch");
+        // (several matrices never get here: cat_gemv)
+        const int rc = rotate_rows(p.x, RotateSuh{{p.suh}}, 1, xr, p.m, p.k, p.x_bf16, nullptr, st,
+                                   "exl3 gemv rotate launch");
         if (rc) return rc;
         p.x = xr;
         p.x_rot = 1;
@@ -294,6 +303,23 @@ GemvParams base_params(const uint16_t* x, const int16_t* trellis, const uint16_t
     p.k = k;
     p.n = n;
     return p;
+}
+
+MatSet one_mat(const int16_t* trellis, const uint16_t* suh, const uint16_t* svh, int n) {
+    MatSet s{};
+    s.count = 1;
+    s.n[0] = n;
+    s.trellis[0] = reinterpret_cast<const uint32_t*>(trellis);
+    s.suh[0] = reinterpret_cast<const __half*>(suh);
+    s.svh[0] = reinterpret_cast<const __half*>(svh);
+    return s;
+}
+
+// exl3_linear_cat takes the GEMV kernels up to exl3_gemm's row count for the
+// whole output's width (unless the GEMV would rotate its rows in a launch of
+// its own, which holds one matrix's rows).
+bool cat_gemv(int m, int k, int n, int K) {
+    return m <= gemm_gemv_rows(n) && m <= kMaxGemvRows && !gemv_pre_rotates(plan_gemv(m, k, n, K, 1), m, 1);
 }
 
 // ----------------------------- dense gate + up on the GEMV kernel (m <= 64)
@@ -443,8 +469,9 @@ extern "C" int exl3_gemm(const uint16_t* x, const int16_t* trellis, const uint16
     EXL3_REQUIRE(aligned(x, 4) && aligned(y, 4) && aligned(suh, 4) && aligned(svh, 4) && aligned(trellis, 16),
                  "exl3_gemm: misaligned pointer");
     hipStream_t st = as_stream(stream);
-    if (m > gemm_gemv_rows(n)) return fat_gemm_rows(x, trellis, suh, svh, y, m, k, n, K, codebook, workspace,
-                                               workspace_bytes, st);
+    if (m > gemm_gemv_rows(n))
+        return fat_gemm_rows("exl3_gemm", x, one_mat(trellis, suh, svh, n), y, m, k, n, K, codebook, 0, 0, workspace,
+                             workspace_bytes, st);
     for (int r0 = 0; r0 < m; r0 += kMaxGemvRows) {
         const int mc = (m - r0) < kMaxGemvRows ? (m - r0) : kMaxGemvRows;
         GemvParams p = base_params(x + (size_t)r0 * k, trellis, suh, svh, y + (size_t)r0 * n, mc, k, n);
@@ -452,6 +479,59 @@ extern "C" int exl3_gemm(const uint16_t* x, const int16_t* trellis, const uint16
         if (rc) return rc;
     }
     return EXL3_OK;
+}
+
+extern "C" size_t exl3_linear_cat_workspace_size(int m, int k, const int* n, int count, int K) {
+    if (m < 1 || k < 128 || !n || count < 1 || count > kMaxMats) return 0;
+    int total = 0;
+    bool n256 = true;
+    for (int j = 0; j < count; ++j) {
+        if (n[j] < 128) return 0;
+        total += n[j];
+        n256 = n256 && n[j] % 256 == 0;
+    }
+    if (cat_gemv(m, k, total, K)) return exl3_gemv_workspace_size(m, k, total, K, 1);
+    return fat_gemm_scratch_bytes(m, k, total, count, n256);
+}
+
+extern "C" int exl3_linear_cat(const void* x, int x_dtype, const int16_t* const* trellis, const uint16_t* const* suh,
+                               const uint16_t* const* svh, const int* n, int count, void* y, int y_dtype, int m, int k,
+                               int K, int codebook, void* workspace, size_t workspace_bytes, void* stream) {
+    clear_error();
+    EXL3_REQUIRE(count >= 1 && count <= kMaxMats, "exl3_linear_cat: %d matrices outside 1..%d", count, kMaxMats);
+    EXL3_REQUIRE(x && trellis && suh && svh && n && y, "exl3_linear_cat: null pointer");
+    EXL3_REQUIRE((x_dtype == EXL3_DTYPE_F16 || x_dtype == EXL3_DTYPE_BF16) &&
+                     (y_dtype == EXL3_DTYPE_F16 || y_dtype == EXL3_DTYPE_BF16),
+                 "exl3_linear_cat: dtypes %d / %d", x_dtype, y_dtype);
+    EXL3_REQUIRE(aligned(x, 4) && aligned(y, 4), "exl3_linear_cat: misaligned pointer");
+    MatSet s{};
+    s.count = count;
+    long long total = 0;
+    for (int j = 0; j < count; ++j) {
+        const int rc = check_common("exl3_linear_cat", m, k, n[j], K, codebook);
+        if (rc) return rc;
+        EXL3_REQUIRE(trellis[j] && suh[j] && svh[j], "exl3_linear_cat: null pointer");
+        EXL3_REQUIRE(aligned(trellis[j], 16) && aligned(suh[j], 4) && aligned(svh[j], 4),
+                     "exl3_linear_cat: misaligned pointer");
+        s.nb0[j] = (int)(total / 128);
+        s.n[j] = n[j];
+        s.trellis[j] = reinterpret_cast<const uint32_t*>(trellis[j]);
+        s.suh[j] = reinterpret_cast<const __half*>(suh[j]);
+        s.svh[j] = reinterpret_cast<const __half*>(svh[j]);
+        total += n[j];
+    }
+    EXL3_REQUIRE(total <= (1 << 30), "exl3_linear_cat: %lld columns", total);
+    const int nt = (int)total, xb = x_dtype == EXL3_DTYPE_BF16, yb = y_dtype == EXL3_DTYPE_BF16;
+    hipStream_t st = as_stream(stream);
+    if (!cat_gemv(m, k, nt, K))
+        return fat_gemm_rows("exl3_linear_cat", static_cast<const uint16_t*>(x), s, static_cast<uint16_t*>(y), m, k, nt,
+                             K, codebook, xb, yb, workspace, workspace_bytes, st);
+    GemvParams p = base_params(static_cast<const uint16_t*>(x), trellis[0], suh[0], svh[0], static_cast<uint16_t*>(y), m,
+                               k, nt);
+    p.mats = s;
+    p.x_bf16 = xb;
+    p.y_bf16 = yb;
+    return run_gemv("exl3_linear_cat", p, K, codebook, 1, workspace, workspace_bytes, st);
 }
 
 extern "C" int exl3_p2b_gemv_batched(const uint16_t* x, int x_per_expert, const int64_t* trellis_ptrs,

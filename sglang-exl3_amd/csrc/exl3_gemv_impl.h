@@ -31,6 +31,38 @@ namespace exl3 {
 constexpr int GV_MAX_THREADS = 512;  // 4 column waves x up to 2 k waves
 constexpr int GV_PRE = 8;            // rotation blocks per wave whose activations are preloaded
 
+// One to kMaxMats matrices over the same input rows, their outputs side by
+// side: column block b (128 columns) of the concatenated output is block
+// b - nb0[j] of matrix j, the last one with nb0[j] <= b.  A layer's output
+// shards (q, k, v) are one launch then: three launches of a few column blocks
+// each leave most of the chip idle (qkv 4096 -> 4096 + 2 x 1024, K = 4, 77 rows
+// bf16: three GEMMs of 26-27 us, casts and concatenation 100.1 us -> 42.6 us).
+constexpr int kMaxMats = 4;
+struct MatSet {
+    int count;
+    int nb0[kMaxMats];
+    int n[kMaxMats];
+    const uint32_t* trellis[kMaxMats];
+    const __half* suh[kMaxMats];
+    const __half* svh[kMaxMats];
+};
+
+struct MatRef {
+    int j, nb0, n;
+    const uint32_t* trellis;
+    const __half* suh;
+    const __half* svh;
+};
+
+// The matrix of column block b (uniform over the workgroup: scalar selects).
+__device__ __forceinline__ MatRef mat_of_block(const MatSet& s, int b) {
+    MatRef r{0, s.nb0[0], s.n[0], s.trellis[0], s.suh[0], s.svh[0]};
+#pragma unroll
+    for (int j = 1; j < kMaxMats; ++j)
+        if (j < s.count && b >= s.nb0[j]) r = MatRef{j, s.nb0[j], s.n[j], s.trellis[j], s.suh[j], s.svh[j]};
+    return r;
+}
+
 struct GemvParams {
     const __half* x;
     long long x_stride_e;  // elements between consecutive experts' x (0 = shared x)
@@ -69,6 +101,10 @@ struct GemvParams {
     // and clears the accumulator (the output rotation is linear).
     int fx;
     unsigned long long* acc;
+    // Several matrices side by side (mats.count > 1, one "expert"): n is the
+    // width of the whole output, the matrix of a column block comes from mats.
+    MatSet mats;
+    int x_bf16, y_bf16;  // x / y are bfloat16 (x_h2, y_bits)
 };
 
 // Steps of weight words a wave keeps in flight.  Measured on MI355X (config 2,
@@ -86,6 +122,26 @@ __device__ __forceinline__ __half2 ld_h2(const EXL3_GLOBAL __half* p) {
 }
 __device__ __forceinline__ void st_h2(EXL3_GLOBAL __half* p, __half2 v) {
     *reinterpret_cast<EXL3_GLOBAL uint32_t*>(p) = *reinterpret_cast<const uint32_t*>(&v);
+}
+
+// Activations in the caller's 16-bit type, as the fp16 pair that the kernels
+// compute with: bfloat16 is rounded to fp16 to nearest, as a cast ahead of the
+// call does.
+__device__ __forceinline__ __half2 x_h2(__half2 v, int bf16) {
+    if (!bf16) return v;
+    const uint32_t u = *reinterpret_cast<const uint32_t*>(&v);
+    return __floats2half2_rn(__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u));
+}
+// An fp16 output pair in the caller's type: the fp16 value rounded to bfloat16,
+// the two roundings of an fp16 result that a cast after the call converts.
+__device__ __forceinline__ uint32_t y_bits(__half2 v, int bf16) {
+    if (!bf16) return *reinterpret_cast<const uint32_t*>(&v);
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    const bf16x2_t r = {(__bf16)__low2float(v), (__bf16)__high2float(v)};
+    return __builtin_bit_cast(uint32_t, r);
+}
+__device__ __forceinline__ void st_y2(EXL3_GLOBAL __half* p, __half2 v, int bf16) {
+    *reinterpret_cast<EXL3_GLOBAL uint32_t*>(p) = y_bits(v, bf16);
 }
 
 // Device-coherent (sc1) store/load: visible to every workgroup of the device
@@ -212,21 +268,21 @@ __device__ __forceinline__ FxPair fx_issue_pair(unsigned long long* acc, float a
 // launch read.
 template <bool COH = false>
 __device__ __forceinline__ void fx_finish_pair(const FxPair& f, unsigned long long* acc, int cnt,
-                                               EXL3_GLOBAL __half* y) {
+                                               EXL3_GLOBAL __half* y, int bf16 = 0) {
     const bool ca = (int)(f.oa >> SK_CNT_SHIFT) == cnt - 1;
     const bool cb = (int)(f.ob >> SK_CNT_SHIFT) == cnt - 1;
     if (!(ca || cb)) return;
     const float va = sk_decode(f.oa + f.ea, cnt), vb = sk_decode(f.ob + f.eb, cnt);
     if (ca && cb) {
-        const __half2 v = __floats2half2_rn(va, vb);
+        const uint32_t v = y_bits(__floats2half2_rn(va, vb), bf16);
         if constexpr (COH)
-            __hip_atomic_store(reinterpret_cast<uint32_t*>((__half*)y), *reinterpret_cast<const uint32_t*>(&v),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(reinterpret_cast<uint32_t*>((__half*)y), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         else
-            st_h2(y, v);
+            *reinterpret_cast<EXL3_GLOBAL uint32_t*>(y) = v;
     } else {
         EXL3_GLOBAL uint16_t* const d = reinterpret_cast<EXL3_GLOBAL uint16_t*>(ca ? y : y + 1);
-        const uint16_t h = __half_as_ushort(__float2half_rn(ca ? va : vb));
+        const float vs = ca ? va : vb;
+        const uint16_t h = (uint16_t)y_bits(__floats2half2_rn(vs, vs), bf16);
         if constexpr (COH)
             __hip_atomic_store((uint16_t*)d, h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         else
@@ -236,8 +292,9 @@ __device__ __forceinline__ void fx_finish_pair(const FxPair& f, unsigned long lo
     if (cb) __hip_atomic_store(acc + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ void fx_add_pair(unsigned long long* acc, float a, float b, int cnt, EXL3_GLOBAL __half* y) {
-    fx_finish_pair(fx_issue_pair(acc, a, b), acc, cnt, y);
+__device__ __forceinline__ void fx_add_pair(unsigned long long* acc, float a, float b, int cnt, EXL3_GLOBAL __half* y,
+                                            int bf16) {
+    fx_finish_pair(fx_issue_pair(acc, a, b), acc, cnt, y, bf16);
 }
 
 // Wait until this wave's outstanding memory operations have completed.
@@ -364,11 +421,19 @@ __global__ __launch_bounds__(GV_MAX_THREADS) void gemv_kernel(GemvParams p) {
     const uint32_t* trellis;
     const __half* suh;
     const __half* svh;
+    int bxm = bx, nm = p.n;  // column block and width inside the matrix
     if (p.t_tab) {
         const int id = gptr(p.ids)[e];
         trellis = reinterpret_cast<const uint32_t*>(gptr(p.t_tab)[id]);
         suh = reinterpret_cast<const __half*>(gptr(p.su_tab)[id]);
         svh = reinterpret_cast<const __half*>(gptr(p.sv_tab)[id]);
+    } else if (!GU && p.mats.count > 1) {
+        const MatRef r = mat_of_block(p.mats, bx);
+        trellis = r.trellis;
+        suh = r.suh;
+        svh = r.svh;
+        bxm = bx - r.nb0;
+        nm = r.n;
     } else if (GU && e) {
         trellis = p.trellis2;
         suh = p.suh2;
@@ -384,11 +449,11 @@ __global__ __launch_bounds__(GV_MAX_THREADS) void gemv_kernel(GemvParams p) {
     constexpr int nsteps = NS;
     const int nthreads = 256 * kw, nwaves = 4 * kw;
     const int kts_wg = 4 * nsteps * kw;  // k-slices of this workgroup
-    const int ntiles = n >> 4;
+    const int ntiles = nm >> 4;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int cw = wave & 3, kwi = wave >> 2;
     const int g = lane >> 4, i = lane & 15, q = i & 7;
-    const int nt = bx * 8 + cw * 2 + (i >> 3);
+    const int nt = bxm * 8 + cw * 2 + (i >> 3);
     const int kt_wg0 = sidx * kts_wg;
     const int kt_w0 = kt_wg0 + kwi * 4 * nsteps;
 
@@ -416,7 +481,7 @@ __global__ __launch_bounds__(GV_MAX_THREADS) void gemv_kernel(GemvParams p) {
     }
     // output scale of this lane's two columns, requested now: the epilogue
     // then needs no extra round trip
-    const __half2 svv = ld_h2(gptr(svh) + bx * 128 + 2 * lane);
+    const __half2 svv = ld_h2(gptr(svh) + bxm * 128 + 2 * lane);
     uint32_t w[D][K];
     const EXL3_GLOBAL uint32_t* tb = gptr(trellis) + ((size_t)(kt_w0 + g) * ntiles + nt) * (8 * K) + K * q;
     const size_t step_stride = (size_t)4 * ntiles * (8 * K);
@@ -432,7 +497,7 @@ __global__ __launch_bounds__(GV_MAX_THREADS) void gemv_kernel(GemvParams p) {
             (void)sv;
             bits = *reinterpret_cast<const uint32_t*>(&xv);
         } else {
-            const __half2 pr = __hmul2(xv, sv);
+            const __half2 pr = __hmul2(x_h2(xv, p.x_bf16), sv);
             float a = __low2float(pr), c = __high2float(pr);
             fwht128_pair_fast(a, c, lane);
             const _Float16 ha = f16_rn(a * kHadNorm), hc = f16_rn(c * kHadNorm);
@@ -520,11 +585,11 @@ __global__ __launch_bounds__(GV_MAX_THREADS) void gemv_kernel(GemvParams p) {
             float a = ybuf[row * 128 + 2 * lane], b = ybuf[row * 128 + 2 * lane + 1];
             fwht128_pair_fast(a, b, lane);
             const FxPair cur = fx_issue_pair(p.acc + (size_t)row * n + c0, a * sva, b * svb);
-            if (prow >= 0) fx_finish_pair(fx, p.acc + (size_t)prow * n + c0, p.splits, yf + (size_t)prow * n + c0);
+            if (prow >= 0) fx_finish_pair(fx, p.acc + (size_t)prow * n + c0, p.splits, yf + (size_t)prow * n + c0, p.y_bf16);
             fx = cur;
             prow = row;
         }
-        if (prow >= 0) fx_finish_pair(fx, p.acc + (size_t)prow * n + c0, p.splits, yf + (size_t)prow * n + c0);
+        if (prow >= 0) fx_finish_pair(fx, p.acc + (size_t)prow * n + c0, p.splits, yf + (size_t)prow * n + c0, p.y_bf16);
         return;
     }
     // Otherwise the last workgroup of the column block finishes.  Partials
@@ -596,32 +661,43 @@ __global__ __launch_bounds__(GV_MAX_THREADS) void gemv_kernel(GemvParams p) {
         float a = ybuf[row * 128 + 2 * lane], b = ybuf[row * 128 + 2 * lane + 1];
         fwht128_pair_fast(a, b, lane);
         const __half2 o = h2_rn(a * kHadNorm * sva, b * kHadNorm * svb);
-        st_h2(y + (size_t)row * n + c0, o);
+        st_y2(y + (size_t)row * n + c0, o, p.y_bf16);
     }
 }
 
 namespace {
 // Input rotation of a row batch: xr = fp16( H(x (.) suh) / sqrt(128) ), one
 // wave per 128-wide chunk (feeds the k-split GEMV's pre-rotated mode and the
-// MFMA GEMM).
+// MFMA GEMM).  blockIdx.y: the matrix whose suh applies; its rotated rows
+// follow those of the matrix before.
 // rs (optional): the sum of each chunk's 128 rotated fp16 values, [row][k/128]
-// (the mul1 raw-entry GEMM's affine correction).
-__global__ __launch_bounds__(256) void rotate_rows_kernel(const __half* x, const __half* suh, __half* xr,
-                                                          long long chunks, int k, float* rs = nullptr) {
+// per matrix (the mul1 raw-entry GEMM's affine correction).
+struct RotateSuh {
+    const __half* suh[kMaxMats];
+};
+__global__ __launch_bounds__(256) void rotate_rows_kernel(const __half* x, RotateSuh suhs, __half* xr,
+                                                          long long chunks, int k, int x_bf16, float* rs) {
     const long long chunk = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (chunk >= chunks) return;
+    const __half* suh = suhs.suh[blockIdx.y];
     const int lane = threadIdx.x & 63, per_row = k >> 7;
     const long long row = chunk / per_row;
     const int c = (int)(chunk - row * per_row) * 128 + 2 * lane;
-    const __half2 pr = __hmul2(ld_h2(gptr(x) + (size_t)row * k + c), ld_h2(gptr(suh) + c));
+    const __half2 pr = __hmul2(x_h2(ld_h2(gptr(x) + (size_t)row * k + c), x_bf16), ld_h2(gptr(suh) + c));
     float a = __low2float(pr), b = __high2float(pr);
     fwht128_pair_fast(a, b, lane);
     const __half2 o = h2_rn(a * kHadNorm, b * kHadNorm);
-    st_h2(gptr(xr) + (size_t)row * k + c, o);
+    st_h2(gptr(xr) + ((size_t)blockIdx.y * chunks + chunk) * 128 + 2 * lane, o);
     if (rs) {
         const float t = wave_sum(__low2float(o) + __high2float(o));
-        if (lane == 0) gptr(rs)[chunk] = t;
+        if (lane == 0) gptr(rs)[(size_t)blockIdx.y * chunks + chunk] = t;
     }
+}
+inline int rotate_rows(const __half* x, const RotateSuh& suhs, int mats, __half* xr, int m, int k, int x_bf16,
+                       float* rs, hipStream_t st, const char* what) {
+    const long long chunks = (long long)m * (k / 128);
+    rotate_rows_kernel<<<dim3((unsigned)((chunks + 3) / 4), mats), 256, 0, st>>>(x, suhs, xr, chunks, k, x_bf16, rs);
+    return launch_status(what);
 }
 }  // namespace
 

@@ -34,13 +34,12 @@ constexpr int SK_THREADS = 256;
 
 struct GemvSkParams {
     const __half* x;          // [m][k]
-    const uint32_t* trellis;  // [k/16][n/16][8K] words
-    const __half* suh;        // [k]
-    const __half* svh;        // [n]
+    MatSet mats;              // trellis [k/16][n/16][8K] words, suh [k], svh [n] of each matrix
     __half* y;                // [m][n]
     unsigned long long* acc;  // [m][n] fixed-point accumulators, zero between calls
-    int m, k, n;
+    int m, k, n;  // n: columns of all matrices
     int pieces;  // P: workgroups per column block (grid.x); grid.y = n / 128
+    int x_bf16, y_bf16;  // x / y are bfloat16
 };
 
 // Rows the kernel is instantiated for (MR >= m): 1, 2 or 4.
@@ -89,11 +88,13 @@ __global__ __launch_bounds__(SK_THREADS) void gemv_sk_kernel(GemvSkParams p) {
 
     const int n = p.n, P = p.pieces, m = p.m, k = p.k;
     const int pi = blockIdx.x, cb = blockIdx.y;
+    const MatRef mat = mat_of_block(p.mats, cb);
+    const int cbm = cb - mat.nb0;  // column block inside its matrix
     const int ks0 = pi * NS;  // first k-step of the piece
 
     const int tid = threadIdx.x, cw = tid >> 6, lane = tid & 63;
     const int g = lane >> 4, i = lane & 15, q = i & 7;
-    const int ntiles = n >> 4;
+    const int ntiles = mat.n >> 4;
 
     constexpr int ROWH = NS * 128;  // staged halves per row
     _Float16* xs = reinterpret_cast<_Float16*>(sk_smem);
@@ -108,17 +109,17 @@ __global__ __launch_bounds__(SK_THREADS) void gemv_sk_kernel(GemvSkParams p) {
 
     // 1. activations of this wave's first job, then the weights
     const EXL3_GLOBAL __half* xg = gptr(p.x) + 2 * lane;
-    const EXL3_GLOBAL __half* suhg = gptr(p.suh) + 2 * lane;
+    const EXL3_GLOBAL __half* suhg = gptr(mat.suh) + 2 * lane;
     __half2 x0 = __float2half2_rn(0.f), s0 = x0;
     if (cw < jobs) {
         const int r0 = cw / nblocks, b0 = cw - r0 * nblocks;
         x0 = ld_h2(xg + (size_t)r0 * k + (j0 + b0) * 128);
         s0 = ld_h2(suhg + (j0 + b0) * 128);
     }
-    const int nt = cb * 8 + cw * 2 + (i >> 3);
+    const int nt = cbm * 8 + cw * 2 + (i >> 3);
     const size_t ss = (size_t)4 * ntiles * (8 * K);  // words between k-steps
-    const EXL3_GLOBAL uint32_t* tb = gptr(p.trellis) + ((size_t)(ks0 * 4 + g) * ntiles + nt) * (8 * K) + K * q;
-    const __half2 svv = ld_h2(gptr(p.svh) + cb * 128 + 2 * lane);
+    const EXL3_GLOBAL uint32_t* tb = gptr(mat.trellis) + ((size_t)(ks0 * 4 + g) * ntiles + nt) * (8 * K) + K * q;
+    const __half2 svv = ld_h2(gptr(mat.svh) + cbm * 128 + 2 * lane);
     // only the first step's words now; the rest of the ring after the
     // staging barrier, so that the burst every wave issues at its start is
     // one step (7.3 MB over the grid at config 2, not 14.7) and the decode
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemv_sk_kernel(GemvSkParams p) {
         const bool mine = l >= 0 && l < NS;
         const __half2 xv = jb == cw ? x0 : ld_h2(xg + (size_t)row * k + j * 128);
         const __half2 sv = jb == cw ? s0 : ld_h2(suhg + j * 128);
-        const __half2 pr = __hmul2(xv, sv);
+        const __half2 pr = __hmul2(x_h2(xv, p.x_bf16), sv);
         float a = __low2float(pr), c = __high2float(pr);
         fwht128_pair_fast(a, c, lane);
         const _Float16 ha = f16_rn(a * kHadNorm), hc = f16_rn(c * kHadNorm);
@@ -235,7 +236,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemv_sk_kernel(GemvSkParams p) {
     a = a * kHadNorm * __low2float(svv);
     b = b * kHadNorm * __high2float(svv);
     const size_t e0 = (size_t)r * n + cb * 128 + 2 * lane;
-    fx_add_pair(p.acc + e0, a, b, P, gptr(p.y) + e0);
+    fx_add_pair(p.acc + e0, a, b, P, gptr(p.y) + e0, p.y_bf16);
 }
 
 // Piece lengths (k-steps) the kernel is instantiated for.

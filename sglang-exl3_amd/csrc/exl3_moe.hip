@@ -200,7 +200,7 @@ __global__ __launch_bounds__(MOE_ROUTE_THREADS) void moe_route_kernel(const int3
 // the operations are the GEMV staging's, so the staged values are the same.
 __global__ __launch_bounds__(MOE_ROUTE_THREADS) void moe_route_rotate_kernel(
     const int32_t* ids, int entries, int E, MoeTables tabs, MoeRoute rt, int topk, int* tok_valid, __half* out,
-    int hidden, int fc, const __half* x, __half* xr) {
+    int hidden, int fc, const __half* x, int x_bf16, __half* xr) {
     if (blockIdx.x == 0) {
         extern __shared__ __align__(16) int rt_smem[];
         route_block(rt_smem, ids, entries, E, tabs, rt, topk, tok_valid, out, hidden, fc);
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(MOE_ROUTE_THREADS) void moe_route_rotate_kernel(
     const int rem = job - entry * per_entry, proj = rem / nblk, j = rem - proj * nblk;
     const __half* suh = reinterpret_cast<const __half*>(gptr(tabs.t[proj == 0 ? 1 : 4])[e]);
     const int kg = j * 128 + 2 * lane;
-    const __half2 pr = __hmul2(ld_h2(gptr(x) + (size_t)(entry / topk) * hidden + kg), ld_h2(gptr(suh) + kg));
+    const __half2 pr = __hmul2(x_h2(ld_h2(gptr(x) + (size_t)(entry / topk) * hidden + kg), x_bf16), ld_h2(gptr(suh) + kg));
     float a = __low2float(pr), c = __high2float(pr);
     fwht128_pair_fast(a, c, lane);
     st_h2(gptr(xr) + ((size_t)proj * entries + entry) * hidden + kg, h2_rn(a * kHadNorm, c * kHadNorm));
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(MOE_ROUTE_THREADS) void moe_route_rotate_kernel(
 // only, fp32 accumulation in slot order.
 __global__ __launch_bounds__(256) void moe_combine_kernel(const __half* y, const int32_t* ids, const void* weights,
                                                           int weights_f16, int topk, int E, int hidden,
-                                                          __half* out) {
+                                                          __half* out, int y_bf16) {
     const int t = blockIdx.y;
     const int c = (blockIdx.x * 256 + threadIdx.x) * 2;
     if (c >= hidden) return;
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const __half* y, const
         a0 += wv * __low2float(v);
         a1 += wv * __high2float(v);
     }
-    st_h2(gptr(out) + (size_t)t * hidden + c, h2_rn(a0, a1));
+    st_y2(gptr(out) + (size_t)t * hidden + c, h2_rn(a0, a1), y_bf16);
 }
 
 static int env_int_once(const char* name) {
@@ -492,7 +492,7 @@ MoeLayout moe_layout(int tokens, int topk, int E, int hidden, int inter) {
 
 int run_moe_decode(const char* fn, const uint16_t* x, const int32_t* ids, const void* weights, int weights_f16,
                    const MoeTables& tb, int E, uint16_t* out, int tokens, int topk, int hidden, int inter, int KG,
-                   int KU, int KD, int cb, float limit, void* ws, size_t ws_bytes, hipStream_t st) {
+                   int KU, int KD, int cb, float limit, int bf16, void* ws, size_t ws_bytes, hipStream_t st) {
     EXL3_REQUIRE((long long)tokens * topk <= kMoeMaxEntries, "%s: tokens*topk=%lld above %d", fn,
                  (long long)tokens * topk, kMoeMaxEntries);
     const MoeLayout L = moe_layout(tokens, topk, E, hidden, inter);
@@ -529,7 +529,7 @@ int run_moe_decode(const char* fn, const uint16_t* x, const int32_t* ids, const 
         const long long blocks = 1 + (jobs + MOE_ROUTE_THREADS / 64 - 1) / (MOE_ROUTE_THREADS / 64);
         moe_route_rotate_kernel<<<(unsigned)blocks, MOE_ROUTE_THREADS, smem, st>>>(
             ids, L.entries, E, tb, rt, topk, tok_valid, reinterpret_cast<__half*>(out), hidden, L.fc,
-            reinterpret_cast<const __half*>(x), xr);
+            reinterpret_cast<const __half*>(x), bf16, xr);
         rc = launch_status("exl3 moe route+rotate launch");
         if (rc) return rc;
     } else if (!direct) {
@@ -543,6 +543,8 @@ int run_moe_decode(const char* fn, const uint16_t* x, const int32_t* ids, const 
     }
 
     MoeParams p{};
+    p.x_bf16 = bf16;
+    p.y_bf16 = bf16;
     p.rt = rt;
     p.topk = topk;
     p.entries = L.entries;
@@ -724,7 +726,7 @@ int run_moe_decode(const char* fn, const uint16_t* x, const int32_t* ids, const 
 
     // 5. weighted combine
     moe_combine_kernel<<<dim3((hidden / 2 + 255) / 256, tokens), 256, 0, st>>>(
-        yslots, ids, weights, weights_f16, topk, E, hidden, reinterpret_cast<__half*>(out));
+        yslots, ids, weights, weights_f16, topk, E, hidden, reinterpret_cast<__half*>(out), bf16);
     return launch_status("exl3 moe combine launch");
 }
 
@@ -820,7 +822,7 @@ __global__ __launch_bounds__(MOE_ROUTE_THREADS) void moe_prefill_route_kernel(co
 // xr[p][crow][k] = fp16(FWHT(x[token][k] (.) suh_p[e][k]) / sqrt(128)), p = 0 gate, 1 up; one wave per
 // (compact row, projection) walking the row's 128-wide blocks (the loads of the next block are issued
 // before the current block's transform); rows past the routed count exit.
-__global__ __launch_bounds__(256) void moe_prefill_rotate_kernel(const __half* x, const int32_t* ids, const int* rows,
+__global__ __launch_bounds__(256) void moe_prefill_rotate_kernel(const __half* x, int x_bf16, const int32_t* ids, const int* rows,
                                                                 const int* counts, const int64_t* suh_g,
                                                                 const int64_t* suh_u, int topk, int hidden,
                                                                 int entries, __half* xr) {
@@ -836,7 +838,7 @@ __global__ __launch_bounds__(256) void moe_prefill_rotate_kernel(const __half* x
     EXL3_GLOBAL __half* dst = gptr(xr) + ((size_t)proj * entries + crow) * hidden + 2 * lane;
     __half2 xv = ld_h2(xs), sv = ld_h2(suh);
     for (int j = 0; j < nblk; ++j) {
-        const __half2 pr = __hmul2(xv, sv);
+        const __half2 pr = __hmul2(x_h2(xv, x_bf16), sv);
         if (j + 1 < nblk) {
             xv = ld_h2(xs + (j + 1) * 128);
             sv = ld_h2(suh + (j + 1) * 128);
@@ -901,7 +903,7 @@ bool moe_use_prefill(int tokens, int topk, int E) {
 
 int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const void* weights, int weights_f16,
                     const MoeTables& tb, int E, uint16_t* out, int tokens, int topk, int hidden, int inter, int KG,
-                    int KU, int KD, int cb, float limit, void* ws, size_t ws_bytes, hipStream_t st) {
+                    int KU, int KD, int cb, float limit, int bf16, void* ws, size_t ws_bytes, hipStream_t st) {
     const PrefillLayout L = prefill_layout(tokens, topk, E, hidden, inter);
     EXL3_REQUIRE_CODE(ws && ws_bytes >= L.total, EXL3_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given",
                       fn, L.total, ws ? ws_bytes : (size_t)0);
@@ -928,7 +930,7 @@ int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const
         if (rc) return rc;
         const long long jobs = (long long)entries * 2;
         moe_prefill_rotate_kernel<<<(unsigned)((jobs + 3) / 4), 256, 0, st>>>(
-            reinterpret_cast<const __half*>(x) + (size_t)t0 * hidden, idc, rows, counts, tb.t[1], tb.t[4], topk,
+            reinterpret_cast<const __half*>(x) + (size_t)t0 * hidden, bf16, idc, rows, counts, tb.t[1], tb.t[4], topk,
             hidden, entries, xr);
         rc = launch_status("exl3 moe prefill rotate launch");
         if (rc) return rc;
@@ -965,7 +967,7 @@ int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const
         if (rc) return rc;
         moe_combine_kernel<<<dim3((hidden / 2 + 255) / 256, T), 256, 0, st>>>(
             y, idc, reinterpret_cast<const char*>(weights) + (size_t)t0 * topk * wsz, weights_f16, topk, E, hidden,
-            reinterpret_cast<__half*>(out) + (size_t)t0 * hidden);
+            reinterpret_cast<__half*>(out) + (size_t)t0 * hidden, bf16);
         rc = launch_status("exl3 moe prefill combine launch");
         if (rc) return rc;
     }
@@ -974,7 +976,7 @@ int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const
 
 int run_moe(const char* fn, const uint16_t* x, const int32_t* ids, const void* weights, int weights_f16,
             const MoeTables& tb, int E, uint16_t* out, int tokens, int topk, int hidden, int inter, int KG,
-            int KU, int KD, int cb, float limit, void* ws, size_t ws_bytes, hipStream_t st) {
+            int KU, int KD, int cb, float limit, int bf16, void* ws, size_t ws_bytes, hipStream_t st) {
     EXL3_REQUIRE(tokens >= 1 && topk >= 1, "%s: tokens=%d topk=%d must be >= 1", fn, tokens, topk);
     EXL3_REQUIRE(E >= 1 && E <= kMoeMaxExperts, "%s: num_experts=%d outside 1..%d", fn, E, kMoeMaxExperts);
     EXL3_REQUIRE(topk <= kMoePrefillChunk, "%s: topk=%d above %d", fn, topk, kMoePrefillChunk);
@@ -989,9 +991,9 @@ int run_moe(const char* fn, const uint16_t* x, const int32_t* ids, const void* w
     EXL3_REQUIRE(aligned(x, 4) && aligned(out, 4), "%s: misaligned x/out", fn);
     if (moe_use_prefill(tokens, topk, E))
         return run_moe_prefill(fn, x, ids, weights, weights_f16, tb, E, out, tokens, topk, hidden, inter, KG, KU, KD,
-                               cb, limit, ws, ws_bytes, st);
+                               cb, limit, bf16, ws, ws_bytes, st);
     return run_moe_decode(fn, x, ids, weights, weights_f16, tb, E, out, tokens, topk, hidden, inter, KG, KU, KD, cb,
-                          limit, ws, ws_bytes, st);
+                          limit, bf16, ws, ws_bytes, st);
 }
 
 }  // namespace
@@ -1033,8 +1035,23 @@ extern "C" int exl3_moe_layer(const uint16_t* x, const int32_t* topk_ids, const 
     clear_error();
     MoeTables tb{{gate_trellis, gate_suh, gate_svh, up_trellis, up_suh, up_svh, down_trellis, down_suh, down_svh}};
     return run_moe("exl3_moe_layer", x, topk_ids, topk_weights, 0, tb, num_experts, out, tokens, topk, hidden,
-                   inter, K_gate, K_up, K_down, codebook, swiglu_limit, workspace, workspace_bytes,
+                   inter, K_gate, K_up, K_down, codebook, swiglu_limit, 0, workspace, workspace_bytes,
                    as_stream(stream));
+}
+
+extern "C" int exl3_moe_layer_typed(const void* x, const int32_t* topk_ids, const float* topk_weights,
+                                    const int64_t* gate_trellis, const int64_t* gate_suh, const int64_t* gate_svh,
+                                    const int64_t* up_trellis, const int64_t* up_suh, const int64_t* up_svh,
+                                    const int64_t* down_trellis, const int64_t* down_suh, const int64_t* down_svh,
+                                    int num_experts, void* out, int tokens, int topk, int hidden, int inter,
+                                    int K_gate, int K_up, int K_down, int codebook, float swiglu_limit, int dtype,
+                                    void* workspace, size_t workspace_bytes, void* stream) {
+    clear_error();
+    EXL3_REQUIRE(dtype == EXL3_DTYPE_F16 || dtype == EXL3_DTYPE_BF16, "exl3_moe_layer_typed: dtype=%d", dtype);
+    MoeTables tb{{gate_trellis, gate_suh, gate_svh, up_trellis, up_suh, up_svh, down_trellis, down_suh, down_svh}};
+    return run_moe("exl3_moe_layer_typed", static_cast<const uint16_t*>(x), topk_ids, topk_weights, 0, tb, num_experts,
+                   static_cast<uint16_t*>(out), tokens, topk, hidden, inter, K_gate, K_up, K_down, codebook,
+                   swiglu_limit, dtype == EXL3_DTYPE_BF16, workspace, workspace_bytes, as_stream(stream));
 }
 
 extern "C" int exl3_p2b_fused_moe(const uint16_t* x, uint16_t* out, const int64_t* gate_trellis,
@@ -1047,6 +1064,6 @@ extern "C" int exl3_p2b_fused_moe(const uint16_t* x, uint16_t* out, const int64_
     clear_error();
     MoeTables tb{{gate_trellis, gate_suh, gate_svh, up_trellis, up_suh, up_svh, down_trellis, down_suh, down_svh}};
     return run_moe("exl3_p2b_fused_moe", x, expert_ids, routing_weights, 1, tb, num_experts, out, 1, num_ids,
-                   hidden, inter, K_gate, K_up, K_down, codebook, swiglu_limit, workspace, workspace_bytes,
+                   hidden, inter, K_gate, K_up, K_down, codebook, swiglu_limit, 0, workspace, workspace_bytes,
                    as_stream(stream));
 }

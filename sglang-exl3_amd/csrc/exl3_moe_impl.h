@@ -148,6 +148,9 @@ struct MoeParams {
     // then stages fp16(silu(min(g, L)) * clamp(u, -L, L)), rotated with its
     // own suh, from those rows.
     int gfx;
+    // the caller's x (gate/up items that rotate their own rows) and final
+    // output (fused combine) are bfloat16
+    int x_bf16, y_bf16;
 };
 
 inline size_t moe_route_smem_bytes(int E, int entries, int tokens) {
@@ -447,7 +450,7 @@ __device__ __forceinline__ void moe_item(const MoeParams& p, int it, unsigned ch
         if (pre_rotated) {
             bits = *reinterpret_cast<const uint32_t*>(&xv);
         } else {
-            const __half2 pr = __hmul2(xv, sv);
+            const __half2 pr = __hmul2(down ? xv : x_h2(xv, p.x_bf16), sv);
             float fa = __low2float(pr), fc = __high2float(pr);
             fwht128_pair_fast(fa, fc, lane);
             const _Float16 ha = f16_rn(fa * kHadNorm), hc = f16_rn(fc * kHadNorm);
@@ -587,7 +590,7 @@ __device__ __forceinline__ void moe_item(const MoeParams& p, int it, unsigned ch
                 const float sa = wv * kHadNorm * __low2float(ev0), sb = wv * kHadNorm * __high2float(ev0);
                 const FxPair cur = fx_issue_pair(p.acc + (size_t)t * n + c0, va * sa, vb * sb);
                 if (ptok >= 0)
-                    fx_finish_pair(fx, p.acc + (size_t)ptok * n + c0, pcnt, gptr(p.final_out) + (size_t)ptok * n + c0);
+                    fx_finish_pair(fx, p.acc + (size_t)ptok * n + c0, pcnt, gptr(p.final_out) + (size_t)ptok * n + c0, p.y_bf16);
                 fx = cur;
                 ptok = t;
                 pcnt = c;
@@ -605,7 +608,7 @@ __device__ __forceinline__ void moe_item(const MoeParams& p, int it, unsigned ch
                                                __HIP_MEMORY_SCOPE_AGENT);
                 }
             } else if (ptok >= 0) {
-                fx_finish_pair(fx, p.acc + (size_t)ptok * n + c0, pcnt, gptr(p.final_out) + (size_t)ptok * n + c0);
+                fx_finish_pair(fx, p.acc + (size_t)ptok * n + c0, pcnt, gptr(p.final_out) + (size_t)ptok * n + c0, p.y_bf16);
             }
             continue;
         }
@@ -767,7 +770,7 @@ __device__ __forceinline__ void moe_item(const MoeParams& p, int it, unsigned ch
                         fx_issue_pair(p.acc + (size_t)t * n + c0, wv * __low2float(yh), wv * __high2float(yh));
                     if (ptok >= 0)
                         fx_finish_pair(fx, p.acc + (size_t)ptok * n + c0, pcnt,
-                                       gptr(p.final_out) + (size_t)ptok * n + c0);
+                                       gptr(p.final_out) + (size_t)ptok * n + c0, p.y_bf16);
                     fx = cur;
                     ptok = t;
                     pcnt = c;
@@ -776,7 +779,7 @@ __device__ __forceinline__ void moe_item(const MoeParams& p, int it, unsigned ch
                 }
             }
             if (ptok >= 0)
-                fx_finish_pair(fx, p.acc + (size_t)ptok * n + c0, pcnt, gptr(p.final_out) + (size_t)ptok * n + c0);
+                fx_finish_pair(fx, p.acc + (size_t)ptok * n + c0, pcnt, gptr(p.final_out) + (size_t)ptok * n + c0, p.y_bf16);
         }
     }
 }

@@ -49,6 +49,8 @@ SIGNATURES = {
     "exl3_gemv": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _SZ, _P]),
     "exl3_gemv_noalloc": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "exl3_gemm": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _SZ, _P]),
+    "exl3_linear_cat_workspace_size": (_SZ, [_I, _I, _P, _I, _I]),
+    "exl3_linear_cat": (_I, [_P, _I, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _P, _SZ, _P]),
     "exl3_p2b_gemv_batched": (_I, [_P, _I, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _P, _SZ, _P]),
     "exl3_hadamard_rows": (_I, [_P, _P, _P, _P, _F, _I, _I, _P]),
     "exl3_hadamard_fast": (_I, [_P, _P, _P, _I, _I, _I, _P]),
@@ -61,6 +63,8 @@ SIGNATURES = {
     "exl3_moe_plan": (_I, [_I, _I, _I, _I, _I, _P]),
     "exl3_moe_layer": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I,
                             _I, _I, _I, _I, _F, _P, _SZ, _P]),
+    "exl3_moe_layer_typed": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I,
+                                  _I, _I, _I, _I, _F, _I, _P, _SZ, _P]),
     "exl3_p2b_fused_moe": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I,
                                 _I, _I, _I, _I, _F, _P, _SZ, _P]),
     "exl3_workspace_status": (_I, [_P, _SZ, _P, _P]),

@@ -160,6 +160,15 @@ def _mgemm_two(layer, x2: torch.Tensor, lin0: EXL3DenseLinear, lin1: EXL3DenseLi
     return lin0.forward(x2), lin1.forward(other)
 
 
+def _cat_compatible(linears: list, *dtypes: torch.dtype) -> bool:
+    """Whether the shards run as one exl3_linear_cat call: up to four of one
+    integer K and codebook over one input width, fp16 or bf16 in and out."""
+    a = linears[0]
+    return (len(linears) <= 4 and isinstance(a.K, int)
+            and all(d in (torch.float16, torch.bfloat16) for d in dtypes)
+            and all(b.K == a.K and b.codebook == a.codebook and b.in_features == a.in_features for b in linears[1:]))
+
+
 class EXL3LinearMethod(LinearMethodBase):
     """SGLang linear method running dense EXL3 weights on the HIP kernels."""
 
@@ -266,8 +275,22 @@ class EXL3LinearMethod(LinearMethodBase):
         linears = getattr(layer, "_exl3_linears", None)
         if not linears:
             raise RuntimeError("EXL3 linear layers were not built after weight load")
+        fuse_on = os.environ.get("SGLANG_EXL3_MGEMM", "1") != "0"
+        out_dtype = getattr(layer, "_exl3_out_dtype", x.dtype)
+        if x.is_cuda and (fuse_on or len(linears) == 1) and not getattr(layer, "_exl3_scale_input", False) \
+                and _cat_compatible(linears, x.dtype, out_dtype):
+            # every shard in one call, the casts inside the kernels
+            from .ops import register_custom_ops
+
+            register_custom_ops()
+            y = torch.ops.sglang_exl3.exl3_linear_cat(
+                x.reshape(-1, x.shape[-1]), [lin.trellis for lin in linears], [lin.suh for lin in linears],
+                [lin.svh for lin in linears], linears[0].K, linears[0].codebook, out_dtype == torch.bfloat16)
+            if bias is not None:
+                y = y + bias.to(out_dtype)
+            return y.view(*x.shape[:-1], y.shape[-1])
         shape, rows, x2, scale = self._prepare(layer, x)
-        fuse = rows <= FUSED_PAIR_MAX_ROWS and os.environ.get("SGLANG_EXL3_MGEMM", "1") != "0"
+        fuse = rows <= FUSED_PAIR_MAX_ROWS and fuse_on
         n = len(linears)
         if n == 2 and fuse and _pair_compatible(linears[0], linears[1]):
             y = torch.cat(fused_pair(layer, x2, linears[0], linears[1]), dim=1)
@@ -278,7 +301,6 @@ class EXL3LinearMethod(LinearMethodBase):
         else:
             outs = [lin.forward(x2) for lin in linears]
             y = torch.cat(outs, dim=1) if len(outs) > 1 else outs[0]
-        out_dtype = getattr(layer, "_exl3_out_dtype", x.dtype)
         y = (y.float() * scale).to(out_dtype) if scale is not None else y.to(out_dtype)
         if bias is not None:
             y = y + bias.to(out_dtype)

@@ -491,15 +491,20 @@ def apply_exl3_experts(x: torch.Tensor, topk_ids: torch.Tensor, topk_weights: to
         raise RuntimeError("EXL3 experts were not built after weight load")
     tokens, hidden = x.shape[-2], x.shape[-1]
     x2d = x.reshape(tokens, hidden)
-    ids = topk_ids.reshape(tokens, -1).to(torch.long)
+    ids = topk_ids.reshape(tokens, -1)
     w = topk_weights.reshape(tokens, -1)
     expert_map = pin_exl3_expert_map(layer, x2d.device)
-    local = map_topk_to_local(ids, len(inners), expert_map)
+    native_ids = expert_map is None and ids.dtype == torch.int32 and fused is not False
+    # local int32 ids go to the kernels as they are, which skip those outside
+    # [0, E) (map_topk_to_local's invalid slot)
+    local = ids if native_ids else map_topk_to_local(ids.to(torch.long), len(inners), expert_map)
     reason = _native_moe_ok(layer, tokens, int(local.shape[-1]))
     if fused is not False and reason is None:
         lim = float(limit)
         lim = 0.0 if (lim != lim or lim == float("inf")) else lim
-        out = torch.ops.sglang_exl3.exl3_moe_layer(
+        op = (torch.ops.sglang_exl3.exl3_moe_layer_typed if x.dtype in (torch.float16, torch.bfloat16)
+              else torch.ops.sglang_exl3.exl3_moe_layer)
+        out = op(
             x2d, local.to(torch.int32), w.to(torch.float32), *[layer._exl3_ptrs[k] for k in _TABLE_ORDER],
             layer._exl3_k_gate, layer._exl3_k_up, layer._exl3_k_down, bool(layer._exl3_use_mcg),
             int(layer._exl3_intermediate_local), lim, int(getattr(layer, "_exl3_codebook", -1)))
@@ -508,6 +513,8 @@ def apply_exl3_experts(x: torch.Tensor, topk_ids: torch.Tensor, topk_weights: to
     if fused is True:
         raise RuntimeError(f"EXL3 fused MoE requested but unavailable: {reason}")
     layer._exl3_last_apply = "loop"
+    if native_ids:
+        local = map_topk_to_local(ids.to(torch.long), len(inners), expert_map)
     return apply_exl3_python_loop(x2d, local, w, inners, None, float(limit)).to(x.dtype)
 
 

@@ -10,8 +10,9 @@ CPU tensors are rejected: there is no CPU fallback in the product.
 
 from __future__ import annotations
 
+import ctypes
 import logging
-from typing import Dict, Tuple
+from typing import Dict, List, Tuple
 
 import torch
 
@@ -103,8 +104,6 @@ def check_waits(device=None) -> None:
     silently.  Synchronises the device; not callable during graph capture.
     A workspace whose status was set is zeroed before the error is raised
     (its counters may have been left non-zero), so later calls run clean."""
-    import ctypes
-
     dev = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
     torch.cuda.synchronize(idx)
@@ -229,6 +228,60 @@ def exl3_linear_impl(x, trellis, suh, svh, K, codebook):
     return _gemv_like("exl3_linear", _lib.lib().exl3_gemm, x, trellis, suh, svh, K, int(codebook))
 
 
+_CAT_DTYPES = {torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16}
+CAT_MAX = 4  # weights of one exl3_linear_cat call
+
+
+def exl3_linear_cat_impl(x, trellis, suh, svh, K, codebook, out_bf16):
+    """[x @ W_0 | x @ W_1 | ..] (rows x sum of widths) for the output shards of
+    one layer: one K and codebook, each its own trellis, suh and svh.  x fp16 or
+    bf16, the output fp16 or bf16, without a cast, copy or concatenation around
+    the kernels (reference: src/sglang_exl3/dense.py:317-371)."""
+    name = "exl3_linear_cat"
+    count = len(trellis)
+    if not 1 <= count <= CAT_MAX or len(suh) != count or len(svh) != count:
+        raise RuntimeError(f"sglang_exl3::{name}: 1 to {CAT_MAX} weights with a suh and svh each")
+    _require_device(name, x, *trellis, *suh, *svh)
+    if x.dim() < 2 or x.dtype not in _CAT_DTYPES:
+        raise RuntimeError(f"sglang_exl3::{name}: x must be float16 or bfloat16 [..., in_features]")
+    if int(codebook) not in (_lib.CB_3INST, _lib.CB_MCG, _lib.CB_MUL1):
+        raise RuntimeError(f"sglang_exl3::{name}: codebook id {codebook} outside 0..2")
+    kdim = x.shape[-1]
+    m = x.numel() // kdim if kdim else 0
+    keep, widths = [], []
+    for t, su, sv in zip(trellis, suh, svh):
+        _check_trellis(name, t, K)
+        n = t.shape[1] * 16
+        if kdim != t.shape[0] * 16:
+            raise RuntimeError(f"sglang_exl3::{name}: x feature dimension does not match trellis")
+        su, sv = _f16(name, su, "suh"), _f16(name, sv, "svh")
+        if su.numel() < kdim or sv.numel() < n:
+            raise RuntimeError(f"sglang_exl3::{name}: suh needs {kdim} and svh {n} elements "
+                               f"(got {su.numel()}, {sv.numel()})")
+        t = t.contiguous()
+        if count > 1:  # views at odd offsets, which the batched launch of two shards takes
+            t, su, sv = (a if a.data_ptr() % q == 0 else a.clone() for a, q in ((t, 16), (su, 4), (sv, 4)))
+        keep.append((t, su, sv))
+        widths.append(n)
+    x2 = x.reshape(m, kdim).contiguous()
+    if x2.dtype == torch.bfloat16 and x2.data_ptr() % 4:
+        x2 = x2.clone()
+    y = torch.empty((m, sum(widths)), dtype=torch.bfloat16 if out_bf16 else torch.float16, device=x.device)
+    if m == 0:
+        return y
+    lib = _lib.lib()
+    ptrs = [(ctypes.c_void_p * count)(*(k[j].data_ptr() for k in keep)) for j in range(3)]
+    ns = (ctypes.c_int * count)(*widths)
+    with torch.cuda.device(x.device):
+        need = int(lib.exl3_linear_cat_workspace_size(m, kdim, ns, count, int(K)))
+        ws = workspace(x.device, need) if need else None
+        rc = lib.exl3_linear_cat(x2.data_ptr(), _CAT_DTYPES[x2.dtype], *ptrs, ns, count, y.data_ptr(),
+                                 _CAT_DTYPES[y.dtype], m, kdim, int(K), int(codebook),
+                                 0 if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream_ptr(x))
+    check_ws(rc, name, ws)
+    return y
+
+
 def p2b_gemv_batched_impl(x, trellis_ptrs, suh_ptrs, svh_ptrs, expert_indices, K, mcg, mmode=1):
     name = "p2b_gemv_batched"
     _require_device(name, x, trellis_ptrs, suh_ptrs, svh_ptrs, expert_indices)
@@ -327,9 +380,30 @@ def exl3_moe_layer_impl(x, topk_ids, topk_weights, gate_trellis_ptrs, gate_suh_p
     topk_ids: [T, topk] local expert ids (outside [0, E) = skipped);
     topk_weights: [T, topk]; swiglu_limit 0 or inf = no clamp; returns fp16 [T, hidden].
     codebook: 0 = 3INST, 1 = MCG, 2 = mul1; -1 = from `mcg` (MCG or mul1)."""
-    name = "exl3_moe_layer"
-    tables = (gate_trellis_ptrs, gate_suh_ptrs, gate_svh_ptrs, up_trellis_ptrs, up_suh_ptrs, up_svh_ptrs,
-              down_trellis_ptrs, down_suh_ptrs, down_svh_ptrs)
+    return _moe_layer("exl3_moe_layer", x.to(torch.float16), topk_ids, topk_weights,
+                      (gate_trellis_ptrs, gate_suh_ptrs, gate_svh_ptrs, up_trellis_ptrs, up_suh_ptrs, up_svh_ptrs,
+                       down_trellis_ptrs, down_suh_ptrs, down_svh_ptrs),
+                      K_gate, K_up, K_down, mcg, intermediate_size, swiglu_limit, codebook)
+
+
+def exl3_moe_layer_typed_impl(x, topk_ids, topk_weights, gate_trellis_ptrs, gate_suh_ptrs, gate_svh_ptrs,
+                              up_trellis_ptrs, up_suh_ptrs, up_svh_ptrs, down_trellis_ptrs, down_suh_ptrs,
+                              down_svh_ptrs, K_gate, K_up, K_down, mcg, intermediate_size, swiglu_limit=0.0,
+                              codebook=-1):
+    """exl3_moe_layer on fp16 or bf16 rows with the output in x's dtype, the
+    casts inside the kernels."""
+    if x.dtype not in _CAT_DTYPES:
+        raise RuntimeError("sglang_exl3::exl3_moe_layer_typed: x must be float16 or bfloat16")
+    if x.dtype == torch.bfloat16 and x.data_ptr() % 4:
+        x = x.clone()
+    return _moe_layer("exl3_moe_layer_typed", x, topk_ids, topk_weights,
+                      (gate_trellis_ptrs, gate_suh_ptrs, gate_svh_ptrs, up_trellis_ptrs, up_suh_ptrs, up_svh_ptrs,
+                       down_trellis_ptrs, down_suh_ptrs, down_svh_ptrs),
+                      K_gate, K_up, K_down, mcg, intermediate_size, swiglu_limit, codebook)
+
+
+def _moe_layer(name, x, topk_ids, topk_weights, tables, K_gate, K_up, K_down, mcg, intermediate_size, swiglu_limit,
+               codebook):
     _require_device(name, x, topk_ids, topk_weights, *tables)
     if x.dim() != 2:
         raise RuntimeError(f"sglang_exl3::{name}: x must be [tokens, hidden]")
@@ -338,9 +412,9 @@ def exl3_moe_layer_impl(x, topk_ids, topk_weights, gate_trellis_ptrs, gate_suh_p
     topk = int(ids.shape[1])
     ids = ids.to(torch.int32).contiguous()
     w = topk_weights.reshape(T, topk).to(torch.float32).contiguous()
-    xh = x.to(torch.float16).contiguous()
+    xh = x.contiguous()
     tabs, E = _moe_tables(name, tables)
-    out = torch.empty((T, hidden), dtype=torch.float16, device=x.device)
+    out = torch.empty((T, hidden), dtype=x.dtype, device=x.device)
     if T == 0 or topk == 0:
         return out.zero_()
     lim = _limit_arg(swiglu_limit)
@@ -348,11 +422,11 @@ def exl3_moe_layer_impl(x, topk_ids, topk_weights, gate_trellis_ptrs, gate_suh_p
     with torch.cuda.device(x.device):
         need = int(lib.exl3_moe_workspace_size(T, topk, E, hidden, int(intermediate_size)))
         ws = workspace(x.device, need)
-        rc = lib.exl3_moe_layer(
+        rc = lib.exl3_moe_layer_typed(
             xh.data_ptr(), ids.data_ptr(), w.data_ptr(), *[t.data_ptr() for t in tabs], E, out.data_ptr(), T, topk,
             hidden, int(intermediate_size), int(K_gate), int(K_up), int(K_down),
-            _lib.codebook_from_mcg(bool(mcg)) if int(codebook) < 0 else int(codebook), lim, ws.data_ptr(),
-            ws.numel(), _stream_ptr(x))
+            _lib.codebook_from_mcg(bool(mcg)) if int(codebook) < 0 else int(codebook), lim, _CAT_DTYPES[x.dtype],
+            ws.data_ptr(), ws.numel(), _stream_ptr(x))
     check_ws(rc, name, ws)
     return out
 
@@ -491,6 +565,17 @@ def register_custom_ops() -> bool:
         rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
         return torch.empty((rows, trellis.size(1) * 16), dtype=torch.float16, device=x.device)
 
+    @torch.library.custom_op("sglang_exl3::exl3_linear_cat", mutates_args=())
+    def exl3_linear_cat(x: torch.Tensor, trellis: List[torch.Tensor], suh: List[torch.Tensor],
+                        svh: List[torch.Tensor], K: int, codebook: int, out_bf16: bool) -> torch.Tensor:
+        return exl3_linear_cat_impl(x, trellis, suh, svh, K, codebook, out_bf16)
+
+    @exl3_linear_cat.register_fake
+    def _(x, trellis, suh, svh, K, codebook, out_bf16):
+        rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
+        return torch.empty((rows, sum(t.size(1) * 16 for t in trellis)),
+                           dtype=torch.bfloat16 if out_bf16 else torch.float16, device=x.device)
+
     @torch.library.custom_op("sglang_exl3::p2b_gemv_batched", mutates_args=())
     def p2b_gemv_batched(x: torch.Tensor, trellis_ptrs: torch.Tensor, suh_ptrs: torch.Tensor,
                          svh_ptrs: torch.Tensor, expert_indices: torch.Tensor, K: int, mcg: bool,
@@ -536,6 +621,23 @@ def register_custom_ops() -> bool:
     @exl3_moe_layer.register_fake
     def _(x, topk_ids, topk_weights, *rest):
         return torch.empty((x.shape[0], x.shape[1]), dtype=torch.float16, device=x.device)
+
+    @torch.library.custom_op("sglang_exl3::exl3_moe_layer_typed", mutates_args=())
+    def exl3_moe_layer_typed(x: torch.Tensor, topk_ids: torch.Tensor, topk_weights: torch.Tensor,
+                             gate_trellis_ptrs: torch.Tensor, gate_suh_ptrs: torch.Tensor,
+                             gate_svh_ptrs: torch.Tensor, up_trellis_ptrs: torch.Tensor, up_suh_ptrs: torch.Tensor,
+                             up_svh_ptrs: torch.Tensor, down_trellis_ptrs: torch.Tensor,
+                             down_suh_ptrs: torch.Tensor, down_svh_ptrs: torch.Tensor, K_gate: int, K_up: int,
+                             K_down: int, mcg: bool, intermediate_size: int, swiglu_limit: float = 0.0,
+                             codebook: int = -1) -> torch.Tensor:
+        return exl3_moe_layer_typed_impl(x, topk_ids, topk_weights, gate_trellis_ptrs, gate_suh_ptrs, gate_svh_ptrs,
+                                         up_trellis_ptrs, up_suh_ptrs, up_svh_ptrs, down_trellis_ptrs, down_suh_ptrs,
+                                         down_svh_ptrs, K_gate, K_up, K_down, mcg, intermediate_size, swiglu_limit,
+                                         codebook)
+
+    @exl3_moe_layer_typed.register_fake
+    def _(x, topk_ids, topk_weights, *rest):
+        return torch.empty((x.shape[0], x.shape[1]), dtype=x.dtype, device=x.device)
 
     @torch.library.custom_op("sglang_exl3::exl3_gate_up_swiglu", mutates_args=())
     def exl3_gate_up_swiglu(x: torch.Tensor, suh: torch.Tensor, gate_trellis: torch.Tensor, gate_svh: torch.Tensor,

@@ -244,3 +244,51 @@ def test_mgemm_two(rows, n0, n1, K0, K1, cb0, cb1, second):
     z0, _ = _mgemm_two(layer, torch.from_numpy(x).cuda(), *lins,
                        x2_b=None if xb is None else torch.from_numpy(xb).cuda())
     assert z0.data_ptr() != y0.data_ptr() and torch.equal(z0, y0)
+
+
+@pytest.mark.parametrize("m,widths,K,cb,x_dtype,y_dtype,env", [
+    (1, (256, 128, 128), 4, 1, torch.bfloat16, torch.bfloat16, {}),   # balanced GEMV
+    (3, (128, 384), 3, 2, torch.bfloat16, torch.float16, {}),         # ... two rows of blocks, mul1
+    (5, (256, 128), 4, 0, torch.float16, torch.bfloat16, {}),         # k-split GEMV, fixed-point hand-off
+    (11, (128, 256, 128, 128), 2, 1, torch.bfloat16, torch.bfloat16, {}),  # k-split GEMV, partial tiles
+    (14, (384, 128), 3, 2, torch.bfloat16, torch.bfloat16, {}),       # 16-row tiles, raw entries, finish launch
+    (40, (128, 256), 4, 1, torch.bfloat16, torch.float16, {}),        # 64-row tiles, split hand-off
+    (70, (128, 256), 5, 2, torch.float16, torch.bfloat16, {"EXL3_FAT_HANDOFF": "0"}),
+    (300, (256, 512), 3, 1, torch.bfloat16, torch.bfloat16, {"EXL3_FAT_WIDE": "2"}),  # wide tiles
+    (300, (128, 512), 3, 1, torch.bfloat16, torch.bfloat16, {"EXL3_FAT_WIDE": "2"}),  # a width the wide tiles refuse
+])
+def test_linear_cat(m, widths, K, cb, x_dtype, y_dtype, env, monkeypatch):
+    """Several weights in one call, each kernel path, against one exl3_linear per weight with the casts
+    around it.  The two only differ in the order of fp32 sums over k (other splits), so an element is at most
+    a few roundings of the output type apart; twice for the clean-workspace contract."""
+    for key, v in env.items():
+        monkeypatch.setenv(key, v)
+    k = 2048
+    packs = [[torch.from_numpy(a).cuda() for a in _scaled(k, n, K, seed=7 * i + m)] for i, n in enumerate(widths)]
+    x = torch.from_numpy(make_x(m, k, seed=m)).cuda().to(x_dtype)
+    ref = torch.cat([torch.ops.sglang_exl3.exl3_linear(x.to(torch.float16), *p, K, cb) for p in packs], dim=1)
+    ref = ref.to(y_dtype).float()
+    for _ in range(2):
+        y = torch.ops.sglang_exl3.exl3_linear_cat(x, *map(list, zip(*packs)), K, cb, y_dtype == torch.bfloat16)
+        assert y.shape == ref.shape and y.dtype == y_dtype
+        # one ulp of the output type, plus the fp32 sums' own error near zero
+        ulp = 2.0 ** (-7 if y_dtype == torch.bfloat16 else -10)
+        rms = float(ref.square().mean().sqrt())
+        assert torch.all((y.float() - ref).abs() <= ulp * ref.abs() + 1e-3 * rms)
+
+
+@pytest.mark.parametrize("T,invalid", [(1, 0), (1, 1), (6, 2), (60, 0), (200, 3)])
+def test_moe_bf16_matches_casts(T, invalid):
+    """bf16 rows in and out of the one-call layer: the bits of the fp16 layer with casts around it (one token
+    without routing, routed with the fused combine, with the combine launch, prefill), ids outside the
+    experts included."""
+    method, layer, _ = _build_moe(8, 256, 256, 3, "mcg", seed=T)
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn((T, 256), generator=g).cuda().to(torch.bfloat16)
+    ids = torch.stack([torch.randperm(8, generator=g)[:2] for _ in range(T)]).to(torch.int32).cuda()
+    for j in range(invalid):
+        ids[j % T, j % 2] = (-1, 8, 1 << 30)[j]
+    w = torch.rand((T, 2), generator=g).cuda()
+    got = method.apply(layer, x, w, ids)
+    want = method.apply(layer, x.to(torch.float16), w, ids.to(torch.long)).to(torch.bfloat16)
+    assert got.dtype == torch.bfloat16 and torch.equal(got, want)

@@ -45,6 +45,11 @@ def test_meta_fake_tensor_dispatch():
         w = torch.empty((6,), dtype=torch.float16)
         assert torch.ops.sglang_exl3.p2b_fused_moe(x[:1], out, ptrs, ptrs, ptrs, ptrs, ptrs, ptrs, ptrs, ptrs,
                                                    ptrs, ids, w, 2, 2, 2, True) is None
+        xb = torch.empty((2, 128), dtype=torch.bfloat16)
+        c = torch.ops.sglang_exl3.exl3_linear_cat(xb, [trellis, trellis], [suh, suh], [svh, svh], 2, 1, False)
+        assert c.shape == (2, 512) and c.dtype == torch.float16
+        mo = torch.ops.sglang_exl3.exl3_moe_layer_typed(xb, ids, w, *[ptrs] * 9, 2, 2, 2, True, 128)
+        assert mo.shape == (2, 128) and mo.dtype == torch.bfloat16
         o32 = torch.empty((2, 256), dtype=torch.float32)
         assert torch.ops.sglang_exl3.exl3_fat_gemm(x, trellis, o32, svh, 2, True, False) is None
 
