@@ -1,7 +1,7 @@
 // C ABI of the many-row EXL3 GEMM: exl3_fat_gemm, exl3_fat_gemm_scatter and
 // the prefill path of exl3_gemm (rotate -> fat GEMM -> fp16), with the launch
 // planner (rows per tile, k-splits).
-#include "exl3_fat_impl.h"
+#include "exl3_tall_impl.h"
 
 namespace exl3 {
 
@@ -13,6 +13,30 @@ int fat_launch_K5(int, int, const FatParams&, int, hipStream_t);
 int fat_launch_K6(int, int, const FatParams&, int, hipStream_t);
 int fat_launch_K7(int, int, const FatParams&, int, hipStream_t);
 int fat_launch_K8(int, int, const FatParams&, int, hipStream_t);
+
+int tall_launch_K1(int, int, const FatParams&, int, int, hipStream_t);
+int tall_launch_K2(int, int, const FatParams&, int, int, hipStream_t);
+int tall_launch_K3(int, int, const FatParams&, int, int, hipStream_t);
+int tall_launch_K4(int, int, const FatParams&, int, int, hipStream_t);
+int tall_launch_K5(int, int, const FatParams&, int, int, hipStream_t);
+int tall_launch_K6(int, int, const FatParams&, int, int, hipStream_t);
+int tall_launch_K7(int, int, const FatParams&, int, int, hipStream_t);
+int tall_launch_K8(int, int, const FatParams&, int, int, hipStream_t);
+
+int tall_launch(int K, int cb, int mt, const FatParams& p, int row_tiles, int splits, hipStream_t st) {
+    switch (K) {
+        case 1: return tall_launch_K1(cb, mt, p, row_tiles, splits, st);
+        case 2: return tall_launch_K2(cb, mt, p, row_tiles, splits, st);
+        case 3: return tall_launch_K3(cb, mt, p, row_tiles, splits, st);
+        case 4: return tall_launch_K4(cb, mt, p, row_tiles, splits, st);
+        case 5: return tall_launch_K5(cb, mt, p, row_tiles, splits, st);
+        case 6: return tall_launch_K6(cb, mt, p, row_tiles, splits, st);
+        case 7: return tall_launch_K7(cb, mt, p, row_tiles, splits, st);
+        case 8: return tall_launch_K8(cb, mt, p, row_tiles, splits, st);
+    }
+    set_error("exl3 gemm: K=%d outside 1..8", K);
+    return EXL3_ERR_UNSUPPORTED;
+}
 
 int fat_launch(int K, int cb, int mt, const FatParams& p, int splits, hipStream_t st) {
     switch (K) {
@@ -45,6 +69,7 @@ __global__ void f32_to_f16_kernel(const float* src, __half* dst, size_t n2, int 
 
 struct FatPlan {
     int mt, splits;
+    bool tall;  // tall_kernel with mt (128 or 256) rows per tile
 };
 
 bool mats_n256(const MatSet& s) {
@@ -67,6 +92,15 @@ bool mats_n256(const MatSet& s) {
 // 222.6 / 129.6, 768: 227.9 / 330.7 / 131.4.  128-row narrow tiles never win
 // (kept as the EXL3_FAT_MT=128 override).
 constexpr int kFatNarrowMaxRows = 256;
+// Rows from which tall tiles replace the 16-row (up to 16 rows), 64-row and
+// wide tiles of an fp16-output call: 17, and 13 for outputs of up to 4096
+// columns, where their k-splits fill more of the chip.  16-row tiles / tall, us:
+// 13 rows, k = n = 2048: 16.7 / 11.8; k = n = 4096: 17.1 / 14.5; k = 14336, n =
+// 4096: 27.5 / 24.9; but k = 4096, n = 6144, K = 3 mul1: 15.6 / 16.4, n = 14336: 20.7 /
+// 21.8.
+constexpr int kTallMinRows = 17;
+constexpr int kTallMinRowsNarrow = 13;
+constexpr int kTallNarrowCols = 4096;
 // ... and only when they make at least this many tiles: a smaller wide grid
 // needs fp32-atomic k-splits, and the narrow kernel with its split hand-off
 // is faster there.  Graph-timed, wide / narrow: k = 14336, n = 4096, M = 320 /
@@ -143,13 +177,64 @@ int wide_tail_tiles(int m, int k, int n, bool gu) {
     return fat_tail_tiles(tiles, k / 64);
 }
 
+// Tall tiles (tall_kernel) for fp16 / bf16 outputs: rows per tile and k-splits
+// by a cost model in us, fitted to 83 shapes from 17 to 4096 rows, 2048^2 to
+// 14336 x 4096 (graph-timed, both tile heights, 1 / 2 / 4 splits; its choice is
+// on average within 2 % of the best of the six).  With W workgroups on the
+// busiest CU, `slots` of them at once, a 64-k step of a tile with rb staged row
+// blocks takes
+//   L = 0.36 + 0.047 rb  alone (decode and MFMAs of one wave per SIMD), and
+//   C = 0.25 + 0.039 rb  per workgroup where enough share the CU;
+// splits add the finish launch and S partial tiles written and read.  Against
+// the narrow and wide kernels before it (us): k = n = 4096, 20 / 64 / 256 /
+// 1024 / 4096 rows: 21.5 / 30.0 / 35.4 / 75.1 / 176.9 -> 17.5 / 21.7 / 34.9 / 63.9 /
+// 147.4; k = 4096, n = 14336: 24.1 / 33.3 / 70.2 / 145.4 / 549.6 -> 22.9 / 32.2 /
+// 58.6 / 125.0 / 473.7; k = 14336, n = 4096, 64 / 1024 rows: 54.6 / 219.4 -> 45.7 /
+// 153.4.  Env EXL3_FAT_TALL: 0 never, 128 / 256 forced (with EXL3_FAT_SPLITS); the
+// overrides that name another kernel (EXL3_FAT_WIDE=2, _MT, _HANDOFF=0) get it.
+constexpr int kTallMaxSplits = 16;
+
+double tall_cost(int M, int k, int n, int mt, int S) {
+    const int rb = 2 * (((M < mt ? M : mt) + 31) / 32), slots = mt == 128 ? 4 : 2;
+    const double L = 0.36 + 0.047 * rb, C = 0.25 + 0.039 * rb;
+    const long long wgs = (long long)(n / 128) * ((M + mt - 1) / mt) * S;
+    const long long W = (wgs + fat_cus() - 1) / fat_cus(), full = W / slots, rest = W % slots;
+    double t = (double)(full * slots) * C;
+    if (t < L * (double)full) t = L * (double)full;
+    if (rest) t += L > rest * C ? L : rest * C;
+    t *= k / 64 / S;
+    if (S > 1) t += 3.0 + (S > 4 ? 0.2 * (S - 4) : 0.0) + (double)S * M * n * 8.0 / 5.0e6;
+    return t;
+}
+
+bool plan_tall(int M, int k, int n, FatPlan* pl) {
+    const int forced = env_int("EXL3_FAT_TALL", -1), fs = env_int("EXL3_FAT_SPLITS", 0);
+    if (forced < 0 && (fat_wide_mode() == 2 || !fat_handoff_on() || env_int("EXL3_FAT_MT", 0) != 0)) return false;
+    if (forced == 0 || (forced < 0 && M < (n <= kTallNarrowCols ? kTallMinRowsNarrow : kTallMinRows))) return false;
+    const int ksteps = k / 64;
+    double best = 1e30;
+    for (int mt = 128; mt <= 256; mt += 128) {
+        if (forced > 0 && forced != mt) continue;
+        for (int S = 1; S <= kTallMaxSplits && ksteps % (2 * S) == 0; S *= 2) {
+            if (fs > 0 && S != fs && ksteps % (2 * fs) == 0) continue;
+            const double c = tall_cost(M, k, n, mt, S);
+            if (c < best - 1e-9) {
+                best = c;
+                *pl = FatPlan{mt, S, true};
+            }
+        }
+    }
+    return pl->tall;
+}
+
 // f16out: a call with fp16 output (exl3_gemm), whose narrow k-splits use the
 // partial-tile hand-off (fat_handoff) unless EXL3_FAT_HANDOFF=0.
 // n256: every matrix of the call is a multiple of 256 columns wide.
 FatPlan plan_fat(int M, int k, int n, bool f16out, bool n256) {
-    FatPlan pl;
+    FatPlan pl{};
     const int ksteps = k / 64;
     pl.splits = 1;
+    if (f16out && plan_tall(M, k, n, &pl)) return pl;
     if (fat_wide_allowed() && M > kFatNarrowMaxRows && n256 &&
         (fat_wide_mode() == 2 || (long long)(n / FB_COLS) * ((M + FB_ROWS - 1) / FB_ROWS) >= kFatWideMinTiles)) {
         pl.mt = FAT_MT_WIDE;
@@ -195,8 +280,8 @@ int check_fat(const char* fn, const void* a, const void* trellis, const void* ou
 // (exl3_gemm K = 3 mul1, n = 14336, M = 256 / 2048: 69.9 / 250.9 -> 70.3 /
 // 250.3 us, each row's sums taken once per 128-column block).
 // EXL3_FAT_RAW=0 turns it off (ablation).
-bool fat_raw(int cb, int mt, bool gu) {
-    return cb == 2 && (mt == 16 || (mt == FAT_MT_WIDE && gu)) && env_int("EXL3_FAT_RAW", 1) != 0;
+bool fat_raw(int cb, int mt, bool gu, bool tall = false) {
+    return cb == 2 && (tall || mt == 16 || (mt == FAT_MT_WIDE && gu)) && env_int("EXL3_FAT_RAW", 1) != 0;
 }
 
 // Narrow plans with k-splits and fp16 output hand partial tiles to the last
@@ -204,7 +289,7 @@ bool fat_raw(int cb, int mt, bool gu) {
 // into a zero-filled buffer that a third launch converts.  EXL3_FAT_HANDOFF=0
 // keeps the atomic path (ablation).
 bool fat_handoff(const FatPlan& pl, int m, int n) {
-    return pl.splits > 1 && pl.mt != FAT_MT_WIDE &&
+    return pl.tall || (pl.splits > 1 && pl.mt != FAT_MT_WIDE) &&
            (size_t)(n / 128) * (size_t)((m + pl.mt - 1) / pl.mt) <= kWsMaxCounters && fat_handoff_on();
 }
 
@@ -257,7 +342,7 @@ int run_fat(const uint16_t* a, const int16_t* trellis, float* out32, __half* out
         p.partials = partials;
         p.counters = counters;
     }
-    if (rowsum && fat_raw(cb, pl.mt, false)) p.rowsum = rowsum;
+    if (rowsum && fat_raw(cb, pl.mt, false, pl.tall)) p.rowsum = rowsum;
     if (tail > 0) {
         p.tiles_x = n / FB_COLS;
         p.tail_tiles = tail;
@@ -290,6 +375,13 @@ int run_fat(const uint16_t* a, const int16_t* trellis, float* out32, __half* out
                                                                                                        0.f);
         const int rc = launch_status("exl3 fat gemm zero fill");
         if (rc) return rc;
+    }
+    if (pl.tall) {
+        p.split_out = pl.splits > 1;
+        p.out_vec = aligned(out16, 16);
+        const int rc = tall_launch(K, cb, pl.mt, p, (M + pl.mt - 1) / pl.mt, pl.splits, st);
+        if (rc || pl.splits == 1) return rc;
+        return fat_split_finish(p, pl.splits, st, "exl3 gemm finish launch");
     }
     // the split-out finish of the gate/up path, on the plain hand-off
     const bool split_out = p.handoff && pl.mt == 16 && M >= kSplitOutMinRows && pl.splits <= 4 &&
@@ -329,7 +421,7 @@ int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_
     __half* xr = reinterpret_cast<__half*>(reinterpret_cast<char*>(ws) + kWsScratchOffset);
     float* o32 = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + kWsScratchOffset + fat_xr_bytes((int)xrows, k));
     const FatPlan pl = plan_rows(m, k, n, mats.count, n256);
-    float* rs = fat_raw(cb, pl.mt, false)
+    float* rs = fat_raw(cb, pl.mt, false, pl.tall)
                     ? reinterpret_cast<float*>(reinterpret_cast<char*>(xr) + fat_xr_only_bytes((int)xrows, k))
                     : nullptr;
     RotateSuh suhs{};

@@ -127,6 +127,7 @@ struct FatParams {
     // for each matrix in turn, and a column block's matrix comes from mats.
     MatSet mats;
     int y_bf16;  // out16 is bfloat16 (plain modes)
+    int out_vec;  // tall tiles: out16 rows are 16-byte aligned
 };
 
 // Sum over chunks [c0, c0 + nc) of row `row` of rowsum (one wave).
@@ -148,6 +149,10 @@ inline size_t fat_smem_bytes(int mt) {
     return a > c ? a : c;
 }
 
+// kMul1Kinv * acc plus the row's bias term sx (raw entries), as one fma: left to
+// contraction, the product folded into it could be either of the two.
+__device__ __forceinline__ float raw_value(float acc, float sx) { return __builtin_fmaf(acc, kMul1Kinv, sx); }
+
 // Gate/up epilogue of one output row segment (two columns per lane of a
 // 128-column block): the summed gate and up partials -> (mul1 map: times
 // kMul1Kinv plus sx, the row's bias term) -> both output rotations, svh ->
@@ -156,10 +161,10 @@ template <bool RAW>
 __device__ __forceinline__ void fat_gu_finish(const FatParams& p, size_t orow, int c0, float ga, float gb, float ua,
                                               float ub, float sx, __half2 svg, __half2 svu, int lane) {
     if constexpr (RAW) {
-        ga = ga * kMul1Kinv + sx;
-        gb = gb * kMul1Kinv + sx;
-        ua = ua * kMul1Kinv + sx;
-        ub = ub * kMul1Kinv + sx;
+        ga = raw_value(ga, sx);
+        gb = raw_value(gb, sx);
+        ua = raw_value(ua, sx);
+        ub = raw_value(ub, sx);
     }
     fwht128_pair_fast(ga, gb, lane);
     fwht128_pair_fast(ua, ub, lane);
@@ -396,8 +401,8 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
                     }
                     if constexpr (RAW) {
                         const float sx = kMul1Bias * wave_sum(L.rs);
-                        va = va * kMul1Kinv + sx;
-                        vb = vb * kMul1Kinv + sx;
+                        va = raw_value(va, sx);
+                        vb = raw_value(vb, sx);
                     }
                     fwht128_pair_fast(va, vb, lane);
                     st_y2(gptr(p.out16) + (size_t)(m0 + row) * p.n + c0, h2_rn((va * kHadNorm) * sva, (vb * kHadNorm) * svb), p.y_bf16);
@@ -421,8 +426,8 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
                 float va = v2[0].x, vb = v2[0].y;
                 if constexpr (RAW) {
                     const float sx = kMul1Bias * fat_row_sum(rowsum, p.k >> 7, m0 + row, 0, p.k >> 7, lane);
-                    va = va * kMul1Kinv + sx;
-                    vb = vb * kMul1Kinv + sx;
+                    va = raw_value(va, sx);
+                    vb = raw_value(vb, sx);
                 }
                 fwht128_pair_fast(va, vb, lane);
                 st_y2(gptr(p.out16) + (size_t)(m0 + row) * p.n + c0, h2_rn((va * kHadNorm) * sva, (vb * kHadNorm) * svb), p.y_bf16);
@@ -504,8 +509,8 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
         if constexpr (RAW) {
             // this split's k range: chunks kt0 / 8 .. + nsteps / 2
             const float sx = kMul1Bias * fat_row_sum(rowsum, p.k >> 7, m0 + row, kt0 >> 3, nsteps >> 1, lane);
-            va = va * kMul1Kinv + sx;
-            vb = vb * kMul1Kinv + sx;
+            va = raw_value(va, sx);
+            vb = raw_value(vb, sx);
         }
         fwht128_pair_fast(va, vb, lane);
         va = (va * kHadNorm) * sva;
@@ -557,12 +562,16 @@ __global__ __launch_bounds__(256) void fat_split_finish_kernel(FatParams p, int 
         return make_float2(__uint_as_float((uint32_t)u), __uint_as_float((uint32_t)(u >> 32)));
     };
     float2 v[NP][4];
+    auto request = [&](int s0) {
 #pragma unroll
-    for (int j = 0; j < NP; ++j) {
-        const float* pj = p.partials + (size_t)(bx * NP + j) * S * rs + (size_t)row * 128 + 2 * lane;
+        for (int j = 0; j < NP; ++j) {
+            const float* pj = p.partials + (size_t)(bx * NP + j) * S * rs + (size_t)row * 128 + 2 * lane;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) v[j][t] = t < S ? ld2(pj + (size_t)t * rs) : make_float2(0.f, 0.f);
-    }
+            for (int t = 0; t < 4; ++t)
+                v[j][t] = s0 + t < S ? ld2(pj + (size_t)(s0 + t) * rs) : make_float2(0.f, 0.f);
+        }
+    };
+    request(0);
     const __half* svh = p.svh;
     const float* rowsum = p.rowsum;
     int cm = c0;
@@ -582,13 +591,16 @@ __global__ __launch_bounds__(256) void fat_split_finish_kernel(FatParams p, int 
     }
     float2 sm[NP];
 #pragma unroll
-    for (int j = 0; j < NP; ++j) {
-        sm[j] = make_float2(0.f, 0.f);
+    for (int j = 0; j < NP; ++j) sm[j] = make_float2(0.f, 0.f);
+    for (int s0 = 0; s0 < S; s0 += 4) {
+        if (s0) request(s0);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            sm[j].x += v[j][t].x;
-            sm[j].y += v[j][t].y;
-        }
+        for (int j = 0; j < NP; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                sm[j].x += v[j][t].x;
+                sm[j].y += v[j][t].y;
+            }
     }
     float sx = 0.f;
     if constexpr (RAW) sx = kMul1Bias * wave_sum(rsum);
@@ -597,8 +609,8 @@ __global__ __launch_bounds__(256) void fat_split_finish_kernel(FatParams p, int 
     } else {
         float va = sm[0].x, vb = sm[0].y;
         if constexpr (RAW) {
-            va = va * kMul1Kinv + sx;
-            vb = vb * kMul1Kinv + sx;
+            va = raw_value(va, sx);
+            vb = raw_value(vb, sx);
         }
         fwht128_pair_fast(va, vb, lane);
         st_y2(gptr(p.out16) + (size_t)row * p.n + c0,
@@ -670,6 +682,22 @@ __device__ __forceinline__ uint32_t nat_pair(const uint32_t* buf, const uint32_t
 // f[h'][j] = tile rows (8h' + 2j, +1) of column q + 8C: run H = j >> 1, pair P = h' + 2 (j & 1).
 template <int K, int CB, int C, bool RAW>
 __device__ __forceinline__ void nat_column(const uint32_t* buf, const uint32_t* mid, uint32_t (&f)[2][4]) {
+    if constexpr (CB != 2) {
+        // the same words, run by run (frag_decode's order: word p of run H is f[p & 1][2 H + (p >> 1)])
+#define EXL3_NAT(H)                                                                      \
+    {                                                                                    \
+        uint32_t t[4];                                                                   \
+        frag_decode<K, CB, false, H, C>(buf, mid, t);                                    \
+        f[0][2 * H] = t[0];                                                              \
+        f[1][2 * H] = t[1];                                                              \
+        f[0][2 * H + 1] = t[2];                                                          \
+        f[1][2 * H + 1] = t[3];                                                          \
+    }
+        EXL3_NAT(0)
+        EXL3_NAT(1)
+#undef EXL3_NAT
+        return;
+    }
     f[0][0] = nat_pair<K, CB, 0, C, 0, RAW>(buf, mid);
     f[0][1] = nat_pair<K, CB, 0, C, 2, RAW>(buf, mid);
     f[0][2] = nat_pair<K, CB, 1, C, 0, RAW>(buf, mid);
@@ -680,17 +708,24 @@ __device__ __forceinline__ void nat_column(const uint32_t* buf, const uint32_t* 
     f[1][3] = nat_pair<K, CB, 1, C, 3, RAW>(buf, mid);
 }
 
-// Decode one 32-value group (words w[0..K-1], previous word from lane q - 1).
-template <int K, int CB, bool RAW = false>
-__device__ __forceinline__ void nat_group(const uint32_t (&w)[K], int prev_addr, uint32_t (&f)[2][2][4]) {
-    uint32_t buf[K + 1], mid[K];
-#pragma unroll
-    for (int j = 0; j < K; ++j) buf[1 + j] = w[j];
-    buf[0] = (uint32_t)__builtin_amdgcn_ds_bpermute(prev_addr, (int)buf[K]);
+// Decode one 32-value group from its word buffer (buf[0] the previous word).
+template <int K, int CB, bool RAW>
+__device__ __forceinline__ void nat_decode(const uint32_t (&buf)[K + 1], uint32_t (&f)[2][2][4]) {
+    uint32_t mid[K];
 #pragma unroll
     for (int j = 0; j < K; ++j) mid[j] = __builtin_amdgcn_alignbit(buf[j], buf[j + 1], 16);
     nat_column<K, CB, 0, RAW>(buf, mid, f[0]);
     nat_column<K, CB, 1, RAW>(buf, mid, f[1]);
+}
+
+// The same from words w[0..K-1], the previous word from lane q - 1.
+template <int K, int CB, bool RAW = false>
+__device__ __forceinline__ void nat_group(const uint32_t (&w)[K], int prev_addr, uint32_t (&f)[2][2][4]) {
+    uint32_t buf[K + 1];
+#pragma unroll
+    for (int j = 0; j < K; ++j) buf[1 + j] = w[j];
+    buf[0] = (uint32_t)__builtin_amdgcn_ds_bpermute(prev_addr, (int)buf[K]);
+    nat_decode<K, CB, RAW>(buf, f);
 }
 
 // mul1 raw entries in the x16 layout (a tile row on 8 lanes, 16 columns
@@ -708,7 +743,7 @@ __device__ __forceinline__ float raw_row_bias(const FatParams& p, int row, int c
 }
 __device__ __forceinline__ void raw_fix16(float (&v)[16], float sx) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = v[e] * kMul1Kinv + sx;
+    for (int e = 0; e < 16; ++e) v[e] = raw_value(v[e], sx);
 }
 
 // GU = true: gate/up mode.  Workgroup bx then covers column block bx of both

@@ -5,7 +5,7 @@
 
 #include <mutex>
 
-#include "exl3_fat_impl.h"
+#include "exl3_tall_impl.h"
 #include "exl3_moe_impl.h"
 
 namespace exl3 {
@@ -851,6 +851,7 @@ __global__ __launch_bounds__(256) void moe_prefill_rotate_kernel(const __half* x
 
 struct PrefillLayout {
     int chunk_tokens, entries, mt, max_tiles;
+    bool tall;
     size_t counts_off, pos_off, rows_off, tiles_off, xr_off, g_off, h_off, y_off, total;
 };
 
@@ -862,7 +863,8 @@ PrefillLayout prefill_layout(int tokens, int topk, int E, int hidden, int inter)
     // 64-row tiles: the 128-row variant holds 67 KB of LDS, so only two
     // workgroups share a CU, and measured slower per row (config 4, 2048
     // tokens: 311 us per grouped GEMM launch against 2 x 120 us at 64 rows)
-    L.mt = 64;
+    L.mt = env_int("EXL3_MOE_PREFILL_MT", 64);
+    L.tall = L.mt > 64;
     L.max_tiles = (E < L.entries ? E : L.entries) + L.entries / L.mt;
     size_t o = kWsScratchOffset;
     L.counts_off = o;
@@ -936,6 +938,10 @@ int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const
         if (rc) return rc;
         FatParams p{};
         p.M = L.max_tiles * L.mt;  // grid.y = max_tiles; rows come from the tiles
+        p.out_vec = 1;             // the scratch rows are
+        auto pass = [&](int K) {
+            return L.tall ? tall_launch(K, cb, L.mt, p, L.max_tiles, 1, st) : fat_launch(K, cb, L.mt, p, 1, st);
+        };
         p.tiles = tiles;
         p.ntiles = counts;
         for (int j = 0; j < 9; ++j) p.tabs[j] = tb.t[j];
@@ -948,13 +954,13 @@ int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const
         p.k = hidden;
         p.n = inter;
         p.ksteps = hidden / 64;
-        rc = fat_launch(KG, cb, L.mt, p, 1, st);
+        rc = pass(KG);
         if (rc) return rc;
         // up, with the SwiGLU and the down projection's input rotation
         p.gmode = 2;
         p.a = xr + (size_t)entries * hidden;
         p.out16 = h;
-        rc = fat_launch(KU, cb, L.mt, p, 1, st);
+        rc = pass(KU);
         if (rc) return rc;
         // down, by (token, slot) entry
         p.gmode = 3;
@@ -963,7 +969,7 @@ int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const
         p.n = hidden;
         p.ksteps = inter / 64;
         p.out16 = y;
-        rc = fat_launch(KD, cb, L.mt, p, 1, st);
+        rc = pass(KD);
         if (rc) return rc;
         moe_combine_kernel<<<dim3((hidden / 2 + 255) / 256, T), 256, 0, st>>>(
             y, idc, reinterpret_cast<const char*>(weights) + (size_t)t0 * topk * wsz, weights_f16, topk, E, hidden,

@@ -8,7 +8,7 @@ import torch
 
 import oracle
 from gpu_util import check_close, make_weight, make_x
-from sglang_exl3 import ops
+from sglang_exl3 import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -245,6 +245,37 @@ def test_mul1_raw_entries(op, m, monkeypatch):
     dec = run()
     torch.cuda.synchronize()
     check_close(raw.float().cpu().numpy(), dec.float().cpu().numpy(), f"raw vs decoded {op} m={m}")
+
+
+@pytest.mark.parametrize("mt", [128, 256])
+@pytest.mark.parametrize("m,k,n,K,cb,splits", [
+    (1, 128, 128, 4, 1, 1), (17, 256, 384, 1, 2, 2), (31, 512, 128, 2, 0, 4), (33, 1024, 256, 3, 2, 8),
+    (64, 2048, 128, 4, 1, 16), (65, 256, 128, 5, 1, 1), (128, 512, 256, 6, 2, 2), (129, 384, 128, 7, 0, 1),
+    (255, 1024, 128, 8, 1, 8), (256, 256, 384, 3, 1, 1), (257, 512, 128, 4, 2, 4), (700, 256, 128, 3, 0, 2)])
+def test_tall_tiles(m, k, n, K, cb, splits, mt, monkeypatch):
+    """Tall tiles of both heights at the edges of their 32-row groups and tiles, every K and codebook, with and
+    without the finish launch: against the oracle, twice (nothing is left behind in the scratch), and an output
+    that is only 4-byte aligned."""
+    print(f"case: tall tiles mt={mt} m={m} k={k} n={n} K={K} cb={cb} splits={splits}", flush=True)
+    monkeypatch.setenv("EXL3_FAT_TALL", str(mt))
+    monkeypatch.setenv("EXL3_FAT_SPLITS", str(splits))
+    monkeypatch.setenv("EXL3_GEMM_GEMV_ROWS", "0")
+    tr, su, sv = make_weight(k, n, K, seed=m + K)
+    x = make_x(m, k, seed=m)
+    d = [torch.from_numpy(v).cuda() for v in (tr, su, sv)]
+    xd = torch.from_numpy(x).cuda()
+    y = torch.ops.sglang_exl3.exl3_linear(xd, *d, K, cb)
+    assert torch.equal(y, torch.ops.sglang_exl3.exl3_linear(xd, *d, K, cb))
+    ref = oracle.matmul(x, oracle.dequant(tr, su, sv, K, cb, rtz=True))
+    check_close(y.float().cpu().numpy(), ref, f"tall m={m}")
+    lib = _lib.lib()
+    need = lib.exl3_gemm_workspace_size(m, k, n, K)
+    ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
+    odd = torch.zeros(m * n + 2, dtype=torch.float16, device="cuda")
+    rc = lib.exl3_gemm(xd.data_ptr(), *[t.data_ptr() for t in d], odd.data_ptr() + 4, m, k, n, K, cb, ws.data_ptr(),
+                       need, int(torch.cuda.current_stream().cuda_stream))
+    _lib.check(rc, "exl3_gemm")
+    assert torch.equal(odd[2:].view(m, n), y)
 
 
 @pytest.mark.parametrize("m,cb", [(16, 1), (64, 2)])
