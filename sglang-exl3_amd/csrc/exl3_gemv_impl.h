@@ -665,11 +665,44 @@ __global__ __launch_bounds__(GV_MAX_THREADS) void gemv_kernel(GemvParams p) {
     }
 }
 
+// One 128-value chunk of an input row on 8 lanes, 16 consecutive values each
+// (lane & 7): o = fp16( H(x (.) suh) / sqrt(128) ), x and suh at this lane's
+// values, only 4-byte aligned by contract (dword-aligned 16-byte loads).
+typedef uint32_t u32x4_a4_t __attribute__((ext_vector_type(4), aligned(4)));
+struct RowChunk {
+    u32x4_t v[2];
+};
+__device__ __forceinline__ RowChunk ld_chunk(const EXL3_GLOBAL __half* p) {
+    const EXL3_GLOBAL u32x4_a4_t* q = reinterpret_cast<const EXL3_GLOBAL u32x4_a4_t*>(p);
+    return RowChunk{{q[0], q[1]}};
+}
+__device__ __forceinline__ RowChunk rotate_chunk(const RowChunk& x, const RowChunk& suh, int x_bf16, int lane) {
+    float v[16];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const uint32_t xu = x.v[e >> 2][e & 3], su = suh.v[e >> 2][e & 3];
+        const __half2 pr = __hmul2(x_h2(*reinterpret_cast<const __half2*>(&xu), x_bf16), *reinterpret_cast<const __half2*>(&su));
+        v[2 * e] = __low2float(pr);
+        v[2 * e + 1] = __high2float(pr);
+    }
+    fwht128_x16(v, lane);
+    const float hn = fwht_x16_norm(lane);
+    RowChunk o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const __half2 h = h2_rn(v[2 * e] * hn, v[2 * e + 1] * hn);
+        o.v[e >> 2][e & 3] = *reinterpret_cast<const uint32_t*>(&h);
+    }
+    return o;
+}
+
 namespace {
-// Input rotation of a row batch: xr = fp16( H(x (.) suh) / sqrt(128) ), one
-// wave per 128-wide chunk (feeds the k-split GEMV's pre-rotated mode and the
-// MFMA GEMM).  blockIdx.y: the matrix whose suh applies; its rotated rows
-// follow those of the matrix before.
+// Input rotation of a row batch: xr = fp16( H(x (.) suh) / sqrt(128) ) (feeds the
+// k-split GEMV's pre-rotated mode and the MFMA GEMM).  A wave takes 8 chunks of
+// 128 values, 8 lanes and 32 bytes a lane each (rotate_chunk); one chunk per
+// wave, 4 bytes a lane, was bound by its instruction count: 1000 x 14336 bf16
+// 19 -> 10.7 us (57 MB).  blockIdx.y: the matrix whose suh applies; its rotated rows follow those of
+// the matrix before.
 // rs (optional): the sum of each chunk's 128 rotated fp16 values, [row][k/128]
 // per matrix (the mul1 raw-entry GEMM's affine correction).
 struct RotateSuh {
@@ -677,26 +710,35 @@ struct RotateSuh {
 };
 __global__ __launch_bounds__(256) void rotate_rows_kernel(const __half* x, RotateSuh suhs, __half* xr,
                                                           long long chunks, int k, int x_bf16, float* rs) {
-    const long long chunk = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (chunk >= chunks) return;
-    const __half* suh = suhs.suh[blockIdx.y];
-    const int lane = threadIdx.x & 63, per_row = k >> 7;
-    const long long row = chunk / per_row;
-    const int c = (int)(chunk - row * per_row) * 128 + 2 * lane;
-    const __half2 pr = __hmul2(x_h2(ld_h2(gptr(x) + (size_t)row * k + c), x_bf16), ld_h2(gptr(suh) + c));
-    float a = __low2float(pr), b = __high2float(pr);
-    fwht128_pair_fast(a, b, lane);
-    const __half2 o = h2_rn(a * kHadNorm, b * kHadNorm);
-    st_h2(gptr(xr) + ((size_t)blockIdx.y * chunks + chunk) * 128 + 2 * lane, o);
+    const int lane = threadIdx.x & 63;
+    const long long chunk = ((long long)blockIdx.x * 4 + (threadIdx.x >> 6)) * 8 + (lane >> 3);
+    const long long cc = chunk < chunks ? chunk : chunks - 1;  // whole waves stay active for the lane exchanges
+    const int c = (int)((unsigned)cc % (unsigned)(k >> 7)) * 128 + (lane & 7) * 16;
+    const RowChunk o = rotate_chunk(ld_chunk(gptr(x) + cc * 128 + (lane & 7) * 16),
+                                    ld_chunk(gptr(suhs.suh[blockIdx.y]) + c), x_bf16, lane);
+    float t = 0.f;
     if (rs) {
-        const float t = wave_sum(__low2float(o) + __high2float(o));
-        if (lane == 0) gptr(rs)[(size_t)blockIdx.y * chunks + chunk] = t;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t u = o.v[e >> 2][e & 3];
+            const __half2 h = *reinterpret_cast<const __half2*>(&u);
+            t += __low2float(h) + __high2float(h);
+        }
+        t += lane_xor<1>(t);
+        t += lane_xor<2>(t);
+        t += lane_xor<4>(t);
     }
+    if (chunk >= chunks) return;
+    EXL3_GLOBAL u32x4_t* dst = reinterpret_cast<EXL3_GLOBAL u32x4_t*>(
+        gptr(xr) + ((size_t)blockIdx.y * chunks + chunk) * 128 + (lane & 7) * 16);
+    dst[0] = o.v[0];
+    dst[1] = o.v[1];
+    if (rs && (lane & 7) == 0) gptr(rs)[(size_t)blockIdx.y * chunks + chunk] = t;
 }
 inline int rotate_rows(const __half* x, const RotateSuh& suhs, int mats, __half* xr, int m, int k, int x_bf16,
                        float* rs, hipStream_t st, const char* what) {
     const long long chunks = (long long)m * (k / 128);
-    rotate_rows_kernel<<<dim3((unsigned)((chunks + 3) / 4), mats), 256, 0, st>>>(x, suhs, xr, chunks, k, x_bf16, rs);
+    rotate_rows_kernel<<<dim3((unsigned)((chunks + 31) / 32), mats), 256, 0, st>>>(x, suhs, xr, chunks, k, x_bf16, rs);
     return launch_status(what);
 }
 }  // namespace
