@@ -14,31 +14,52 @@ int fat_launch_K6(int, int, const FatParams&, int, hipStream_t);
 int fat_launch_K7(int, int, const FatParams&, int, hipStream_t);
 int fat_launch_K8(int, int, const FatParams&, int, hipStream_t);
 
-int tall_launch_K1(int, int, const FatParams&, int, int, hipStream_t);
-int tall_launch_K2(int, int, const FatParams&, int, int, hipStream_t);
-int tall_launch_K3(int, int, const FatParams&, int, int, hipStream_t);
-int tall_launch_K4(int, int, const FatParams&, int, int, hipStream_t);
-int tall_launch_K5(int, int, const FatParams&, int, int, hipStream_t);
-int tall_launch_K6(int, int, const FatParams&, int, int, hipStream_t);
-int tall_launch_K7(int, int, const FatParams&, int, int, hipStream_t);
-int tall_launch_K8(int, int, const FatParams&, int, int, hipStream_t);
+int tall_launch_K1(int, int, const FatParams&, int, int, bool, hipStream_t);
+int tall_launch_K2(int, int, const FatParams&, int, int, bool, hipStream_t);
+int tall_launch_K3(int, int, const FatParams&, int, int, bool, hipStream_t);
+int tall_launch_K4(int, int, const FatParams&, int, int, bool, hipStream_t);
+int tall_launch_K5(int, int, const FatParams&, int, int, bool, hipStream_t);
+int tall_launch_K6(int, int, const FatParams&, int, int, bool, hipStream_t);
+int tall_launch_K7(int, int, const FatParams&, int, int, bool, hipStream_t);
+int tall_launch_K8(int, int, const FatParams&, int, int, bool, hipStream_t);
 
-int tall_launch(int K, int cb, int mt, const FatParams& p, int row_tiles, int splits, hipStream_t st) {
+// What the kernels read through without a check of their own.
+int check_fat_params(const FatParams& p, const char* what) {
+    bool tabs = true;
+    for (int j = 0; j < 9; ++j) tabs = tabs && p.tabs[j];
+    if (!p.a || (p.gmode ? !(p.tiles && p.ntiles && tabs) : !(p.trellis && p.svh)) ||
+        (p.gu && !(p.trellis2 && p.svh2)) || (p.gmode == 3 && !p.rows_map) || (p.split_out && !p.partials) ||
+        p.ksteps < 1) {
+        set_error("%s: incomplete launch parameters", what);
+        return EXL3_ERR_ARG;
+    }
+    return EXL3_OK;
+}
+
+int tall_launch(int K, int cb, int mt, const FatParams& p, int row_tiles, int splits, bool gu_fused, hipStream_t st) {
+    const int rc = check_fat_params(p, "exl3 gemm (tall tiles)");
+    if (rc) return rc;
+    if (p.ksteps % 2) {
+        set_error("exl3 gemm (tall tiles): %d steps per split", p.ksteps);
+        return EXL3_ERR_ARG;
+    }
     switch (K) {
-        case 1: return tall_launch_K1(cb, mt, p, row_tiles, splits, st);
-        case 2: return tall_launch_K2(cb, mt, p, row_tiles, splits, st);
-        case 3: return tall_launch_K3(cb, mt, p, row_tiles, splits, st);
-        case 4: return tall_launch_K4(cb, mt, p, row_tiles, splits, st);
-        case 5: return tall_launch_K5(cb, mt, p, row_tiles, splits, st);
-        case 6: return tall_launch_K6(cb, mt, p, row_tiles, splits, st);
-        case 7: return tall_launch_K7(cb, mt, p, row_tiles, splits, st);
-        case 8: return tall_launch_K8(cb, mt, p, row_tiles, splits, st);
+        case 1: return tall_launch_K1(cb, mt, p, row_tiles, splits, gu_fused, st);
+        case 2: return tall_launch_K2(cb, mt, p, row_tiles, splits, gu_fused, st);
+        case 3: return tall_launch_K3(cb, mt, p, row_tiles, splits, gu_fused, st);
+        case 4: return tall_launch_K4(cb, mt, p, row_tiles, splits, gu_fused, st);
+        case 5: return tall_launch_K5(cb, mt, p, row_tiles, splits, gu_fused, st);
+        case 6: return tall_launch_K6(cb, mt, p, row_tiles, splits, gu_fused, st);
+        case 7: return tall_launch_K7(cb, mt, p, row_tiles, splits, gu_fused, st);
+        case 8: return tall_launch_K8(cb, mt, p, row_tiles, splits, gu_fused, st);
     }
     set_error("exl3 gemm: K=%d outside 1..8", K);
     return EXL3_ERR_UNSUPPORTED;
 }
 
 int fat_launch(int K, int cb, int mt, const FatParams& p, int splits, hipStream_t st) {
+    const int rc = check_fat_params(p, "exl3 fat gemm");
+    if (rc) return rc;
     switch (K) {
         case 1: return fat_launch_K1(cb, mt, p, splits, st);
         case 2: return fat_launch_K2(cb, mt, p, splits, st);
@@ -379,7 +400,7 @@ int run_fat(const uint16_t* a, const int16_t* trellis, float* out32, __half* out
     if (pl.tall) {
         p.split_out = pl.splits > 1;
         p.out_vec = aligned(out16, 16);
-        const int rc = tall_launch(K, cb, pl.mt, p, (M + pl.mt - 1) / pl.mt, pl.splits, st);
+        const int rc = tall_launch(K, cb, pl.mt, p, (M + pl.mt - 1) / pl.mt, pl.splits, false, st);
         if (rc || pl.splits == 1) return rc;
         return fat_split_finish(p, pl.splits, st, "exl3 gemm finish launch");
     }

@@ -127,7 +127,9 @@ struct FatParams {
     // for each matrix in turn, and a column block's matrix comes from mats.
     MatSet mats;
     int y_bf16;  // out16 is bfloat16 (plain modes)
+    int tail_parts;  // tall dense gate/up: workgroups per tail tile
     int out_vec;  // tall tiles: out16 rows are 16-byte aligned
+    int up_rows;  // tall grouped gate/up: rows between the gate's and the up projection's rotated rows in a
 };
 
 // Sum over chunks [c0, c0 + nc) of row `row` of rowsum (one wave).

@@ -225,14 +225,19 @@ __global__ __launch_bounds__(MOE_ROUTE_THREADS) void moe_route_rotate_kernel(
 // ------------------------------------------------------------------ combine
 
 // out[t][c] = fp16( sum_slot w[t][slot] * y[t*topk + slot][c] ), valid slots
-// only, fp32 accumulation in slot order.
+// only, fp32 accumulation in slot order.  8 columns (16 bytes of y) a thread
+// where the caller's rows allow 16-byte stores, else 2; y is workspace.
+template <int V>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const __half* y, const int32_t* ids, const void* weights,
                                                           int weights_f16, int topk, int E, int hidden,
                                                           __half* out, int y_bf16) {
     const int t = blockIdx.y;
-    const int c = (blockIdx.x * 256 + threadIdx.x) * 2;
+    const int c = (blockIdx.x * 256 + threadIdx.x) * V;
     if (c >= hidden) return;
-    float a0 = 0.f, a1 = 0.f;
+    float a[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) a[v] = 0.f;
+#pragma unroll 4
     for (int s = 0; s < topk; ++s) {
         const int ent = t * topk + s;
         const int id = gptr(ids)[ent];
@@ -240,11 +245,37 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const __half* y, const
         const float wv = weights_f16
                              ? __half2float(__ushort_as_half(gptr(reinterpret_cast<const uint16_t*>(weights))[ent]))
                              : gptr(reinterpret_cast<const float*>(weights))[ent];
-        const __half2 v = ld_h2(gptr(y) + (size_t)ent * hidden + c);
-        a0 += wv * __low2float(v);
-        a1 += wv * __high2float(v);
+        uint32_t u[V / 2];
+        if constexpr (V == 8) {
+            const u32x4_t q = *reinterpret_cast<const EXL3_GLOBAL u32x4_t*>(gptr(y) + (size_t)ent * hidden + c);
+            u[0] = q.x; u[1] = q.y; u[2] = q.z; u[3] = q.w;
+        } else {
+            u[0] = *reinterpret_cast<const EXL3_GLOBAL uint32_t*>(gptr(y) + (size_t)ent * hidden + c);
+        }
+#pragma unroll
+        for (int v = 0; v < V / 2; ++v) {
+            const __half2 h = *reinterpret_cast<const __half2*>(&u[v]);
+            a[2 * v] += wv * __low2float(h);
+            a[2 * v + 1] += wv * __high2float(h);
+        }
     }
-    st_y2(gptr(out) + (size_t)t * hidden + c, h2_rn(a0, a1), y_bf16);
+    uint32_t o[V / 2];
+#pragma unroll
+    for (int v = 0; v < V / 2; ++v) o[v] = y_bits(h2_rn(a[2 * v], a[2 * v + 1]), y_bf16);
+    EXL3_GLOBAL uint32_t* dst = reinterpret_cast<EXL3_GLOBAL uint32_t*>(gptr(out) + (size_t)t * hidden + c);
+    if constexpr (V == 8) *reinterpret_cast<EXL3_GLOBAL u32x4_t*>(dst) = u32x4_t{o[0], o[1], o[2], o[3]};
+    else dst[0] = o[0];
+}
+
+static int moe_combine(const __half* y, const int32_t* ids, const void* weights, int weights_f16, int topk, int E,
+                       int hidden, __half* out, int tokens, int y_bf16, hipStream_t st, const char* what) {
+    if (aligned(out, 16))
+        moe_combine_kernel<8><<<dim3((hidden / 8 + 255) / 256, tokens), 256, 0, st>>>(y, ids, weights, weights_f16, topk,
+                                                                                     E, hidden, out, y_bf16);
+    else
+        moe_combine_kernel<2><<<dim3((hidden / 2 + 255) / 256, tokens), 256, 0, st>>>(y, ids, weights, weights_f16, topk,
+                                                                                     E, hidden, out, y_bf16);
+    return launch_status(what);
 }
 
 static int env_int_once(const char* name) {
@@ -725,9 +756,8 @@ int run_moe_decode(const char* fn, const uint16_t* x, const int32_t* ids, const 
     if (L.fc) return EXL3_OK;
 
     // 5. weighted combine
-    moe_combine_kernel<<<dim3((hidden / 2 + 255) / 256, tokens), 256, 0, st>>>(
-        yslots, ids, weights, weights_f16, topk, E, hidden, reinterpret_cast<__half*>(out), bf16);
-    return launch_status("exl3 moe combine launch");
+    return moe_combine(yslots, ids, weights, weights_f16, topk, E, hidden, reinterpret_cast<__half*>(out), tokens, bf16,
+                       st, "exl3 moe combine launch");
 }
 
 // ------------------------------------------------------------ prefill path
@@ -735,15 +765,16 @@ int run_moe_decode(const char* fn, const uint16_t* x, const int32_t* ids, const 
 // For batches whose experts get many rows each, the 16-row work units of the
 // decode path decode every expert's weights once per 16 rows with the
 // pair-form GEMV.  The prefill path groups the rows of each expert into tiles
-// of up to 64 / 128 rows and runs the MFMA GEMM kernel (real-valued B
+// of up to 128 (or 64) rows and runs the MFMA GEMM kernel (real-valued B
 // fragments, decode once per tile) in its grouped mode:
 //   route    one workgroup: counting sort of the (token, slot) entries by
 //            expert -> compact row -> entry map, row tiles (expert, first row,
 //            rows), the tile count
 //   rotate   xr[p][crow] = fp16(H(x[token] (.) suh_p[e]) / sqrt(128)) for the
-//            gate and up projections, one wave per (row, projection, block)
-//   gate     g32[crow] = fp32 gate output
-//   up       h[crow] = fp16 silu(min(g, L)) * clamp(u, -L, L), rotated with the
+//            gate and up projections, one wave per (row, projection)
+//   gate/up  of one bit width: 128-row tall tiles, both in one workgroup;
+//            otherwise 64-row tiles, the gate's fp32 output in g32, then up
+//            h[crow] = fp16 silu(min(g, L)) * clamp(u, -L, L), rotated with the
 //            down projection's suh
 //   down     y[entry] = fp16 down output
 //   combine  out[t] = sum over the token's valid slots of w * y, fp32, slot order
@@ -755,30 +786,49 @@ int run_moe_decode(const char* fn, const uint16_t* x, const int32_t* ids, const 
 // 1234-1344).
 constexpr int kMoePrefillChunk = 16384;  // (token, slot) entries per pipeline pass
 
+// Routing of one chunk, in one workgroup: every thread keeps its up to
+// kRouteEntries entries' experts and ranks in registers (one round trip for the
+// ids, LDS counters, no pass over memory in between: 16384 entries 21.1 -> 10.2 us).
+// Tiles are listed by rows, full ones first, then the partial ones from many
+// rows to few, so the last round of the GEMM grids is made of cheap tiles.
+constexpr int kRouteEntries = kMoePrefillChunk / MOE_ROUTE_THREADS;
+constexpr int kRouteGroup = 16;  // rows by which partial tiles are told apart
+
 __global__ __launch_bounds__(MOE_ROUTE_THREADS) void moe_prefill_route_kernel(const int32_t* ids, int entries,
-                                                                             int E, int mt, int* pos, int* rows,
+                                                                             int E, int mt, int* rows,
                                                                              FatTile* tiles, int* counts) {
     extern __shared__ __align__(16) int prs[];
     int* cnt = prs;       // [E]
     int* off = cnt + E;   // [E] first compact row
-    int* toff = off + E;  // [E] first tile
+    int* toff = off + E;  // [E] first full tile
+    __shared__ int group[16], gstart[16];  // partial tiles by ceil(rows / kRouteGroup) (mt <= 256)
     const int tid = threadIdx.x;
-    for (int e = tid; e < E; e += MOE_ROUTE_THREADS) cnt[e] = 0;
-    __syncthreads();
     const EXL3_GLOBAL int32_t* idg = gptr(ids);
-    EXL3_GLOBAL int* posg = gptr(pos);
-    for (int i = tid; i < entries; i += MOE_ROUTE_THREADS) {
-        const int e = idg[i];
-        posg[i] = (e >= 0 && e < E) ? atomicAdd(&cnt[e], 1) : -1;
+    int eid[kRouteEntries], pos[kRouteEntries];
+#pragma unroll
+    for (int j = 0; j < kRouteEntries; ++j) {
+        const int i = tid + j * MOE_ROUTE_THREADS;
+        const int e = i < entries ? idg[i] : -1;
+        eid[j] = e >= 0 && e < E ? e : -1;
+    }
+    for (int e = tid; e < E; e += MOE_ROUTE_THREADS) cnt[e] = 0;
+    if (tid < 16) group[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kRouteEntries; ++j) pos[j] = eid[j] >= 0 ? atomicAdd(&cnt[eid[j]], 1) : 0;
+    __syncthreads();
+    for (int e = tid; e < E; e += MOE_ROUTE_THREADS) {
+        const int r = cnt[e] % mt;
+        if (r) atomicAdd(&group[(r - 1) / kRouteGroup], 1);
     }
     __syncthreads();
-    if (tid < 64) {  // exclusive scans of rows and tiles over the experts, one wave
+    if (tid < 64) {  // exclusive scans of rows and full tiles over the experts, one wave
         const int chunk = (E + 63) / 64;
         const int e0 = tid * chunk, e1 = min(E, e0 + chunk);
         int sr = 0, st = 0;
         for (int e = e0; e < e1; ++e) {
             sr += cnt[e];
-            st += (cnt[e] + mt - 1) / mt;
+            st += cnt[e] / mt;
         }
         int ir = sr, it = st;
 #pragma unroll
@@ -794,18 +844,22 @@ __global__ __launch_bounds__(MOE_ROUTE_THREADS) void moe_prefill_route_kernel(co
             off[e] = r;
             toff[e] = t;
             r += cnt[e];
-            t += (cnt[e] + mt - 1) / mt;
+            t += cnt[e] / mt;
         }
         if (tid == 63) {
-            gptr(counts)[0] = it;  // row tiles
-            gptr(counts)[1] = ir;  // routed rows
+            int start = it;
+            for (int q = 15; q >= 0; --q) {
+                gstart[q] = start;
+                start += group[q];
+            }
+            gptr(counts)[0] = start;  // row tiles
+            gptr(counts)[1] = ir;     // routed rows
         }
     }
     __syncthreads();
-    for (int i = tid; i < entries; i += MOE_ROUTE_THREADS) {  // the same i as above: own pos[] write
-        const int ps = posg[i];
-        if (ps >= 0) gptr(rows)[off[idg[i]] + ps] = i;
-    }
+#pragma unroll
+    for (int j = 0; j < kRouteEntries; ++j)
+        if (eid[j] >= 0) gptr(rows)[off[eid[j]] + pos[j]] = tid + j * MOE_ROUTE_THREADS;
     for (int e = tid; e < E; e += MOE_ROUTE_THREADS) {
         const int c = cnt[e];
         for (int t = 0; t * mt < c; ++t) {
@@ -814,14 +868,16 @@ __global__ __launch_bounds__(MOE_ROUTE_THREADS) void moe_prefill_route_kernel(co
             tl.crow0 = off[e] + t * mt;
             tl.nrows = min(mt, c - t * mt);
             tl.pad = 0;
-            *reinterpret_cast<EXL3_GLOBAL u32x4_t*>(gptr(tiles) + toff[e] + t) = *reinterpret_cast<const u32x4_t*>(&tl);
+            const int slot = tl.nrows == mt ? toff[e] + t : atomicAdd(&gstart[(tl.nrows - 1) / kRouteGroup], 1);
+            *reinterpret_cast<EXL3_GLOBAL u32x4_t*>(gptr(tiles) + slot) = *reinterpret_cast<const u32x4_t*>(&tl);
         }
     }
 }
 
 // xr[p][crow][k] = fp16(FWHT(x[token][k] (.) suh_p[e][k]) / sqrt(128)), p = 0 gate, 1 up; one wave per
-// (compact row, projection) walking the row's 128-wide blocks (the loads of the next block are issued
-// before the current block's transform); rows past the routed count exit.
+// (compact row, projection), 8 of the row's 128-wide blocks at a time, 32 bytes a lane (rotate_chunk); rows
+// past the routed count exit.  2048 tokens x 8 slots, hidden 2048 (134 MB written): one chunk
+// per wave and 4 bytes a lane 58.0 us, now 36.3.
 __global__ __launch_bounds__(256) void moe_prefill_rotate_kernel(const __half* x, int x_bf16, const int32_t* ids, const int* rows,
                                                                 const int* counts, const int64_t* suh_g,
                                                                 const int64_t* suh_u, int topk, int hidden,
@@ -833,26 +889,23 @@ __global__ __launch_bounds__(256) void moe_prefill_rotate_kernel(const __half* x
     if (crow >= gptr(counts)[1]) return;
     const int entry = gptr(rows)[crow];
     const int e = gptr(ids)[entry];
-    const EXL3_GLOBAL __half* suh = gptr(reinterpret_cast<const __half*>(gptr(proj ? suh_u : suh_g)[e])) + 2 * lane;
-    const EXL3_GLOBAL __half* xs = gptr(x) + (size_t)(entry / topk) * hidden + 2 * lane;
-    EXL3_GLOBAL __half* dst = gptr(xr) + ((size_t)proj * entries + crow) * hidden + 2 * lane;
-    __half2 xv = ld_h2(xs), sv = ld_h2(suh);
-    for (int j = 0; j < nblk; ++j) {
-        const __half2 pr = __hmul2(x_h2(xv, x_bf16), sv);
-        if (j + 1 < nblk) {
-            xv = ld_h2(xs + (j + 1) * 128);
-            sv = ld_h2(suh + (j + 1) * 128);
+    const int c0 = (lane & 7) * 16;
+    const EXL3_GLOBAL __half* suh = gptr(reinterpret_cast<const __half*>(gptr(proj ? suh_u : suh_g)[e])) + c0;
+    const EXL3_GLOBAL __half* xs = gptr(x) + (size_t)(entry / topk) * hidden + c0;
+    EXL3_GLOBAL __half* dst = gptr(xr) + ((size_t)proj * entries + crow) * hidden + c0;
+    for (int j0 = 0; j0 < nblk; j0 += 8) {
+        const int j = j0 + (lane >> 3), jc = min(j, nblk - 1) * 128;  // whole waves stay active
+        const RowChunk o = rotate_chunk(ld_chunk(xs + jc), ld_chunk(suh + jc), x_bf16, lane);
+        if (j < nblk) {
+            reinterpret_cast<EXL3_GLOBAL u32x4_t*>(dst + j * 128)[0] = o.v[0];
+            reinterpret_cast<EXL3_GLOBAL u32x4_t*>(dst + j * 128)[1] = o.v[1];
         }
-        float a = __low2float(pr), c = __high2float(pr);
-        fwht128_pair_fast(a, c, lane);
-        st_h2(dst + j * 128, h2_rn(a * kHadNorm, c * kHadNorm));
     }
 }
 
 struct PrefillLayout {
-    int chunk_tokens, entries, mt, max_tiles;
-    bool tall;
-    size_t counts_off, pos_off, rows_off, tiles_off, xr_off, g_off, h_off, y_off, total;
+    int chunk_tokens, entries, max_tiles;
+    size_t counts_off, rows_off, tiles_off, xr_off, g_off, h_off, y_off, total;
 };
 
 PrefillLayout prefill_layout(int tokens, int topk, int E, int hidden, int inter) {
@@ -860,17 +913,10 @@ PrefillLayout prefill_layout(int tokens, int topk, int E, int hidden, int inter)
     L.chunk_tokens = kMoePrefillChunk / topk < 1 ? 1 : kMoePrefillChunk / topk;
     if (L.chunk_tokens > tokens) L.chunk_tokens = tokens;
     L.entries = L.chunk_tokens * topk;
-    // 64-row tiles: the 128-row variant holds 67 KB of LDS, so only two
-    // workgroups share a CU, and measured slower per row (config 4, 2048
-    // tokens: 311 us per grouped GEMM launch against 2 x 120 us at 64 rows)
-    L.mt = env_int("EXL3_MOE_PREFILL_MT", 64);
-    L.tall = L.mt > 64;
-    L.max_tiles = (E < L.entries ? E : L.entries) + L.entries / L.mt;
+    L.max_tiles = (E < L.entries ? E : L.entries) + L.entries / 64;  // enough for either tile height
     size_t o = kWsScratchOffset;
     L.counts_off = o;
     o = align256(o + 4 * sizeof(int));
-    L.pos_off = o;
-    o = align256(o + (size_t)L.entries * sizeof(int));
     L.rows_off = o;
     o = align256(o + (size_t)L.entries * sizeof(int));
     L.tiles_off = o;
@@ -889,18 +935,33 @@ PrefillLayout prefill_layout(int tokens, int topk, int E, int hidden, int inter)
 
 // Rows per active expert (uniform routing estimate) from which a batch takes
 // the prefill path; every batch above the decode path's entry limit does.
-// Graph-timed on config 4 (decode path -> prefill path): B = 64 / 128: 92 /
-// 151 us -> 135 / 158 us; B = 256 / 512 / 1024: 243 / 398 / 772 us -> 217 /
-// 298 / 437 us.
+// 64-row tiles pay from 16 rows; 128-row tiles (gate and up of one bit width) from
+// 5, if the active experts' projections are at least 2^25 weights each, below
+// which the path's five launches (~30 us) cost more than its tiles save.
+// Graph-timed, us, 64-row tiles / 128-row tiles / decode path: config 4 (skewed
+// router, 201M weights), 64 tokens (4 rows) 122 / 82 / 83, 96 (6 rows) 123 / 87 / 106,
+// 128 128 / 95 / 126, 256 144 / 108 / 204, 512 182 / 157 / 358; 16 experts, hidden 2048,
+// inter 1408, top 2, K = 4 (46M): 48 tokens (6 rows) 75 / 54 / 68, 100 90 / 56 / 78, 200
+// 108 / 64 / 119.  128-row tiles / decode path: 64 experts, 2048 x 1408 (184M), 6
+// rows: 103 / 152; 8 experts, 4096 x 14336 (470M), 6 rows: 273 / 310; 60 experts, 1024 x
+// 512 (31M), 5.3 rows: 40 / 39; 16 experts, 1024 x 1024 (16M), 6 rows: 39 / 28; 8 experts,
+// 1024 x 512 (4M), 8 rows: 33 / 25.
 constexpr double kMoePrefillRowsPerExpert = 16.0;
+constexpr double kMoeTallRowsPerExpert = 5.0, kMoeTallMinWeights = 33554432.0;
 
-bool moe_use_prefill(int tokens, int topk, int E) {
+// Env EXL3_MOE_TALL=0: the 64-row tiles always.
+bool moe_use_tall(int KG, int KU) { return KG == KU && env_int("EXL3_MOE_TALL", 1) != 0; }
+
+bool moe_use_prefill(int tokens, int topk, int E, int hidden, int inter, bool tall) {
     const int forced = env_int("EXL3_MOE_PREFILL", -1);  // 0: never (decode path), 1: always
     const long long entries = (long long)tokens * topk;
     if (entries > kMoeMaxEntries) return true;
     if (forced >= 0) return forced != 0;
     const double act = expected_active(tokens, topk, E);
-    return act > 0 && (double)entries / act >= kMoePrefillRowsPerExpert;
+    if (act <= 0) return false;
+    const double per = (double)entries / act;
+    return per >= kMoePrefillRowsPerExpert ||
+           (tall && per >= kMoeTallRowsPerExpert && act * hidden * inter >= kMoeTallMinWeights);
 }
 
 int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const void* weights, int weights_f16,
@@ -911,7 +972,6 @@ int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const
                       fn, L.total, ws ? ws_bytes : (size_t)0);
     char* w8 = reinterpret_cast<char*>(ws);
     int* counts = reinterpret_cast<int*>(w8 + L.counts_off);
-    int* pos = reinterpret_cast<int*>(w8 + L.pos_off);
     int* rows = reinterpret_cast<int*>(w8 + L.rows_off);
     FatTile* tiles = reinterpret_cast<FatTile*>(w8 + L.tiles_off);
     __half* xr = reinterpret_cast<__half*>(w8 + L.xr_off);
@@ -922,12 +982,17 @@ int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const
     int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&moe_prefill_route_kernel), rsmem, "exl3 moe prefill route");
     if (rc) return rc;
     const size_t wsz = weights_f16 ? 2 : 4;
+    // 128-row tall tiles, gate and up in one workgroup, where the two share a
+    // bit width; else the 64-row tiles, gate and up in turn, with the gate's fp32
+    // rows through memory (config 4, 2048 tokens: gate/up 211 us and down 101,
+    // the layer 461 -> 343)
+    const bool tall = moe_use_tall(KG, KU);
+    const int mt = tall ? 128 : 64, row_tiles = (E < L.entries ? E : L.entries) + L.entries / mt;
     for (int t0 = 0; t0 < tokens; t0 += L.chunk_tokens) {
         const int T = tokens - t0 < L.chunk_tokens ? tokens - t0 : L.chunk_tokens;
         const int entries = T * topk;
         const int32_t* idc = ids + (size_t)t0 * topk;
-        moe_prefill_route_kernel<<<1, MOE_ROUTE_THREADS, rsmem, st>>>(idc, entries, E, L.mt, pos, rows, tiles,
-                                                                       counts);
+        moe_prefill_route_kernel<<<1, MOE_ROUTE_THREADS, rsmem, st>>>(idc, entries, E, mt, rows, tiles, counts);
         rc = launch_status("exl3 moe prefill route launch");
         if (rc) return rc;
         const long long jobs = (long long)entries * 2;
@@ -937,30 +1002,39 @@ int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const
         rc = launch_status("exl3 moe prefill rotate launch");
         if (rc) return rc;
         FatParams p{};
-        p.M = L.max_tiles * L.mt;  // grid.y = max_tiles; rows come from the tiles
+        p.M = row_tiles * mt;  // grid.y = row_tiles; rows come from the tiles
         p.out_vec = 1;             // the scratch rows are
-        auto pass = [&](int K) {
-            return L.tall ? tall_launch(K, cb, L.mt, p, L.max_tiles, 1, st) : fat_launch(K, cb, L.mt, p, 1, st);
-        };
         p.tiles = tiles;
         p.ntiles = counts;
         for (int j = 0; j < 9; ++j) p.tabs[j] = tb.t[j];
         p.g32 = g32;
         p.rows_map = rows;
         p.limit = limit;
-        // gate
-        p.gmode = 1;
-        p.a = xr;
-        p.k = hidden;
-        p.n = inter;
-        p.ksteps = hidden / 64;
-        rc = pass(KG);
-        if (rc) return rc;
-        // up, with the SwiGLU and the down projection's input rotation
-        p.gmode = 2;
-        p.a = xr + (size_t)entries * hidden;
-        p.out16 = h;
-        rc = pass(KU);
+        if (tall) {
+            // gate and up of a column block in one workgroup
+            p.gmode = 4;
+            p.a = xr;
+            p.up_rows = entries;
+            p.out16 = h;
+            p.k = hidden;
+            p.n = inter;
+            p.ksteps = hidden / 64;
+            rc = tall_launch(KG, cb, mt, p, row_tiles, 1, true, st);
+        } else {
+            // gate
+            p.gmode = 1;
+            p.a = xr;
+            p.k = hidden;
+            p.n = inter;
+            p.ksteps = hidden / 64;
+            rc = fat_launch(KG, cb, mt, p, 1, st);
+            if (rc) return rc;
+            // up, with the SwiGLU and the down projection's input rotation
+            p.gmode = 2;
+            p.a = xr + (size_t)entries * hidden;
+            p.out16 = h;
+            rc = fat_launch(KU, cb, mt, p, 1, st);
+        }
         if (rc) return rc;
         // down, by (token, slot) entry
         p.gmode = 3;
@@ -969,12 +1043,11 @@ int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const
         p.n = hidden;
         p.ksteps = inter / 64;
         p.out16 = y;
-        rc = pass(KD);
+        rc = tall ? tall_launch(KD, cb, mt, p, row_tiles, 1, false, st) : fat_launch(KD, cb, mt, p, 1, st);
         if (rc) return rc;
-        moe_combine_kernel<<<dim3((hidden / 2 + 255) / 256, T), 256, 0, st>>>(
-            y, idc, reinterpret_cast<const char*>(weights) + (size_t)t0 * topk * wsz, weights_f16, topk, E, hidden,
-            reinterpret_cast<__half*>(out) + (size_t)t0 * hidden, bf16);
-        rc = launch_status("exl3 moe prefill combine launch");
+        rc = moe_combine(y, idc, reinterpret_cast<const char*>(weights) + (size_t)t0 * topk * wsz, weights_f16, topk, E,
+                         hidden, reinterpret_cast<__half*>(out) + (size_t)t0 * hidden, T, bf16, st,
+                         "exl3 moe prefill combine launch");
         if (rc) return rc;
     }
     return EXL3_OK;
@@ -995,7 +1068,7 @@ int run_moe(const char* fn, const uint16_t* x, const int32_t* ids, const void* w
     for (int j = 0; j < 9; ++j) tabs_ok = tabs_ok && tb.t[j];
     EXL3_REQUIRE(x && ids && weights && out && tabs_ok, "%s: null pointer", fn);
     EXL3_REQUIRE(aligned(x, 4) && aligned(out, 4), "%s: misaligned x/out", fn);
-    if (moe_use_prefill(tokens, topk, E))
+    if (moe_use_prefill(tokens, topk, E, hidden, inter, moe_use_tall(KG, KU)))
         return run_moe_prefill(fn, x, ids, weights, weights_f16, tb, E, out, tokens, topk, hidden, inter, KG, KU, KD,
                                cb, limit, bf16, ws, ws_bytes, st);
     return run_moe_decode(fn, x, ids, weights, weights_f16, tb, E, out, tokens, topk, hidden, inter, KG, KU, KD, cb,
@@ -1009,8 +1082,15 @@ using namespace exl3;
 
 extern "C" size_t exl3_moe_workspace_size(int tokens, int topk, int num_experts, int hidden, int inter) {
     if (tokens < 1 || topk < 1 || num_experts < 1 || hidden < 128 || inter < 128) return 0;
-    if (moe_use_prefill(tokens, topk, num_experts)) return prefill_layout(tokens, topk, num_experts, hidden, inter).total;
-    return moe_layout(tokens, topk, num_experts, hidden, inter).total;
+    // room for either path where the bit widths decide (K is not known here)
+    size_t need = 0;
+    if (moe_use_prefill(tokens, topk, num_experts, hidden, inter, true))
+        need = prefill_layout(tokens, topk, num_experts, hidden, inter).total;
+    if (!moe_use_prefill(tokens, topk, num_experts, hidden, inter, false)) {
+        const size_t d = moe_layout(tokens, topk, num_experts, hidden, inter).total;
+        need = need > d ? need : d;
+    }
+    return need;
 }
 
 extern "C" int exl3_moe_plan(int tokens, int topk, int num_experts, int hidden, int inter, int* out) {

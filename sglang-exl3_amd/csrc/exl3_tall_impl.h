@@ -46,74 +46,39 @@ __device__ __forceinline__ void copy_to_lds16(const EXL3_GLOBAL char* base, uint
         : "memory");
 }
 
-template <int K, int CB, int MT, bool RAW>
-__global__ __launch_bounds__(TL_THREADS, MT == 256 ? 2 : (MT == 192 ? 3 : 4)) void tall_kernel(FatParams p) {
-    static_assert(!RAW || CB == 2, "raw entries: mul1");
+// The k loop of one wave: `rows` rows (up to MT) x the wave's 32 columns over
+// nsteps (even) 64-k steps.  tb: the wave's words of step 0; abase: row 0 of the
+// tile at the split's first k; lds: the byte offset of the two A buffers in
+// the workgroup's LDS, copied by SW waves, of which this is wave sw.
+template <int K, int CB, int MT, int SW, bool RAW>
+__device__ __forceinline__ void tall_loop(float4_t (&acc)[MT / 16][2], const EXL3_GLOBAL uint32_t* tb,
+                                          size_t step_stride, int nsteps, const EXL3_GLOBAL char* abase, int k,
+                                          int rows, unsigned char* smem, uint32_t lds, int sw, int lane) {
     constexpr int RB = MT / 16;
     constexpr int PF = MT == 128 ? 1 : 2;  // row blocks whose fragments are read ahead
-    extern __shared__ __align__(16) unsigned char fat_smem[];
-
-    const int bx = blockIdx.x, sidx = blockIdx.z;
-    const uint32_t* trel = p.trellis;
-    const __half* svh_p = p.svh;
-    const __half* dsuh = nullptr;  // grouped up pass: the down projection's suh
-    const __half* arows = p.a;
-    const float* rowsum = p.rowsum;
-    int bxm = bx, nm = p.n;  // column block and width inside the matrix
-    int m0 = blockIdx.y * MT;
-    int rows = min(MT, p.M - m0);
-    if (p.gmode) {
-        if ((int)blockIdx.y >= __builtin_amdgcn_readfirstlane(*gptr(p.ntiles))) return;
-        const EXL3_GLOBAL FatTile* tl = gptr(p.tiles) + blockIdx.y;
-        const int e = __builtin_amdgcn_readfirstlane(tl->e);
-        m0 = __builtin_amdgcn_readfirstlane(tl->crow0);
-        rows = __builtin_amdgcn_readfirstlane(tl->nrows);
-        const int pb = p.gmode == 1 ? 0 : (p.gmode == 2 ? 3 : 6);
-        trel = reinterpret_cast<const uint32_t*>(gptr(p.tabs[pb])[e]);
-        svh_p = reinterpret_cast<const __half*>(gptr(p.tabs[pb + 2])[e]);
-        if (p.gmode == 2) dsuh = reinterpret_cast<const __half*>(gptr(p.tabs[7])[e]);
-    } else if (p.mats.count > 1) {
-        const MatRef r = mat_of_block(p.mats, bx);
-        trel = r.trellis;
-        svh_p = r.svh;
-        bxm = bx - r.nb0;
-        nm = r.n;
-        arows += (size_t)r.j * p.M * p.k;
-        if constexpr (RAW) rowsum += (size_t)r.j * p.M * (p.k >> 7);
-    }
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int cw = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int g = lane >> 4, i = lane & 15, q = i & 7;
-    const int ntiles = nm >> 4;
-    const int nsteps = p.ksteps;
-    const int kt0 = sidx * nsteps * 4;
-    const int nt = bxm * 8 + cw * 2 + (i >> 3);
-    const EXL3_GLOBAL uint32_t* tb = gptr(trel) + ((size_t)(kt0 + g) * ntiles + nt) * (8 * K) + K * q;
-    const size_t step_stride = (size_t)4 * ntiles * (8 * K);
+    constexpr int GR = 8 * SW;             // rows copied by one instruction of each wave
+    const int g = lane >> 4, i = lane & 15;
     const int prev_addr = ((lane & ~7) | ((lane + 7) & 7)) << 2;
-
-    // A copies: wave w's j-th instruction of a step moves rows 32j + 8w .. + 7;
+    // A copies: wave w's j-th instruction of a step moves rows GR j + 8w .. + 7;
     // rows past the tile repeat its last row (never stored)
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)fat_smem;
-    const EXL3_GLOBAL char* abase =
-        reinterpret_cast<const EXL3_GLOBAL char*>(gptr(arows)) + ((size_t)m0 * p.k + (size_t)kt0 * 16) * 2;
-    uint32_t aoff[MT / 32];
-    const uint32_t achunk = 16u * (uint32_t)((lane & 7) ^ (lane >> 3) ^ (cw & 1));
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + lds;
+    uint32_t aoff[MT / GR];
+    const uint32_t achunk = 16u * (uint32_t)((lane & 7) ^ (lane >> 3) ^ (sw & 1));
 #pragma unroll
-    for (int j = 0; j < MT / 32; ++j)
-        aoff[j] = (uint32_t)min(32 * j + 8 * cw + (lane >> 3), rows - 1) * (uint32_t)p.k * 2u + achunk;
+    for (int j = 0; j < MT / GR; ++j)
+        aoff[j] = (uint32_t)min(GR * j + 8 * sw + (lane >> 3), rows - 1) * (uint32_t)k * 2u + achunk;
     auto copy_a = [&](int step, int bufi) {
         const EXL3_GLOBAL char* src = abase + (size_t)step * 128;
 #pragma unroll
-        for (int j = 0; j < MT / 32; ++j)
-            if (32 * j < rows) copy_to_lds16(src, aoff[j], lds0 + bufi * (MT * 128) + (32 * j + 8 * cw) * 128);
+        for (int j = 0; j < MT / GR; ++j)
+            if (GR * j < rows) copy_to_lds16(src, aoff[j], lds0 + bufi * (MT * 128) + (GR * j + 8 * sw) * 128);
     };
     // A fragment reads: row 16 rb + i, logical chunk 2g + h
     uint32_t rd_off[2];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) rd_off[h] = (uint32_t)i * 128u + 16u * (uint32_t)((2 * g + h) ^ (i & 7) ^ (i >> 3));
+    for (int h = 0; h < 2; ++h)
+        rd_off[h] = lds + (uint32_t)i * 128u + 16u * (uint32_t)((2 * g + h) ^ (i & 7) ^ (i >> 3));
 
-    float4_t acc[RB][2];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
         acc[rb][0] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -135,7 +100,7 @@ __global__ __launch_bounds__(TL_THREADS, MT == 256 ? 2 : (MT == 192 ? 3 : 4)) vo
 
     auto step_body = [&](int s, auto slot_c, uint32_t (&w)[K], uint32_t (&wn)[K]) {
         constexpr int SL = decltype(slot_c)::value;
-        const unsigned char* ab = fat_smem + SL * (MT * 128);
+        const unsigned char* ab = smem + SL * (MT * 128);
         half8_t A[PF + 1][2];
         auto read_a = [&](int rb) {
 #pragma unroll
@@ -179,6 +144,54 @@ __global__ __launch_bounds__(TL_THREADS, MT == 256 ? 2 : (MT == 192 ? 3 : 4)) vo
         step_body(s, std::integral_constant<int, 0>{}, wa, wb);
         step_body(s + 1, std::integral_constant<int, 1>{}, wb, wa);
     }
+}
+
+template <int K, int CB, int MT, bool RAW>
+__global__ __launch_bounds__(TL_THREADS, MT == 256 ? 2 : 4) void tall_kernel(FatParams p) {
+    static_assert(!RAW || CB == 2, "raw entries: mul1");
+    constexpr int RB = MT / 16;
+    extern __shared__ __align__(16) unsigned char fat_smem[];
+
+    const int bx = blockIdx.x, sidx = blockIdx.z;
+    // gate/up mode: block bx is column block bx / 2 of the gate (even) or up
+    // (odd) projection, and its partial tile goes to the finish launch
+    const uint32_t* trel = (p.gu && (bx & 1)) ? p.trellis2 : p.trellis;
+    const __half* svh_p = p.svh;
+    const __half* arows = p.a;
+    const float* rowsum = p.rowsum;
+    int bxm = p.gu ? bx >> 1 : bx, nm = p.n;  // column block and width inside the matrix
+    int m0 = blockIdx.y * MT;
+    int rows = min(MT, p.M - m0);
+    if (p.gmode) {
+        if ((int)blockIdx.y >= __builtin_amdgcn_readfirstlane(*gptr(p.ntiles))) return;
+        const EXL3_GLOBAL FatTile* tl = gptr(p.tiles) + blockIdx.y;
+        const int e = __builtin_amdgcn_readfirstlane(tl->e);
+        m0 = __builtin_amdgcn_readfirstlane(tl->crow0);
+        rows = __builtin_amdgcn_readfirstlane(tl->nrows);
+        trel = reinterpret_cast<const uint32_t*>(gptr(p.tabs[6])[e]);  // down (gmode 3)
+        svh_p = reinterpret_cast<const __half*>(gptr(p.tabs[8])[e]);
+    } else if (p.mats.count > 1) {
+        const MatRef r = mat_of_block(p.mats, bx);
+        trel = r.trellis;
+        svh_p = r.svh;
+        bxm = bx - r.nb0;
+        nm = r.n;
+        arows += (size_t)r.j * p.M * p.k;
+        if constexpr (RAW) rowsum += (size_t)r.j * p.M * (p.k >> 7);
+    }
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int cw = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, i = lane & 15, q = i & 7;
+    const int ntiles = nm >> 4;
+    const int nsteps = p.ksteps;
+    const int kt0 = sidx * nsteps * 4;
+    const int nt = bxm * 8 + cw * 2 + (i >> 3);
+    const EXL3_GLOBAL uint32_t* tb = gptr(trel) + ((size_t)(kt0 + g) * ntiles + nt) * (8 * K) + K * q;
+    const size_t step_stride = (size_t)4 * ntiles * (8 * K);
+    const EXL3_GLOBAL char* abase =
+        reinterpret_cast<const EXL3_GLOBAL char*>(gptr(arows)) + ((size_t)m0 * p.k + (size_t)kt0 * 16) * 2;
+    float4_t acc[RB][2];
+    tall_loop<K, CB, MT, 4, RAW>(acc, tb, step_stride, nsteps, abase, p.k, rows, fat_smem, 0, cw, lane);
 
     // epilogue: passes of 64 rows through LDS; 8 lanes hold a row, 16
     // consecutive columns each (fwht128_x16)
@@ -247,45 +260,9 @@ __global__ __launch_bounds__(TL_THREADS, MT == 256 ? 2 : (MT == 192 ? 3 : 4)) vo
             fwht128_x16(v, lane);
 #pragma unroll
             for (int e = 0; e < 16; ++e) v[e] = (v[e] * hn) * sv[e];
-            if (p.gmode == 1) {
-                if (row < rows)
-#pragma unroll
-                    for (int q4 = 0; q4 < 4; ++q4)
-                        *reinterpret_cast<EXL3_GLOBAL u32x4_t*>(gptr(p.g32) + (size_t)crow * p.n + c0 + 4 * q4) =
-                            *reinterpret_cast<const u32x4_t*>(v + 4 * q4);
-                continue;
-            }
             uint32_t ow[8];
             size_t orow = (size_t)crow;
-            if (p.gmode == 2) {
-                float gv[16];
-#pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4)
-                    *reinterpret_cast<u32x4_t*>(gv + 4 * q4) =
-                        *reinterpret_cast<const EXL3_GLOBAL u32x4_t*>(gptr(p.g32) + (size_t)crow * p.n + c0 + 4 * q4);
-                if (p.limit > 0.0f && p.limit < __builtin_huge_valf()) {
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        gv[e] = fminf(gv[e], p.limit);
-                        v[e] = fminf(fmaxf(v[e], -p.limit), p.limit);
-                    }
-                }
-                // the activation in fp16, then the down projection's input rotation of this 128-wide chunk
-                const EXL3_GLOBAL uint32_t* dsp = reinterpret_cast<const EXL3_GLOBAL uint32_t*>(gptr(dsuh) + c0);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const uint32_t du = dsp[e];
-                    const __half2 pr = __hmul2(h2_rn(silu_f(gv[2 * e]) * v[2 * e], silu_f(gv[2 * e + 1]) * v[2 * e + 1]),
-                                               *reinterpret_cast<const __half2*>(&du));
-                    v[2 * e] = __low2float(pr);
-                    v[2 * e + 1] = __high2float(pr);
-                }
-                fwht128_x16(v, lane);
-#pragma unroll
-                for (int e = 0; e < 16; ++e) v[e] *= hn;
-            } else if (p.gmode == 3) {
-                orow = (size_t)gptr(p.rows_map)[crow];
-            }
+            if (p.gmode) orow = (size_t)gptr(p.rows_map)[crow];  // by (token, slot) entry
 #pragma unroll
             for (int e = 0; e < 8; ++e) ow[e] = y_bits(h2_rn(v[2 * e], v[2 * e + 1]), p.y_bf16);
             if (row >= rows) continue;
@@ -301,29 +278,194 @@ __global__ __launch_bounds__(TL_THREADS, MT == 256 ? 2 : (MT == 192 ? 3 : 4)) vo
     }
 }
 
-// Tiles of `mt` (128 or 256) rows; grouped mode and plain fp16 output, with
-// k-splits handed to fat_split_finish_kernel (split_out).
+// Gate and up of a 128-column block in one workgroup of 8 waves (waves 0-3
+// gate, 4-7 up), so the SwiGLU runs on the accumulators: no partial tiles or
+// fp32 gate rows through memory.  Dense (GRP = false): both halves read one
+// staged A (the projections share their input rotation); p.out16 = the activation;
+// tiles_x, tail_first, tail_tiles and tail_parts describe the linear grid.
+// Grouped (MoE prefill): each half stages its own projection's rotated rows
+// (p.a, then p.a + p.up_rows * k for up), the weights are the tile's expert's, and
+// out16[crow] is the activation rotated for the down projection.
+template <int MT, bool GRP>
+constexpr size_t tall_gu_smem_bytes() {
+    constexpr size_t stage = (GRP ? 4 : 2) * (size_t)MT * 128, tile = (size_t)TL_PASS_ROWS * (256 + 4) * sizeof(float);
+    return stage > tile ? stage : tile;
+}
+
+template <int K, int CB, int MT, bool RAW, bool GRP>
+__global__ __launch_bounds__(2 * TL_THREADS, MT == 256 ? 2 : 4) void tall_gu_kernel(FatParams p) {
+    static_assert(!RAW || (CB == 2 && !GRP), "raw entries: mul1, dense");
+    constexpr int RB = MT / 16, CTS = 256 + 4;
+    extern __shared__ __align__(16) unsigned char fat_smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), up = wv >> 2, cw = wv & 3;
+    const int g = lane >> 4, i = lane & 15, q = i & 7;
+    const uint32_t* trel = up ? p.trellis2 : p.trellis;
+    const __half *svg = p.svh, *svu = p.svh2, *dsuh = nullptr;
+    const __half* arows = p.a;
+    int bx = blockIdx.x, m0 = 0, rows = 0;
+    if constexpr (!GRP) {
+        // linear grid, column blocks fastest; the tiles from tail_first on run
+        // as tail_parts workgroups of MT / tail_parts rows each
+        int lin = blockIdx.x, part = 0, mt = MT;
+        if (lin >= p.tail_first) {
+            const int o = lin - p.tail_first, t = o / p.tail_parts;
+            part = o - t * p.tail_parts;
+            mt = MT / p.tail_parts;
+            lin = p.tail_first + t;
+        }
+        const int by = __builtin_amdgcn_readfirstlane(lin / p.tiles_x);
+        bx = __builtin_amdgcn_readfirstlane(lin - by * p.tiles_x);
+        m0 = __builtin_amdgcn_readfirstlane(by * MT + part * mt);
+        rows = __builtin_amdgcn_readfirstlane(min(mt, p.M - m0));
+        if (rows <= 0) return;
+    }
+    if constexpr (GRP) {
+        if ((int)blockIdx.y >= __builtin_amdgcn_readfirstlane(*gptr(p.ntiles))) return;
+        const EXL3_GLOBAL FatTile* tl = gptr(p.tiles) + blockIdx.y;
+        const int e = __builtin_amdgcn_readfirstlane(tl->e);
+        m0 = __builtin_amdgcn_readfirstlane(tl->crow0);
+        rows = __builtin_amdgcn_readfirstlane(tl->nrows);
+        trel = reinterpret_cast<const uint32_t*>(gptr(p.tabs[up ? 3 : 0])[e]);
+        svg = reinterpret_cast<const __half*>(gptr(p.tabs[2])[e]);
+        svu = reinterpret_cast<const __half*>(gptr(p.tabs[5])[e]);
+        dsuh = reinterpret_cast<const __half*>(gptr(p.tabs[7])[e]);
+        if (up) arows += (size_t)p.up_rows * p.k;
+    }
+    const int ntiles = p.n >> 4;
+    const int nt = bx * 8 + cw * 2 + (i >> 3);
+    const EXL3_GLOBAL uint32_t* tb = gptr(trel) + ((size_t)g * ntiles + nt) * (8 * K) + K * q;
+    const EXL3_GLOBAL char* abase = reinterpret_cast<const EXL3_GLOBAL char*>(gptr(arows)) + (size_t)m0 * p.k * 2;
+    float4_t acc[RB][2];
+    tall_loop<K, CB, MT, GRP ? 4 : 8, RAW>(acc, tb, (size_t)4 * ntiles * (8 * K), p.ksteps, abase, p.k, rows, fat_smem,
+                                           GRP ? up * (2 * MT * 128) : 0, GRP ? cw : wv, lane);
+
+    // passes of 64 rows through LDS, gate in the left and up in the right 128
+    // columns; 8 rows per wave, 16 consecutive columns of both per lane
+    float* ct = reinterpret_cast<float*>(fat_smem);
+    const int col = (lane & 7) * 16, c0 = bx * 128 + col;
+    const float hn = fwht_x16_norm(lane);
+#pragma unroll
+    for (int pass = 0; pass < MT / TL_PASS_ROWS; ++pass) {
+        if (pass * TL_PASS_ROWS >= rows) break;
+        if (pass) __syncthreads();
+#pragma unroll
+        for (int rr = 0; rr < TL_PASS_ROWS / 16; ++rr)
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    ct[(rr * 16 + 4 * g + r) * CTS + up * 128 + cw * 32 + (i >> 3) * 16 + (i & 7) + 8 * c] =
+                        acc[pass * (TL_PASS_ROWS / 16) + rr][c][r];
+        __syncthreads();
+        if (pass * TL_PASS_ROWS + wv * 8 >= rows) continue;
+        const int lr = wv * 8 + (lane >> 3), row = pass * TL_PASS_ROWS + lr;
+        const int crow = m0 + (row < rows ? row : rows - 1);
+        float gv[16], uv[16];
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+            *reinterpret_cast<float4*>(gv + 4 * q4) = *reinterpret_cast<const float4*>(ct + lr * CTS + col + 4 * q4);
+            *reinterpret_cast<float4*>(uv + 4 * q4) = *reinterpret_cast<const float4*>(ct + lr * CTS + 128 + col + 4 * q4);
+        }
+        if constexpr (RAW) {
+            const float sx = raw_row_bias(p, crow, 0, p.k >> 7, lane);
+            raw_fix16(gv, sx);
+            raw_fix16(uv, sx);
+        }
+        fwht128_x16(gv, lane);
+        fwht128_x16(uv, lane);
+        // svh and suh are only 4-byte aligned by contract
+        const EXL3_GLOBAL uint32_t* sgp = reinterpret_cast<const EXL3_GLOBAL uint32_t*>(gptr(svg) + c0);
+        const EXL3_GLOBAL uint32_t* sup = reinterpret_cast<const EXL3_GLOBAL uint32_t*>(gptr(svu) + c0);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            gv[e] = (gv[e] * hn) * __half2float(__ushort_as_half((unsigned short)(sgp[e >> 1] >> (16 * (e & 1)))));
+            uv[e] = (uv[e] * hn) * __half2float(__ushort_as_half((unsigned short)(sup[e >> 1] >> (16 * (e & 1)))));
+        }
+        if (p.limit > 0.0f && p.limit < __builtin_huge_valf()) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                gv[e] = fminf(gv[e], p.limit);
+                uv[e] = fminf(fmaxf(uv[e], -p.limit), p.limit);
+            }
+        }
+        uint32_t ow[8];
+        if constexpr (GRP) {
+            // the activation in fp16, then the down projection's input rotation of this 128-wide chunk
+            const EXL3_GLOBAL uint32_t* dsp = reinterpret_cast<const EXL3_GLOBAL uint32_t*>(gptr(dsuh) + c0);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t du = dsp[e];
+                const __half2 pr = __hmul2(h2_rn(silu_f(gv[2 * e]) * uv[2 * e], silu_f(gv[2 * e + 1]) * uv[2 * e + 1]),
+                                           *reinterpret_cast<const __half2*>(&du));
+                gv[2 * e] = __low2float(pr);
+                gv[2 * e + 1] = __high2float(pr);
+            }
+            fwht128_x16(gv, lane);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const __half2 o = h2_rn(gv[2 * e] * hn, gv[2 * e + 1] * hn);
+                ow[e] = *reinterpret_cast<const uint32_t*>(&o);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const __half2 o = h2_rn(silu_f(gv[2 * e]) * uv[2 * e], silu_f(gv[2 * e + 1]) * uv[2 * e + 1]);
+                ow[e] = *reinterpret_cast<const uint32_t*>(&o);
+            }
+        }
+        if (row >= rows) continue;
+        EXL3_GLOBAL uint32_t* o = reinterpret_cast<EXL3_GLOBAL uint32_t*>(gptr(p.out16) + (size_t)crow * p.n + c0);
+        if (p.out_vec) {
+            reinterpret_cast<EXL3_GLOBAL u32x4_t*>(o)[0] = u32x4_t{ow[0], ow[1], ow[2], ow[3]};
+            reinterpret_cast<EXL3_GLOBAL u32x4_t*>(o)[1] = u32x4_t{ow[4], ow[5], ow[6], ow[7]};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = ow[e];
+        }
+    }
+}
+
+// Tiles of `mt` (128 or 256) rows.  gu_fused: tall_gu_kernel (dense with 256-row
+// tiles, or grouped, p.gmode = 4, with 128), else tall_kernel: plain fp16 output,
+// grouped down pass (p.gmode = 3), or partial tiles for
+// fat_split_finish_kernel (p.split_out; always in gate/up mode).
 template <int K>
-int tall_launch_k(int cb, int mt, const FatParams& p, int row_tiles, int splits, hipStream_t st) {
-    const dim3 grid(p.n / 128, row_tiles, splits);
-    const size_t smem = tall_smem_bytes(mt);
-#define EXL3_TALL(CBV, MTV, RAWV)                                                                      \
-    if (cb == CBV && mt == MTV && (p.rowsum != nullptr) == RAWV) {                                     \
-        const void* fn = reinterpret_cast<const void*>(&tall_kernel<K, CBV, MTV, RAWV>);               \
-        const int lrc = allow_dynamic_lds(fn, smem, "exl3 gemm (tall tiles)");                         \
+int tall_launch_k(int cb, int mt, const FatParams& p, int row_tiles, int splits, bool gu_fused, hipStream_t st) {
+#define EXL3_TALL_GO(FN, GRID, THREADS, SMEM)                                                          \
+    {                                                                                                  \
+        const void* fn = reinterpret_cast<const void*>(&FN);                                           \
+        const int lrc = allow_dynamic_lds(fn, SMEM, "exl3 gemm (tall tiles)");                         \
         if (lrc) return lrc;                                                                           \
-        tall_kernel<K, CBV, MTV, RAWV><<<grid, TL_THREADS, smem, st>>>(p);                             \
+        FN<<<GRID, THREADS, SMEM, st>>>(p);                                                            \
         return launch_status("exl3 gemm (tall tiles) launch");                                         \
     }
-    EXL3_TALL(0, 128, false) EXL3_TALL(1, 128, false) EXL3_TALL(2, 128, false) EXL3_TALL(2, 128, true)
-    EXL3_TALL(0, 192, false) EXL3_TALL(1, 192, false) EXL3_TALL(2, 192, false) EXL3_TALL(2, 192, true)
-    EXL3_TALL(0, 256, false) EXL3_TALL(1, 256, false) EXL3_TALL(2, 256, false) EXL3_TALL(2, 256, true)
+#define EXL3_TALL_GU(CBV, MTV, RAWV, GRPV)                                                             \
+    if (cb == CBV && mt == MTV && (p.rowsum != nullptr) == RAWV && (p.gmode != 0) == GRPV)             \
+    EXL3_TALL_GO((tall_gu_kernel<K, CBV, MTV, RAWV, GRPV>),                                            \
+                 GRPV ? dim3(p.n / 128, row_tiles) : dim3(p.tail_first + p.tail_tiles * p.tail_parts),         \
+                 2 * TL_THREADS,                                                                       \
+                 (tall_gu_smem_bytes<MTV, GRPV>()))
+#define EXL3_TALL(CBV, MTV, RAWV)                                                                      \
+    if (cb == CBV && mt == MTV && (p.rowsum != nullptr) == RAWV)                                       \
+    EXL3_TALL_GO((tall_kernel<K, CBV, MTV, RAWV>), dim3((p.gu ? 2 : 1) * (p.n / 128), row_tiles, splits), TL_THREADS, \
+                 tall_smem_bytes(MTV))
+    if (gu_fused) {
+        EXL3_TALL_GU(0, 256, false, false) EXL3_TALL_GU(1, 256, false, false)
+        EXL3_TALL_GU(2, 256, false, false) EXL3_TALL_GU(2, 256, true, false)
+        EXL3_TALL_GU(0, 128, false, true) EXL3_TALL_GU(1, 128, false, true) EXL3_TALL_GU(2, 128, false, true)
+    } else {
+        EXL3_TALL(0, 128, false) EXL3_TALL(1, 128, false) EXL3_TALL(2, 128, false) EXL3_TALL(2, 128, true)
+        EXL3_TALL(0, 256, false) EXL3_TALL(1, 256, false) EXL3_TALL(2, 256, false) EXL3_TALL(2, 256, true)
+    }
 #undef EXL3_TALL
+#undef EXL3_TALL_GU
+#undef EXL3_TALL_GO
     set_error("exl3 gemm: no tall kernel for codebook %d tile rows %d", cb, mt);
     return EXL3_ERR_UNSUPPORTED;
 }
 
 // One instantiation unit per K (exl3_tall_inst.hip built with -DEXL3_K=K).
-int tall_launch(int K, int cb, int mt, const FatParams& p, int row_tiles, int splits, hipStream_t st);
+int tall_launch(int K, int cb, int mt, const FatParams& p, int row_tiles, int splits, bool gu_fused, hipStream_t st);
 
 }  // namespace exl3

@@ -651,6 +651,40 @@ def test_moe_prefill_swiglu_limit(monkeypatch):
     check_close(out.float().cpu().numpy(), ex.ref(x, ids, w, limit=2.0), "moe prefill limit")
 
 
+@pytest.mark.parametrize("K,cb,limit", [(1, 1, 0.0), (2, 2, 1.5), (3, 1, 0.0), (4, 0, 0.0), (5, 2, 0.0), (6, 1, 2.0),
+                                        (7, 0, 0.0), (8, 2, 0.0)])
+def test_moe_prefill_tile_edges(K, cb, limit, monkeypatch):
+    """128-row tiles with gate and up in one workgroup: experts with 0, 1, 31, 32, 33, 127, 128, 129 and 300 rows,
+    two skipped ids, hidden of three 128-chunks, every K: against the oracle, bit-equal when repeated (tiles may
+    be listed in another order) and into an output that is only 4-byte aligned, close to the 64-row tiles
+    (EXL3_MOE_TALL=0)."""
+    monkeypatch.setenv("EXL3_MOE_PREFILL", "1")
+    print(f"case: moe prefill tile edges K={K} cb={cb}", flush=True)
+    counts = (0, 1, 31, 32, 33, 127, 128, 129, 300)
+    E, hidden, inter = len(counts), 384, 256
+    ids = np.concatenate([np.full(c, e, np.int32) for e, c in enumerate(counts)] + [np.array([-1, E], np.int32)])
+    T = len(ids)
+    ids = np.random.default_rng(K).permutation(ids)[:, None]
+    w = np.random.default_rng(K + 1).random((T, 1)).astype(np.float32) + 0.1
+    ex = Experts(E, hidden, inter, (K, K, K), cb, seed=60 + K)
+    x = make_x(T, hidden, seed=61 + K)
+    out = _layer_capi(ex, x, ids, w, cb=cb, limit=limit)
+    assert torch.equal(_layer_capi(ex, x, ids, w, cb=cb, limit=limit), out)
+    check_close(out.float().cpu().numpy(), ex.ref(x, ids, w, limit=limit or float("inf")), f"moe prefill edges K={K}")
+    L = _lib.lib()
+    xd, idd, wd = (torch.from_numpy(v).cuda() for v in (x, ids, w))
+    odd = torch.zeros(T * hidden + 2, dtype=torch.float16, device="cuda")
+    ws = ops.workspace(xd.device, int(L.exl3_moe_workspace_size(T, 1, E, hidden, inter)))
+    rc = L.exl3_moe_layer(xd.data_ptr(), idd.data_ptr(), wd.data_ptr(), *[t.data_ptr() for t in ex.tables], E,
+                          odd.data_ptr() + 4, T, 1, hidden, inter, K, K, K, cb, limit, ws.data_ptr(), ws.numel(),
+                          torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "exl3_moe_layer")
+    assert torch.equal(odd[2:].view(T, hidden), out)
+    monkeypatch.setenv("EXL3_MOE_TALL", "0")
+    small = _layer_capi(ex, x, ids, w, cb=cb, limit=limit)
+    check_close(out.float().cpu().numpy(), small.float().cpu().numpy(), f"128-row vs 64-row tiles K={K}")
+
+
 def test_moe_prefill_token_chunks_vs_oracle_subset():
     """16800 routed rows: above one pipeline pass (16384), so two token chunks; checked on 64
     seeded tokens from both chunks (tokens are independent)."""
