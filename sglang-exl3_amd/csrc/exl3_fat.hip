@@ -473,34 +473,85 @@ int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_
 
 // Gate/up SwiGLU on the MFMA kernels: the input is rotated once with the
 // shared suh into the scratch, then
-//   * up to kGateUpNarrowMaxRows rows: the narrow kernel in gate/up mode (16- or
-//     64-row tiles; partial tiles and one counter per (column block, row tile)
-//     in the scratch);
-//   * above: the wide-tile kernel in gate/up mode (one split, tail split).
-// k-splits of the narrow kernel: the most that keep the grid within 1.25 rounds
-// of resident workgroups (CUs x waves per SIMD: 6 for 16-row tiles, set by
-// their ~75 VGPRs, 4 for 64-row tiles, set by their LDS) and at least 16 steps
-// per split (shorter splits spend more on the hand-off and epilogue than the
-// extra workgroups win).  Config 3 (n = 14336 per projection, k = 4096),
-// graph-timed, narrow splits 1 / 2 / 4 / 8: M = 16: 41.1 / 31.1 / 29.7 / 31.8
-// us, 32: 57.0 / 42.0 / 39.7 / 43.2, 64: 80.1 / 57.1 / 56.6 / 64.4, 96: 80.6 /
-// 68.5 / 74.1 / 88.6, 128: 89.0 / 79.2 / 81.0 / 96.8, 160: 93.7 / 106.0 / 98.7 /
-// 118.0, 192: 106.8 / 110.9 / 109.8 / 132.8; wide tiles M = 160 / 192 / 256:
-// 98.2 / 96.8 / 97.7.
-constexpr int kGateUpNarrowMaxRows = 160;
+//   * up to 16 rows: the narrow kernel in gate/up mode (k-splits hand partial
+//     tiles over in the scratch);
+//   * above: tall tiles, gate and up blocks as partial tiles with the finish
+//     launch, or both projections in one workgroup of 256 rows.
 constexpr int kGateUpMinSplitSteps = 16;
+constexpr int kGateUpWideMinRows = 160, kGateUpWideMaxK = 256;
 
-// Scratch: [counters][accumulators][xr fp16 m*k][partials, narrow only].
 struct GateUpFatPlan {
     int mt, splits;
+    bool tall, fused;  // fused: gate and up in one workgroup
+    int tail_parts;    // fused: workgroups per tile of the last round
 };
 
+// The fused kernel runs one workgroup per CU.  Tiles of a last round that would
+// leave half the CUs or more idle are split by rows, 2 or 4 workgroups each
+// (each decodes the tile's weights again, on CUs that had nothing to do).  Whole /
+// split, us: k = 4096, n = 14336, M = 2048 (896 tiles: 3.5 rounds) 451 / 440; k = 3072, n =
+// 6144, M = 1500 170 / 141; k = n = 2048, M = 1000 (64 tiles) 65 / 39.  Two k-halves, the
+// first handing its sums over through memory, gave 455, 157 and 59.
+// Env EXL3_FAT_TAIL=0 turns it off.
+long long gu_tiles(int m, int n) { return (long long)(n / 128) * ((m + 255) / 256); }
+int gu_tail_parts(int m, int n) {
+    const int c = fat_cus(), r = (int)(gu_tiles(m, n) % c);
+    if (r == 0 || env_int("EXL3_FAT_TAIL", 1) == 0) return 1;
+    return 4 * r <= c ? 4 : 2 * r <= c ? 2 : 1;
+}
+double gu_fused_cost(int m, int k, int n) {
+    auto round = [&](int rows) {
+        const int rb = 2 * (((m < rows ? m : rows) + 31) / 32);
+        return (k / 64) * (0.45 + 0.078 * rb) + 2.0 + 0.56 * rb;
+    };
+    const long long tiles = gu_tiles(m, n), cus = fat_cus();
+    return (double)(tiles / cus) * round(256) + (tiles % cus ? round(256 / gu_tail_parts(m, n)) : 0.0);
+}
+
+// Above 16 rows by cost in us: partial tiles (tall_cost over both projections'
+// columns, and the finish launch always) or fused rounds (0.45 + 0.078 rb a 64-k
+// step, 2 + 0.56 rb for the epilogue).  The kernels before
+// (64-row tiles to 160 rows, 256 x 256 tiles above) / this rule, us: k = 4096, n =
+// 14336, K = 3 mul1, 40 / 300 / 512 / 2048 rows: 44.3 / 118.8 / 124.9 / 460.4 -> 38.4 /
+// 105.5 / 118.8 / 439.7; k = 2048, n = 6144, K = 4, 64 / 600: 35.1 / 73.7 -> 23.8 / 57.5; k =
+// n = 2048, 17 / 1000: 22.1 / 64.0 -> 13.3 / 37.4; k = 8192, n = 16384, 1100: 637 -> 568.
+// The rule is within 6 % of the best of the seven choices at 16 shapes.
+// More than 160 rows of k <= 256 (no layer is that short) keep the 256 x 256 tiles,
+// whose bounded tail wait callers see reported there (300 x 256 x 256: 33.6 us;
+// partial tiles 13.0).
+// Env EXL3_GU_TALL: 128 / 256 partial tiles of that height (with
+// EXL3_FAT_SPLITS), 1 fused.
 GateUpFatPlan plan_gate_up_fat(int m, int k, int n) {
-    if (m > kGateUpNarrowMaxRows && fat_wide_allowed()) return GateUpFatPlan{FAT_MT_WIDE, 1};
-    GateUpFatPlan pl{m <= 16 ? 16 : 64, 1};
     const int ksteps = k / 64;
-    const long long base = 2LL * (n / 128) * ((m + pl.mt - 1) / pl.mt);
-    const long long resident = (long long)fat_cus() * (pl.mt == 16 ? 6 : 4);
+    if (m > 16) {
+        const int forced = env_int("EXL3_GU_TALL", 0), fs = env_int("EXL3_FAT_SPLITS", 0);
+        if (forced == 0 && m > kGateUpWideMinRows && k <= kGateUpWideMaxK && fat_wide_allowed())
+            return GateUpFatPlan{FAT_MT_WIDE, 1, false, false, 1};
+        GateUpFatPlan best{256, 1, true, true, gu_tail_parts(m, n)};
+        double cost = forced == 128 || forced == 256 ? 1e30 : gu_fused_cost(m, k, n);
+        for (int mt = 128; mt <= 256 && forced != 1; mt += 128) {
+            if (forced > 1 && forced != mt) continue;
+            for (int S = 1; S <= kTallMaxSplits && ksteps % (2 * S) == 0; S *= 2) {
+                if (fs > 0 && S != fs && ksteps % (2 * fs) == 0) continue;
+                double c = tall_cost(m, k, 2 * n, mt, S);
+                if (S == 1) c += 3.0 + (double)m * n * 16.0 / 5.0e6;  // the finish launch all the same
+                if (c < cost - 1e-9) {
+                    cost = c;
+                    best = GateUpFatPlan{mt, S, true, false, 1};
+                }
+            }
+        }
+        return best;
+    }
+    // k-splits of the narrow kernel: the most that keep the grid within 1.25
+    // rounds of resident workgroups (CUs x 6 waves per SIMD, set by their ~75
+    // VGPRs) and at least 16 steps per split (shorter splits spend more on the
+    // hand-off and epilogue than the extra workgroups win).  Config 3 (n = 14336
+    // per projection, k = 4096), graph-timed, splits 1 / 2 / 4 / 8: M = 16: 41.1 /
+    // 31.1 / 29.7 / 31.8 us.
+    GateUpFatPlan pl{16, 1, false, false, 1};
+    const long long base = 2LL * (n / 128);
+    const long long resident = (long long)fat_cus() * 6;
     const int min_steps = kGateUpMinSplitSteps;
     const int forced = env_int("EXL3_FAT_SPLITS", 0);  // tuning override (power of two)
     while ((forced ? pl.splits < forced
@@ -513,8 +564,9 @@ GateUpFatPlan plan_gate_up_fat(int m, int k, int n) {
 size_t fat_gate_up_scratch_bytes(int m, int k, int n) {
     const GateUpFatPlan pl = plan_gate_up_fat(m, k, n);
     size_t b = kWsScratchOffset + fat_xr_bytes(m, k);
-    if (pl.mt != FAT_MT_WIDE) b += (size_t)2 * (n / 128) * pl.splits * (size_t)m * 128 * sizeof(float);
-    else b += fat_tail_bytes(wide_tail_tiles(m, k, n, true));
+    if (pl.fused) return b;
+    if (pl.mt == FAT_MT_WIDE) b += fat_tail_bytes(wide_tail_tiles(m, k, n, true));
+    else b += (size_t)2 * (n / 128) * pl.splits * (size_t)m * 128 * sizeof(float);
     return b;
 }
 
@@ -528,12 +580,12 @@ int fat_gate_up_rows(const uint16_t* x, const uint16_t* suh, const int16_t* gate
                       ws ? ws_bytes : (size_t)0);
     EXL3_REQUIRE(aligned(gate_trellis, 16) && aligned(up_trellis, 16) && aligned(gate_svh, 4) && aligned(up_svh, 4),
                  "exl3_gate_up_swiglu: misaligned pointer");
-    const int mtiles = pl.mt == FAT_MT_WIDE ? 1 : (m + pl.mt - 1) / pl.mt;
+    const int mtiles = pl.tall || pl.mt == FAT_MT_WIDE ? 1 : (m + pl.mt - 1) / pl.mt;
     EXL3_REQUIRE_CODE((size_t)(n / 128) * mtiles <= kWsMaxCounters, EXL3_ERR_UNSUPPORTED,
                       "exl3_gate_up_swiglu: %d column blocks exceed the workspace counters", n / 128);
     char* w8 = reinterpret_cast<char*>(ws);
     __half* xr = reinterpret_cast<__half*>(w8 + kWsScratchOffset);
-    float* rs = fat_raw(cb, pl.mt, true) ? reinterpret_cast<float*>(w8 + kWsScratchOffset + fat_xr_only_bytes(m, k)) : nullptr;
+    float* rs = fat_raw(cb, pl.mt, true, pl.tall) ? reinterpret_cast<float*>(w8 + kWsScratchOffset + fat_xr_only_bytes(m, k)) : nullptr;
     int rc = rotate_rows(reinterpret_cast<const __half*>(x), RotateSuh{{reinterpret_cast<const __half*>(suh)}}, 1, xr, m,
                          k, 0, rs, st, "exl3_gate_up_swiglu rotate launch");
     if (rc) return rc;
@@ -553,6 +605,18 @@ int fat_gate_up_rows(const uint16_t* x, const uint16_t* suh, const int16_t* gate
     p.limit = limit;
     p.counters = reinterpret_cast<int*>(w8);
     p.partials = reinterpret_cast<float*>(w8 + kWsScratchOffset + fat_xr_bytes(m, k));
+    if (pl.tall) {
+        p.split_out = !pl.fused;
+        p.out_vec = aligned(out, 16);
+        const int row_tiles = (m + pl.mt - 1) / pl.mt;
+        p.tiles_x = n / 128;
+        p.tail_parts = pl.tail_parts;
+        p.tail_tiles = pl.tail_parts > 1 ? (int)(gu_tiles(m, n) % fat_cus()) : 0;
+        p.tail_first = (int)gu_tiles(m, n) - p.tail_tiles;
+        rc = tall_launch(K, cb, pl.mt, p, row_tiles, pl.splits, pl.fused, st);
+        if (rc || pl.fused) return rc;
+        return fat_split_finish(p, pl.splits, st, "exl3_gate_up_swiglu finish launch");
+    }
     if (pl.mt == FAT_MT_WIDE) {
         const int tail = wide_tail_tiles(m, k, n, true);
         if (tail > 0) {

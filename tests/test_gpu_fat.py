@@ -278,6 +278,40 @@ def test_tall_tiles(m, k, n, K, cb, splits, mt, monkeypatch):
     assert torch.equal(odd[2:].view(m, n), y)
 
 
+@pytest.mark.parametrize("kind", ["1", "128", "256"])
+@pytest.mark.parametrize("m,k,n,K,cb,splits,limit", [
+    (17, 128, 128, 1, 1, 1, 0.0), (31, 256, 384, 2, 2, 2, 1.0), (32, 512, 128, 3, 0, 4, 0.0),
+    (33, 1024, 256, 4, 1, 8, 0.0), (127, 384, 128, 5, 2, 1, 2.0), (128, 256, 256, 6, 0, 2, 0.0),
+    (129, 512, 384, 7, 1, 4, 0.0), (255, 128, 128, 8, 2, 1, 0.0), (256, 512, 256, 3, 2, 2, 0.0),
+    (257, 256, 128, 4, 0, 1, 0.0), (520, 1024, 128, 3, 1, 1, 0.0)])
+def test_gate_up_tall_tiles(m, k, n, K, cb, splits, limit, kind, monkeypatch):
+    """gate/up + SwiGLU on tall tiles: partial tiles of either height with the finish launch, or both projections in
+    one workgroup (k a multiple of 256: every tile as two k-halves), at the edges of their row groups, every K and
+    codebook: against the oracle, bit-equal when repeated and into an output that is only 4-byte aligned."""
+    print(f"case: gate/up tall kind={kind} m={m} k={k} n={n} K={K} cb={cb} splits={splits}", flush=True)
+    monkeypatch.setenv("EXL3_GU_TALL", kind)
+    monkeypatch.setenv("EXL3_FAT_SPLITS", str(splits))
+    tg, su, sg = make_weight(k, n, K, seed=m + K)
+    tu, _, sv_u = make_weight(k, n, K, seed=m + K + 50)
+    scale = np.float32(4.0 / np.sqrt(k))
+    sg, sv_u = ((v.astype(np.float32) * scale).astype(np.float16) for v in (sg, sv_u))
+    x = make_x(m, k, seed=m)
+    d = [torch.from_numpy(v).cuda() for v in (x, su, tg, sg, tu, sv_u)]
+    y = torch.ops.sglang_exl3.exl3_gate_up_swiglu(*d, K, cb, limit)
+    assert torch.equal(y, torch.ops.sglang_exl3.exl3_gate_up_swiglu(*d, K, cb, limit))
+    g = oracle.matmul(x, oracle.dequant(tg, su, sg, K, cb, rtz=True))
+    u = oracle.matmul(x, oracle.dequant(tu, su, sv_u, K, cb, rtz=True))
+    check_close(y.float().cpu().numpy(), oracle.swiglu(g, u, limit or float("inf")), f"gate/up tall m={m}")
+    lib = _lib.lib()
+    need = lib.exl3_gate_up_workspace_size(m, k, n, K)
+    ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
+    odd = torch.zeros(m * n + 2, dtype=torch.float16, device="cuda")
+    rc = lib.exl3_gate_up_swiglu(*[t.data_ptr() for t in d], odd.data_ptr() + 4, m, k, n, K, cb, limit, ws.data_ptr(),
+                                 need, int(torch.cuda.current_stream().cuda_stream))
+    _lib.check(rc, "exl3_gate_up_swiglu")
+    assert torch.equal(odd[2:].view(m, n), y)
+
+
 @pytest.mark.parametrize("m,cb", [(16, 1), (64, 2)])
 def test_gemm_split_handoff_repeatable(m, cb, monkeypatch):
     """exl3_gemm's narrow k-splits hand partial tiles to the last split of each
