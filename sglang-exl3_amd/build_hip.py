@@ -2,13 +2,14 @@
 
 Compiles every csrc/*.hip (the GEMV instantiation unit once per bit width)
 with hipcc for gfx950 and links one shared library into
-sglang_exl3/_lib/.  Run directly (python build_hip.py) or through
+sglang_exl3/_lib/, and csrc/torch_ops.cpp (host code) with g++ into a second.  Run directly (python build_hip.py) or through
 __graft_entry__.build().
 """
 
 from __future__ import annotations
 
 import concurrent.futures as cf
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -19,6 +20,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIBDIR = os.path.join(HERE, "sglang_exl3", "_lib")
 LIBNAME = "libsglang_exl3_amd.so"
+OPS_LIBNAME = "libsglang_exl3_ops.so"
 ARCH = os.environ.get("EXL3_OFFLOAD_ARCH", "gfx950")
 
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
@@ -79,7 +81,26 @@ def build(force: bool = False, jobs: int | None = None) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr[-6000:]}")
     os.replace(tmp, out)
+    _build_ops(force)
     return out
+
+
+def _build_ops(force: bool) -> None:
+    """The operators' native entry (host code, linked against PyTorch)."""
+    src, out = os.path.join(CSRC, "torch_ops.cpp"), os.path.join(LIBDIR, OPS_LIBNAME)
+    if not force and os.path.exists(out) and os.path.getmtime(out) >= max(os.path.getmtime(src), _headers_mtime()):
+        return
+    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
+    inc = [os.path.join(torch_dir, "include"), os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+           os.path.join(rocm, "include")]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           *(f"-I{i}" for i in inc), src, "-o", out + ".tmp", f"-L{os.path.join(torch_dir, 'lib')}",
+           "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", f"-L{os.path.join(rocm, 'lib')}", "-lamdhip64"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for torch_ops.cpp:\n{r.stderr[-6000:]}")
+    os.replace(out + ".tmp", out)
 
 
 if __name__ == "__main__":

@@ -13,6 +13,8 @@ import threading
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("SGLANG_EXL3_AMD_LIB", os.path.join(_HERE, "_lib", "libsglang_exl3_amd.so"))
 
+OPS_LIB_PATH = os.path.join(_HERE, "_lib", "libsglang_exl3_ops.so")
+
 EXL3_OK = 0
 EXL3_ERR_ARG = 1
 EXL3_ERR_UNSUPPORTED = 2
@@ -96,6 +98,24 @@ def lib() -> ctypes.CDLL:
                 fn.argtypes = args
             _lib = L
     return _lib
+
+
+# the entry points of the operators' native path, in the order exl3_ops_bind takes them
+_OPS_BOUND = ("exl3_gemv", "exl3_gemv_workspace_size", "exl3_linear_cat", "exl3_linear_cat_workspace_size",
+              "exl3_gate_up_swiglu", "exl3_gate_up_workspace_size")
+
+
+def load_ops() -> ctypes.CDLL:
+    """Load the operators' native path (csrc/torch_ops.cpp; needs torch) and bind it to the HIP library."""
+    if not os.path.exists(OPS_LIB_PATH):
+        raise RuntimeError(f"sglang_exl3 operator library not found at {OPS_LIB_PATH}; build it with "
+                           "`python sglang-exl3_amd/build_hip.py` (or __graft_entry__.build())")
+    L = lib()
+    ops = ctypes.CDLL(OPS_LIB_PATH)
+    ops.exl3_ops_bind.restype = None
+    ops.exl3_ops_bind.argtypes = [_P]
+    ops.exl3_ops_bind((_P * len(_OPS_BOUND))(*(ctypes.cast(getattr(L, f), _P).value for f in _OPS_BOUND)))
+    return ops
 
 
 def check(rc: int, what: str) -> None:

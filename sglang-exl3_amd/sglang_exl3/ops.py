@@ -44,6 +44,7 @@ _WORKSPACES: Dict[Tuple[int, int], torch.Tensor] = {}
 # (stream-ordered, on the stream it was used on).
 _CAPTURED: Dict[int, torch.Tensor] = {}
 _RETIRED_WORKSPACES: list = []
+_FRAGMENT = torch.library.Library("sglang_exl3", "FRAGMENT")
 
 
 def _stream_ptr(t: torch.Tensor) -> int:
@@ -83,6 +84,8 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
             _RETIRED_WORKSPACES.append((key, ws))
         ws = torch.zeros(size, dtype=torch.uint8, device=device)
         _WORKSPACES[key] = ws
+        if _OPS_REGISTERED:
+            torch.ops.sglang_exl3.keep_workspace(ws, key[1])
     elif capturing:
         _CAPTURED[id(ws)] = ws
     return ws
@@ -540,6 +543,12 @@ def register_custom_ops() -> bool:
                   mcg: bool, mmode: int = 1) -> torch.Tensor:
         return exl3_gemv_impl(x, trellis, suh, svh, K, mcg, mmode)
 
+    @torch.library.custom_op("sglang_exl3::exl3_gemv_general", mutates_args=())
+    def exl3_gemv_general(x: torch.Tensor, trellis: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor, K: int,
+                          mcg: bool, mmode: int = 1) -> torch.Tensor:
+        return exl3_gemv_impl(x, trellis, suh, svh, K, mcg, mmode)
+
+    @exl3_gemv_general.register_fake
     @exl3_gemv.register_fake
     def _(x, trellis, suh, svh, K, mcg, mmode=1):
         out_dim = svh.size(0) if svh.ndim == 1 else trellis.size(1) * 16
@@ -570,6 +579,12 @@ def register_custom_ops() -> bool:
                         svh: List[torch.Tensor], K: int, codebook: int, out_bf16: bool) -> torch.Tensor:
         return exl3_linear_cat_impl(x, trellis, suh, svh, K, codebook, out_bf16)
 
+    @torch.library.custom_op("sglang_exl3::exl3_linear_cat_general", mutates_args=())
+    def exl3_linear_cat_general(x: torch.Tensor, trellis: List[torch.Tensor], suh: List[torch.Tensor],
+                                svh: List[torch.Tensor], K: int, codebook: int, out_bf16: bool) -> torch.Tensor:
+        return exl3_linear_cat_impl(x, trellis, suh, svh, K, codebook, out_bf16)
+
+    @exl3_linear_cat_general.register_fake
     @exl3_linear_cat.register_fake
     def _(x, trellis, suh, svh, K, codebook, out_bf16):
         rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
@@ -646,6 +661,14 @@ def register_custom_ops() -> bool:
         return exl3_gate_up_swiglu_impl(x, suh, gate_trellis, gate_svh, up_trellis, up_svh, K, codebook,
                                         swiglu_limit)
 
+    @torch.library.custom_op("sglang_exl3::exl3_gate_up_swiglu_general", mutates_args=())
+    def exl3_gate_up_swiglu_general(x: torch.Tensor, suh: torch.Tensor, gate_trellis: torch.Tensor,
+                                    gate_svh: torch.Tensor, up_trellis: torch.Tensor, up_svh: torch.Tensor, K: int,
+                                    codebook: int, swiglu_limit: float = 0.0) -> torch.Tensor:
+        return exl3_gate_up_swiglu_impl(x, suh, gate_trellis, gate_svh, up_trellis, up_svh, K, codebook,
+                                        swiglu_limit)
+
+    @exl3_gate_up_swiglu_general.register_fake
     @exl3_gate_up_swiglu.register_fake
     def _(x, suh, gate_trellis, gate_svh, up_trellis, up_svh, K, codebook, swiglu_limit=0.0):
         rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
@@ -670,6 +693,11 @@ def register_custom_ops() -> bool:
     def _(a, packed, out, svh, token_idx, route_weight, K, mcg, mul1):
         return None
 
+    # the native path of the *_general twins' operators (csrc/torch_ops.cpp), and the workspaces it runs on
+    _FRAGMENT.define("keep_workspace(Tensor ws, int stream) -> ()")
+    _lib.load_ops()
     _OPS_REGISTERED = True
+    for (_, stream), ws in _WORKSPACES.items():
+        torch.ops.sglang_exl3.keep_workspace(ws, stream)
     logger.info("registered sglang_exl3 custom ops (gfx950 HIP backend)")
     return True
