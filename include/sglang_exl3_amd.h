@@ -152,7 +152,8 @@ int exl3_gemm(const uint16_t* x, const int16_t* trellis, const uint16_t* suh, co
 /* Scratch bytes exl3_gemm needs for m rows: the GEMV workspace where the
  * GEMV kernels run, above that the prefill scratch (rotated input m*k fp16
  * and its per-128 row sums, then the k-splits' fp32 partial tiles or the
- * wide kernel's tail hand-off).  It depends on the current device's CU
+ * wide kernel's tail hand-off).  Above 16 rows exl3_gemm also runs, with
+ * fewer k-splits, in a workspace that holds just the rotated rows.  It depends on the current device's CU
  * count.  The workspace must start zero-filled (counters), as for exl3_gemv;
  * every call leaves the counters zero. */
 size_t exl3_gemm_workspace_size(int m, int k, int n, int K);
@@ -209,10 +210,11 @@ size_t exl3_gate_up_workspace_size(int m, int k, int n, int K);
  * reference's batched decode path returns them, exl3.py:1018-1034); above,
  * the input is rotated once and an MFMA kernel computes both projections of
  * a column block and applies the SwiGLU in its epilogue (g and u in fp32):
- * up to 160 rows the narrow kernel in gate/up mode (its k-splits hand fp32
- * partial tiles to the last split of each column block and row tile, or,
- * from 6 to 16 rows, to a finish launch that completes every row), above
- * it the wide-tile kernel, one workgroup holding the gate and up columns.  Replaces the gate/up half of
+ * up to 16 rows the narrow kernel in gate/up mode (its k-splits hand fp32
+ * partial tiles to the last split of each column block, or, from 6 rows, to
+ * a finish launch that completes every row), above it tall tiles with the
+ * finish launch or with gate and up in one workgroup.  A workspace that only
+ * holds the rotated rows is taken too (fewer splits).  Replaces the gate/up half of
  * apply_exl3_batched_fat (src/sglang_exl3/exl3.py:1154-1206). */
 int exl3_gate_up_swiglu(const uint16_t* x, const uint16_t* suh, const int16_t* gate_trellis,
                         const uint16_t* gate_svh, const int16_t* up_trellis, const uint16_t* up_svh,

@@ -228,7 +228,9 @@ double tall_cost(int M, int k, int n, int mt, int S) {
     return t;
 }
 
-bool plan_tall(int M, int k, int n, FatPlan* pl) {
+// limit: bytes for partial tiles; what does not fit is not chosen (one split
+// needs none).
+bool plan_tall(int M, int k, int n, FatPlan* pl, size_t limit) {
     const int forced = env_int("EXL3_FAT_TALL", -1), fs = env_int("EXL3_FAT_SPLITS", 0);
     if (forced < 0 && (fat_wide_mode() == 2 || !fat_handoff_on() || env_int("EXL3_FAT_MT", 0) != 0)) return false;
     if (forced == 0 || (forced < 0 && M < (n <= kTallNarrowCols ? kTallMinRowsNarrow : kTallMinRows))) return false;
@@ -239,6 +241,7 @@ bool plan_tall(int M, int k, int n, FatPlan* pl) {
         for (int S = 1; S <= kTallMaxSplits && ksteps % (2 * S) == 0; S *= 2) {
             if (fs > 0 && S != fs && ksteps % (2 * fs) == 0) continue;
             const double c = tall_cost(M, k, n, mt, S);
+            if (S > 1 && (size_t)S * M * n * 4 > limit) continue;
             if (c < best - 1e-9) {
                 best = c;
                 *pl = FatPlan{mt, S, true};
@@ -251,11 +254,11 @@ bool plan_tall(int M, int k, int n, FatPlan* pl) {
 // f16out: a call with fp16 output (exl3_gemm), whose narrow k-splits use the
 // partial-tile hand-off (fat_handoff) unless EXL3_FAT_HANDOFF=0.
 // n256: every matrix of the call is a multiple of 256 columns wide.
-FatPlan plan_fat(int M, int k, int n, bool f16out, bool n256) {
+FatPlan plan_fat(int M, int k, int n, bool f16out, bool n256, size_t limit = SIZE_MAX) {
     FatPlan pl{};
     const int ksteps = k / 64;
     pl.splits = 1;
-    if (f16out && plan_tall(M, k, n, &pl)) return pl;
+    if (f16out && plan_tall(M, k, n, &pl, limit)) return pl;
     if (fat_wide_allowed() && M > kFatNarrowMaxRows && n256 &&
         (fat_wide_mode() == 2 || (long long)(n / FB_COLS) * ((M + FB_ROWS - 1) / FB_ROWS) >= kFatWideMinTiles)) {
         pl.mt = FAT_MT_WIDE;
@@ -317,8 +320,8 @@ bool fat_handoff(const FatPlan& pl, int m, int n) {
 // Plan of an fp16-output call over `mats` matrices: several matrices do not
 // take the fp32 atomics (only reached by the tuning overrides), so such a plan
 // runs unsplit.
-FatPlan plan_rows(int m, int k, int n, int mats, bool n256, bool f16out = true) {
-    FatPlan pl = plan_fat(m, k, n, f16out, n256);
+FatPlan plan_rows(int m, int k, int n, int mats, bool n256, bool f16out = true, size_t limit = SIZE_MAX) {
+    FatPlan pl = plan_fat(m, k, n, f16out, n256, limit);
     if (mats > 1 && pl.splits > 1 && !fat_handoff(pl, m, n)) pl.splits = 1;
     return pl;
 }
@@ -352,8 +355,8 @@ int run_fat(const uint16_t* a, const int16_t* trellis, float* out32, __half* out
             const int64_t* token_idx, const uint16_t* route_w, int M, int k, int n, int K, int cb, bool zero_first,
             hipStream_t st, int tail = 0, char* tail_part = nullptr, int* tail_sync = nullptr,
             const float* rowsum = nullptr, float* partials = nullptr, int* counters = nullptr,
-            const MatSet* mats = nullptr, int y_bf16 = 0) {
-    const FatPlan pl = mats ? plan_rows(M, k, n, mats->count, mats_n256(*mats), out16 != nullptr)
+            const MatSet* mats = nullptr, int y_bf16 = 0, const FatPlan* plan = nullptr) {
+    const FatPlan pl = plan ? *plan : mats ? plan_rows(M, k, n, mats->count, mats_n256(*mats), out16 != nullptr)
                             : plan_fat(M, k, n, out16 != nullptr, n % FB_COLS == 0);
     FatParams p{};
     if (mats && mats->count > 1) p.mats = *mats;
@@ -424,24 +427,31 @@ size_t fat_xr_bytes(int m, int k) { return fat_xr_only_bytes(m, k) + (((size_t)m
 // [counters][accumulators][xr][split partial tiles S*m*n fp32 (narrow
 // hand-off) | out fp32 m*n (wide plan with k-splits) | tail-split hand-off
 // tiles (unsplit wide launch)].
-size_t fat_gemm_scratch_bytes(int m, int k, int n, int mats, bool n256) {
-    const FatPlan pl = plan_rows(m, k, n, mats, n256);
+size_t fat_gemm_plan_bytes(const FatPlan& pl, int m, int k, int n, int mats) {
     const bool split = pl.splits > 1;
     const size_t tail = (!split && pl.mt == FAT_MT_WIDE) ? fat_tail_bytes(wide_tail_tiles(m, k, n, false)) : 0;
     const size_t out = fat_handoff(pl, m, n) ? (size_t)pl.splits * m * n * 4 : (size_t)m * n * 4;
     return kWsScratchOffset + fat_xr_bytes(m * mats, k) + (split ? out : tail);
 }
+size_t fat_gemm_scratch_bytes(int m, int k, int n, int mats, bool n256) {
+    return fat_gemm_plan_bytes(plan_rows(m, k, n, mats, n256), m, k, n, mats);
+}
 
 int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_t* y, int m, int k, int n, int K,
                   int cb, int x_bf16, int y_bf16, void* ws, size_t ws_bytes, hipStream_t st) {
     const bool n256 = mats_n256(mats);
-    const size_t need = fat_gemm_scratch_bytes(m, k, n, mats.count, n256);
+    FatPlan pl = plan_rows(m, k, n, mats.count, n256);
+    size_t need = fat_gemm_plan_bytes(pl, m, k, n, mats.count);
+    const size_t base = kWsScratchOffset + fat_xr_bytes(m * mats.count, k);
+    if (pl.tall && ws_bytes < need && ws_bytes >= base) {  // a buffer sized for other rows: the splits that fit
+        pl = plan_rows(m, k, n, mats.count, n256, true, ws_bytes - base);
+        need = fat_gemm_plan_bytes(pl, m, k, n, mats.count);
+    }
     EXL3_REQUIRE_CODE(ws && ws_bytes >= need, EXL3_ERR_WORKSPACE,
                       "%s: %zu workspace bytes needed for m=%d, %zu given", fn, need, m, ws ? ws_bytes : (size_t)0);
     const size_t xrows = (size_t)m * mats.count;
     __half* xr = reinterpret_cast<__half*>(reinterpret_cast<char*>(ws) + kWsScratchOffset);
     float* o32 = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + kWsScratchOffset + fat_xr_bytes((int)xrows, k));
-    const FatPlan pl = plan_rows(m, k, n, mats.count, n256);
     float* rs = fat_raw(cb, pl.mt, false, pl.tall)
                     ? reinterpret_cast<float*>(reinterpret_cast<char*>(xr) + fat_xr_only_bytes((int)xrows, k))
                     : nullptr;
@@ -456,14 +466,14 @@ int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_
         const int tail = pl.mt == FAT_MT_WIDE ? wide_tail_tiles(m, k, n, false) : 0;
         return run_fat(reinterpret_cast<const uint16_t*>(xr), trellis, nullptr, reinterpret_cast<__half*>(y), svh,
                        nullptr, nullptr, m, k, n, K, cb, false, st, tail, reinterpret_cast<char*>(o32),
-                       reinterpret_cast<int*>(ws), rs, nullptr, nullptr, &mats, y_bf16);
+                       reinterpret_cast<int*>(ws), rs, nullptr, nullptr, &mats, y_bf16, &pl);
     }
     if (fat_handoff(pl, m, n))
         return run_fat(reinterpret_cast<const uint16_t*>(xr), trellis, nullptr, reinterpret_cast<__half*>(y), svh,
                        nullptr, nullptr, m, k, n, K, cb, false, st, 0, nullptr, nullptr, rs, o32,
-                       reinterpret_cast<int*>(ws), &mats, y_bf16);
+                       reinterpret_cast<int*>(ws), &mats, y_bf16, &pl);
     rc = run_fat(reinterpret_cast<const uint16_t*>(xr), trellis, o32, nullptr, svh, nullptr, nullptr, m, k, n, K, cb,
-                 true, st, 0, nullptr, nullptr, rs, nullptr, nullptr, &mats);
+                 true, st, 0, nullptr, nullptr, rs, nullptr, nullptr, &mats, 0, &pl);
     if (rc) return rc;
     const size_t n2 = (size_t)m * n / 2;
     f32_to_f16_kernel<<<(unsigned)((n2 + 255) / 256 < 8192 ? (n2 + 255) / 256 : 8192), 256, 0, st>>>(
@@ -521,7 +531,8 @@ double gu_fused_cost(int m, int k, int n) {
 // partial tiles 13.0).
 // Env EXL3_GU_TALL: 128 / 256 partial tiles of that height (with
 // EXL3_FAT_SPLITS), 1 fused.
-GateUpFatPlan plan_gate_up_fat(int m, int k, int n) {
+// limit: bytes for partial tiles, as for plan_tall (the fused kernel needs none).
+GateUpFatPlan plan_gate_up_fat(int m, int k, int n, size_t limit = SIZE_MAX) {
     const int ksteps = k / 64;
     if (m > 16) {
         const int forced = env_int("EXL3_GU_TALL", 0), fs = env_int("EXL3_FAT_SPLITS", 0);
@@ -535,6 +546,7 @@ GateUpFatPlan plan_gate_up_fat(int m, int k, int n) {
                 if (fs > 0 && S != fs && ksteps % (2 * fs) == 0) continue;
                 double c = tall_cost(m, k, 2 * n, mt, S);
                 if (S == 1) c += 3.0 + (double)m * n * 16.0 / 5.0e6;  // the finish launch all the same
+                if ((size_t)2 * S * m * n * 4 > limit) continue;
                 if (c < cost - 1e-9) {
                     cost = c;
                     best = GateUpFatPlan{mt, S, true, false, 1};
@@ -561,8 +573,7 @@ GateUpFatPlan plan_gate_up_fat(int m, int k, int n) {
     return pl;
 }
 
-size_t fat_gate_up_scratch_bytes(int m, int k, int n) {
-    const GateUpFatPlan pl = plan_gate_up_fat(m, k, n);
+size_t fat_gate_up_plan_bytes(const GateUpFatPlan& pl, int m, int k, int n) {
     size_t b = kWsScratchOffset + fat_xr_bytes(m, k);
     if (pl.fused) return b;
     if (pl.mt == FAT_MT_WIDE) b += fat_tail_bytes(wide_tail_tiles(m, k, n, true));
@@ -570,11 +581,20 @@ size_t fat_gate_up_scratch_bytes(int m, int k, int n) {
     return b;
 }
 
+size_t fat_gate_up_scratch_bytes(int m, int k, int n) {
+    return fat_gate_up_plan_bytes(plan_gate_up_fat(m, k, n), m, k, n);
+}
+
 int fat_gate_up_rows(const uint16_t* x, const uint16_t* suh, const int16_t* gate_trellis, const uint16_t* gate_svh,
                      const int16_t* up_trellis, const uint16_t* up_svh, uint16_t* out, int m, int k, int n, int K,
                      int cb, float limit, void* ws, size_t ws_bytes, hipStream_t st) {
-    const GateUpFatPlan pl = plan_gate_up_fat(m, k, n);
-    const size_t need = fat_gate_up_scratch_bytes(m, k, n);
+    GateUpFatPlan pl = plan_gate_up_fat(m, k, n);
+    size_t need = fat_gate_up_plan_bytes(pl, m, k, n);
+    const size_t base = kWsScratchOffset + fat_xr_bytes(m, k);
+    if (pl.tall && ws_bytes < need && ws_bytes >= base) {  // a buffer sized for other rows: what fits
+        pl = plan_gate_up_fat(m, k, n, ws_bytes - base);
+        need = fat_gate_up_plan_bytes(pl, m, k, n);
+    }
     EXL3_REQUIRE_CODE(ws && ws_bytes >= need, EXL3_ERR_WORKSPACE,
                       "exl3_gate_up_swiglu: %zu workspace bytes needed for m=%d, %zu given", need, m,
                       ws ? ws_bytes : (size_t)0);

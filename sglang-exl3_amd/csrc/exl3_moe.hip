@@ -1068,7 +1068,10 @@ int run_moe(const char* fn, const uint16_t* x, const int32_t* ids, const void* w
     for (int j = 0; j < 9; ++j) tabs_ok = tabs_ok && tb.t[j];
     EXL3_REQUIRE(x && ids && weights && out && tabs_ok, "%s: null pointer", fn);
     EXL3_REQUIRE(aligned(x, 4) && aligned(out, 4), "%s: misaligned x/out", fn);
-    if (moe_use_prefill(tokens, topk, E, hidden, inter, moe_use_tall(KG, KU)))
+    // a buffer sized for another batch that only the decode path fits keeps that path
+    if (moe_use_prefill(tokens, topk, E, hidden, inter, false) ||
+        (moe_use_prefill(tokens, topk, E, hidden, inter, moe_use_tall(KG, KU)) &&
+         ws_bytes >= prefill_layout(tokens, topk, E, hidden, inter).total))
         return run_moe_prefill(fn, x, ids, weights, weights_f16, tb, E, out, tokens, topk, hidden, inter, KG, KU, KD,
                                cb, limit, bf16, ws, ws_bytes, st);
     return run_moe_decode(fn, x, ids, weights, weights_f16, tb, E, out, tokens, topk, hidden, inter, KG, KU, KD, cb,

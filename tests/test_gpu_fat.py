@@ -278,6 +278,39 @@ def test_tall_tiles(m, k, n, K, cb, splits, mt, monkeypatch):
     assert torch.equal(odd[2:].view(m, n), y)
 
 
+@pytest.mark.parametrize("m", [40, 200])
+def test_tall_tiles_take_the_splits_that_fit(m):
+    """A workspace that holds the rotated rows but not all the partial tiles the plan wants (a buffer sized for
+    other rows): plain and gate/up calls run with what fits, against the oracle; one without room for the rows
+    is refused."""
+    k, n, K = 2048, 256, 3
+    print(f"case: small workspace m={m}", flush=True)
+    lib = _lib.lib()
+    tg, su, sg = make_weight(k, n, K, seed=m)
+    tu, _, sv_u = make_weight(k, n, K, seed=m + 1)
+    sg, sv_u = ((v.astype(np.float32) * np.float32(4.0 / np.sqrt(k))).astype(np.float16) for v in (sg, sv_u))
+    x = make_x(m, k, seed=m)
+    xd, sud, tgd, sgd, tud, svd = (torch.from_numpy(v).cuda() for v in (x, su, tg, sg, tu, sv_u))
+    base = (256 << 10) + (4 << 20) + m * k * 2 + ((m * (k // 128) * 4 + 255) & ~255)
+    g = oracle.matmul(x, oracle.dequant(tg, su, sg, K, 1, rtz=True))
+    u = oracle.matmul(x, oracle.dequant(tu, su, sv_u, K, 1, rtz=True))
+    st = int(torch.cuda.current_stream().cuda_stream)
+    assert base < lib.exl3_gemm_workspace_size(m, k, n, K) and base < lib.exl3_gate_up_workspace_size(m, k, n, K)
+    for size in (base - 256, base, base + 2 * m * n * 4):
+        ws = torch.zeros(size, dtype=torch.uint8, device="cuda")
+        y, z = (torch.zeros((m, n), dtype=torch.float16, device="cuda") for _ in range(2))
+        rc = lib.exl3_gemm(xd.data_ptr(), tgd.data_ptr(), sud.data_ptr(), sgd.data_ptr(), y.data_ptr(), m, k, n, K, 1,
+                           ws.data_ptr(), size, st)
+        rc2 = lib.exl3_gate_up_swiglu(xd.data_ptr(), sud.data_ptr(), tgd.data_ptr(), sgd.data_ptr(), tud.data_ptr(),
+                                      svd.data_ptr(), z.data_ptr(), m, k, n, K, 1, 0.0, ws.data_ptr(), size, st)
+        if size < base:
+            assert rc == rc2 == _lib.EXL3_ERR_WORKSPACE
+            continue
+        assert rc == rc2 == _lib.EXL3_OK
+        check_close(y.float().cpu().numpy(), g, f"gemm m={m} in {size} bytes")
+        check_close(z.float().cpu().numpy(), oracle.swiglu(g, u, float("inf")), f"gate/up m={m} in {size} bytes")
+
+
 @pytest.mark.parametrize("kind", ["1", "128", "256"])
 @pytest.mark.parametrize("m,k,n,K,cb,splits,limit", [
     (17, 128, 128, 1, 1, 1, 0.0), (31, 256, 384, 2, 2, 2, 1.0), (32, 512, 128, 3, 0, 4, 0.0),
