@@ -937,7 +937,11 @@ PrefillLayout prefill_layout(int tokens, int topk, int E, int hidden, int inter)
 // the prefill path; every batch above the decode path's entry limit does.
 // 64-row tiles pay from 16 rows; 128-row tiles (gate and up of one bit width) from
 // 5, if the active experts' projections are at least 2^25 weights each, below
-// which the path's five launches (~30 us) cost more than its tiles save.
+// which the path's five launches (~30 us) cost more than its tiles save, and rows
+// and outputs are bfloat16: the tiles round a decoded weight to fp16 where the
+// decode path's pair form sums its two halves exactly, which an fp16 output
+// shows (160 experts, 15 rows: error against 64 bits 6.1e-4 -> 6.5e-4) and a
+// bfloat16 one does not (1.8e-3 either way).
 // Graph-timed, us, 64-row tiles / 128-row tiles / decode path: config 4 (skewed
 // router, 201M weights), 64 tokens (4 rows) 122 / 82 / 83, 96 (6 rows) 123 / 87 / 106,
 // 128 128 / 95 / 126, 256 144 / 108 / 204, 512 182 / 157 / 358; 16 experts, hidden 2048,
@@ -1070,7 +1074,7 @@ int run_moe(const char* fn, const uint16_t* x, const int32_t* ids, const void* w
     EXL3_REQUIRE(aligned(x, 4) && aligned(out, 4), "%s: misaligned x/out", fn);
     // a buffer sized for another batch that only the decode path fits keeps that path
     if (moe_use_prefill(tokens, topk, E, hidden, inter, false) ||
-        (moe_use_prefill(tokens, topk, E, hidden, inter, moe_use_tall(KG, KU)) &&
+        (moe_use_prefill(tokens, topk, E, hidden, inter, bf16 && moe_use_tall(KG, KU)) &&
          ws_bytes >= prefill_layout(tokens, topk, E, hidden, inter).total))
         return run_moe_prefill(fn, x, ids, weights, weights_f16, tb, E, out, tokens, topk, hidden, inter, KG, KU, KD,
                                cb, limit, bf16, ws, ws_bytes, st);
@@ -1085,7 +1089,7 @@ using namespace exl3;
 
 extern "C" size_t exl3_moe_workspace_size(int tokens, int topk, int num_experts, int hidden, int inter) {
     if (tokens < 1 || topk < 1 || num_experts < 1 || hidden < 128 || inter < 128) return 0;
-    // room for either path where the bit widths decide (K is not known here)
+    // room for either path where bit widths and types decide (they are not known here)
     size_t need = 0;
     if (moe_use_prefill(tokens, topk, num_experts, hidden, inter, true))
         need = prefill_layout(tokens, topk, num_experts, hidden, inter).total;

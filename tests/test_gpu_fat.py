@@ -278,6 +278,27 @@ def test_tall_tiles(m, k, n, K, cb, splits, mt, monkeypatch):
     assert torch.equal(odd[2:].view(m, n), y)
 
 
+@pytest.mark.parametrize("m,k,cb", [(17, 384, 1), (33, 128, 2), (70, 1152, 2)])
+def test_rotation_of_dword_aligned_rows(m, k, cb):
+    """The input rotation's 16-byte loads on x and suh that are only 4-byte aligned, with chunk counts that do not
+    fill its waves (51, 33, 630), and the chunk sums that mul1 tiles read: the aligned call's bits, fp16 and bf16."""
+    n, K = 128, 4
+    print(f"case: rotation alignment m={m} k={k} cb={cb}", flush=True)
+    tr, su, sv = (torch.from_numpy(v).cuda() for v in make_weight(k, n, K, seed=m))
+    xs = torch.from_numpy(make_x(m, k, seed=m)).cuda()
+    su_odd = torch.zeros(k + 2, dtype=torch.float16, device="cuda")
+    su_odd[2:] = su
+    for dtype in (torch.float16, torch.bfloat16):
+        x = xs.to(dtype)
+        x_odd = torch.zeros(m * k + 2, dtype=dtype, device="cuda")
+        x_odd[2:] = x.reshape(-1)
+        cat = torch.ops.sglang_exl3.exl3_linear_cat
+        want = cat(x, [tr], [su], [sv], K, cb, False)
+        assert torch.equal(cat(x_odd[2:].view(m, k), [tr], [su_odd[2:]], [sv], K, cb, False), want)
+    ref = oracle.matmul(xs.cpu().numpy(), oracle.dequant(*(t.cpu().numpy() for t in (tr, su, sv)), K, cb, rtz=True))
+    check_close(cat(xs, [tr], [su], [sv], K, cb, False).float().cpu().numpy(), ref, f"rotation m={m} k={k}")
+
+
 @pytest.mark.parametrize("m", [40, 200])
 def test_tall_tiles_take_the_splits_that_fit(m):
     """A workspace that holds the rotated rows but not all the partial tiles the plan wants (a buffer sized for
