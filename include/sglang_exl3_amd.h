@@ -166,9 +166,12 @@ size_t exl3_linear_cat_workspace_size(int m, int k, const int* n, int count, int
  * outputs side by side: y[m][n[0] + n[1] + ..] = [x . W_0 | x . W_1 | ..], any
  * m >= 1, each weight with its own suh and svh.  x_dtype and y_dtype:
  * EXL3_DTYPE_F16 or EXL3_DTYPE_BF16; bfloat16 inputs are rounded to f16, and a
- * bfloat16 output is the f16 result rounded, as casts around exl3_gemm give
- * it.  trellis / suh / svh / n: host arrays of `count` entries.  The kernels
- * and row thresholds are exl3_gemm's for the width of the whole output.
+ * bfloat16 output is the f16 result rounded, as casts around the call would
+ * round them.  trellis / suh / svh / n: host arrays of `count` entries.  The
+ * kernels are exl3_gemm's, planned for the width of the whole output: sums run
+ * in another order than in one exl3_gemm per weight, so the bits differ.  MCG
+ * and 3INST calls leave the GEMV, which multiplies by unrounded codebook values,
+ * at the row count of the narrowest weight.
  * Replaces the linear per output shard with the casts and torch.cat around
  * them (src/sglang_exl3/dense.py:317-371). */
 int exl3_linear_cat(const void* x, int x_dtype, const int16_t* const* trellis, const uint16_t* const* suh,

@@ -315,11 +315,24 @@ MatSet one_mat(const int16_t* trellis, const uint16_t* suh, const uint16_t* svh,
     return s;
 }
 
-// exl3_linear_cat takes the GEMV kernels up to exl3_gemm's row count for the
-// whole output's width (unless the GEMV would rotate its rows in a launch of
-// its own, which holds one matrix's rows).
-bool cat_gemv(int m, int k, int n, int K) {
-    return m <= gemm_gemv_rows(n) && m <= kMaxGemvRows && !gemv_pre_rotates(plan_gemv(m, k, n, K, 1), m, 1);
+// exl3_linear_cat takes the GEMV kernels (unless the GEMV would rotate its rows
+// in a launch of its own, which holds one matrix's rows) up to the row count at
+// which exl3_gemm leaves them
+//   * for its narrowest matrix, for MCG and 3INST: the pair form adds the two
+//     fp16 halves of a codebook value in the MFMA, the tiles round the sum to
+//     fp16 first, so a matrix keeps the pair form as long as it has it alone;
+//   * for the whole output's width, for mul1, whose tiles read exact raw
+//     entries.
+// k = 1024, n = 8192 + 4096, MCG, 12 rows: error of an fp16 output against 64 bits
+// 2.1e-4 (pair form), 3.1e-4 (tiles).
+bool cat_gemv(int m, int k, const int* n, int count, int K, int cb) {
+    int total = 0, narrow = n[0];
+    for (int j = 0; j < count; ++j) {
+        total += n[j];
+        narrow = n[j] < narrow ? n[j] : narrow;
+    }
+    return m <= gemm_gemv_rows(cb == EXL3_CB_MUL1 ? total : narrow) && m <= kMaxGemvRows &&
+           !gemv_pre_rotates(plan_gemv(m, k, total, K, 1), m, 1);
 }
 
 // ----------------------------- dense gate + up on the GEMV kernel (m <= 64)
@@ -490,8 +503,15 @@ extern "C" size_t exl3_linear_cat_workspace_size(int m, int k, const int* n, int
         total += n[j];
         n256 = n256 && n[j] % 256 == 0;
     }
-    if (cat_gemv(m, k, total, K)) return exl3_gemv_workspace_size(m, k, total, K, 1);
-    return fat_gemm_scratch_bytes(m, k, total, count, n256);
+    // room for either path where the codebook decides (it is not known here)
+    size_t need = 0;
+    const bool wide = cat_gemv(m, k, n, count, K, EXL3_CB_MUL1), narrow = cat_gemv(m, k, n, count, K, EXL3_CB_MCG);
+    if (wide || narrow) need = exl3_gemv_workspace_size(m, k, total, K, 1);
+    if (!wide || !narrow) {
+        const size_t f = fat_gemm_scratch_bytes(m, k, total, count, n256);
+        need = need > f ? need : f;
+    }
+    return need;
 }
 
 extern "C" int exl3_linear_cat(const void* x, int x_dtype, const int16_t* const* trellis, const uint16_t* const* suh,
@@ -523,7 +543,7 @@ extern "C" int exl3_linear_cat(const void* x, int x_dtype, const int16_t* const*
     EXL3_REQUIRE(total <= (1 << 30), "exl3_linear_cat: %lld columns", total);
     const int nt = (int)total, xb = x_dtype == EXL3_DTYPE_BF16, yb = y_dtype == EXL3_DTYPE_BF16;
     hipStream_t st = as_stream(stream);
-    if (!cat_gemv(m, k, nt, K))
+    if (!cat_gemv(m, k, n, count, K, codebook))
         return fat_gemm_rows("exl3_linear_cat", static_cast<const uint16_t*>(x), s, static_cast<uint16_t*>(y), m, k, nt,
                              K, codebook, xb, yb, workspace, workspace_bytes, st);
     GemvParams p = base_params(static_cast<const uint16_t*>(x), trellis[0], suh[0], svh[0], static_cast<uint16_t*>(y), m,

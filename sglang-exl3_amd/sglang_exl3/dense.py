@@ -169,6 +169,32 @@ def _cat_compatible(linears: list, *dtypes: torch.dtype) -> bool:
             and all(b.K == a.K and b.codebook == a.codebook and b.in_features == a.in_features for b in linears[1:]))
 
 
+def _batched_pair(linears: list) -> Optional[tuple]:
+    """The two shards of a 2- or 3-shard layer (gate/up, k/v) that run as one
+    batched launch, or None."""
+    if len(linears) in (2, 3) and _pair_compatible(linears[-2], linears[-1]):
+        return linears[-2], linears[-1]
+    return None
+
+
+def _gemv_rows(width: int) -> int:
+    """Rows up to which exl3_gemm runs the pair-form GEMV (csrc/exl3_gemv.hip, gemm_gemv_rows)."""
+    return 12 if width < 12288 else (8 if width < 24576 else 7)
+
+
+def _cat_exact(linears: list, rows: int) -> bool:
+    """Whether exl3_linear_cat multiplies by weights as exact as the separate
+    calls do.  The GEMV and the batched launch (pair form) add the two fp16
+    halves of an MCG codebook value exactly; the MFMA tiles round the sum to
+    fp16 (error of an fp16 output against 64 bits: 2.1e-4 -> 3.1e-4).
+    exl3_linear_cat leaves the GEMV at the row count of the narrowest shard,
+    which is where separate calls leave it too, except a batched pair, which
+    keeps the pair form up to FUSED_PAIR_MAX_ROWS rows.  mul1 tiles read exact
+    entries."""
+    return (linears[0].codebook != _lib.CB_MCG or _batched_pair(linears) is None
+            or rows <= _gemv_rows(min(lin.out_features for lin in linears)) or rows > FUSED_PAIR_MAX_ROWS)
+
+
 class EXL3LinearMethod(LinearMethodBase):
     """SGLang linear method running dense EXL3 weights on the HIP kernels."""
 
@@ -278,7 +304,7 @@ class EXL3LinearMethod(LinearMethodBase):
         fuse_on = os.environ.get("SGLANG_EXL3_MGEMM", "1") != "0"
         out_dtype = getattr(layer, "_exl3_out_dtype", x.dtype)
         if x.is_cuda and (fuse_on or len(linears) == 1) and not getattr(layer, "_exl3_scale_input", False) \
-                and _cat_compatible(linears, x.dtype, out_dtype):
+                and _cat_compatible(linears, x.dtype, out_dtype) and _cat_exact(linears, math.prod(x.shape[:-1])):
             # every shard in one call, the casts inside the kernels
             from .ops import register_custom_ops
 
@@ -290,14 +316,9 @@ class EXL3LinearMethod(LinearMethodBase):
                 y = y + bias.to(out_dtype)
             return y.view(*x.shape[:-1], y.shape[-1])
         shape, rows, x2, scale = self._prepare(layer, x)
-        fuse = rows <= FUSED_PAIR_MAX_ROWS and fuse_on
-        n = len(linears)
-        if n == 2 and fuse and _pair_compatible(linears[0], linears[1]):
-            y = torch.cat(fused_pair(layer, x2, linears[0], linears[1]), dim=1)
-        elif n == 3 and fuse and _pair_compatible(linears[1], linears[2]):
-            q = linears[0].forward(x2)
-            k, v = fused_pair(layer, x2, linears[1], linears[2])
-            y = torch.cat((q, k, v), dim=1)
+        pair = _batched_pair(linears) if rows <= FUSED_PAIR_MAX_ROWS and fuse_on else None
+        if pair:
+            y = torch.cat([lin.forward(x2) for lin in linears[:-2]] + list(fused_pair(layer, x2, *pair)), dim=1)
         else:
             outs = [lin.forward(x2) for lin in linears]
             y = torch.cat(outs, dim=1) if len(outs) > 1 else outs[0]

@@ -9,7 +9,7 @@ import torch
 import torch.nn as nn
 
 import oracle
-from gpu_util import check_close, make_weight, make_x
+from gpu_util import EXACT_WEIGHTS_REL, check_close, make_weight, make_x, product64, rel_error
 from sglang_exl3 import ops
 from sglang_exl3.exl3 import (
     MCG_MARKER_SIGNED_INT32,
@@ -275,6 +275,50 @@ def test_linear_cat(m, widths, K, cb, x_dtype, y_dtype, env, monkeypatch):
         ulp = 2.0 ** (-7 if y_dtype == torch.bfloat16 else -10)
         rms = float(ref.square().mean().sqrt())
         assert torch.all((y.float() - ref).abs() <= ulp * ref.abs() + 1e-3 * rms)
+
+
+def _linear_layer(outs, k, K, cb, dtype, seed):
+    """An EXL3LinearMethod layer of seeded shards, and the shards on the device."""
+    method = EXL3LinearMethod(EXL3Config(bits=K, codebook="mul1" if cb == 2 else "mcg"), bits=K)
+    layer = nn.Module()
+    method.create_weights(layer, k, outs, k, sum(outs), dtype)
+    packs = []
+    for i, n in enumerate(outs):
+        pack = [torch.from_numpy(a).cuda() for a in _scaled(k, n, K, seed=seed + i)]
+        packs.append(pack)
+        for suffix, t in zip(("trellis", "suh", "svh"), pack):
+            method._load_linear(getattr(layer, f"exl3_{i}_{suffix}"), t, i)
+        if cb:
+            marker = "mcg" if cb == 1 else "mul1"
+            val = MCG_MARKER_SIGNED_INT32 if cb == 1 else MUL1_MARKER_SIGNED_INT32
+            method._load_linear(getattr(layer, f"exl3_{i}_{marker}"), torch.tensor(val, dtype=torch.int32), i)
+    method.process_weights_after_loading(layer)
+    return method, layer, packs
+
+
+@pytest.mark.parametrize("rows,outs,cb,exact", [
+    (8, [256, 256], 1, (0, 1)),
+    (13, [256, 256], 1, (0, 1)),              # a pair keeps the pair form to 64 rows
+    (64, [384, 384], 1, (0, 1)),
+    (13, [512, 128, 128], 1, (1, 2)), (40, [512, 128, 128], 1, (1, 2)),
+    (12, [8192, 4096], 1, (0, 1)),            # a sum of widths from 12288 on, each shard below it
+    (9, [4096, 4096, 4096, 128], 0, (0, 1, 2, 3)),
+    (12, [12288, 256], 1, (1,)),
+    (8, [24576, 128], 1, (1,)),
+    (16, [256, 256], 2, (0, 1)), (40, [512, 128, 128], 2, (0, 1, 2)), (12, [8192, 4096], 2, (0, 1)),
+])
+def test_linear_layer_weights_are_not_rounded(rows, outs, cb, exact):
+    """Shards that separate calls and the batched launch multiply by exact codebook values (the pair-form GEMV, mul1's
+    raw entries) have them in the one call too, for fp16 outputs where it shows."""
+    print(f"case: exact weights rows={rows} outs={outs} cb={cb}", flush=True)
+    k, K = 1024, 3
+    method, layer, packs = _linear_layer(outs, k, K, cb, torch.float16, seed=rows)
+    x = torch.from_numpy(make_x(rows, k, seed=rows)).cuda()
+    got = method.apply(layer, x).split(outs, dim=1)
+    for i in exact:
+        err = rel_error(got[i], product64(x, *packs[i], K, cb))
+        print(f"shard {i}: {err:.2e}", flush=True)
+        assert err < EXACT_WEIGHTS_REL
 
 
 @pytest.mark.parametrize("T,invalid", [(1, 0), (1, 1), (6, 2), (60, 0), (200, 3)])
