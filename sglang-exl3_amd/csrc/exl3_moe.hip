@@ -935,37 +935,25 @@ PrefillLayout prefill_layout(int tokens, int topk, int E, int hidden, int inter)
 
 // Rows per active expert (uniform routing estimate) from which a batch takes
 // the prefill path; every batch above the decode path's entry limit does.
-// 64-row tiles pay from 16 rows; 128-row tiles (gate and up of one bit width) from
-// 5, if the active experts' projections are at least 2^25 weights each, below
-// which the path's five launches (~30 us) cost more than its tiles save, and rows
-// and outputs are bfloat16: the tiles round a decoded weight to fp16 where the
-// decode path's pair form sums its two halves exactly, which an fp16 output
-// shows (160 experts, 15 rows: error against 64 bits 6.1e-4 -> 6.5e-4) and a
-// bfloat16 one does not (1.8e-3 either way).
-// Graph-timed, us, 64-row tiles / 128-row tiles / decode path: config 4 (skewed
-// router, 201M weights), 64 tokens (4 rows) 122 / 82 / 83, 96 (6 rows) 123 / 87 / 106,
-// 128 128 / 95 / 126, 256 144 / 108 / 204, 512 182 / 157 / 358; 16 experts, hidden 2048,
-// inter 1408, top 2, K = 4 (46M): 48 tokens (6 rows) 75 / 54 / 68, 100 90 / 56 / 78, 200
-// 108 / 64 / 119.  128-row tiles / decode path: 64 experts, 2048 x 1408 (184M), 6
-// rows: 103 / 152; 8 experts, 4096 x 14336 (470M), 6 rows: 273 / 310; 60 experts, 1024 x
-// 512 (31M), 5.3 rows: 40 / 39; 16 experts, 1024 x 1024 (16M), 6 rows: 39 / 28; 8 experts,
-// 1024 x 512 (4M), 8 rows: 33 / 25.
+// The tiles round a decoded weight to fp16 where the decode path's pair form adds
+// its two halves exactly, so a batch that ran the pair form before 128-row tiles
+// were there keeps it, although those would be faster from ~5 rows: graph-timed,
+// us, 64-row tiles / 128-row tiles / decode path, config 4 (skewed router):
+// 64 tokens (4 rows) 122 / 82 / 83, 128 128 / 95 / 126, 256 (16 rows) 144 / 108 /
+// 204, 512 182 / 157 / 358; 160 experts, 15 rows: error of an fp16 output against
+// 64 bits 6.1e-4 (decode path), 6.5e-4 (tiles).
 constexpr double kMoePrefillRowsPerExpert = 16.0;
-constexpr double kMoeTallRowsPerExpert = 5.0, kMoeTallMinWeights = 33554432.0;
 
 // Env EXL3_MOE_TALL=0: the 64-row tiles always.
 bool moe_use_tall(int KG, int KU) { return KG == KU && env_int("EXL3_MOE_TALL", 1) != 0; }
 
-bool moe_use_prefill(int tokens, int topk, int E, int hidden, int inter, bool tall) {
+bool moe_use_prefill(int tokens, int topk, int E) {
     const int forced = env_int("EXL3_MOE_PREFILL", -1);  // 0: never (decode path), 1: always
     const long long entries = (long long)tokens * topk;
     if (entries > kMoeMaxEntries) return true;
     if (forced >= 0) return forced != 0;
     const double act = expected_active(tokens, topk, E);
-    if (act <= 0) return false;
-    const double per = (double)entries / act;
-    return per >= kMoePrefillRowsPerExpert ||
-           (tall && per >= kMoeTallRowsPerExpert && act * hidden * inter >= kMoeTallMinWeights);
+    return act > 0 && (double)entries / act >= kMoePrefillRowsPerExpert;
 }
 
 int run_moe_prefill(const char* fn, const uint16_t* x, const int32_t* ids, const void* weights, int weights_f16,
@@ -1072,10 +1060,7 @@ int run_moe(const char* fn, const uint16_t* x, const int32_t* ids, const void* w
     for (int j = 0; j < 9; ++j) tabs_ok = tabs_ok && tb.t[j];
     EXL3_REQUIRE(x && ids && weights && out && tabs_ok, "%s: null pointer", fn);
     EXL3_REQUIRE(aligned(x, 4) && aligned(out, 4), "%s: misaligned x/out", fn);
-    // a buffer sized for another batch that only the decode path fits keeps that path
-    if (moe_use_prefill(tokens, topk, E, hidden, inter, false) ||
-        (moe_use_prefill(tokens, topk, E, hidden, inter, bf16 && moe_use_tall(KG, KU)) &&
-         ws_bytes >= prefill_layout(tokens, topk, E, hidden, inter).total))
+    if (moe_use_prefill(tokens, topk, E))
         return run_moe_prefill(fn, x, ids, weights, weights_f16, tb, E, out, tokens, topk, hidden, inter, KG, KU, KD,
                                cb, limit, bf16, ws, ws_bytes, st);
     return run_moe_decode(fn, x, ids, weights, weights_f16, tb, E, out, tokens, topk, hidden, inter, KG, KU, KD, cb,
@@ -1089,15 +1074,8 @@ using namespace exl3;
 
 extern "C" size_t exl3_moe_workspace_size(int tokens, int topk, int num_experts, int hidden, int inter) {
     if (tokens < 1 || topk < 1 || num_experts < 1 || hidden < 128 || inter < 128) return 0;
-    // room for either path where bit widths and types decide (they are not known here)
-    size_t need = 0;
-    if (moe_use_prefill(tokens, topk, num_experts, hidden, inter, true))
-        need = prefill_layout(tokens, topk, num_experts, hidden, inter).total;
-    if (!moe_use_prefill(tokens, topk, num_experts, hidden, inter, false)) {
-        const size_t d = moe_layout(tokens, topk, num_experts, hidden, inter).total;
-        need = need > d ? need : d;
-    }
-    return need;
+    if (moe_use_prefill(tokens, topk, num_experts)) return prefill_layout(tokens, topk, num_experts, hidden, inter).total;
+    return moe_layout(tokens, topk, num_experts, hidden, inter).total;
 }
 
 extern "C" int exl3_moe_plan(int tokens, int topk, int num_experts, int hidden, int inter, int* out) {
