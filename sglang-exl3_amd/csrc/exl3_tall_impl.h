@@ -87,13 +87,19 @@ __device__ __forceinline__ void tall_loop(float4_t (&acc)[MT / 16][2], const EXL
     uint32_t wa[K], wb[K];  // the words of this step and of the next one
     copy_a(0, 0);
     load_words<K>(tb, wa);
-    load_words<K>(tb + (size_t)(nsteps > 1 ? 1 : 0) * step_stride, wb);
-    // wait for everything but the last request, and pass the next step's words
-    // through, so that the compiler adds no wait of its own behind the copies
+    load_words<K>(tb + step_stride, wb);
+    // Wait for everything but the last weight request, and pass the next step's
+    // words through, so that the compiler adds no wait of its own behind the
+    // copies.  A request is at least WL load instructions (of 16 bytes at most)
+    // behind the step's copies, and all its words are used (after the loop, the
+    // last two's), so WL operations left in flight are never a copy.  With one
+    // for every K, each step of 5 to 8 bits waited for half of the request that it
+    // had just made.
+    constexpr int WL = (K + 3) / 4;
     auto step_end = [&](uint32_t (&wn)[K]) {
 #pragma unroll
         for (int j = 0; j < K; ++j) asm volatile("" : "+v"(wn[j]));
-        asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(WL) : "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
     step_end(wa);
@@ -144,6 +150,8 @@ __device__ __forceinline__ void tall_loop(float4_t (&acc)[MT / 16][2], const EXL
         step_body(s, std::integral_constant<int, 0>{}, wa, wb);
         step_body(s + 1, std::integral_constant<int, 1>{}, wb, wa);
     }
+#pragma unroll
+    for (int j = 0; j < K; ++j) asm volatile("" ::"v"(wa[j]), "v"(wb[j]));
 }
 
 template <int K, int CB, int MT, bool RAW>
