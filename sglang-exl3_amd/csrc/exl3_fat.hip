@@ -199,32 +199,34 @@ int wide_tail_tiles(int m, int k, int n, bool gu) {
 }
 
 // Tall tiles (tall_kernel) for fp16 / bf16 outputs: rows per tile and k-splits
-// by a cost model in us, fitted to 83 shapes from 17 to 4096 rows, 2048^2 to
-// 14336 x 4096 (graph-timed, both tile heights, 1 / 2 / 4 splits; its choice is
-// on average within 2 % of the best of the six).  With W workgroups on the
-// busiest CU, `slots` of them at once, a 64-k step of a tile with rb staged row
-// blocks takes
-//   L = 0.36 + 0.047 rb  alone (decode and MFMAs of one wave per SIMD), and
-//   C = 0.25 + 0.039 rb  per workgroup where enough share the CU;
-// splits add the finish launch and S partial tiles written and read.  Against
-// the narrow and wide kernels before it (us): k = n = 4096, 20 / 64 / 256 /
-// 1024 / 4096 rows: 21.5 / 30.0 / 35.4 / 75.1 / 176.9 -> 17.5 / 21.7 / 34.9 / 63.9 /
-// 147.4; k = 4096, n = 14336: 24.1 / 33.3 / 70.2 / 145.4 / 549.6 -> 22.9 / 32.2 /
-// 58.6 / 125.0 / 473.7; k = 14336, n = 4096, 64 / 1024 rows: 54.6 / 219.4 -> 45.7 /
-// 153.4.  Env EXL3_FAT_TALL: 0 never, 128 / 256 forced (with EXL3_FAT_SPLITS); the
+// by a cost model in us, fitted to 1600 times of both tile heights with 1 / 2 / 4 / 8
+// splits, plain and gate/up (17 to 2048 rows, 2048^2 to 4096 x 14336 and 14336 x
+// 4096, K = 3 to 8, every codebook; its choice is on average within 0.6 % of the
+// best of them, at worst 8 %).  With W workgroups on the busiest CU, `slots` of
+// them at once, a 64-k step of a tile with rb staged row blocks takes
+//   L = 0.347 + 0.064 rb  alone (decode and MFMAs of one wave per SIMD), and
+//   C = 0.269 + 0.027 rb  per workgroup where enough share the CU;
+// a tile's epilogue 0.327 rb; splits add the finish launch and S partial tiles
+// written and read.  K and codebook move a step by up to 10 %, for every choice
+// alike.  Against the narrow and wide kernels before it (us, K = 4 MCG): k = 4096, n =
+// 6144, 24 / 64 / 200 / 700 / 2048 rows: 20.7 / 29.1 / 39.6 / 98.2 / 133.9 -> 17.0 / 22.7 /
+// 37.9 / 60.8 / 113.8; k = 4096, n = 14336: 23.5 / 31.6 / 71.0 / 128.8 / 272.9 -> 23.2 /
+// 30.3 / 53.1 / 96.8 / 237.1; k = 14336, n = 4096, 64 / 1000 rows: 51.8 / 238.3 -> 33.3 /
+// 146.2.
+// Env EXL3_FAT_TALL: 0 never, 128 / 256 forced (with EXL3_FAT_SPLITS); the
 // overrides that name another kernel (EXL3_FAT_WIDE=2, _MT, _HANDOFF=0) get it.
 constexpr int kTallMaxSplits = 16;
 
 double tall_cost(int M, int k, int n, int mt, int S) {
     const int rb = 2 * (((M < mt ? M : mt) + 31) / 32), slots = mt == 128 ? 4 : 2;
-    const double L = 0.36 + 0.047 * rb, C = 0.25 + 0.039 * rb;
+    const double L = 0.347 + 0.064 * rb, C = 0.269 + 0.027 * rb;
     const long long wgs = (long long)(n / 128) * ((M + mt - 1) / mt) * S;
     const long long W = (wgs + fat_cus() - 1) / fat_cus(), full = W / slots, rest = W % slots;
     double t = (double)(full * slots) * C;
     if (t < L * (double)full) t = L * (double)full;
     if (rest) t += L > rest * C ? L : rest * C;
-    t *= k / 64 / S;
-    if (S > 1) t += 3.0 + (S > 4 ? 0.2 * (S - 4) : 0.0) + (double)S * M * n * 8.0 / 5.0e6;
+    t = t * (k / 64 / S) + 0.327 * rb * (double)(full + (rest != 0));
+    if (S > 1) t += 3.0 + (S > 4 ? 0.2 * (S - 4) : 0.0) + (double)S * M * n * 8.0 / 3.17e6;
     return t;
 }
 
@@ -545,7 +547,7 @@ GateUpFatPlan plan_gate_up_fat(int m, int k, int n, size_t limit = SIZE_MAX) {
             for (int S = 1; S <= kTallMaxSplits && ksteps % (2 * S) == 0; S *= 2) {
                 if (fs > 0 && S != fs && ksteps % (2 * fs) == 0) continue;
                 double c = tall_cost(m, k, 2 * n, mt, S);
-                if (S == 1) c += 3.0 + (double)m * n * 16.0 / 5.0e6;  // the finish launch all the same
+                if (S == 1) c += 3.0 + (double)m * n * 16.0 / 3.17e6;  // the finish launch all the same
                 if ((size_t)2 * S * m * n * 4 > limit) continue;
                 if (c < cost - 1e-9) {
                     cost = c;
