@@ -343,9 +343,8 @@ __device__ __forceinline__ uint32_t decode2_rn(uint32_t s0, uint32_t s1) {
         __half2 b = *reinterpret_cast<__half2*>(&y1);
         __half v0 = __hadd(__low2half(a), __high2half(a));
         __half v1 = __hadd(__low2half(b), __high2half(b));
-        __half2 r2 = __halves2half2(v0, v1);
-        const uint32_t r = *reinterpret_cast<uint32_t*>(&r2);
-        return r;
+        __half2 r = __halves2half2(v0, v1);
+        return *reinterpret_cast<uint32_t*>(&r);
     }
 }
 
@@ -460,9 +459,15 @@ __device__ __forceinline__ uint32_t frag_pair(const uint32_t* buf, const uint32_
     }
 }
 
-template <int K, int CB, bool RZ, int H, int C, bool RAW = false>
+// SDWA: pairs by decode4_rn.  It pays where a wave decodes beside other waves'
+// MFMAs (tall tiles) or does nothing else (dequant); in the narrow and wide MFMA
+// kernels the fixed order of its adds costs more than the instruction it saves
+// (kernel alone, k = 4096, n = 6144, MCG, K = 3 / 6: 16-row tiles 11.2 / 11.6 us
+// without, 12.8 / 13.6 with; 64-row tiles 28.2 / 28.6 and 29.0 / 29.2).
+template <int K, int CB, bool RZ, int H, int C, bool RAW = false, bool SDWA = false>
 __device__ __forceinline__ void frag_decode(const uint32_t* buf, const uint32_t* mid, uint32_t* f) {
-    if constexpr (CB != 2 && !RZ) {
+    static_assert(!SDWA || !RZ, "decode4_rn: round to nearest");
+    if constexpr (CB != 2 && SDWA) {
         constexpr int u = 16 * H + 4 * C;  // pairs (u, u + 1), (u + 2, u + 3), (u + 8, u + 9), (u + 10, u + 11)
         decode4_rn<CB>(window_mid<K, u>(buf, mid), window_mid<K, u + 1>(buf, mid), window_mid<K, u + 2>(buf, mid),
                        window_mid<K, u + 3>(buf, mid), f[0], f[1]);
@@ -481,15 +486,15 @@ __device__ __forceinline__ void frag_decode(const uint32_t* buf, const uint32_t*
 // straddling windows are cut from one middle word per word boundary (a
 // single v_bfe each instead of v_alignbit + mask: config 3 gate/up M = 16 /
 // 128 30.3 / 81.6 -> 29.6 / 79.5 us, MoE prefill 2048 tokens 528.6 -> 515.7).
-template <int K, int CB, bool RZ, bool RAW = false>
+template <int K, int CB, bool RZ, bool RAW = false, bool SDWA = false>
 __device__ __forceinline__ void decode_group(const uint32_t* buf, uint32_t frag[2][2][4]) {
     uint32_t mid[K];
 #pragma unroll
     for (int j = 0; j < K; ++j) mid[j] = __builtin_amdgcn_alignbit(buf[j], buf[j + 1], 16);
-    frag_decode<K, CB, RZ, 0, 0, RAW>(buf, mid, frag[0][0]);
-    frag_decode<K, CB, RZ, 1, 0, RAW>(buf, mid, frag[0][1]);
-    frag_decode<K, CB, RZ, 0, 1, RAW>(buf, mid, frag[1][0]);
-    frag_decode<K, CB, RZ, 1, 1, RAW>(buf, mid, frag[1][1]);
+    frag_decode<K, CB, RZ, 0, 0, RAW, SDWA>(buf, mid, frag[0][0]);
+    frag_decode<K, CB, RZ, 1, 0, RAW, SDWA>(buf, mid, frag[0][1]);
+    frag_decode<K, CB, RZ, 0, 1, RAW, SDWA>(buf, mid, frag[1][0]);
+    frag_decode<K, CB, RZ, 1, 1, RAW, SDWA>(buf, mid, frag[1][1]);
 }
 
 }  // namespace exl3

@@ -107,7 +107,7 @@ __global__ __launch_bounds__(DQ_THREADS, 4) void dequant_kernel(const uint32_t* 
 #pragma unroll
         for (int j = 1; j <= K; ++j) asm volatile("" : "+v"(buf[j]));
         uint32_t frag[2][2][4];
-        decode_group<K, CB, false>(buf, frag);
+        decode_group<K, CB, false, false, true>(buf, frag);
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll

@@ -682,14 +682,14 @@ __device__ __forceinline__ uint32_t nat_pair(const uint32_t* buf, const uint32_t
 }
 
 // f[h'][j] = tile rows (8h' + 2j, +1) of column q + 8C: run H = j >> 1, pair P = h' + 2 (j & 1).
-template <int K, int CB, int C, bool RAW>
+template <int K, int CB, int C, bool RAW, bool SDWA>
 __device__ __forceinline__ void nat_column(const uint32_t* buf, const uint32_t* mid, uint32_t (&f)[2][4]) {
-    if constexpr (CB != 2) {
+    if constexpr (CB != 2 && SDWA) {
         // the same words, run by run (frag_decode's order: word p of run H is f[p & 1][2 H + (p >> 1)])
 #define EXL3_NAT(H)                                                                      \
     {                                                                                    \
         uint32_t t[4];                                                                   \
-        frag_decode<K, CB, false, H, C>(buf, mid, t);                                    \
+        frag_decode<K, CB, false, H, C, false, true>(buf, mid, t);                       \
         f[0][2 * H] = t[0];                                                              \
         f[1][2 * H] = t[1];                                                              \
         f[0][2 * H + 1] = t[2];                                                          \
@@ -711,13 +711,13 @@ __device__ __forceinline__ void nat_column(const uint32_t* buf, const uint32_t* 
 }
 
 // Decode one 32-value group from its word buffer (buf[0] the previous word).
-template <int K, int CB, bool RAW>
+template <int K, int CB, bool RAW, bool SDWA = false>
 __device__ __forceinline__ void nat_decode(const uint32_t (&buf)[K + 1], uint32_t (&f)[2][2][4]) {
     uint32_t mid[K];
 #pragma unroll
     for (int j = 0; j < K; ++j) mid[j] = __builtin_amdgcn_alignbit(buf[j], buf[j + 1], 16);
-    nat_column<K, CB, 0, RAW>(buf, mid, f[0]);
-    nat_column<K, CB, 1, RAW>(buf, mid, f[1]);
+    nat_column<K, CB, 0, RAW, SDWA>(buf, mid, f[0]);
+    nat_column<K, CB, 1, RAW, SDWA>(buf, mid, f[1]);
 }
 
 // The same from words w[0..K-1], the previous word from lane q - 1.
