@@ -1,6 +1,7 @@
 // C ABI of the many-row EXL3 GEMM: exl3_fat_gemm, exl3_fat_gemm_scatter and
 // the prefill path of exl3_gemm (rotate -> fat GEMM -> fp16), with the launch
 // planner (rows per tile, k-splits).
+#include "exl3_rotate.h"
 #include "exl3_tall_impl.h"
 
 namespace exl3 {

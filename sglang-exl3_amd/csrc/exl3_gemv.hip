@@ -5,6 +5,7 @@
 #include <stdlib.h>
 
 #include "exl3_gemv_sk.h"
+#include "exl3_rotate.h"
 
 namespace exl3 {
 

@@ -696,53 +696,6 @@ __device__ __forceinline__ RowChunk rotate_chunk(const RowChunk& x, const RowChu
     return o;
 }
 
-namespace {
-// Input rotation of a row batch: xr = fp16( H(x (.) suh) / sqrt(128) ) (feeds the
-// k-split GEMV's pre-rotated mode and the MFMA GEMM).  A wave takes 8 chunks of
-// 128 values, 8 lanes and 32 bytes a lane each (rotate_chunk); one chunk per
-// wave, 4 bytes a lane, was bound by its instruction count: 1000 x 14336 bf16
-// 19 -> 10.7 us (57 MB).  blockIdx.y: the matrix whose suh applies; its rotated rows follow those of
-// the matrix before.
-// rs (optional): the sum of each chunk's 128 rotated fp16 values, [row][k/128]
-// per matrix (the mul1 raw-entry GEMM's affine correction).
-struct RotateSuh {
-    const __half* suh[kMaxMats];
-};
-__global__ __launch_bounds__(256) void rotate_rows_kernel(const __half* x, RotateSuh suhs, __half* xr,
-                                                          long long chunks, int k, int x_bf16, float* rs) {
-    const int lane = threadIdx.x & 63;
-    const long long chunk = ((long long)blockIdx.x * 4 + (threadIdx.x >> 6)) * 8 + (lane >> 3);
-    const long long cc = chunk < chunks ? chunk : chunks - 1;  // whole waves stay active for the lane exchanges
-    const int c = (int)((unsigned)cc % (unsigned)(k >> 7)) * 128 + (lane & 7) * 16;
-    const RowChunk o = rotate_chunk(ld_chunk(gptr(x) + cc * 128 + (lane & 7) * 16),
-                                    ld_chunk(gptr(suhs.suh[blockIdx.y]) + c), x_bf16, lane);
-    float t = 0.f;
-    if (rs) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const uint32_t u = o.v[e >> 2][e & 3];
-            const __half2 h = *reinterpret_cast<const __half2*>(&u);
-            t += __low2float(h) + __high2float(h);
-        }
-        t += lane_xor<1>(t);
-        t += lane_xor<2>(t);
-        t += lane_xor<4>(t);
-    }
-    if (chunk >= chunks) return;
-    EXL3_GLOBAL u32x4_t* dst = reinterpret_cast<EXL3_GLOBAL u32x4_t*>(
-        gptr(xr) + ((size_t)blockIdx.y * chunks + chunk) * 128 + (lane & 7) * 16);
-    dst[0] = o.v[0];
-    dst[1] = o.v[1];
-    if (rs && (lane & 7) == 0) gptr(rs)[(size_t)blockIdx.y * chunks + chunk] = t;
-}
-inline int rotate_rows(const __half* x, const RotateSuh& suhs, int mats, __half* xr, int m, int k, int x_bf16,
-                       float* rs, hipStream_t st, const char* what) {
-    const long long chunks = (long long)m * (k / 128);
-    rotate_rows_kernel<<<dim3((unsigned)((chunks + 31) / 32), mats), 256, 0, st>>>(x, suhs, xr, chunks, k, x_bf16, rs);
-    return launch_status(what);
-}
-}  // namespace
-
 // Dynamic LDS bytes of gemv_kernel for (m, k-slices per workgroup, kw).
 inline size_t gemv_smem_bytes(int m, int kts_wg, int kw) {
     const size_t xs = ((size_t)kts_wg * 4 * m * 8 * 2 + 16 + 15) & ~(size_t)15;

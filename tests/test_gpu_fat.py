@@ -278,12 +278,15 @@ def test_tall_tiles(m, k, n, K, cb, splits, mt, monkeypatch):
     assert torch.equal(odd[2:].view(m, n), y)
 
 
+@pytest.mark.parametrize("few", ["0", "1000000"])
 @pytest.mark.parametrize("m,k,cb", [(17, 384, 1), (33, 128, 2), (70, 1152, 2)])
-def test_rotation_of_dword_aligned_rows(m, k, cb):
-    """The input rotation's 16-byte loads on x and suh that are only 4-byte aligned, with chunk counts that do not
-    fill its waves (51, 33, 630), and the chunk sums that mul1 tiles read: the aligned call's bits, fp16 and bf16."""
+def test_rotation_of_dword_aligned_rows(m, k, cb, few, monkeypatch):
+    """Both input rotations (8 chunks a wave, one a wave) on x and suh that are only 4-byte aligned, with chunk counts
+    that do not fill their waves or workgroups (51, 33, 630), and the chunk sums that mul1 tiles read: the aligned
+    call's bits, fp16 and bf16."""
     n, K = 128, 4
-    print(f"case: rotation alignment m={m} k={k} cb={cb}", flush=True)
+    print(f"case: rotation alignment m={m} k={k} cb={cb} few={few}", flush=True)
+    monkeypatch.setenv("EXL3_ROTATE_FEW", few)
     tr, su, sv = (torch.from_numpy(v).cuda() for v in make_weight(k, n, K, seed=m))
     xs = torch.from_numpy(make_x(m, k, seed=m)).cuda()
     su_odd = torch.zeros(k + 2, dtype=torch.float16, device="cuda")
