@@ -94,12 +94,6 @@ struct FatPlan {
     bool tall;  // tall_kernel with mt (128 or 256) rows per tile
 };
 
-bool mats_n256(const MatSet& s) {
-    for (int j = 0; j < s.count; ++j)
-        if (s.n[j] % FB_COLS) return false;
-    return true;
-}
-
 // Wide tiles (256 x 256, fat_big_kernel) above kFatNarrowMaxRows rows (env
 // EXL3_FAT_WIDE=0 turns them off); up to there the narrow kernel with 16-row
 // tiles up to 16 rows and 64-row tiles above.  k-splits for the narrow kernel
@@ -180,11 +174,9 @@ int fat_cus() {
 // Tiles of a one-split wide-tile launch that run as two k-halves (the tail
 // split): the tiles of a last round that would fill at most half the CUs
 // (or all tiles, when there are at most half as many as CUs).  Graph-timed,
-// split vs whole (k = 4096, K = 3): gate/up n = 14336, M = 160 / 256 / 2048 /
-// 2560: 96.7 / 99.9 / 546.9 / 678.0 vs 130.4 / 133.1 / 551.9 / 696.6 us;
-// exl3_gemm n = 14336, M = 300 / 512: 91.8 / 95.4 vs 126.7 / 130.0, n = 28672,
-// M = 768 / 2048: 221.7 / 522.2 vs 257.8 / 534.1.  Env EXL3_FAT_TAIL=0 turns
-// it off.
+// split vs whole (k = 4096, K = 3): exl3_gemm n = 14336, M = 300 / 512: 91.8 /
+// 95.4 vs 126.7 / 130.0, n = 28672, M = 768 / 2048: 221.7 / 522.2 vs 257.8 /
+// 534.1.  Env EXL3_FAT_TAIL=0 turns it off.
 int fat_tail_tiles(int tiles, int ksteps) {
     if (ksteps % 4 != 0 || env_int("EXL3_FAT_TAIL", 1) == 0) return 0;
     const int c = fat_cus(), r = tiles % c;
@@ -192,11 +184,9 @@ int fat_tail_tiles(int tiles, int ksteps) {
 }
 size_t fat_tail_bytes(int tail) { return (size_t)tail * FB_TAIL_FLOATS * sizeof(float); }
 
-// Tail tiles of the wide kernel for an unsplit (m, k, n) call (gate/up mode:
-// n per projection, one tile per 128-column block of each).
-int wide_tail_tiles(int m, int k, int n, bool gu) {
-    const int tiles = (gu ? n / 128 : n / FB_COLS) * ((m + FB_ROWS - 1) / FB_ROWS);
-    return fat_tail_tiles(tiles, k / 64);
+// Tail tiles of the wide kernel for an unsplit (m, k, n) call.
+int wide_tail_tiles(int m, int k, int n) {
+    return fat_tail_tiles((n / FB_COLS) * ((m + FB_ROWS - 1) / FB_ROWS), k / 64);
 }
 
 // Tall tiles (tall_kernel) for fp16 / bf16 outputs: rows per tile and k-splits
@@ -232,11 +222,17 @@ double tall_cost(int M, int k, int n, int mt, int S) {
 }
 
 // limit: bytes for partial tiles; what does not fit is not chosen (one split
-// needs none).
-bool plan_tall(int M, int k, int n, FatPlan* pl, size_t limit) {
-    const int forced = env_int("EXL3_FAT_TALL", -1), fs = env_int("EXL3_FAT_SPLITS", 0);
-    if (forced < 0 && (fat_wide_mode() == 2 || !fat_handoff_on() || env_int("EXL3_FAT_MT", 0) != 0)) return false;
-    if (forced == 0 || (forced < 0 && M < (n <= kTallNarrowCols ? kTallMinRowsNarrow : kTallMinRows))) return false;
+// needs none).  mats: of several matrices, which the 64-row and wide tiles do not
+// take, only up to 16 rows may go elsewhere.
+bool plan_tall(int M, int k, int n, int mats, FatPlan* pl, size_t limit) {
+    int forced = env_int("EXL3_FAT_TALL", -1);
+    const int fs = env_int("EXL3_FAT_SPLITS", 0);
+    if (mats > 1 && M > 16) {
+        if (forced != 128 && forced != 256) forced = -1;
+    } else {
+        if (forced < 0 && (fat_wide_mode() == 2 || !fat_handoff_on() || env_int("EXL3_FAT_MT", 0) != 0)) return false;
+        if (forced == 0 || (forced < 0 && M < (n <= kTallNarrowCols ? kTallMinRowsNarrow : kTallMinRows))) return false;
+    }
     const int ksteps = k / 64;
     double best = 1e30;
     for (int mt = 128; mt <= 256; mt += 128) {
@@ -256,13 +252,12 @@ bool plan_tall(int M, int k, int n, FatPlan* pl, size_t limit) {
 
 // f16out: a call with fp16 output (exl3_gemm), whose narrow k-splits use the
 // partial-tile hand-off (fat_handoff) unless EXL3_FAT_HANDOFF=0.
-// n256: every matrix of the call is a multiple of 256 columns wide.
-FatPlan plan_fat(int M, int k, int n, bool f16out, bool n256, size_t limit = SIZE_MAX) {
+FatPlan plan_fat(int M, int k, int n, bool f16out, int mats, size_t limit = SIZE_MAX) {
     FatPlan pl{};
     const int ksteps = k / 64;
     pl.splits = 1;
-    if (f16out && plan_tall(M, k, n, &pl, limit)) return pl;
-    if (fat_wide_allowed() && M > kFatNarrowMaxRows && n256 &&
+    if (f16out && plan_tall(M, k, n, mats, &pl, limit)) return pl;
+    if (fat_wide_allowed() && M > kFatNarrowMaxRows && n % FB_COLS == 0 &&
         (fat_wide_mode() == 2 || (long long)(n / FB_COLS) * ((M + FB_ROWS - 1) / FB_ROWS) >= kFatWideMinTiles)) {
         pl.mt = FAT_MT_WIDE;
         const long long base = (long long)(n / FB_COLS) * ((M + FB_ROWS - 1) / FB_ROWS);
@@ -271,7 +266,7 @@ FatPlan plan_fat(int M, int k, int n, bool f16out, bool n256, size_t limit = SIZ
     }
     pl.mt = M > 16 ? 64 : 16;
     const int fmt = env_int("EXL3_FAT_MT", 0);  // tuning override: 16, 64 or 128 rows per tile
-    if (fmt == 16 || fmt == 64 || fmt == 128) pl.mt = fmt;
+    if (mats == 1 && (fmt == 16 || fmt == 64 || fmt == 128)) pl.mt = fmt;
     const long long base = (long long)(n / 128) * ((M + pl.mt - 1) / pl.mt);
     const bool ho = f16out && fat_handoff_on();
     const long long wgs = ho ? kFatHandoffWgs : kFatNarrowWgs;
@@ -296,20 +291,15 @@ int check_fat(const char* fn, const void* a, const void* trellis, const void* ou
     return EXL3_OK;
 }
 
-// Narrow 16-row tiles and wide tiles on mul1 weights read the raw entries
-// (two VALU ops per two weights instead of four) and correct in the epilogue
-// from the rotated rows' chunk sums.  Graph-timed, raw / decoded: config 3
-// gate/up M = 16: 29.3 / 31.6 us, exl3_gemm k = 4096, n = 14336, M = 16:
-// 22.7 / 23.2 us; on 64-row tiles the per-row sums cost more than the
-// decode saves (gate/up M = 64: 55.8 / 53.7 us).  Wide tiles in gate/up mode
-// sum a row's chunks in the epilogue, on the row's 8 lanes (config 3 M = 256
-// / 2048: 89.4 / 478.9 -> 87.7 / 467.6 us); plain wide tiles stay decoded
-// (exl3_gemm K = 3 mul1, n = 14336, M = 256 / 2048: 69.9 / 250.9 -> 70.3 /
-// 250.3 us, each row's sums taken once per 128-column block).
+// Narrow 16-row tiles and tall tiles on mul1 weights read the raw entries (two
+// VALU ops per two weights instead of four) and correct in the epilogue from the
+// rotated rows' chunk sums.  Graph-timed, raw / decoded: config 3 gate/up M = 16:
+// 29.3 / 31.6 us, exl3_gemm k = 4096, n = 14336, M = 16: 22.7 / 23.2 us; on
+// 64-row tiles the per-row sums cost more than the decode saves (gate/up M = 64:
+// 55.8 / 53.7 us), and wide tiles do not gain (exl3_gemm K = 3 mul1, n = 14336,
+// M = 256 / 2048: 69.9 / 250.9 -> 70.3 / 250.3 us).
 // EXL3_FAT_RAW=0 turns it off (ablation).
-bool fat_raw(int cb, int mt, bool gu, bool tall = false) {
-    return cb == 2 && (tall || mt == 16 || (mt == FAT_MT_WIDE && gu)) && env_int("EXL3_FAT_RAW", 1) != 0;
-}
+bool fat_raw(int cb, int mt, bool tall) { return cb == 2 && (tall || mt == 16) && env_int("EXL3_FAT_RAW", 1) != 0; }
 
 // Narrow plans with k-splits and fp16 output hand partial tiles to the last
 // split of each (column block, row tile) instead of adding fp32 atomically
@@ -323,8 +313,8 @@ bool fat_handoff(const FatPlan& pl, int m, int n) {
 // Plan of an fp16-output call over `mats` matrices: several matrices do not
 // take the fp32 atomics (only reached by the tuning overrides), so such a plan
 // runs unsplit.
-FatPlan plan_rows(int m, int k, int n, int mats, bool n256, bool f16out = true, size_t limit = SIZE_MAX) {
-    FatPlan pl = plan_fat(m, k, n, f16out, n256, limit);
+FatPlan plan_rows(int m, int k, int n, int mats, size_t limit = SIZE_MAX) {
+    FatPlan pl = plan_fat(m, k, n, true, mats, limit);
     if (mats > 1 && pl.splits > 1 && !fat_handoff(pl, m, n)) pl.splits = 1;
     return pl;
 }
@@ -359,8 +349,7 @@ int run_fat(const uint16_t* a, const int16_t* trellis, float* out32, __half* out
             hipStream_t st, int tail = 0, char* tail_part = nullptr, int* tail_sync = nullptr,
             const float* rowsum = nullptr, float* partials = nullptr, int* counters = nullptr,
             const MatSet* mats = nullptr, int y_bf16 = 0, const FatPlan* plan = nullptr) {
-    const FatPlan pl = plan ? *plan : mats ? plan_rows(M, k, n, mats->count, mats_n256(*mats), out16 != nullptr)
-                            : plan_fat(M, k, n, out16 != nullptr, n % FB_COLS == 0);
+    const FatPlan pl = plan ? *plan : plan_fat(M, k, n, out16 != nullptr, 1);
     FatParams p{};
     if (mats && mats->count > 1) p.mats = *mats;
     p.y_bf16 = y_bf16;
@@ -369,7 +358,7 @@ int run_fat(const uint16_t* a, const int16_t* trellis, float* out32, __half* out
         p.partials = partials;
         p.counters = counters;
     }
-    if (rowsum && fat_raw(cb, pl.mt, false, pl.tall)) p.rowsum = rowsum;
+    if (rowsum && fat_raw(cb, pl.mt, pl.tall)) p.rowsum = rowsum;
     if (tail > 0) {
         p.tiles_x = n / FB_COLS;
         p.tail_tiles = tail;
@@ -432,22 +421,21 @@ size_t fat_xr_bytes(int m, int k) { return fat_xr_only_bytes(m, k) + (((size_t)m
 // tiles (unsplit wide launch)].
 size_t fat_gemm_plan_bytes(const FatPlan& pl, int m, int k, int n, int mats) {
     const bool split = pl.splits > 1;
-    const size_t tail = (!split && pl.mt == FAT_MT_WIDE) ? fat_tail_bytes(wide_tail_tiles(m, k, n, false)) : 0;
+    const size_t tail = (!split && pl.mt == FAT_MT_WIDE) ? fat_tail_bytes(wide_tail_tiles(m, k, n)) : 0;
     const size_t out = fat_handoff(pl, m, n) ? (size_t)pl.splits * m * n * 4 : (size_t)m * n * 4;
     return kWsScratchOffset + fat_xr_bytes(m * mats, k) + (split ? out : tail);
 }
-size_t fat_gemm_scratch_bytes(int m, int k, int n, int mats, bool n256) {
-    return fat_gemm_plan_bytes(plan_rows(m, k, n, mats, n256), m, k, n, mats);
+size_t fat_gemm_scratch_bytes(int m, int k, int n, int mats) {
+    return fat_gemm_plan_bytes(plan_rows(m, k, n, mats), m, k, n, mats);
 }
 
 int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_t* y, int m, int k, int n, int K,
                   int cb, int x_bf16, int y_bf16, void* ws, size_t ws_bytes, hipStream_t st) {
-    const bool n256 = mats_n256(mats);
-    FatPlan pl = plan_rows(m, k, n, mats.count, n256);
+    FatPlan pl = plan_rows(m, k, n, mats.count);
     size_t need = fat_gemm_plan_bytes(pl, m, k, n, mats.count);
     const size_t base = kWsScratchOffset + fat_xr_bytes(m * mats.count, k);
     if (pl.tall && ws_bytes < need && ws_bytes >= base) {  // a buffer sized for other rows: the splits that fit
-        pl = plan_rows(m, k, n, mats.count, n256, true, ws_bytes - base);
+        pl = plan_rows(m, k, n, mats.count, ws_bytes - base);
         need = fat_gemm_plan_bytes(pl, m, k, n, mats.count);
     }
     EXL3_REQUIRE_CODE(ws && ws_bytes >= need, EXL3_ERR_WORKSPACE,
@@ -455,7 +443,7 @@ int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_
     const size_t xrows = (size_t)m * mats.count;
     __half* xr = reinterpret_cast<__half*>(reinterpret_cast<char*>(ws) + kWsScratchOffset);
     float* o32 = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + kWsScratchOffset + fat_xr_bytes((int)xrows, k));
-    float* rs = fat_raw(cb, pl.mt, false, pl.tall)
+    float* rs = fat_raw(cb, pl.mt, pl.tall)
                     ? reinterpret_cast<float*>(reinterpret_cast<char*>(xr) + fat_xr_only_bytes((int)xrows, k))
                     : nullptr;
     RotateSuh suhs{};
@@ -466,7 +454,7 @@ int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_
     const int16_t* trellis = reinterpret_cast<const int16_t*>(mats.trellis[0]);
     const uint16_t* svh = reinterpret_cast<const uint16_t*>(mats.svh[0]);
     if (pl.splits == 1) {
-        const int tail = pl.mt == FAT_MT_WIDE ? wide_tail_tiles(m, k, n, false) : 0;
+        const int tail = pl.mt == FAT_MT_WIDE ? wide_tail_tiles(m, k, n) : 0;
         return run_fat(reinterpret_cast<const uint16_t*>(xr), trellis, nullptr, reinterpret_cast<__half*>(y), svh,
                        nullptr, nullptr, m, k, n, K, cb, false, st, tail, reinterpret_cast<char*>(o32),
                        reinterpret_cast<int*>(ws), rs, nullptr, nullptr, &mats, y_bf16, &pl);
@@ -491,7 +479,6 @@ int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_
 //   * above: tall tiles, gate and up blocks as partial tiles with the finish
 //     launch, or both projections in one workgroup of 256 rows.
 constexpr int kGateUpMinSplitSteps = 16;
-constexpr int kGateUpWideMinRows = 160, kGateUpWideMaxK = 256;
 
 struct GateUpFatPlan {
     int mt, splits;
@@ -528,10 +515,7 @@ double gu_fused_cost(int m, int k, int n) {
 // 14336, K = 3 mul1, 40 / 300 / 512 / 2048 rows: 44.3 / 118.8 / 124.9 / 460.4 -> 38.4 /
 // 105.5 / 118.8 / 439.7; k = 2048, n = 6144, K = 4, 64 / 600: 35.1 / 73.7 -> 23.8 / 57.5; k =
 // n = 2048, 17 / 1000: 22.1 / 64.0 -> 13.3 / 37.4; k = 8192, n = 16384, 1100: 637 -> 568.
-// The rule is within 6 % of the best of the seven choices at 16 shapes.
-// More than 160 rows of k <= 256 (no layer is that short) keep the 256 x 256 tiles,
-// whose bounded tail wait callers see reported there (300 x 256 x 256: 33.6 us;
-// partial tiles 13.0).
+// 300 x 256 x 256: 33.6 -> 10.6.
 // Env EXL3_GU_TALL: 128 / 256 partial tiles of that height (with
 // EXL3_FAT_SPLITS), 1 fused.
 // limit: bytes for partial tiles, as for plan_tall (the fused kernel needs none).
@@ -539,8 +523,6 @@ GateUpFatPlan plan_gate_up_fat(int m, int k, int n, size_t limit = SIZE_MAX) {
     const int ksteps = k / 64;
     if (m > 16) {
         const int forced = env_int("EXL3_GU_TALL", 0), fs = env_int("EXL3_FAT_SPLITS", 0);
-        if (forced == 0 && m > kGateUpWideMinRows && k <= kGateUpWideMaxK && fat_wide_allowed())
-            return GateUpFatPlan{FAT_MT_WIDE, 1, false, false, 1};
         GateUpFatPlan best{256, 1, true, true, gu_tail_parts(m, n)};
         double cost = forced == 128 || forced == 256 ? 1e30 : gu_fused_cost(m, k, n);
         for (int mt = 128; mt <= 256 && forced != 1; mt += 128) {
@@ -578,9 +560,7 @@ GateUpFatPlan plan_gate_up_fat(int m, int k, int n, size_t limit = SIZE_MAX) {
 
 size_t fat_gate_up_plan_bytes(const GateUpFatPlan& pl, int m, int k, int n) {
     size_t b = kWsScratchOffset + fat_xr_bytes(m, k);
-    if (pl.fused) return b;
-    if (pl.mt == FAT_MT_WIDE) b += fat_tail_bytes(wide_tail_tiles(m, k, n, true));
-    else b += (size_t)2 * (n / 128) * pl.splits * (size_t)m * 128 * sizeof(float);
+    if (!pl.fused) b += (size_t)2 * (n / 128) * pl.splits * (size_t)m * 128 * sizeof(float);
     return b;
 }
 
@@ -603,12 +583,11 @@ int fat_gate_up_rows(const uint16_t* x, const uint16_t* suh, const int16_t* gate
                       ws ? ws_bytes : (size_t)0);
     EXL3_REQUIRE(aligned(gate_trellis, 16) && aligned(up_trellis, 16) && aligned(gate_svh, 4) && aligned(up_svh, 4),
                  "exl3_gate_up_swiglu: misaligned pointer");
-    const int mtiles = pl.tall || pl.mt == FAT_MT_WIDE ? 1 : (m + pl.mt - 1) / pl.mt;
-    EXL3_REQUIRE_CODE((size_t)(n / 128) * mtiles <= kWsMaxCounters, EXL3_ERR_UNSUPPORTED,
+    EXL3_REQUIRE_CODE((size_t)(n / 128) <= kWsMaxCounters, EXL3_ERR_UNSUPPORTED,
                       "exl3_gate_up_swiglu: %d column blocks exceed the workspace counters", n / 128);
     char* w8 = reinterpret_cast<char*>(ws);
     __half* xr = reinterpret_cast<__half*>(w8 + kWsScratchOffset);
-    float* rs = fat_raw(cb, pl.mt, true, pl.tall) ? reinterpret_cast<float*>(w8 + kWsScratchOffset + fat_xr_only_bytes(m, k)) : nullptr;
+    float* rs = fat_raw(cb, pl.mt, pl.tall) ? reinterpret_cast<float*>(w8 + kWsScratchOffset + fat_xr_only_bytes(m, k)) : nullptr;
     int rc = rotate_rows(reinterpret_cast<const __half*>(x), RotateSuh{{reinterpret_cast<const __half*>(suh)}}, 1, xr, m,
                          k, 0, rs, st, "exl3_gate_up_swiglu rotate launch");
     if (rc) return rc;
@@ -640,18 +619,6 @@ int fat_gate_up_rows(const uint16_t* x, const uint16_t* suh, const int16_t* gate
         if (rc || pl.fused) return rc;
         return fat_split_finish(p, pl.splits, st, "exl3_gate_up_swiglu finish launch");
     }
-    if (pl.mt == FAT_MT_WIDE) {
-        const int tail = wide_tail_tiles(m, k, n, true);
-        if (tail > 0) {
-            p.tiles_x = n / 128;
-            p.tail_tiles = tail;
-            p.tail_first = p.tiles_x * ((m + FB_ROWS - 1) / FB_ROWS) - tail;
-            p.tail_part = p.partials;
-            p.tail_sync = p.counters;
-            p.max_polls = wait_polls();
-            p.status = p.counters + kWsStatusIndex;
-        }
-    }
     // One 16-row tile of 6 to 16 rows with up to 4 k-splits: the splits store
     // their partial tiles and exit, and fat_split_finish_kernel finishes every
     // (row, column block) in a launch of its own (env EXL3_FAT_SPLIT_OUT=0:
@@ -660,8 +627,7 @@ int fat_gate_up_rows(const uint16_t* x, const uint16_t* suh, const int16_t* gate
     // 24.48 / 24.95 / 26.1 / 26.21 / 27.1 / 27.22 -> 23.25 / 24.20 / 24.75 /
     // 25.07 / 25.45 / 25.8 / 26.1 us (with four rows the last arrival's chain
     // is short and the extra boundary does not pay).
-    const bool split_out = pl.mt == 16 && m >= kSplitOutMinRows && pl.splits <= 4 &&
-                           env_int("EXL3_FAT_SPLIT_OUT", 1) != 0;
+    const bool split_out = m >= kSplitOutMinRows && pl.splits <= 4 && env_int("EXL3_FAT_SPLIT_OUT", 1) != 0;
     p.split_out = split_out ? 1 : 0;
     rc = fat_launch(K, cb, pl.mt, p, pl.splits, st);
     if (rc || !split_out) return rc;
@@ -694,5 +660,5 @@ extern "C" int exl3_fat_gemm_scatter(const uint16_t* a, const int16_t* trellis, 
 extern "C" size_t exl3_gemm_workspace_size(int m, int k, int n, int K) {
     if (m < 1 || k < 128 || n < 128) return 0;
     if (m <= gemm_gemv_rows(n)) return exl3_gemv_workspace_size(m, k, n, K, 1);
-    return fat_gemm_scratch_bytes(m, k, n, 1, n % 256 == 0);
+    return fat_gemm_scratch_bytes(m, k, n, 1);
 }

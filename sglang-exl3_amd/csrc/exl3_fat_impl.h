@@ -67,13 +67,13 @@ struct FatParams {
     int M, k, n;
     int ksteps;      // steps (4 k-slices) per k-split
     int accumulate;  // add atomically into out32 instead of storing
-    // Gate/up mode (fat_big_kernel<.., GU = true>): `trellis`/`svh` are the
-    // gate projection, `trellis2`/`svh2` the up projection, both n wide;
+    // Gate/up mode (16-row tiles; tall tiles): `trellis`/`svh` are the gate
+    // projection, `trellis2`/`svh2` the up projection, both n wide;
     // out16[m][n] = fp16( silu(min(g, limit)) * clamp(u, -limit, limit) ).
     // fat_gemm_kernel in gate/up mode: grid.x enumerates (column block,
     // projection) pairs (even: gate, odd: up); each workgroup stores its fp32
-    // partial tile, and the last of the 2 S arrivals of a (column block, row
-    // tile) sums them, applies both output rotations and the SwiGLU.
+    // partial tile, and the last of the 2 S arrivals of a column block sums
+    // them, applies both output rotations and the SwiGLU.
     int gu;
     // Narrow split hand-off (gate/up mode, or plain mode with handoff) with
     // split_out != 0: each workgroup stores its partial tile and exits (no
@@ -117,13 +117,12 @@ struct FatParams {
     int* tail_sync;    // [tail_tiles] arrival counts, then [tail_tiles] flags; zero between calls
     int max_polls;     // polls before the second half's wait gives up
     int* status;       // workspace status word: EXL3_WAIT_FAT_TAIL when a wait gave up
-    // Narrow kernel on mul1 weights (fat_gemm_kernel<.., RAW = true>, plain
-    // and gate/up modes): B holds the raw entries (mul1_raw_pair) and the
+    // 16-row and tall tiles on mul1 weights (RAW = true, plain and gate/up modes): B holds the raw entries (mul1_raw_pair) and the
     // epilogue applies kMul1Kinv * acc + kMul1Bias * (sum of the rows' x over
     // the k range), from rowsum[row][k/128] (rotate_rows_kernel's chunk sums).
     const float* rowsum;
-    // Several matrices side by side (mats.count > 1, plain mode with out16): n
-    // is the width of the whole output, `a` (and rowsum) holds the rows rotated
+    // Several matrices side by side (mats.count > 1, 16-row and tall tiles with
+    // out16): n is the width of the whole output, `a` (and rowsum) holds the rows rotated
     // for each matrix in turn, and a column block's matrix comes from mats.
     MatSet mats;
     int y_bf16;  // out16 is bfloat16 (plain modes)
@@ -195,15 +194,16 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
     extern __shared__ __align__(16) unsigned char fat_smem[];
 
     const int sidx = blockIdx.z;
-    // gate/up mode: blockIdx.x = 2 * column block + projection
-    const int bx = p.gu ? (int)(blockIdx.x >> 1) : (int)blockIdx.x;
-    const uint32_t* trel = (p.gu && (blockIdx.x & 1)) ? p.trellis2 : p.trellis;
+    // gate/up mode (16-row tiles only): blockIdx.x = 2 * column block + projection
+    const bool gu = MT == 16 && p.gu;
+    const int bx = gu ? (int)(blockIdx.x >> 1) : (int)blockIdx.x;
+    const uint32_t* trel = (gu && (blockIdx.x & 1)) ? p.trellis2 : p.trellis;
     const __half* svh_p = p.svh;
     const __half* dsuh = nullptr;  // grouped up pass: the down projection's suh
     const __half* arows = p.a;
     const float* rowsum = p.rowsum;
     int bxm = bx, nm = p.n;  // column block and width inside the matrix
-    if (p.mats.count > 1) {
+    if (MT == 16 && p.mats.count > 1) {
         const MatRef r = mat_of_block(p.mats, bx);
         trel = r.trellis;
         svh_p = r.svh;
@@ -348,13 +348,13 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
         }
         return;
     }
-    if (p.gu || p.handoff) {
+    if (gu || p.handoff) {
         // partial-tile hand-off (gate/up mode, or plain mode with k-splits):
         // partial tile out (device-coherent stores), one counter per (column
         // block, row tile); the last of the np x S arrivals sums each row's
         // splits in split order (deterministic)
-        const int np = p.gu ? 2 : 1;
-        const int S = gridDim.z, proj = p.gu ? (int)(blockIdx.x & 1) : 0;
+        const int np = gu ? 2 : 1;
+        const int S = gridDim.z, proj = gu ? (int)(blockIdx.x & 1) : 0;
         const size_t rs = (size_t)p.M * 128;  // between splits
         float* part = p.partials + ((size_t)(bx * np + proj) * S + sidx) * rs + (size_t)m0 * 128;
         for (int idx = 2 * tid; idx < rows * 128; idx += 2 * FAT_THREADS) {
@@ -374,7 +374,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
         __syncthreads();
         if (!gu_last) return;
         if (tid == 0) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (!p.gu) {
+        if (!gu) {
             const float* pv = p.partials + (size_t)bx * S * rs + (size_t)m0 * 128 + 2 * lane;
             const float sva = __low2float(svv), svb = __high2float(svv);
             if (S <= 4) {
@@ -721,13 +721,13 @@ __device__ __forceinline__ void nat_decode(const uint32_t (&buf)[K + 1], uint32_
 }
 
 // The same from words w[0..K-1], the previous word from lane q - 1.
-template <int K, int CB, bool RAW = false>
+template <int K, int CB>
 __device__ __forceinline__ void nat_group(const uint32_t (&w)[K], int prev_addr, uint32_t (&f)[2][2][4]) {
     uint32_t buf[K + 1];
 #pragma unroll
     for (int j = 0; j < K; ++j) buf[1 + j] = w[j];
     buf[0] = (uint32_t)__builtin_amdgcn_ds_bpermute(prev_addr, (int)buf[K]);
-    nat_decode<K, CB, RAW>(buf, f);
+    nat_decode<K, CB, false>(buf, f);
 }
 
 // mul1 raw entries in the x16 layout (a tile row on 8 lanes, 16 columns
@@ -748,18 +748,7 @@ __device__ __forceinline__ void raw_fix16(float (&v)[16], float sx) {
     for (int e = 0; e < 16; ++e) v[e] = raw_value(v[e], sx);
 }
 
-// GU = true: gate/up mode.  Workgroup bx then covers column block bx of both
-// projections: its left 128 columns (column quarters 0, 1) decode the gate
-// trellis, its right 128 (quarters 2, 3) the up trellis, so the epilogue
-// holds the gate and up values of the same columns and applies the SwiGLU
-// in registers.  The reference's fused path concatenates the two packs per
-// call and combines them with separate torch kernels
-// (src/sglang_exl3/exl3.py:1184-1206).
-// RAW (mul1, p.rowsum set): B holds the raw entries (mul1_raw_pair) and the
-// epilogue applies kMul1Kinv * acc + kMul1Bias * (the row's x sum over the
-// k range) before the output rotation, two VALU per pair of states fewer in
-// the decode (config 3 M = 2048, whole-tile harness: 497.6 -> 483.2 us).
-template <int K, int CB, bool GU, bool RAW = false>
+template <int K, int CB>
 __global__ __launch_bounds__(FB_THREADS, 2) void fat_big_kernel(FatParams p) {
     constexpr int RB = FB_ROWS / 2 / 16;  // row blocks per wave
     static_assert(FB_A_BYTES == 4 * 16 * FB_THREADS, "four 16-byte A chunks per thread and step");
@@ -787,26 +776,12 @@ __global__ __launch_bounds__(FB_THREADS, 2) void fat_big_kernel(FatParams p) {
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
     const int rh = wv >> 2, cq = wv & 3;
     const int g = lane >> 4, i = lane & 15, q = i & 7;
-    int ntiles = p.n >> 4;
+    const int ntiles = p.n >> 4;
     const int nsteps = half >= 0 ? p.ksteps / 2 : p.ksteps;  // even
     const int kt0 = sidx * p.ksteps * 4 + (half > 0 ? nsteps * 4 : 0);
     // this wave decodes group rh of quarter cq: column tiles 4cq + 2rh + (i >> 3)
-    // (gate/up mode: quarters 0, 1 of the gate block bx, 2, 3 of the up block bx)
-    int nt = GU ? bx * 8 + (cq & 1) * 4 + rh * 2 + (i >> 3) : bx * (FB_COLS / 16) + cq * 4 + rh * 2 + (i >> 3);
-    const uint32_t* trel = (GU && cq >= 2) ? p.trellis2 : p.trellis;
-    const __half* arows = p.a;
-    const __half* svh_p = p.svh;
-    int svc0 = bx * FB_COLS;  // the tile's first column inside its matrix
-    if (!GU && p.mats.count > 1) {  // every matrix a multiple of FB_COLS wide
-        const MatRef r = mat_of_block(p.mats, bx * (FB_COLS / 128));
-        trel = r.trellis;
-        svh_p = r.svh;
-        arows += (size_t)r.j * p.M * p.k;
-        nt -= r.nb0 * 8;
-        svc0 -= r.nb0 * 128;
-        ntiles = r.n >> 4;
-    }
-    const EXL3_GLOBAL uint32_t* tb = gptr(trel) + ((size_t)(kt0 + g) * ntiles + nt) * (8 * K) + K * q;
+    const int nt = bx * (FB_COLS / 16) + cq * 4 + rh * 2 + (i >> 3);
+    const EXL3_GLOBAL uint32_t* tb = gptr(p.trellis) + ((size_t)(kt0 + g) * ntiles + nt) * (8 * K) + K * q;
     const size_t step_stride = (size_t)4 * ntiles * (8 * K);
     const int prev_addr = ((lane & ~7) | ((lane + 7) & 7)) << 2;
 
@@ -814,7 +789,7 @@ __global__ __launch_bounds__(FB_THREADS, 2) void fat_big_kernel(FatParams p) {
     // physical chunk u & 7, which holds logical chunk (u & 7) ^ (row & 7) ^
     // ((row >> 3) & 1).  Rows past M repeat the last row (never stored).
     const EXL3_GLOBAL char* abase =
-        reinterpret_cast<const EXL3_GLOBAL char*>(gptr(arows)) + ((size_t)m0 * p.k + (size_t)kt0 * 16) * 2;
+        reinterpret_cast<const EXL3_GLOBAL char*>(gptr(p.a)) + ((size_t)m0 * p.k + (size_t)kt0 * 16) * 2;
     uint32_t aoff[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -855,7 +830,7 @@ __global__ __launch_bounds__(FB_THREADS, 2) void fat_big_kernel(FatParams p) {
     auto load_step = [&](int step) { load_words<K>(tb + (size_t)step * step_stride, w); };
     auto decode_post = [&](int bufi) {
         uint32_t fr[2][2][4];  // [column half][h'][j]
-        nat_group<K, CB, RAW>(w, prev_addr, fr);
+        nat_group<K, CB>(w, prev_addr, fr);
         unsigned char* bb = bsm + (size_t)bufi * FB_B_BYTES;
 #pragma unroll
         for (int c = 0; c < 2; ++c)
@@ -1037,66 +1012,6 @@ __global__ __launch_bounds__(FB_THREADS, 2) void fat_big_kernel(FatParams p) {
                     }
                 }
         __syncthreads();
-        if constexpr (GU) {
-            // 8 rows per wave, gate and up of one 128-column block: lane l
-            // holds 16 consecutive columns (16 (l & 7) ..) of each, LDS row
-            // 8 wv + (l >> 3); output FWHT, norm and svh of both, then SwiGLU
-            static_assert(FB_PASS_ROWS / 8 == FB_THREADS / 64, "one row group per wave");
-            const int ctr = wv * 8 + (lane >> 3);
-            const int trow = (ctr >> 5) * 128 + pass * 32 + (ctr & 31);
-            const int col = (lane & 7) * 16;
-            float gv[16], uv[16];
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const float4 a = *reinterpret_cast<const float4*>(ct + ctr * FB_CTS + col + 4 * q4);
-                const float4 b = *reinterpret_cast<const float4*>(ct + ctr * FB_CTS + 128 + col + 4 * q4);
-                gv[4 * q4] = a.x; gv[4 * q4 + 1] = a.y; gv[4 * q4 + 2] = a.z; gv[4 * q4 + 3] = a.w;
-                uv[4 * q4] = b.x; uv[4 * q4 + 1] = b.y; uv[4 * q4 + 2] = b.z; uv[4 * q4 + 3] = b.w;
-            }
-            if constexpr (RAW) {
-                const float sx = raw_row_bias(p, m0 + (trow < rows ? trow : rows - 1), sidx * (p.ksteps >> 1),
-                                              p.ksteps >> 1, lane);
-                raw_fix16(gv, sx);
-                raw_fix16(uv, sx);
-            }
-            fwht128_x16(gv, lane);
-            fwht128_x16(uv, lane);
-            const float hn = fwht_x16_norm(lane);
-            const int c0 = bx * 128 + col;
-            const EXL3_GLOBAL uint32_t* sgp = reinterpret_cast<const EXL3_GLOBAL uint32_t*>(gptr(p.svh) + c0);
-            const EXL3_GLOBAL uint32_t* sup = reinterpret_cast<const EXL3_GLOBAL uint32_t*>(gptr(p.svh2) + c0);
-#pragma unroll
-            for (int e2 = 0; e2 < 8; ++e2) {
-                const uint32_t sgw = sgp[e2], suw = sup[e2];
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int e = 2 * e2 + h;
-                    gv[e] = (gv[e] * hn) * __half2float(__ushort_as_half((unsigned short)(sgw >> (16 * h))));
-                    uv[e] = (uv[e] * hn) * __half2float(__ushort_as_half((unsigned short)(suw >> (16 * h))));
-                }
-            }
-            // one uniform branch around all 32 values: a per-value test is
-            // turned into selects that cost 80 VALU per pass without a clamp
-            if (p.limit > 0.0f && p.limit < __builtin_huge_valf()) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    gv[e] = fminf(gv[e], p.limit);
-                    uv[e] = fminf(fmaxf(uv[e], -p.limit), p.limit);
-                }
-            }
-            uint32_t ow[8];
-#pragma unroll
-            for (int e2 = 0; e2 < 8; ++e2) {
-                const __half2 o = h2_rn(silu_f(gv[2 * e2]) * uv[2 * e2], silu_f(gv[2 * e2 + 1]) * uv[2 * e2 + 1]);
-                ow[e2] = *reinterpret_cast<const uint32_t*>(&o);
-            }
-            if (trow < rows) {
-                EXL3_GLOBAL uint32_t* o = reinterpret_cast<EXL3_GLOBAL uint32_t*>(gptr(p.out16) + (size_t)(m0 + trow) * p.n + c0);
-#pragma unroll
-                for (int e2 = 0; e2 < 8; ++e2) o[e2] = ow[e2];
-            }
-            continue;
-        }
         // 8 rows x one 128-block per wave at a time: lane l holds 16 consecutive
         // columns (16 (l & 7) ..) of LDS row 8 rg + (l >> 3)
 #pragma unroll
@@ -1114,14 +1029,11 @@ __global__ __launch_bounds__(FB_THREADS, 2) void fat_big_kernel(FatParams p) {
                 v[4 * q + 2] = t.z;
                 v[4 * q + 3] = t.w;
             }
-            if constexpr (RAW)
-                raw_fix16(v, raw_row_bias(p, m0 + (trow < rows ? trow : rows - 1), sidx * (p.ksteps >> 1),
-                                          p.ksteps >> 1, lane));
             fwht128_x16(v, lane);
             const float hn = fwht_x16_norm(lane);
             const int c0 = bx * FB_COLS + col;
             // svh and the outputs are only 4- (8-) byte aligned by contract
-            const EXL3_GLOBAL uint32_t* svp = reinterpret_cast<const EXL3_GLOBAL uint32_t*>(gptr(svh_p) + svc0 + col);
+            const EXL3_GLOBAL uint32_t* svp = reinterpret_cast<const EXL3_GLOBAL uint32_t*>(gptr(p.svh) + c0);
             uint32_t sw[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) sw[e] = svp[e];
@@ -1177,21 +1089,23 @@ __global__ __launch_bounds__(FB_THREADS, 2) void fat_big_kernel(FatParams p) {
 
 template <int K>
 int fat_launch_k(int cb, int mt, const FatParams& p, int splits, hipStream_t st) {
+    if (mt != 16 && (p.gu || p.mats.count > 1)) {
+        set_error("exl3 fat gemm: gate/up and several matrices run on 16-row tiles here");
+        return EXL3_ERR_UNSUPPORTED;
+    }
     if (mt == FAT_MT_WIDE) {
-        dim3 grid(p.gu ? p.n / 128 : p.n / FB_COLS, (p.M + FB_ROWS - 1) / FB_ROWS, splits);
+        dim3 grid(p.n / FB_COLS, (p.M + FB_ROWS - 1) / FB_ROWS, splits);
         if (p.tail_tiles > 0) grid = dim3(p.tail_first + 2 * p.tail_tiles, 1, 1);
         const size_t smem = fat_big_smem_bytes();
-#define EXL3_FATB(CBV, GUV, RAWV)                                                                      \
-    if (cb == CBV && (p.gu != 0) == GUV && (p.rowsum != nullptr) == RAWV) {                            \
-        const void* fn = reinterpret_cast<const void*>(&fat_big_kernel<K, CBV, GUV, RAWV>);            \
+#define EXL3_FATB(CBV)                                                                                 \
+    if (cb == CBV) {                                                                                   \
+        const void* fn = reinterpret_cast<const void*>(&fat_big_kernel<K, CBV>);                       \
         const int lrc = allow_dynamic_lds(fn, smem, "exl3 fat gemm (wide tiles)");                     \
         if (lrc) return lrc;                                                                           \
-        fat_big_kernel<K, CBV, GUV, RAWV><<<grid, FB_THREADS, smem, st>>>(p);                          \
+        fat_big_kernel<K, CBV><<<grid, FB_THREADS, smem, st>>>(p);                                     \
         return launch_status("exl3 fat gemm launch");                                                  \
     }
-        EXL3_FATB(0, false, false) EXL3_FATB(1, false, false) EXL3_FATB(2, false, false)
-        EXL3_FATB(0, true, false) EXL3_FATB(1, true, false) EXL3_FATB(2, true, false)
-        EXL3_FATB(2, true, true)
+        EXL3_FATB(0) EXL3_FATB(1) EXL3_FATB(2)
 #undef EXL3_FATB
     }
     dim3 grid((p.gu ? 2 : 1) * (p.n / 128), (p.M + mt - 1) / mt, splits);

@@ -57,7 +57,7 @@ int gemv_launch(int K, int cb, int mb, const GemvParams& p, int experts, hipStre
     return EXL3_ERR_UNSUPPORTED;
 }
 
-size_t fat_gemm_scratch_bytes(int m, int k, int n, int mats, bool n256);
+size_t fat_gemm_scratch_bytes(int m, int k, int n, int mats);
 int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_t* y, int m, int k, int n, int K,
                   int cb, int x_bf16, int y_bf16, void* ws, size_t ws_bytes, hipStream_t st);
 
@@ -498,18 +498,16 @@ extern "C" int exl3_gemm(const uint16_t* x, const int16_t* trellis, const uint16
 extern "C" size_t exl3_linear_cat_workspace_size(int m, int k, const int* n, int count, int K) {
     if (m < 1 || k < 128 || !n || count < 1 || count > kMaxMats) return 0;
     int total = 0;
-    bool n256 = true;
     for (int j = 0; j < count; ++j) {
         if (n[j] < 128) return 0;
         total += n[j];
-        n256 = n256 && n[j] % 256 == 0;
     }
     // room for either path where the codebook decides (it is not known here)
     size_t need = 0;
     const bool wide = cat_gemv(m, k, n, count, K, EXL3_CB_MUL1), narrow = cat_gemv(m, k, n, count, K, EXL3_CB_MCG);
     if (wide || narrow) need = exl3_gemv_workspace_size(m, k, total, K, 1);
     if (!wide || !narrow) {
-        const size_t f = fat_gemm_scratch_bytes(m, k, total, count, n256);
+        const size_t f = fat_gemm_scratch_bytes(m, k, total, count);
         need = need > f ? need : f;
     }
     return need;

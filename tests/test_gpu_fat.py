@@ -172,10 +172,10 @@ def test_fat_then_gemv_workspace_stays_clean():
 @pytest.mark.parametrize("cb", [1, 2])
 @pytest.mark.parametrize("op", ["gemm", "gate_up"])
 def test_tail_split_repeatable(op, cb, monkeypatch):
-    """Tail split of the wide-tile kernel (every tile of a one-round launch runs as
-    two k-halves, the first half hands its sums to the second): against the
-    oracle, bit-identical over repeated calls (the hand-off counts and flags
-    reset themselves), and close to the unsplit kernel (EXL3_FAT_TAIL=0)."""
+    """The last round's tiles in parts: of the wide-tile kernel (exl3_gemm, EXL3_FAT_WIDE=2) as two k-halves, the first
+    half handing its sums to the second, of the fused gate/up kernel (EXL3_GU_TALL=1) as row parts.  Every tile of
+    these one-round launches: against the oracle, bit-identical over repeated calls (the hand-off counts and flags
+    reset themselves), and close to the launch of whole tiles (EXL3_FAT_TAIL=0)."""
     # gemm: 56 x 2 tiles, enough for one k-split (smaller grids split k with
     # fp32 atomics instead); gate/up: 2 x 2 tiles, always one split
     m, k, K = (512, 1024, 3) if op == "gemm" else (300, 1024, 3)
@@ -183,11 +183,13 @@ def test_tail_split_repeatable(op, cb, monkeypatch):
     print(f"case: tail split {op} m={m} k={k} n={n} cb={cb}", flush=True)
     x = torch.from_numpy(make_x(m, k, seed=31)).cuda()
     if op == "gemm":
+        monkeypatch.setenv("EXL3_FAT_WIDE", "2")
         tr, su, sv = make_weight(k, n, K, seed=32)
         d = [torch.from_numpy(v).cuda() for v in (tr, su, sv)]
         run = lambda: torch.ops.sglang_exl3.exl3_gemm(x, *d, K, cb == 1)
         ref = oracle.matmul(x.cpu().numpy(), oracle.dequant(tr, su, sv, K, cb, rtz=True))
     else:
+        monkeypatch.setenv("EXL3_GU_TALL", "1")
         tg, su, sg = make_weight(k, n, K, seed=33)
         tu, _, su2 = make_weight(k, n, K, seed=34)
         d = [torch.from_numpy(v).cuda() for v in (su, tg, sg, tu, su2)]
@@ -204,6 +206,8 @@ def test_tail_split_repeatable(op, cb, monkeypatch):
     whole = run()
     torch.cuda.synchronize()
     check_close(outs[0].float().cpu().numpy(), whole.float().cpu().numpy(), f"tail split vs whole {op}")
+    if op == "gate_up":  # the same sums, other workgroups
+        assert torch.equal(outs[0], whole)
 
 
 @pytest.mark.parametrize("op,m", [("gemm", 16), ("gemm", 48), ("gemm", 300), ("gate_up", 16), ("gate_up", 48),

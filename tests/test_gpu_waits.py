@@ -44,20 +44,17 @@ def test_workspace_status_starts_clear_and_capi_checks_arguments():
 
 
 def test_fat_tail_wait_that_gives_up_is_reported(monkeypatch):
-    """Gate/up SwiGLU at m=300 takes the wide-tile kernel, whose 4 tiles all run as
-    tail-split k-halves (k=256: 4 steps)."""
-    m, k, n, K, cb = 300, 256, 256, 3, 1
+    """exl3_gemm on the wide-tile kernel (EXL3_FAT_WIDE=2) at m=300, n=12288: one k-split, 96 tiles, which all run
+    as tail-split k-halves (k=256: 4 steps)."""
+    m, k, n, K, cb = 300, 256, 12288, 3, 1
     print(f"case: fat tail wait m={m} k={k} n={n} K={K} cb={cb}", flush=True)
-    tg, su, sg = make_weight(k, n, K, seed=501)
-    tu, _, sv_u = make_weight(k, n, K, seed=502)
-    scale = np.float32(4.0 / np.sqrt(k))
-    sg = (sg.astype(np.float32) * scale).astype(np.float16)
-    sv_u = (sv_u.astype(np.float32) * scale).astype(np.float16)
+    monkeypatch.setenv("EXL3_FAT_WIDE", "2")
+    tr, su, sv = make_weight(k, n, K, seed=501)
     x = make_x(m, k, seed=503)
-    d = [torch.from_numpy(a).cuda() for a in (x, su, tg, sg, tu, sv_u)]
+    d = [torch.from_numpy(a).cuda() for a in (x, tr, su, sv)]
 
     def run():
-        out = torch.ops.sglang_exl3.exl3_gate_up_swiglu(*d, K, cb, 0.0)
+        out = torch.ops.sglang_exl3.exl3_gemm(*d, K, cb == 1)
         torch.cuda.synchronize()
         return out
 
@@ -71,9 +68,8 @@ def test_fat_tail_wait_that_gives_up_is_reported(monkeypatch):
     again = run()
     ops.check_waits()
     assert torch.equal(again, clean)
-    g = oracle.matmul(x, oracle.dequant(tg, su, sg, K, cb, rtz=True))
-    u = oracle.matmul(x, oracle.dequant(tu, su, sv_u, K, cb, rtz=True))
-    check_close(again.float().cpu().numpy(), oracle.swiglu(g, u, float("inf")), "gate_up after a reported wait")
+    ref = oracle.matmul(x, oracle.dequant(tr, su, sv, K, cb, rtz=True))
+    check_close(again.float().cpu().numpy(), ref, "gemm after a reported wait")
 
 
 def test_moe_fused_wait_that_gives_up_is_reported(monkeypatch):
