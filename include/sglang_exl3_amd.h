@@ -178,6 +178,15 @@ int exl3_linear_cat(const void* x, int x_dtype, const int16_t* const* trellis, c
                     const uint16_t* const* svh, const int* n, int count, void* y, int y_dtype, int m, int k, int K,
                     int codebook, void* workspace, size_t workspace_bytes, void* stream);
 
+/* exl3_linear_cat without its first `first` weights, with the bits that the
+ * others' columns have in the whole call (K and V of a qkv projection,
+ * src/sglang_exl3/dense.py:373-398).  apart 0: outputs side by side, y[m][n[first]
+ * + ..]; 1: each packed, y = [m][n[first]], then [m][n[first + 1]], ..  All `count`
+ * weights are given; same workspace size as the whole call. */
+int exl3_linear_cat_part(const void* x, int x_dtype, const int16_t* const* trellis, const uint16_t* const* suh,
+                         const uint16_t* const* svh, const int* n, int count, int first, int apart, void* y, int y_dtype,
+                         int m, int k, int K, int codebook, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Many-row EXL3 GEMM on MFMA with the input already rotated:
  *   out[m][n] (f32) = svh[n] * (H . (a . T)[m][128-block])[n] / sqrt(128)
  * a: f16 [M][k] = fp16(H(x (.) suh) / sqrt(128)) per 128 block; trellis

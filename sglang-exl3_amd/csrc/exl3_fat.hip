@@ -429,14 +429,16 @@ size_t fat_gemm_scratch_bytes(int m, int k, int n, int mats) {
     return fat_gemm_plan_bytes(plan_rows(m, k, n, mats), m, k, n, mats);
 }
 
+// plan_n, plan_mats: the width and number of matrices that the call is planned
+// for (n and mats.count, or more where it is part of another).
 int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_t* y, int m, int k, int n, int K,
-                  int cb, int x_bf16, int y_bf16, void* ws, size_t ws_bytes, hipStream_t st) {
-    FatPlan pl = plan_rows(m, k, n, mats.count);
-    size_t need = fat_gemm_plan_bytes(pl, m, k, n, mats.count);
-    const size_t base = kWsScratchOffset + fat_xr_bytes(m * mats.count, k);
+                  int cb, int x_bf16, int y_bf16, int plan_n, int plan_mats, void* ws, size_t ws_bytes, hipStream_t st) {
+    FatPlan pl = plan_rows(m, k, plan_n, plan_mats);
+    size_t need = fat_gemm_plan_bytes(pl, m, k, plan_n, plan_mats);
+    const size_t base = kWsScratchOffset + fat_xr_bytes(m * plan_mats, k);
     if (pl.tall && ws_bytes < need && ws_bytes >= base) {  // a buffer sized for other rows: the splits that fit
-        pl = plan_rows(m, k, n, mats.count, ws_bytes - base);
-        need = fat_gemm_plan_bytes(pl, m, k, n, mats.count);
+        pl = plan_rows(m, k, plan_n, plan_mats, ws_bytes - base);
+        need = fat_gemm_plan_bytes(pl, m, k, plan_n, plan_mats);
     }
     EXL3_REQUIRE_CODE(ws && ws_bytes >= need, EXL3_ERR_WORKSPACE,
                       "%s: %zu workspace bytes needed for m=%d, %zu given", fn, need, m, ws ? ws_bytes : (size_t)0);
@@ -459,7 +461,7 @@ int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_
                        nullptr, nullptr, m, k, n, K, cb, false, st, tail, reinterpret_cast<char*>(o32),
                        reinterpret_cast<int*>(ws), rs, nullptr, nullptr, &mats, y_bf16, &pl);
     }
-    if (fat_handoff(pl, m, n))
+    if (fat_handoff(pl, m, plan_n))
         return run_fat(reinterpret_cast<const uint16_t*>(xr), trellis, nullptr, reinterpret_cast<__half*>(y), svh,
                        nullptr, nullptr, m, k, n, K, cb, false, st, 0, nullptr, nullptr, rs, o32,
                        reinterpret_cast<int*>(ws), &mats, y_bf16, &pl);

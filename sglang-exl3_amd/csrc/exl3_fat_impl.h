@@ -203,12 +203,16 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
     const __half* arows = p.a;
     const float* rowsum = p.rowsum;
     int bxm = bx, nm = p.n;  // column block and width inside the matrix
+    long long y0 = 0;        // its output, rows ys apart
+    int ys = p.n;
     if (MT == 16 && p.mats.count > 1) {
         const MatRef r = mat_of_block(p.mats, bx);
         trel = r.trellis;
         svh_p = r.svh;
         bxm = bx - r.nb0;
         nm = r.n;
+        y0 = r.y0;
+        ys = r.ys;
         arows += (size_t)r.j * p.M * p.k;
         if constexpr (RAW) rowsum += (size_t)r.j * p.M * (p.k >> 7);
     }
@@ -311,6 +315,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
             }
     __syncthreads();
     const int c0 = bx * 128 + 2 * lane;
+    EXL3_GLOBAL __half* const yo = gptr(p.out16) + y0 + (size_t)m0 * ys + bxm * 128 + 2 * lane;  // plain fp16 / bf16 output
     if (p.gmode) {
         const float sva = __low2float(svv), svb = __high2float(svv);
         const bool clamp = p.limit > 0.0f && p.limit < __builtin_huge_valf();
@@ -407,7 +412,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
                         vb = raw_value(vb, sx);
                     }
                     fwht128_pair_fast(va, vb, lane);
-                    st_y2(gptr(p.out16) + (size_t)(m0 + row) * p.n + c0, h2_rn((va * kHadNorm) * sva, (vb * kHadNorm) * svb), p.y_bf16);
+                    st_y2(yo + (size_t)row * ys, h2_rn((va * kHadNorm) * sva, (vb * kHadNorm) * svb), p.y_bf16);
                 };
                 constexpr int RS = FAT_THREADS / 64;
                 RowLoads1 la, lb;
@@ -432,7 +437,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
                     vb = raw_value(vb, sx);
                 }
                 fwht128_pair_fast(va, vb, lane);
-                st_y2(gptr(p.out16) + (size_t)(m0 + row) * p.n + c0, h2_rn((va * kHadNorm) * sva, (vb * kHadNorm) * svb), p.y_bf16);
+                st_y2(yo + (size_t)row * ys, h2_rn((va * kHadNorm) * sva, (vb * kHadNorm) * svb), p.y_bf16);
             }
             return;
         }
@@ -519,7 +524,7 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
         vb = (vb * kHadNorm) * svb;
         const int src = m0 + row;
         if (p.out16) {
-            st_y2(gptr(p.out16) + (size_t)src * p.n + c0, h2_rn(va, vb), p.y_bf16);
+            st_y2(yo + (size_t)row * ys, h2_rn(va, vb), p.y_bf16);
             continue;
         }
         size_t dst = (size_t)src;
@@ -540,11 +545,12 @@ __global__ __launch_bounds__(FAT_THREADS, MT <= 64 ? 4 : 1) void fat_gemm_kernel
     }
 }
 
-// Finish of the narrow kernel's split hand-off with split_out (one 16-row
-// tile, up to 4 k-splits; GU: gate/up mode, else plain mode with fp16
-// output): one wave per (row, column block) sums the partial rows in split
-// order, from zero, as the in-kernel hand-off does, and applies the same
-// epilogue, so the results are bit-identical to it.  The extra launch costs a
+// Finish of split_out partial tiles: of the narrow kernel's hand-off (one 16-row
+// tile, up to 4 k-splits) and of tall tiles (any rows, up to 16 splits; gate/up
+// mode: 1 to 16).  GU: gate/up mode, else plain mode with fp16 or bf16 output.
+// One wave per (row, column block) sums the partial rows in split order, from
+// zero, as the in-kernel hand-off does, and applies the same epilogue, so the
+// results are bit-identical to it.  The extra launch costs a
 // kernel boundary, but every row's chain then runs at once, where the last
 // arrival of a column block runs its rows on four waves behind a store /
 // counter / load chain (config 3 M = 16, kernel plus finish against the
@@ -576,11 +582,14 @@ __global__ __launch_bounds__(256) void fat_split_finish_kernel(FatParams p, int 
     request(0);
     const __half* svh = p.svh;
     const float* rowsum = p.rowsum;
-    int cm = c0;
+    int cm = c0, ys = p.n;
+    long long y0 = 0;
     if (!GU && p.mats.count > 1) {
         const MatRef r = mat_of_block(p.mats, bx);
         svh = r.svh;
         cm = c0 - r.nb0 * 128;
+        y0 = r.y0;
+        ys = r.ys;
         if constexpr (RAW) rowsum += (size_t)r.j * p.M * (p.k >> 7);
     }
     const __half2 sv0 = ld_h2(gptr(svh) + cm);
@@ -615,7 +624,7 @@ __global__ __launch_bounds__(256) void fat_split_finish_kernel(FatParams p, int 
             vb = raw_value(vb, sx);
         }
         fwht128_pair_fast(va, vb, lane);
-        st_y2(gptr(p.out16) + (size_t)row * p.n + c0,
+        st_y2(gptr(p.out16) + y0 + (size_t)row * ys + cm,
               h2_rn((va * kHadNorm) * __low2float(sv0), (vb * kHadNorm) * __high2float(sv0)), p.y_bf16);
     }
 }

@@ -59,7 +59,7 @@ int gemv_launch(int K, int cb, int mb, const GemvParams& p, int experts, hipStre
 
 size_t fat_gemm_scratch_bytes(int m, int k, int n, int mats);
 int fat_gemm_rows(const char* fn, const uint16_t* x, const MatSet& mats, uint16_t* y, int m, int k, int n, int K,
-                  int cb, int x_bf16, int y_bf16, void* ws, size_t ws_bytes, hipStream_t st);
+                  int cb, int x_bf16, int y_bf16, int plan_n, int plan_mats, void* ws, size_t ws_bytes, hipStream_t st);
 
 // Rows up to which exl3_gemm runs the GEMV kernels; above, the input is
 // rotated once and the MFMA GEMM runs (env EXL3_GEMM_GEMV_ROWS, at most 64).
@@ -234,10 +234,12 @@ int check_common(const char* fn, int m, int k, int n, int K, int codebook) {
     return EXL3_OK;
 }
 
-int run_gemv(const char* fn, GemvParams p, int K, int codebook, int experts, void* ws, size_t ws_bytes,
+// plan_n: the width that the launch shape and the workspace are planned for (p.n,
+// or wider where the call is part of another).
+int run_gemv(const char* fn, GemvParams p, int K, int codebook, int experts, int plan_n, void* ws, size_t ws_bytes,
              hipStream_t st) {
-    GemvPlan pl = plan_gemv(p.m, p.k, p.n, K, experts);
-    const size_t need = workspace_bytes_for(pl, p.m, p.k, p.n, experts);
+    GemvPlan pl = plan_gemv(p.m, p.k, plan_n, K, experts);
+    const size_t need = workspace_bytes_for(pl, p.m, p.k, plan_n, experts);
     EXL3_REQUIRE_CODE(need == 0 || (ws && ws_bytes >= need), EXL3_ERR_WORKSPACE,
                       "%s: workspace of %zu bytes needed, %zu given", fn, need, ws ? ws_bytes : (size_t)0);
     if (pl.sk) {
@@ -247,7 +249,7 @@ int run_gemv(const char* fn, GemvParams p, int K, int codebook, int experts, voi
             q.mats = p.mats;
         } else {
             q.mats.count = 1;
-            q.mats.n[0] = p.n;
+            q.mats.n[0] = q.mats.ys[0] = p.n;
             q.mats.trellis[0] = p.trellis;
             q.mats.suh[0] = p.suh;
             q.mats.svh[0] = p.svh;
@@ -265,7 +267,7 @@ int run_gemv(const char* fn, GemvParams p, int K, int codebook, int experts, voi
     p.nsteps = pl.nsteps;
     p.kw = pl.kw;
     p.splits = pl.splits;
-    if (gemv_fx(pl, p.m, p.n, experts) && !p.gu) {
+    if (gemv_fx(pl, p.m, plan_n, experts) && !p.gu) {
         p.fx = 1;
         p.acc = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(ws) + kWsAccOffset);
     }
@@ -281,7 +283,7 @@ int run_gemv(const char* fn, GemvParams p, int K, int codebook, int experts, voi
     }
     if (gemv_pre_rotates(pl, p.m, experts) && !p.gu) {
         __half* xr = reinterpret_cast<__half*>(reinterpret_cast<char*>(ws) + kWsScratchOffset +
-                                               gemv_partials_bytes(pl, p.m, p.n, experts));
+                                               gemv_partials_bytes(pl, p.m, plan_n, experts));
         // (several matrices never get here: cat_gemv)
         const int rc = rotate_rows(p.x, RotateSuh{{p.suh}}, 1, xr, p.m, p.k, p.x_bf16, nullptr, st,
                                    "exl3 gemv rotate launch");
@@ -470,7 +472,7 @@ extern "C" int exl3_gemv(const uint16_t* x, const int16_t* trellis, const uint16
     EXL3_REQUIRE(aligned(x, 4) && aligned(y, 4) && aligned(suh, 4) && aligned(svh, 4) && aligned(trellis, 16),
                  "exl3_gemv: misaligned pointer");
     GemvParams p = base_params(x, trellis, suh, svh, y, m, k, n);
-    return run_gemv("exl3_gemv", p, K, codebook, 1, workspace, workspace_bytes, as_stream(stream));
+    return run_gemv("exl3_gemv", p, K, codebook, 1, n, workspace, workspace_bytes, as_stream(stream));
 }
 
 extern "C" int exl3_gemm(const uint16_t* x, const int16_t* trellis, const uint16_t* suh, const uint16_t* svh,
@@ -484,12 +486,12 @@ extern "C" int exl3_gemm(const uint16_t* x, const int16_t* trellis, const uint16
                  "exl3_gemm: misaligned pointer");
     hipStream_t st = as_stream(stream);
     if (m > gemm_gemv_rows(n))
-        return fat_gemm_rows("exl3_gemm", x, one_mat(trellis, suh, svh, n), y, m, k, n, K, codebook, 0, 0, workspace,
-                             workspace_bytes, st);
+        return fat_gemm_rows("exl3_gemm", x, one_mat(trellis, suh, svh, n), y, m, k, n, K, codebook, 0, 0, n, 1,
+                             workspace, workspace_bytes, st);
     for (int r0 = 0; r0 < m; r0 += kMaxGemvRows) {
         const int mc = (m - r0) < kMaxGemvRows ? (m - r0) : kMaxGemvRows;
         GemvParams p = base_params(x + (size_t)r0 * k, trellis, suh, svh, y + (size_t)r0 * n, mc, k, n);
-        rc = run_gemv("exl3_gemm", p, K, codebook, 1, workspace, workspace_bytes, st);
+        rc = run_gemv("exl3_gemm", p, K, codebook, 1, n, workspace, workspace_bytes, st);
         if (rc) return rc;
     }
     return EXL3_OK;
@@ -513,44 +515,63 @@ extern "C" size_t exl3_linear_cat_workspace_size(int m, int k, const int* n, int
     return need;
 }
 
-extern "C" int exl3_linear_cat(const void* x, int x_dtype, const int16_t* const* trellis, const uint16_t* const* suh,
-                               const uint16_t* const* svh, const int* n, int count, void* y, int y_dtype, int m, int k,
-                               int K, int codebook, void* workspace, size_t workspace_bytes, void* stream) {
+extern "C" int exl3_linear_cat_part(const void* x, int x_dtype, const int16_t* const* trellis,
+                                    const uint16_t* const* suh, const uint16_t* const* svh, const int* n, int count,
+                                    int first, int apart, void* y, int y_dtype, int m, int k, int K, int codebook, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
     clear_error();
     EXL3_REQUIRE(count >= 1 && count <= kMaxMats, "exl3_linear_cat: %d matrices outside 1..%d", count, kMaxMats);
+    EXL3_REQUIRE(first >= 0 && first < count, "exl3_linear_cat: first matrix %d of %d", first, count);
     EXL3_REQUIRE(x && trellis && suh && svh && n && y, "exl3_linear_cat: null pointer");
     EXL3_REQUIRE((x_dtype == EXL3_DTYPE_F16 || x_dtype == EXL3_DTYPE_BF16) &&
                      (y_dtype == EXL3_DTYPE_F16 || y_dtype == EXL3_DTYPE_BF16),
                  "exl3_linear_cat: dtypes %d / %d", x_dtype, y_dtype);
     EXL3_REQUIRE(aligned(x, 4) && aligned(y, 4), "exl3_linear_cat: misaligned pointer");
+    // matrices first .. count - 1 run; the plan is that of all of them
     MatSet s{};
-    s.count = count;
-    long long total = 0;
+    s.count = count - first;
+    long long total = 0, skipped = 0;
     for (int j = 0; j < count; ++j) {
         const int rc = check_common("exl3_linear_cat", m, k, n[j], K, codebook);
         if (rc) return rc;
         EXL3_REQUIRE(trellis[j] && suh[j] && svh[j], "exl3_linear_cat: null pointer");
         EXL3_REQUIRE(aligned(trellis[j], 16) && aligned(suh[j], 4) && aligned(svh[j], 4),
                      "exl3_linear_cat: misaligned pointer");
-        s.nb0[j] = (int)(total / 128);
-        s.n[j] = n[j];
-        s.trellis[j] = reinterpret_cast<const uint32_t*>(trellis[j]);
-        s.suh[j] = reinterpret_cast<const __half*>(suh[j]);
-        s.svh[j] = reinterpret_cast<const __half*>(svh[j]);
         total += n[j];
+        if (j < first) {
+            skipped = total;
+            continue;
+        }
+        const int i = j - first;
+        s.nb0[i] = (int)((total - n[j] - skipped) / 128);
+        s.n[i] = n[j];
+        s.trellis[i] = reinterpret_cast<const uint32_t*>(trellis[j]);
+        s.suh[i] = reinterpret_cast<const __half*>(suh[j]);
+        s.svh[i] = reinterpret_cast<const __half*>(svh[j]);
     }
     EXL3_REQUIRE(total <= (1 << 30), "exl3_linear_cat: %lld columns", total);
-    const int nt = (int)total, xb = x_dtype == EXL3_DTYPE_BF16, yb = y_dtype == EXL3_DTYPE_BF16;
+    for (int i = 0; i < s.count; ++i) {
+        s.ys[i] = apart ? s.n[i] : (int)(total - skipped);
+        s.y0[i] = (long long)s.nb0[i] * 128 * (apart ? m : 1);
+    }
+    const int plan_n = (int)total, nt = (int)(total - skipped), xb = x_dtype == EXL3_DTYPE_BF16, yb = y_dtype == EXL3_DTYPE_BF16;
     hipStream_t st = as_stream(stream);
     if (!cat_gemv(m, k, n, count, K, codebook))
         return fat_gemm_rows("exl3_linear_cat", static_cast<const uint16_t*>(x), s, static_cast<uint16_t*>(y), m, k, nt,
-                             K, codebook, xb, yb, workspace, workspace_bytes, st);
-    GemvParams p = base_params(static_cast<const uint16_t*>(x), trellis[0], suh[0], svh[0], static_cast<uint16_t*>(y), m,
-                               k, nt);
-    p.mats = s;
+                             K, codebook, xb, yb, plan_n, count, workspace, workspace_bytes, st);
+    GemvParams p = base_params(static_cast<const uint16_t*>(x), trellis[first], suh[first], svh[first],
+                               static_cast<uint16_t*>(y), m, k, nt);
+    if (s.count > 1) p.mats = s;
     p.x_bf16 = xb;
     p.y_bf16 = yb;
-    return run_gemv("exl3_linear_cat", p, K, codebook, 1, workspace, workspace_bytes, st);
+    return run_gemv("exl3_linear_cat", p, K, codebook, 1, plan_n, workspace, workspace_bytes, st);
+}
+
+extern "C" int exl3_linear_cat(const void* x, int x_dtype, const int16_t* const* trellis, const uint16_t* const* suh,
+                               const uint16_t* const* svh, const int* n, int count, void* y, int y_dtype, int m, int k,
+                               int K, int codebook, void* workspace, size_t workspace_bytes, void* stream) {
+    return exl3_linear_cat_part(x, x_dtype, trellis, suh, svh, n, count, 0, 0, y, y_dtype, m, k, K, codebook, workspace,
+                                workspace_bytes, stream);
 }
 
 extern "C" int exl3_p2b_gemv_batched(const uint16_t* x, int x_per_expert, const int64_t* trellis_ptrs,
@@ -570,6 +591,6 @@ extern "C" int exl3_p2b_gemv_batched(const uint16_t* x, int x_per_expert, const 
     p.ids = ids;
     p.x_stride_e = x_per_expert ? (long long)m * k : 0;
     p.y_stride_e = (long long)m * n;
-    return run_gemv("exl3_p2b_gemv_batched", p, K, codebook, num_active, workspace, workspace_bytes,
+    return run_gemv("exl3_p2b_gemv_batched", p, K, codebook, num_active, n, workspace, workspace_bytes,
                     as_stream(stream));
 }

@@ -236,7 +236,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemv_sk_kernel(GemvSkParams p) {
     a = a * kHadNorm * __low2float(svv);
     b = b * kHadNorm * __high2float(svv);
     const size_t e0 = (size_t)r * n + cb * 128 + 2 * lane;
-    fx_add_pair(p.acc + e0, a, b, P, gptr(p.y) + e0, p.y_bf16);
+    fx_add_pair(p.acc + e0, a, b, P, gptr(p.y) + mat.y0 + (size_t)r * mat.ys + cbm * 128 + 2 * lane, p.y_bf16);
 }
 
 // Piece lengths (k-steps) the kernel is instantiated for.

@@ -169,6 +169,8 @@ __global__ __launch_bounds__(TL_THREADS, MT == 256 ? 2 : 4) void tall_kernel(Fat
     const __half* arows = p.a;
     const float* rowsum = p.rowsum;
     int bxm = p.gu ? bx >> 1 : bx, nm = p.n;  // column block and width inside the matrix
+    long long y0 = 0;                         // its output, rows ys apart
+    int ys = p.n;
     int m0 = blockIdx.y * MT;
     int rows = min(MT, p.M - m0);
     if (p.gmode) {
@@ -185,6 +187,8 @@ __global__ __launch_bounds__(TL_THREADS, MT == 256 ? 2 : 4) void tall_kernel(Fat
         svh_p = r.svh;
         bxm = bx - r.nb0;
         nm = r.n;
+        y0 = r.y0;
+        ys = r.ys;
         arows += (size_t)r.j * p.M * p.k;
         if constexpr (RAW) rowsum += (size_t)r.j * p.M * (p.k >> 7);
     }
@@ -206,7 +210,6 @@ __global__ __launch_bounds__(TL_THREADS, MT == 256 ? 2 : 4) void tall_kernel(Fat
     // consecutive columns each (fwht128_x16)
     float* ct = reinterpret_cast<float*>(fat_smem);
     const int col = (lane & 7) * 16;
-    const int c0 = bx * 128 + col;
     const float hn = fwht_x16_norm(lane);
     float sv[16];
     {
@@ -275,7 +278,8 @@ __global__ __launch_bounds__(TL_THREADS, MT == 256 ? 2 : 4) void tall_kernel(Fat
 #pragma unroll
             for (int e = 0; e < 8; ++e) ow[e] = y_bits(h2_rn(v[2 * e], v[2 * e + 1]), p.y_bf16);
             if (row >= rows) continue;
-            EXL3_GLOBAL uint32_t* o = reinterpret_cast<EXL3_GLOBAL uint32_t*>(gptr(p.out16) + orow * p.n + c0);
+            EXL3_GLOBAL uint32_t* o =
+                reinterpret_cast<EXL3_GLOBAL uint32_t*>(gptr(p.out16) + y0 + orow * ys + bxm * 128 + col);
             if (p.out_vec) {
                 reinterpret_cast<EXL3_GLOBAL u32x4_t*>(o)[0] = u32x4_t{ow[0], ow[1], ow[2], ow[3]};
                 reinterpret_cast<EXL3_GLOBAL u32x4_t*>(o)[1] = u32x4_t{ow[4], ow[5], ow[6], ow[7]};

@@ -1,5 +1,5 @@
 // Native entry of the operators that programs call eagerly, one per layer:
-// exl3_gemv, exl3_linear_cat and exl3_gate_up_swiglu.
+// exl3_gemv, exl3_linear_cat, exl3_linear_part and exl3_gate_up_swiglu.
 //
 // A one-token call is bound by its host path: from Python (operator wrapper,
 // checks, two ctypes calls, stream and device queries) exl3_gemv took 20.5 us
@@ -32,7 +32,7 @@ namespace {
 struct Abi {
     decltype(&exl3_gemv) gemv;
     decltype(&exl3_gemv_workspace_size) gemv_ws;
-    decltype(&exl3_linear_cat) cat;
+    decltype(&exl3_linear_cat_part) cat;
     decltype(&exl3_linear_cat_workspace_size) cat_ws;
     decltype(&exl3_gate_up_swiglu) gate_up;
     decltype(&exl3_gate_up_workspace_size) gate_up_ws;
@@ -140,13 +140,21 @@ struct Cat {
     static constexpr const char *name = "sglang_exl3::exl3_linear_cat",
                                 *general = "sglang_exl3::exl3_linear_cat_general";
 };
+using PartFn = at::Tensor(const at::Tensor&, at::TensorList, at::TensorList, at::TensorList, c10::SymInt, c10::SymInt,
+                          bool, c10::SymInt);
+struct Part {
+    static constexpr const char *name = "sglang_exl3::exl3_linear_part",
+                                *general = "sglang_exl3::exl3_linear_part_general";
+};
 
-at::Tensor linear_cat(const at::Tensor& x, at::TensorList trellis, at::TensorList suh, at::TensorList svh, int64_t K,
-                      int64_t codebook, bool out_bf16) {
+// Weights from `first` on, side by side [m, n] or (apart) packed one after the
+// other [m * n]; an undefined tensor: the general path.
+at::Tensor linear_weights(const at::Tensor& x, at::TensorList trellis, at::TensorList suh, at::TensorList svh,
+                          int64_t K, int64_t codebook, bool out_bf16, int64_t first, bool apart) {
     const int64_t m = rows_of(x, true), k = m ? x.size(-1) : 0, dev = m ? x.get_device() : -1;
     const size_t count = trellis.size();
     bool ok = m >= 1 && count >= 1 && count <= 4 && suh.size() == count && svh.size() == count && K >= 1 && K <= 8 &&
-              codebook >= 0 && codebook <= 2;
+              codebook >= 0 && codebook <= 2 && first >= 0 && first < (int64_t)count;
     const int16_t* tr[4];
     const uint16_t *su[4], *sv[4];
     int ns[4];
@@ -159,19 +167,35 @@ at::Tensor linear_cat(const at::Tensor& x, at::TensorList trellis, at::TensorLis
         su[j] = u16(suh[j]);
         sv[j] = u16(svh[j]);
         ns[j] = (int)(trellis[j].size(1) * 16);
-        n += ns[j];
+        if ((int64_t)j >= first) n += ns[j];
     }
     Launch l;
     if (ok && l.get(dev, abi.cat_ws((int)m, (int)k, ns, (int)count, (int)K))) {
-        at::Tensor y = at::empty({m, n}, x.options().dtype(out_bf16 ? at::kBFloat16 : at::kHalf));
+        const auto options = x.options().dtype(out_bf16 ? at::kBFloat16 : at::kHalf);
+        at::Tensor y = apart ? at::empty({m * n}, options) : at::empty({m, n}, options);
         if (done(abi.cat(x.const_data_ptr(), x.scalar_type() == at::kBFloat16 ? 1 : 0, tr, su, sv, ns, (int)count,
-                         y.mutable_data_ptr(), out_bf16 ? 1 : 0, (int)m, (int)k, (int)K, (int)codebook,
-                         l.ws.mutable_data_ptr(), l.ws.numel(), l.stream),
+                         (int)first, apart ? 1 : 0, y.mutable_data_ptr(), out_bf16 ? 1 : 0, (int)m, (int)k, (int)K,
+                         (int)codebook, l.ws.mutable_data_ptr(), l.ws.numel(), l.stream),
                  l))
             return y;
     }
+    return {};
+}
+
+at::Tensor linear_cat(const at::Tensor& x, at::TensorList trellis, at::TensorList suh, at::TensorList svh, int64_t K,
+                      int64_t codebook, bool out_bf16) {
+    at::Tensor y = linear_weights(x, trellis, suh, svh, K, codebook, out_bf16, 0, false);
+    if (y.defined()) return y;
     static const auto h = c10::Dispatcher::singleton().findSchemaOrThrow(Cat::general, "").typed<CatFn>();
     return h.call(x, trellis, suh, svh, K, codebook, out_bf16);
+}
+
+at::Tensor linear_part(const at::Tensor& x, at::TensorList trellis, at::TensorList suh, at::TensorList svh, int64_t K,
+                       int64_t codebook, bool out_bf16, int64_t first) {
+    at::Tensor y = linear_weights(x, trellis, suh, svh, K, codebook, out_bf16, first, true);
+    if (y.defined()) return y;
+    static const auto h = c10::Dispatcher::singleton().findSchemaOrThrow(Part::general, "").typed<PartFn>();
+    return h.call(x, trellis, suh, svh, K, codebook, out_bf16, first);
 }
 
 // -------------------------------------------------------- exl3_gate_up_swiglu
@@ -240,6 +264,7 @@ struct Autograd<Op, R(A...)> {
 TORCH_LIBRARY_IMPL(sglang_exl3, CUDA, m) {
     m.impl("exl3_gemv", gemv);
     m.impl("exl3_linear_cat", linear_cat);
+    m.impl("exl3_linear_part", linear_part);
     m.impl("exl3_gate_up_swiglu", gate_up);
     m.impl("keep_workspace", keep_workspace);
 }
@@ -247,10 +272,11 @@ TORCH_LIBRARY_IMPL(sglang_exl3, CUDA, m) {
 TORCH_LIBRARY_IMPL(sglang_exl3, AutogradCUDA, m) {
     m.impl("exl3_gemv", Autograd<Gemv, GemvFn>::call);
     m.impl("exl3_linear_cat", Autograd<Cat, CatFn>::call);
+    m.impl("exl3_linear_part", Autograd<Part, PartFn>::call);
     m.impl("exl3_gate_up_swiglu", Autograd<GateUp, GateUpFn>::call);
 }
 
-// Addresses of the C ABI: gemv, its workspace size, linear_cat, .., gate_up, ..
+// Addresses of the C ABI: gemv, its workspace size, linear_cat_part, .., gate_up, ..
 extern "C" void exl3_ops_bind(void* const* fn) {
     abi.gemv = reinterpret_cast<decltype(abi.gemv)>(fn[0]);
     abi.gemv_ws = reinterpret_cast<decltype(abi.gemv_ws)>(fn[1]);

@@ -53,6 +53,7 @@ SIGNATURES = {
     "exl3_gemm": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _SZ, _P]),
     "exl3_linear_cat_workspace_size": (_SZ, [_I, _I, _P, _I, _I]),
     "exl3_linear_cat": (_I, [_P, _I, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _P, _SZ, _P]),
+    "exl3_linear_cat_part": (_I, [_P, _I, _P, _P, _P, _P, _I, _I, _I, _P, _I, _I, _I, _I, _I, _P, _SZ, _P]),
     "exl3_p2b_gemv_batched": (_I, [_P, _I, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _P, _SZ, _P]),
     "exl3_hadamard_rows": (_I, [_P, _P, _P, _P, _F, _I, _I, _P]),
     "exl3_hadamard_fast": (_I, [_P, _P, _P, _I, _I, _I, _P]),
@@ -101,7 +102,7 @@ def lib() -> ctypes.CDLL:
 
 
 # the entry points of the operators' native path, in the order exl3_ops_bind takes them
-_OPS_BOUND = ("exl3_gemv", "exl3_gemv_workspace_size", "exl3_linear_cat", "exl3_linear_cat_workspace_size",
+_OPS_BOUND = ("exl3_gemv", "exl3_gemv_workspace_size", "exl3_linear_cat_part", "exl3_linear_cat_workspace_size",
               "exl3_gate_up_swiglu", "exl3_gate_up_workspace_size")
 
 

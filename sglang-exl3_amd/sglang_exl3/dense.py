@@ -182,17 +182,19 @@ def _gemv_rows(width: int) -> int:
     return 12 if width < 12288 else (8 if width < 24576 else 7)
 
 
-def _cat_exact(linears: list, rows: int) -> bool:
-    """Whether exl3_linear_cat multiplies by weights as exact as the separate
-    calls do.  The GEMV and the batched launch (pair form) add the two fp16
-    halves of an MCG codebook value exactly; the MFMA tiles round the sum to
-    fp16 (error of an fp16 output against 64 bits: 2.1e-4 -> 3.1e-4).
+def _separate_rows(linears: list) -> tuple:
+    """(lo, hi): from lo + 1 to hi rows the shards run as separate calls, whose
+    weights are more exact than exl3_linear_cat's there.  The GEMV and the
+    batched launch (pair form) add the two fp16 halves of an MCG codebook value
+    exactly; the MFMA tiles round the sum to fp16 (error of an fp16 output
+    against 64 bits: 2.1e-4 -> 3.1e-4).
     exl3_linear_cat leaves the GEMV at the row count of the narrowest shard,
     which is where separate calls leave it too, except a batched pair, which
     keeps the pair form up to FUSED_PAIR_MAX_ROWS rows.  mul1 tiles read exact
     entries."""
-    return (linears[0].codebook != _lib.CB_MCG or _batched_pair(linears) is None
-            or rows <= _gemv_rows(min(lin.out_features for lin in linears)) or rows > FUSED_PAIR_MAX_ROWS)
+    if linears[0].codebook != _lib.CB_MCG or _batched_pair(linears) is None:
+        return 0, 0
+    return _gemv_rows(min(lin.out_features for lin in linears)), FUSED_PAIR_MAX_ROWS
 
 
 class EXL3LinearMethod(LinearMethodBase):
@@ -277,6 +279,7 @@ class EXL3LinearMethod(LinearMethodBase):
             linears.append(EXL3DenseLinear(pack["trellis"], pack["suh"], pack["svh"], pack.get("mcg"),
                                            pack.get("mul1")))
         layer._exl3_linears = linears
+        layer._exl3_separate_rows = _separate_rows(linears)
         if not self._logged:
             self._logged = True
             logger.info("EXL3 dense linears engaged: shards=%d K=%s", len(linears), [lin.K for lin in linears])
@@ -297,21 +300,33 @@ class EXL3LinearMethod(LinearMethodBase):
                 x2 = x2.to(torch.float16).contiguous()
         return shape, rows, x2, scale
 
+    @staticmethod
+    def _cat(layer, linears: list, x: torch.Tensor, fuse_on: bool, kv_only: bool = False) -> Optional[torch.Tensor]:
+        """Every shard in one call, the casts inside the kernels: [rows, widths]
+        in the layer's dtype (kv_only: the second and third alone, packed one
+        after the other, with the same bits); None where they run separately."""
+        lo, hi = getattr(layer, "_exl3_separate_rows", None) or _separate_rows(linears)
+        if lo < math.prod(x.shape[:-1]) <= hi or not x.is_cuda or not (fuse_on or len(linears) == 1):
+            return None
+        out_dtype = getattr(layer, "_exl3_out_dtype", x.dtype)
+        if getattr(layer, "_exl3_scale_input", False) or not _cat_compatible(linears, x.dtype, out_dtype):
+            return None
+        from .ops import register_custom_ops
+
+        register_custom_ops()
+        args = (x.reshape(-1, x.shape[-1]), [lin.trellis for lin in linears], [lin.suh for lin in linears],
+                [lin.svh for lin in linears], linears[0].K, linears[0].codebook, out_dtype == torch.bfloat16)
+        return torch.ops.sglang_exl3.exl3_linear_part(*args, 1) if kv_only \
+            else torch.ops.sglang_exl3.exl3_linear_cat(*args)
+
     def apply(self, layer, x: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         linears = getattr(layer, "_exl3_linears", None)
         if not linears:
             raise RuntimeError("EXL3 linear layers were not built after weight load")
         fuse_on = os.environ.get("SGLANG_EXL3_MGEMM", "1") != "0"
         out_dtype = getattr(layer, "_exl3_out_dtype", x.dtype)
-        if x.is_cuda and (fuse_on or len(linears) == 1) and not getattr(layer, "_exl3_scale_input", False) \
-                and _cat_compatible(linears, x.dtype, out_dtype) and _cat_exact(linears, math.prod(x.shape[:-1])):
-            # every shard in one call, the casts inside the kernels
-            from .ops import register_custom_ops
-
-            register_custom_ops()
-            y = torch.ops.sglang_exl3.exl3_linear_cat(
-                x.reshape(-1, x.shape[-1]), [lin.trellis for lin in linears], [lin.suh for lin in linears],
-                [lin.svh for lin in linears], linears[0].K, linears[0].codebook, out_dtype == torch.bfloat16)
+        y = self._cat(layer, linears, x, fuse_on)
+        if y is not None:
             if bias is not None:
                 y = y + bias.to(out_dtype)
             return y.view(*x.shape[:-1], y.shape[-1])
@@ -328,13 +343,20 @@ class EXL3LinearMethod(LinearMethodBase):
         return y.view(*shape[:-1], y.shape[-1])
 
     def apply_kv_only(self, layer, x: torch.Tensor):
-        """K and V shards of a 3-shard qkv projection only (Q skipped)."""
+        """K and V shards of a 3-shard qkv projection only (Q skipped): the
+        bits of apply's K and V columns."""
         linears = getattr(layer, "_exl3_linears", None)
         if not linears or len(linears) != 3:
             raise RuntimeError("apply_kv_only requires a 3-shard qkv_proj")
-        shape, rows, x2, _ = self._prepare(layer, x)
         kl, vl = linears[1], linears[2]
-        if rows <= FUSED_PAIR_MAX_ROWS and _pair_compatible(kl, vl) and os.environ.get("SGLANG_EXL3_MGEMM", "1") != "0":
+        fuse_on = os.environ.get("SGLANG_EXL3_MGEMM", "1") != "0"
+        y = self._cat(layer, linears, x, fuse_on, kv_only=True)
+        if y is not None:
+            rows = math.prod(x.shape[:-1])
+            k, v = y.split((rows * kl.out_features, rows * vl.out_features))
+            return k.view(*x.shape[:-1], kl.out_features), v.view(*x.shape[:-1], vl.out_features)
+        shape, rows, x2, _ = self._prepare(layer, x)
+        if rows <= FUSED_PAIR_MAX_ROWS and _pair_compatible(kl, vl) and fuse_on:
             k, v = fused_pair(layer, x2, kl, vl)
         else:
             k, v = kl.forward(x2), vl.forward(x2)

@@ -240,10 +240,23 @@ def exl3_linear_cat_impl(x, trellis, suh, svh, K, codebook, out_bf16):
     one layer: one K and codebook, each its own trellis, suh and svh.  x fp16 or
     bf16, the output fp16 or bf16, without a cast, copy or concatenation around
     the kernels (reference: src/sglang_exl3/dense.py:317-371)."""
-    name = "exl3_linear_cat"
+    return _linear_weights("exl3_linear_cat", x, trellis, suh, svh, K, codebook, out_bf16, 0, False)
+
+
+def exl3_linear_part_impl(x, trellis, suh, svh, K, codebook, out_bf16, first):
+    """The weights of exl3_linear_cat from `first` on, with the bits that their
+    columns have there, each output packed: [rows x width_first, then rows x
+    width_(first + 1), ..] in one dimension (reference:
+    src/sglang_exl3/dense.py:373-398)."""
+    return _linear_weights("exl3_linear_part", x, trellis, suh, svh, K, codebook, out_bf16, int(first), True)
+
+
+def _linear_weights(name, x, trellis, suh, svh, K, codebook, out_bf16, first, apart):
     count = len(trellis)
     if not 1 <= count <= CAT_MAX or len(suh) != count or len(svh) != count:
         raise RuntimeError(f"sglang_exl3::{name}: 1 to {CAT_MAX} weights with a suh and svh each")
+    if not 0 <= first < count:
+        raise RuntimeError(f"sglang_exl3::{name}: first weight {first} of {count}")
     _require_device(name, x, *trellis, *suh, *svh)
     if x.dim() < 2 or x.dtype not in _CAT_DTYPES:
         raise RuntimeError(f"sglang_exl3::{name}: x must be float16 or bfloat16 [..., in_features]")
@@ -269,7 +282,8 @@ def exl3_linear_cat_impl(x, trellis, suh, svh, K, codebook, out_bf16):
     x2 = x.reshape(m, kdim).contiguous()
     if x2.dtype == torch.bfloat16 and x2.data_ptr() % 4:
         x2 = x2.clone()
-    y = torch.empty((m, sum(widths)), dtype=torch.bfloat16 if out_bf16 else torch.float16, device=x.device)
+    n = sum(widths[first:])
+    y = torch.empty((m * n,) if apart else (m, n), dtype=torch.bfloat16 if out_bf16 else torch.float16, device=x.device)
     if m == 0:
         return y
     lib = _lib.lib()
@@ -278,9 +292,10 @@ def exl3_linear_cat_impl(x, trellis, suh, svh, K, codebook, out_bf16):
     with torch.cuda.device(x.device):
         need = int(lib.exl3_linear_cat_workspace_size(m, kdim, ns, count, int(K)))
         ws = workspace(x.device, need) if need else None
-        rc = lib.exl3_linear_cat(x2.data_ptr(), _CAT_DTYPES[x2.dtype], *ptrs, ns, count, y.data_ptr(),
-                                 _CAT_DTYPES[y.dtype], m, kdim, int(K), int(codebook),
-                                 0 if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream_ptr(x))
+        rc = lib.exl3_linear_cat_part(x2.data_ptr(), _CAT_DTYPES[x2.dtype], *ptrs, ns, count, first, int(apart),
+                                      y.data_ptr(), _CAT_DTYPES[y.dtype], m, kdim, int(K), int(codebook),
+                                      0 if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+                                      _stream_ptr(x))
     check_ws(rc, name, ws)
     return y
 
@@ -589,6 +604,24 @@ def register_custom_ops() -> bool:
     def _(x, trellis, suh, svh, K, codebook, out_bf16):
         rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
         return torch.empty((rows, sum(t.size(1) * 16 for t in trellis)),
+                           dtype=torch.bfloat16 if out_bf16 else torch.float16, device=x.device)
+
+    @torch.library.custom_op("sglang_exl3::exl3_linear_part", mutates_args=())
+    def exl3_linear_part(x: torch.Tensor, trellis: List[torch.Tensor], suh: List[torch.Tensor],
+                         svh: List[torch.Tensor], K: int, codebook: int, out_bf16: bool, first: int) -> torch.Tensor:
+        return exl3_linear_part_impl(x, trellis, suh, svh, K, codebook, out_bf16, first)
+
+    @torch.library.custom_op("sglang_exl3::exl3_linear_part_general", mutates_args=())
+    def exl3_linear_part_general(x: torch.Tensor, trellis: List[torch.Tensor], suh: List[torch.Tensor],
+                                 svh: List[torch.Tensor], K: int, codebook: int, out_bf16: bool,
+                                 first: int) -> torch.Tensor:
+        return exl3_linear_part_impl(x, trellis, suh, svh, K, codebook, out_bf16, first)
+
+    @exl3_linear_part_general.register_fake
+    @exl3_linear_part.register_fake
+    def _(x, trellis, suh, svh, K, codebook, out_bf16, first):
+        rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
+        return torch.empty((rows * sum(t.size(1) * 16 for t in trellis[first:]),),
                            dtype=torch.bfloat16 if out_bf16 else torch.float16, device=x.device)
 
     @torch.library.custom_op("sglang_exl3::p2b_gemv_batched", mutates_args=())

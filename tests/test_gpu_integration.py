@@ -321,6 +321,25 @@ def test_linear_layer_weights_are_not_rounded(rows, outs, cb, exact):
         assert err < EXACT_WEIGHTS_REL
 
 
+@pytest.mark.parametrize("outs,cb,dtype", [
+    ([512, 128, 128], 1, torch.bfloat16), ([512, 128, 128], 2, torch.float16), ([384, 256, 128], 0, torch.bfloat16),
+    ([4096, 128, 256], 2, torch.bfloat16),
+])
+def test_kv_only_has_the_bits_of_apply(outs, cb, dtype):
+    """apply_kv_only returns apply's K and V, packed, at every row count: GEMV plans, 16-row and tall tiles with and
+    without k-splits, the batched pair (MCG, 13 to 64 rows)."""
+    k, K = 2048, 3
+    method, layer, packs = _linear_layer(outs, k, K, cb, dtype, seed=11)
+    for rows in (1, 2, 4, 7, 11, 12, 13, 16, 17, 40, 64, 65, 200, 600):
+        print(f"case: kv only outs={outs} cb={cb} rows={rows}", flush=True)
+        x = torch.from_numpy(make_x(rows, k, seed=rows)).cuda().to(dtype).view(1, rows, k)
+        want = method.apply(layer, x).split(outs, dim=-1)[1:]
+        got = method.apply_kv_only(layer, x)
+        for g, w in zip(got, want):
+            assert g.is_contiguous() and g.dtype == dtype and torch.equal(g, w)
+    assert method.apply_kv_only(layer, x[:, :0])[0].shape == (1, 0, outs[1])
+
+
 @pytest.mark.parametrize("T,invalid", [(1, 0), (1, 1), (6, 2), (60, 0), (200, 3)])
 def test_moe_bf16_matches_casts(T, invalid):
     """bf16 rows in and out of the one-call layer: the bits of the fp16 layer with casts around it (one token

@@ -29,6 +29,7 @@ def _calls(w, x):
     return {
         "gemv": (o.exl3_gemv, o.exl3_gemv_general, (x, *w[0], K, True, 1)),
         "cat": (o.exl3_linear_cat, o.exl3_linear_cat_general, (x, tr, su, sv, K, 1, True)),
+        "part": (o.exl3_linear_part, o.exl3_linear_part_general, (x, tr, su, sv, K, 2, False, 1)),
         "cat1": (o.exl3_linear_cat, o.exl3_linear_cat_general, (x.bfloat16(), tr[:1], su[:1], sv[:1], K, 2, False)),
         "gate_up": (o.exl3_gate_up_swiglu, o.exl3_gate_up_swiglu_general, (x, su[0], tr[0], sv[0], tr[1], sv[1], K, 1, 2.0)),
     }
@@ -44,7 +45,7 @@ def _same(op, general, args):
     assert torch.equal(*outs) if isinstance(outs[0], torch.Tensor) else outs[0] == outs[1]
 
 
-@pytest.mark.parametrize("name", ["gemv", "cat", "cat1", "gate_up"])
+@pytest.mark.parametrize("name", ["gemv", "cat", "part", "cat1", "gate_up"])
 @pytest.mark.parametrize("m", [1, 17, 64])
 def test_native_equals_general(weights, name, m):
     print(f"case: native op {name} m={m}", flush=True)
@@ -85,7 +86,7 @@ def test_native_refuses_what_general_refuses(weights):
     for name, (op, general, args) in _calls(weights, x).items():
         for bad in ((x[:, :128], *args[1:]), (x.float(), *args[1:]), (x[0], *args[1:]), (x.cpu(), *args[1:])):
             _same(op, general, bad)
-        empty = op(x[:0], *args[1:]) if name in ("cat", "cat1", "gate_up") else None
+        empty = op(x[:0], *args[1:]) if name in ("cat", "part", "cat1", "gate_up") else None
         assert empty is None or empty.shape == general(x[:0], *args[1:]).shape
         xg = args[0].detach().clone().requires_grad_()
         y = op(xg, *args[1:])

@@ -48,6 +48,8 @@ def test_meta_fake_tensor_dispatch():
         xb = torch.empty((2, 128), dtype=torch.bfloat16)
         c = torch.ops.sglang_exl3.exl3_linear_cat(xb, [trellis, trellis], [suh, suh], [svh, svh], 2, 1, False)
         assert c.shape == (2, 512) and c.dtype == torch.float16
+        c = torch.ops.sglang_exl3.exl3_linear_part(xb, [trellis] * 3, [suh] * 3, [svh] * 3, 2, 1, True, 1)
+        assert c.shape == (1024,) and c.dtype == torch.bfloat16
         mo = torch.ops.sglang_exl3.exl3_moe_layer_typed(xb, ids, w, *[ptrs] * 9, 2, 2, 2, True, 128)
         assert mo.shape == (2, 128) and mo.dtype == torch.bfloat16
         o32 = torch.empty((2, 256), dtype=torch.float32)
