@@ -2,13 +2,15 @@
 
 Compiles every csrc/*.hip (the GEMV instantiation unit once per bit width)
 with hipcc for gfx950 and links one shared library into
-sglang_exl3/_lib/, and csrc/torch_ops.cpp (host code) with g++ into a second.  Run directly (python build_hip.py) or through
-__graft_entry__.build().
+sglang_exl3/_lib/, and csrc/torch_ops.cpp (host code) with g++ into a second,
+which the operators can do without.  Run directly (python build_hip.py) or
+through __graft_entry__.build().
 """
 
 from __future__ import annotations
 
 import concurrent.futures as cf
+import importlib.metadata
 import importlib.util
 import os
 import shutil
@@ -86,20 +88,34 @@ def build(force: bool = False, jobs: int | None = None) -> str:
 
 
 def _build_ops(force: bool) -> None:
-    """The operators' native entry (host code, linked against PyTorch)."""
+    """The operators' native entry (host code, linked against PyTorch, whose
+    version it names).  Where PyTorch cannot be built against, a
+    warning: the operators then run without it."""
     src, out = os.path.join(CSRC, "torch_ops.cpp"), os.path.join(LIBDIR, OPS_LIBNAME)
-    if not force and os.path.exists(out) and os.path.getmtime(out) >= max(os.path.getmtime(src), _headers_mtime()):
+    header = os.path.join(HERE, "..", "include", "sglang_exl3_amd.h")
+    try:
+        version = importlib.metadata.version("torch")
+        torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    except (importlib.metadata.PackageNotFoundError, AttributeError):
+        print("warning: no PyTorch, the operators' native entry is not built", file=sys.stderr)
         return
-    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    if not force and os.path.exists(out) and os.path.getmtime(out) >= max(map(os.path.getmtime, (src, header))):
+        with open(out, "rb") as f:
+            if b"exl3-ops-torch:" + version.encode() + b"\0" in f.read():
+                return
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
     inc = [os.path.join(torch_dir, "include"), os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
            os.path.join(rocm, "include")]
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", f'-DEXL3_TORCH_VERSION="{version}"',
            *(f"-I{i}" for i in inc), src, "-o", out + ".tmp", f"-L{os.path.join(torch_dir, 'lib')}",
            "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", f"-L{os.path.join(rocm, 'lib')}", "-lamdhip64"]
     r = subprocess.run(cmd, capture_output=True, text=True)
+    if os.path.exists(out):
+        os.remove(out)
     if r.returncode != 0:
-        raise RuntimeError(f"g++ failed for torch_ops.cpp:\n{r.stderr[-6000:]}")
+        print(f"warning: the operators' native entry is not built, g++ failed for torch_ops.cpp:\n{r.stderr[-6000:]}",
+              file=sys.stderr)
+        return
     os.replace(out + ".tmp", out)
 
 

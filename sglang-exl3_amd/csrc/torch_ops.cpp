@@ -276,6 +276,10 @@ TORCH_LIBRARY_IMPL(sglang_exl3, AutogradCUDA, m) {
     m.impl("exl3_gate_up_swiglu", Autograd<GateUp, GateUpFn>::call);
 }
 
+// The PyTorch that this was built for (EXL3_TORCH_VERSION), looked up in the file
+// before it is loaded: another one's ABI need not fit.
+extern "C" __attribute__((used)) const char exl3_ops_torch[] = "exl3-ops-torch:" EXL3_TORCH_VERSION;
+
 // Addresses of the C ABI: gemv, its workspace size, linear_cat_part, .., gate_up, ..
 extern "C" void exl3_ops_bind(void* const* fn) {
     abi.gemv = reinterpret_cast<decltype(abi.gemv)>(fn[0]);

@@ -7,6 +7,7 @@ if the library is missing or fails to load, every op raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.metadata
 import os
 import threading
 
@@ -14,6 +15,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("SGLANG_EXL3_AMD_LIB", os.path.join(_HERE, "_lib", "libsglang_exl3_amd.so"))
 
 OPS_LIB_PATH = os.path.join(_HERE, "_lib", "libsglang_exl3_ops.so")
+OPS_TORCH_MARK = b"exl3-ops-torch:"  # in the operator library, followed by the PyTorch version it was built for
 
 EXL3_OK = 0
 EXL3_ERR_ARG = 1
@@ -107,11 +109,16 @@ _OPS_BOUND = ("exl3_gemv", "exl3_gemv_workspace_size", "exl3_linear_cat_part", "
 
 
 def load_ops() -> ctypes.CDLL:
-    """Load the operators' native path (csrc/torch_ops.cpp; needs torch) and bind it to the HIP library."""
+    """Load the operators' native path (csrc/torch_ops.cpp; needs torch) and bind it to the HIP library.
+    RuntimeError or OSError where it is not there, was built for another PyTorch or does not load."""
     if not os.path.exists(OPS_LIB_PATH):
         raise RuntimeError(f"sglang_exl3 operator library not found at {OPS_LIB_PATH}; build it with "
                            "`python sglang-exl3_amd/build_hip.py` (or __graft_entry__.build())")
     L = lib()
+    version = importlib.metadata.version("torch")
+    with open(OPS_LIB_PATH, "rb") as f:
+        if OPS_TORCH_MARK + version.encode() + b"\0" not in f.read():
+            raise RuntimeError(f"{OPS_LIB_PATH} was not built for PyTorch {version}")
     ops = ctypes.CDLL(OPS_LIB_PATH)
     ops.exl3_ops_bind.restype = None
     ops.exl3_ops_bind.argtypes = [_P]

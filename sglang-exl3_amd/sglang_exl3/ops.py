@@ -21,6 +21,7 @@ from . import _lib
 logger = logging.getLogger("sglang.exl3.ops")
 
 _OPS_REGISTERED = False
+_NATIVE_PATH = False  # the operators' native path (csrc/torch_ops.cpp) is loaded
 
 # Reference op list (tests/test_cuda_graph.py:15-23)
 OP_NAMES = (
@@ -84,7 +85,7 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
             _RETIRED_WORKSPACES.append((key, ws))
         ws = torch.zeros(size, dtype=torch.uint8, device=device)
         _WORKSPACES[key] = ws
-        if _OPS_REGISTERED:
+        if _NATIVE_PATH:
             torch.ops.sglang_exl3.keep_workspace(ws, key[1])
     elif capturing:
         _CAPTURED[id(ws)] = ws
@@ -539,7 +540,7 @@ def exl3_fat_gemm_scatter_impl(a, packed, out, svh, token_idx, route_weight, K, 
 def register_custom_ops() -> bool:
     """Register the EXL3 kernels in torch.ops.sglang_exl3 with fake kernels
     (same schemas as src/sglang_exl3/ops.py:38-226)."""
-    global _OPS_REGISTERED
+    global _OPS_REGISTERED, _NATIVE_PATH
     if _OPS_REGISTERED:
         return True
 
@@ -726,11 +727,17 @@ def register_custom_ops() -> bool:
     def _(a, packed, out, svh, token_idx, route_weight, K, mcg, mul1):
         return None
 
-    # the native path of the *_general twins' operators (csrc/torch_ops.cpp), and the workspaces it runs on
+    # the native path of the *_general twins' operators (csrc/torch_ops.cpp), and the workspaces it runs on;
+    # without it the operators run their Python implementation, on the same kernels
     _FRAGMENT.define("keep_workspace(Tensor ws, int stream) -> ()")
-    _lib.load_ops()
+    try:
+        _lib.load_ops()
+        _NATIVE_PATH = True
+    except (OSError, RuntimeError) as e:
+        logger.warning("sglang_exl3: the operators' native path is not used (eager calls cost more host time): %s", e)
     _OPS_REGISTERED = True
-    for (_, stream), ws in _WORKSPACES.items():
-        torch.ops.sglang_exl3.keep_workspace(ws, stream)
+    if _NATIVE_PATH:
+        for (_, stream), ws in _WORKSPACES.items():
+            torch.ops.sglang_exl3.keep_workspace(ws, stream)
     logger.info("registered sglang_exl3 custom ops (gfx950 HIP backend)")
     return True

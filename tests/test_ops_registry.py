@@ -3,11 +3,18 @@
 Mirrors the reference's tests/test_cuda_graph.py:13-68 (same op list, same fake
 shapes), and checks that CPU tensors are refused (no CPU fallback)."""
 
+import importlib.metadata
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
 import sglang_exl3
 from sglang_exl3 import ops
+
+PKG = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "sglang-exl3_amd")
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -54,6 +61,35 @@ def test_meta_fake_tensor_dispatch():
         assert mo.shape == (2, 128) and mo.dtype == torch.bfloat16
         o32 = torch.empty((2, 256), dtype=torch.float32)
         assert torch.ops.sglang_exl3.exl3_fat_gemm(x, trellis, o32, svh, 2, True, False) is None
+
+
+@pytest.mark.parametrize("fault", ["missing", "other torch", "does not load"])
+def test_operators_register_without_the_native_path(fault, tmp_path):
+    """Without the second library, with one built for another PyTorch or one that does not load, the operators are
+    registered all the same and keep their Python implementation."""
+    lib = tmp_path / "libsglang_exl3_ops.so"
+    if fault != "missing":
+        version = importlib.metadata.version("torch") if fault == "does not load" else "0.0.1"
+        lib.write_bytes(b"not a library exl3-ops-torch:" + version.encode() + b"\0")
+    code = f"""
+import sys
+sys.path.insert(0, {PKG!r})
+import torch
+from sglang_exl3 import _lib, ops
+_lib.OPS_LIB_PATH = {str(lib)!r}
+assert ops.register_custom_ops() and not ops._NATIVE_PATH
+x = torch.empty((2, 128), dtype=torch.float16, device="meta")
+t, h = (torch.empty(s, dtype=d, device="meta") for s, d in (((8, 16, 32), torch.int16), ((256,), torch.float16)))
+assert torch.ops.sglang_exl3.exl3_linear_cat(x, [t], [h], [h], 2, 1, False).shape == (2, 256)
+try:
+    torch.ops.sglang_exl3.exl3_gemv(torch.zeros((1, 128)), torch.zeros((8, 16, 32)), torch.zeros(128), torch.zeros(256), 2, True)
+except RuntimeError as e:
+    assert "HIP device" in str(e)
+else:
+    raise AssertionError
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
 
 
 def test_cpu_tensors_are_refused():
