@@ -43,7 +43,7 @@ __device__ __forceinline__ void copy_to_lds16(const EXL3_GLOBAL char* base, uint
         "s_nop 0\n\t"
         "global_load_lds_dwordx4 %0, %1" ::"v"(off),
         "s"(base), "s"(lds)
-        : "memory");
+        : "memory", "m0");
 }
 
 // The k loop of one wave: `rows` rows (up to MT) x the wave's 32 columns over
