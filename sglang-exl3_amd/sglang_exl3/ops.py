@@ -69,17 +69,18 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     per-stream workspace in src/sglang_exl3/dense.py:45-58) and keeps the old
     one alive for graphs that captured it.
 
-    Growth is refused while the stream is being captured: the zero fill would
+    It does not grow while the stream is being captured: the zero fill would
     then only run at graph replay, and eager calls on the stream would find
-    an uninitialised buffer.  Run each op shape once before capture."""
+    an uninitialised buffer.  A call that needs less at its least (tall tiles
+    run with the k-splits whose partial tiles fit) then takes the buffer that is
+    there - the size asked for can be larger for fewer rows - and only one that
+    refuses it raises (check_ws): run such an op once before capture."""
     key = (device.index or 0, int(torch.cuda.current_stream(device).cuda_stream))
     ws = _WORKSPACES.get(key)
     capturing = torch.cuda.is_current_stream_capturing()
-    if ws is None or ws.numel() < nbytes:
-        if capturing:
-            raise RuntimeError(
-                f"sglang_exl3: the workspace of this stream must grow to {nbytes} bytes during HIP graph "
-                "capture; run the op once (same shape) on this stream before capturing")
+    if capturing and ws is None:
+        raise _growth_error(nbytes)
+    if not capturing and (ws is None or ws.numel() < nbytes):
         size = max(nbytes, 1 << 20, 0 if ws is None else 2 * ws.numel())
         if ws is not None and id(ws) in _CAPTURED:
             _RETIRED_WORKSPACES.append((key, ws))
@@ -90,6 +91,11 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     elif capturing:
         _CAPTURED[id(ws)] = ws
     return ws
+
+
+def _growth_error(nbytes: int) -> RuntimeError:
+    return RuntimeError(f"sglang_exl3: the workspace of this stream must grow to {nbytes} bytes during HIP graph "
+                        "capture; run the op once (same shape) on this stream before capturing")
 
 
 WAIT_CAUSES = {
@@ -129,13 +135,16 @@ def check_waits(device=None) -> None:
                            "last check_waits() are not valid")
 
 
-def check_ws(rc: int, what: str, ws) -> None:
+def check_ws(rc: int, what: str, ws, need: int = 0) -> None:
     """Raise for a non-zero status after re-zeroing the workspace the call
     used: a call that failed after some of its launches were enqueued can
     leave split-k counters or fixed-point accumulators non-zero, and every
     later call on the stream relies on them being zero."""
-    if rc != _lib.EXL3_OK and ws is not None and not torch.cuda.is_current_stream_capturing():
-        ws.zero_()
+    if rc != _lib.EXL3_OK and ws is not None:
+        if not torch.cuda.is_current_stream_capturing():
+            ws.zero_()
+        elif rc == _lib.EXL3_ERR_WORKSPACE and need > ws.numel():
+            raise _growth_error(need)
     _lib.check(rc, what)
 
 
@@ -209,7 +218,7 @@ def _gemv_like(name, fn, x, trellis, suh, svh, K, cb, max_rows=None, gemv=False)
         rc = fn(x2.data_ptr(), tr.data_ptr(), suh.data_ptr(), svh.data_ptr(), y.data_ptr(), m, kdim, n,
                 int(K), int(cb), 0 if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
                 _stream_ptr(x))
-    check_ws(rc, name, ws)
+    check_ws(rc, name, ws, need)
     return y
 
 
@@ -297,7 +306,7 @@ def _linear_weights(name, x, trellis, suh, svh, K, codebook, out_bf16, first, ap
                                       y.data_ptr(), _CAT_DTYPES[y.dtype], m, kdim, int(K), int(codebook),
                                       0 if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
                                       _stream_ptr(x))
-    check_ws(rc, name, ws)
+    check_ws(rc, name, ws, need)
     return y
 
 
@@ -328,7 +337,7 @@ def p2b_gemv_batched_impl(x, trellis_ptrs, suh_ptrs, svh_ptrs, expert_indices, K
             suh_ptrs.contiguous().data_ptr(), svh_ptrs.contiguous().data_ptr(), ids.data_ptr(), e,
             out.data_ptr(), m, kdim, n, int(K), _lib.codebook_from_mcg(bool(mcg)),
             0 if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream_ptr(x))
-    check_ws(rc, name, ws)
+    check_ws(rc, name, ws, need)
     return out
 
 
@@ -388,7 +397,7 @@ def p2b_fused_moe_impl(x, out, gate_trellis_ptrs, gate_suh_ptrs, gate_svh_ptrs, 
             x.data_ptr(), out.data_ptr(), *[t.data_ptr() for t in tabs], E, ids.data_ptr(), rw.data_ptr(),
             ids.numel(), hidden, inter, int(K_gate), int(K_up), int(K_down), _lib.codebook_from_mcg(bool(mcg)),
             _limit_arg(swiglu_limit), ws.data_ptr(), ws.numel(), _stream_ptr(x))
-    check_ws(rc, name, ws)
+    check_ws(rc, name, ws, need)
     return out
 
 
@@ -446,7 +455,7 @@ def _moe_layer(name, x, topk_ids, topk_weights, tables, K_gate, K_up, K_down, mc
             hidden, int(intermediate_size), int(K_gate), int(K_up), int(K_down),
             _lib.codebook_from_mcg(bool(mcg)) if int(codebook) < 0 else int(codebook), lim, _CAT_DTYPES[x.dtype],
             ws.data_ptr(), ws.numel(), _stream_ptr(x))
-    check_ws(rc, name, ws)
+    check_ws(rc, name, ws, need)
     return out
 
 
@@ -482,7 +491,7 @@ def exl3_gate_up_swiglu_impl(x, suh, gate_trellis, gate_svh, up_trellis, up_svh,
         rc = lib.exl3_gate_up_swiglu(x2.data_ptr(), suh.data_ptr(), gt.data_ptr(), gsv.data_ptr(), ut.data_ptr(),
                                      usv.data_ptr(), out.data_ptr(), m, kdim, n, int(K), int(codebook),
                                      _limit_arg(swiglu_limit), ws.data_ptr(), ws.numel(), _stream_ptr(x))
-    check_ws(rc, name, ws)
+    check_ws(rc, name, ws, need)
     return out
 
 
