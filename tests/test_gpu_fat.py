@@ -210,21 +210,21 @@ def test_tail_split_repeatable(op, cb, monkeypatch):
         assert torch.equal(outs[0], whole)
 
 
-@pytest.mark.parametrize("op,m", [("gemm", 16), ("gemm", 48), ("gemm", 300), ("gate_up", 16), ("gate_up", 48),
+@pytest.mark.parametrize("op,m", [("gemm", 16), ("gemm", 20), ("gemm", 48), ("gemm", 300), ("gate_up", 16), ("gate_up", 48),
                                   ("gate_up", 200)])
 def test_mul1_raw_entries(op, m, monkeypatch):
-    """Narrow 16-row MFMA tiles on mul1 weights read raw entries (1024 + byte
-    sum, no affine step) and correct in the epilogue with kinv * acc + bias *
-    (row sum of the rotated x over the split's k range).  k = 14336 (112 chunk
-    sums per row), 16-row tiles with k-splits (m = 16): against the oracle and
-    close to the decoded path (EXL3_FAT_RAW=0).  The wide tiles in gate/up mode
-    (m = 200: tail-split k-halves, the row sums taken in the epilogue) read
-    raw entries too; the 64-row tiles (m = 48) and the plain wide tiles (gemm
-    m = 300, forced by EXL3_FAT_WIDE=2: 16 fp32-atomic k-splits) decode values
-    and are checked at the same k."""
+    """Narrow 16-row MFMA tiles and tall tiles on mul1 weights read raw entries
+    (1024 + byte sum, no affine step) and correct in the epilogue with kinv * acc
+    + bias * (row sum of the rotated x over the split's k range).  k = 14336 (112
+    chunk sums per row), 16-row tiles with k-splits (m = 16; EXL3_FAT_TALL=0 for
+    gemm, which takes tall tiles there at this width), tall tiles (gemm m = 20,
+    gate/up m = 48 and 200): against the oracle and close to the decoded path
+    (EXL3_FAT_RAW=0).  The 64-row tiles (gemm m = 48, EXL3_FAT_TALL=0) and the
+    plain wide tiles (gemm m = 300, EXL3_FAT_WIDE=2: 16 fp32-atomic k-splits)
+    decode values and are checked at the same k."""
     k, n, K, cb = 14336, 256, 3, 2
-    if op == "gemm" and m > 256:
-        monkeypatch.setenv("EXL3_FAT_WIDE", "2")
+    if op == "gemm" and m != 20:
+        monkeypatch.setenv(*(("EXL3_FAT_WIDE", "2") if m > 256 else ("EXL3_FAT_TALL", "0")))
     print(f"case: raw mul1 {op} m={m} k={k} n={n}", flush=True)
     x = torch.from_numpy(make_x(m, k, seed=51 + m)).cuda()
     if op == "gemm":
@@ -339,7 +339,7 @@ def test_tall_tiles_take_the_splits_that_fit(m):
         check_close(z.float().cpu().numpy(), oracle.swiglu(g, u, float("inf")), f"gate/up m={m} in {size} bytes")
 
 
-@pytest.mark.parametrize("kind", ["1", "128", "256"])
+@pytest.mark.parametrize("kind", ["1", "1 whole", "128", "256"])
 @pytest.mark.parametrize("m,k,n,K,cb,splits,limit", [
     (17, 128, 128, 1, 1, 1, 0.0), (31, 256, 384, 2, 2, 2, 1.0), (32, 512, 128, 3, 0, 4, 0.0),
     (33, 1024, 256, 4, 1, 8, 0.0), (127, 384, 128, 5, 2, 1, 2.0), (128, 256, 256, 6, 0, 2, 0.0),
@@ -347,10 +347,13 @@ def test_tall_tiles_take_the_splits_that_fit(m):
     (257, 256, 128, 4, 0, 1, 0.0), (520, 1024, 128, 3, 1, 1, 0.0)])
 def test_gate_up_tall_tiles(m, k, n, K, cb, splits, limit, kind, monkeypatch):
     """gate/up + SwiGLU on tall tiles: partial tiles of either height with the finish launch, or both projections in
-    one workgroup (k a multiple of 256: every tile as two k-halves), at the edges of their row groups, every K and
-    codebook: against the oracle, bit-equal when repeated and into an output that is only 4-byte aligned."""
+    one workgroup of up to 256 rows ("1 whole") or of a quarter of them ("1": these grids leave most CUs idle, so
+    every tile runs as four row parts), at the edges of their row groups, every K and codebook: against the oracle,
+    bit-equal when repeated and into an output that is only 4-byte aligned."""
     print(f"case: gate/up tall kind={kind} m={m} k={k} n={n} K={K} cb={cb} splits={splits}", flush=True)
-    monkeypatch.setenv("EXL3_GU_TALL", kind)
+    monkeypatch.setenv("EXL3_GU_TALL", kind.split()[0])
+    if kind == "1 whole":
+        monkeypatch.setenv("EXL3_FAT_TAIL", "0")
     monkeypatch.setenv("EXL3_FAT_SPLITS", str(splits))
     tg, su, sg = make_weight(k, n, K, seed=m + K)
     tu, _, sv_u = make_weight(k, n, K, seed=m + K + 50)
@@ -373,14 +376,43 @@ def test_gate_up_tall_tiles(m, k, n, K, cb, splits, limit, kind, monkeypatch):
     assert torch.equal(odd[2:].view(m, n), y)
 
 
-@pytest.mark.parametrize("m,cb", [(16, 1), (64, 2)])
-def test_gemm_split_handoff_repeatable(m, cb, monkeypatch):
+@pytest.mark.parametrize("m,k,n,K,cb,limit", [(1300, 128, 7168, 3, 1, 0.0), (1300, 256, 7168, 2, 2, 1.0),
+                                              (1100, 128, 8192, 4, 0, 0.0)])
+def test_gate_up_fused_whole_tiles_and_parts(m, k, n, K, cb, limit, monkeypatch):
+    """The fused gate/up kernel with a full round of whole tiles before the tail's (256 CUs: 336 tiles, the last 80 in
+    two row parts each; 320 tiles, the last 64 in four) and a ragged last row tile: against the oracle, and the bits
+    of whole tiles throughout (EXL3_FAT_TAIL=0)."""
+    print(f"case: fused gate/up tail m={m} k={k} n={n} K={K} cb={cb}", flush=True)
+    monkeypatch.setenv("EXL3_GU_TALL", "1")
+    tg, su, sg = make_weight(k, n, K, seed=m + K)
+    tu, _, sv_u = make_weight(k, n, K, seed=m + K + 50)
+    scale = np.float32(4.0 / np.sqrt(k))
+    sg, sv_u = ((v.astype(np.float32) * scale).astype(np.float16) for v in (sg, sv_u))
+    x = make_x(m, k, seed=m)
+    d = [torch.from_numpy(v).cuda() for v in (x, su, tg, sg, tu, sv_u)]
+    y = torch.ops.sglang_exl3.exl3_gate_up_swiglu(*d, K, cb, limit)
+    assert torch.equal(y, torch.ops.sglang_exl3.exl3_gate_up_swiglu(*d, K, cb, limit))
+    g = oracle.matmul(x, oracle.dequant(tg, su, sg, K, cb, rtz=True))
+    u = oracle.matmul(x, oracle.dequant(tu, su, sv_u, K, cb, rtz=True))
+    check_close(y.float().cpu().numpy(), oracle.swiglu(g, u, limit or float("inf")), f"fused gate/up m={m}")
+    monkeypatch.setenv("EXL3_FAT_TAIL", "0")
+    assert torch.equal(y, torch.ops.sglang_exl3.exl3_gate_up_swiglu(*d, K, cb, limit))
+
+
+@pytest.mark.parametrize("m,k,n,cb", [(16, 4096, 2048, 1), (64, 4096, 2048, 2), (14, 14336, 4608, 2),
+                                      (16, 14336, 4608, 1)])
+def test_gemm_split_handoff_repeatable(m, k, n, cb, monkeypatch):
     """exl3_gemm's narrow k-splits hand partial tiles to the last split of each
-    (column block, row tile): against the oracle, bit-identical over repeated
-    calls (the counters reset themselves), and close to the fp32-atomic path
-    (EXL3_FAT_HANDOFF=0).  k = 4096, n = 2048: four splits of 16 steps."""
-    k, n, K = 4096, 2048, 3
-    print(f"case: gemm split hand-off m={m} cb={cb}", flush=True)
+    (column block, row tile), in the kernel or (16 rows, up to four splits) in a
+    finish launch: against the oracle, bit-identical over repeated calls (the
+    counters reset themselves), and close to the fp32-atomic path
+    (EXL3_FAT_HANDOFF=0).  k = 4096, n = 2048: four splits of 16 steps
+    (EXL3_FAT_TALL=0, which tall tiles would take); k = 14336, n = 4608: eight of
+    28, the hand-off that a default plan runs in the kernel."""
+    K = 3
+    if n <= 4096:
+        monkeypatch.setenv("EXL3_FAT_TALL", "0")
+    print(f"case: gemm split hand-off m={m} k={k} n={n} cb={cb}", flush=True)
     x = torch.from_numpy(make_x(m, k, seed=61 + m)).cuda()
     tr, su, sv = make_weight(k, n, K, seed=62)
     d = [torch.from_numpy(v).cuda() for v in (tr, su, sv)]
@@ -406,6 +438,7 @@ def test_gemm_split_out_finish_matches_in_kernel_handoff(m, cb, monkeypatch):
     k, n, K = 2048, 384, 3
     print(f"case: gemm split-out finish m={m} cb={cb}", flush=True)
     monkeypatch.setenv("EXL3_GEMM_GEMV_ROWS", "0")  # the MFMA path at every m
+    monkeypatch.setenv("EXL3_FAT_TALL", "0")  # 16-row tiles at 13 and 16 rows too
     x = torch.from_numpy(make_x(m, k, seed=81 + m)).cuda()
     tr, su, sv = make_weight(k, n, K, seed=82 + cb)
     d = [torch.from_numpy(v).cuda() for v in (tr, su, sv)]
@@ -421,12 +454,14 @@ def test_gemm_split_out_finish_matches_in_kernel_handoff(m, cb, monkeypatch):
 
 @pytest.mark.parametrize("m", [13, 40, 100, 250])
 @pytest.mark.parametrize("cb", [0, 1, 2])
-def test_gemm_split_handoff_ragged_rows(m, cb):
-    """The split hand-off on row counts that leave the last row tile partial
-    (16-row tiles at 13 rows, 64-row tiles above), every codebook (3INST
-    through exl3_linear): k = 2048 gives two splits of 16 steps, n = 384 three
-    column blocks.  Against the oracle, and bit-identical on a repeat call."""
+def test_gemm_split_handoff_ragged_rows(m, cb, monkeypatch):
+    """The split hand-off of the narrow kernel (EXL3_FAT_TALL=0) on row counts
+    that leave the last row tile partial (16-row tiles at 13 rows, 64-row tiles
+    above), every codebook (3INST through exl3_linear): k = 2048 gives two splits
+    of 16 steps, n = 384 three column blocks.  Against the oracle, and
+    bit-identical on a repeat call."""
     k, n, K = 2048, 384, 4
+    monkeypatch.setenv("EXL3_FAT_TALL", "0")
     print(f"case: gemm split hand-off ragged m={m} cb={cb}", flush=True)
     x = torch.from_numpy(make_x(m, k, seed=71 + m)).cuda()
     tr, su, sv = make_weight(k, n, K, seed=72 + cb)
@@ -454,10 +489,12 @@ def test_fat_narrow_every_width(K, cb):
 
 @pytest.mark.parametrize("K", range(1, 9))
 @pytest.mark.parametrize("cb", [1, 2])
-def test_gemm_16_rows_every_width(K, cb):
-    """exl3_gemm at 16 rows (16-row tiles, k-split hand-off; mul1 reads raw
-    entries) at every bit width, against the oracle."""
+def test_gemm_16_rows_every_width(K, cb, monkeypatch):
+    """exl3_gemm at 16 rows (16-row tiles, which tall tiles replace at this width
+    unless EXL3_FAT_TALL=0; mul1 reads raw entries) at every bit width, against
+    the oracle."""
     m, k, n = 16, 1024, 256
+    monkeypatch.setenv("EXL3_FAT_TALL", "0")
     print(f"case: gemm 16 rows K={K} cb={cb}", flush=True)
     tr, su, sv = make_weight(k, n, K, seed=300 + 3 * K + cb)
     x = make_x(m, k, seed=301 + K)

@@ -2,10 +2,11 @@
 oracle: out = silu(min(x W_g, L)) * clamp(x W_u, -L, L), both weights sharing
 the input rotation suh, as the reference's fused gate/up path does
 (src/sglang_exl3/exl3.py:1184-1206).  Up to 3 rows the GEMV kernel (gate and
-up rounded to fp16 first), up to 160 the narrow MFMA kernel in gate/up mode
-(k-splits hand partial tiles to the last split, or up to 16 rows to a finish
-launch), above the wide-tile MFMA kernel (fp32 accumulators throughout).  Bar: max-abs-err <= 2e-2 * rms(ref),
-cosine >= 0.9999."""
+up rounded to fp16 first), up to 16 the narrow MFMA kernel in gate/up mode
+(k-splits hand partial tiles to the last split, or from 6 rows to a finish
+launch), above tall tiles (partial tiles with the finish launch, or both
+projections in one workgroup; fp32 accumulators throughout).  Bar: max-abs-err
+<= 2e-2 * rms(ref), cosine >= 0.9999."""
 
 import numpy as np
 import pytest
@@ -62,10 +63,10 @@ def test_gate_up_swiglu_vs_oracle(m, k, n, K, cb):
 
 @pytest.mark.parametrize("m,cb", [(5, 2), (13, 0), (40, 1), (100, 2), (150, 0), (160, 1)])
 def test_gate_up_split_handoff_ragged_rows(m, cb):
-    """The narrow kernel's gate/up k-splits (k = 2048: two splits of 16 steps,
-    n = 384: three column blocks per projection) on row counts that leave the
-    last row tile partial; bit-identical on a repeat call (the counters reset
-    themselves)."""
+    """Gate/up k-splits (k = 2048, n = 384: three column blocks per projection) on
+    row counts that leave the last row tile partial: the narrow kernel's hand-off
+    (5 rows), its finish launch (13), tall tiles' partial tiles (above);
+    bit-identical on a repeat call (the counters reset themselves)."""
     k, n, K = 2048, 384, 3
     print(f"case: gate_up split hand-off ragged m={m} cb={cb}", flush=True)
     tg, su, sg, tu, sv_u = _pair(k, n, K, seed=110 + m)
@@ -80,7 +81,7 @@ def test_gate_up_split_handoff_ragged_rows(m, cb):
 @pytest.mark.parametrize("m,cb,limit", [(6, 2, 0.0), (9, 1, 1.5), (16, 2, 0.0), (16, 0, 2.0)])
 def test_gate_up_split_out_finish_matches_in_kernel_handoff(m, cb, limit, monkeypatch):
     """From 6 to 16 rows the narrow gate/up k-splits store their partial tiles and
-    a second launch (fat_gu_finish_kernel) finishes every row; its sums and
+    a second launch (fat_split_finish_kernel) finishes every row; its sums and
     epilogue are the in-kernel hand-off's, so both give the same bits
     (EXL3_FAT_SPLIT_OUT=0 keeps the hand-off), also with a clamp and the
     mul1 raw-entry map (cb 2)."""

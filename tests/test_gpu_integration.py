@@ -251,11 +251,16 @@ def test_mgemm_two(rows, n0, n1, K0, K1, cb0, cb1, second):
     (3, (128, 384), 3, 2, torch.bfloat16, torch.float16, {}),         # ... two rows of blocks, mul1
     (5, (256, 128), 4, 0, torch.float16, torch.bfloat16, {}),         # k-split GEMV, fixed-point hand-off
     (11, (128, 256, 128, 128), 2, 1, torch.bfloat16, torch.bfloat16, {}),  # k-split GEMV, partial tiles
-    (14, (384, 128), 3, 2, torch.bfloat16, torch.bfloat16, {}),       # 16-row tiles, raw entries, finish launch
-    (40, (128, 256), 4, 1, torch.bfloat16, torch.float16, {}),        # 64-row tiles, split hand-off
-    (70, (128, 256), 5, 2, torch.float16, torch.bfloat16, {"EXL3_FAT_HANDOFF": "0"}),
-    (300, (256, 512), 3, 1, torch.bfloat16, torch.bfloat16, {"EXL3_FAT_WIDE": "2"}),  # wide tiles
-    (300, (128, 512), 3, 1, torch.bfloat16, torch.bfloat16, {"EXL3_FAT_WIDE": "2"}),  # a width the wide tiles refuse
+    # 16-row tiles, raw entries: finish launch, hand-off in the kernel, unsplit
+    (14, (384, 128), 3, 2, torch.bfloat16, torch.bfloat16, {"EXL3_FAT_TALL": "0"}),
+    (14, (384, 128), 3, 2, torch.bfloat16, torch.bfloat16, {"EXL3_FAT_TALL": "0", "EXL3_FAT_SPLIT_OUT": "0"}),
+    (16, (256, 128), 5, 2, torch.float16, torch.bfloat16, {"EXL3_FAT_TALL": "0", "EXL3_FAT_HANDOFF": "0"}),
+    (13, (4096, 128, 256), 4, 0, torch.bfloat16, torch.bfloat16, {}),  # ... by default above 4096 columns, decoded values
+    (14, (384, 128), 3, 2, torch.bfloat16, torch.bfloat16, {}),       # tall tiles from 13 rows, raw entries
+    (40, (128, 256), 4, 1, torch.bfloat16, torch.float16, {}),        # tall tiles, finish launch
+    (300, (256, 128), 3, 2, torch.bfloat16, torch.bfloat16, {"EXL3_FAT_TALL": "256", "EXL3_FAT_SPLITS": "1"}),  # no splits
+    (70, (128, 256), 5, 2, torch.float16, torch.bfloat16, {"EXL3_FAT_HANDOFF": "0"}),  # the switches of other kernels
+    (300, (256, 512), 3, 1, torch.bfloat16, torch.bfloat16, {"EXL3_FAT_WIDE": "2"}),   # name one weight's (tall tiles here)
 ])
 def test_linear_cat(m, widths, K, cb, x_dtype, y_dtype, env, monkeypatch):
     """Several weights in one call, each kernel path, against one exl3_linear per weight with the casts

@@ -618,14 +618,14 @@ def test_moe_rejects_bad_arguments():
 # ------------------------------------------------------------- prefill path
 #
 # Batches whose experts get many rows each (or more than 8192 routed rows) run
-# the prefill pipeline: device-side sort into 64/128-row tiles, one rotation
-# pass, the grouped MFMA GEMM for gate, up (+ SwiGLU + down rotation) and down,
-# then the slot-ordered combine.  EXL3_MOE_PREFILL=1 forces it for small cases.
+# the prefill pipeline: device-side sort into 128-row tiles (64 where gate and up
+# have different bit widths), one rotation pass, the grouped MFMA GEMM for gate
+# and up (+ SwiGLU + down rotation) and down, then the slot-ordered combine.  EXL3_MOE_PREFILL=1 forces it for small cases.
 
 
 @pytest.mark.parametrize("T,topk,E,hidden,inter,Ks,cb,invalid", [
-    (40, 4, 8, 256, 256, (3, 3, 3), 1, 0),     # ~20 rows per expert: 64-row tiles
-    (300, 2, 4, 256, 128, (2, 3, 4), 2, 3),    # ~150 rows per expert: several 128-row tiles; per-projection K
+    (40, 4, 8, 256, 256, (3, 3, 3), 1, 0),     # ~20 rows per expert: one partial 128-row tile each
+    (300, 2, 4, 256, 128, (2, 3, 4), 2, 3),    # ~150 rows per expert; per-projection K: 64-row tiles
     (64, 8, 16, 512, 384, (4, 4, 4), 0, 5),    # 3INST codebook, invalid ids
     (1, 3, 4, 256, 256, (3, 3, 3), 1, 0),      # a single token through the prefill pipeline
 ])

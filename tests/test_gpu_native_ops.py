@@ -47,14 +47,17 @@ def _same(op, general, args):
 
 @pytest.mark.parametrize("name", ["gemv", "cat", "part", "cat1", "gate_up"])
 @pytest.mark.parametrize("m", [1, 17, 64])
-def test_native_equals_general(weights, name, m):
+def test_native_equals_general(weights, name, m, monkeypatch):
     print(f"case: native op {name} m={m}", flush=True)
     x = torch.from_numpy(make_x(m, k, seed=m)).cuda()
     op, general, args = _calls(weights, x)[name]
     want = general(*args)
-    for _ in range(2):
-        got = op(*args)
-        assert got.dtype == want.dtype and torch.equal(got, want)
+    with monkeypatch.context() as mp:  # the Python implementation is not reached: the call is the native path's
+        for impl in ("exl3_gemv_impl", "exl3_linear_cat_impl", "exl3_linear_part_impl", "exl3_gate_up_swiglu_impl"):
+            mp.setattr(ops, impl, lambda *a: pytest.fail("general path"))
+        for _ in range(2):
+            got = op(*args)
+            assert got.dtype == want.dtype and torch.equal(got, want)
     with torch.inference_mode():
         assert torch.equal(op(*args), want)
     # strided rows, three-dimensional rows, rows at an odd element offset
