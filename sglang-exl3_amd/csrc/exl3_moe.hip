@@ -923,12 +923,12 @@ PrefillLayout prefill_layout(int tokens, int topk, int E, int hidden, int inter)
     o = align256(o + (size_t)L.max_tiles * sizeof(FatTile));
     L.xr_off = o;
     o = align256(o + (size_t)2 * L.entries * hidden * 2);
-    L.g_off = o;
-    o = align256(o + (size_t)L.entries * inter * 4);
     L.h_off = o;
     o = align256(o + (size_t)L.entries * inter * 2);
-    L.y_off = o;
-    o = align256(o + (size_t)L.entries * hidden * 2);
+    // the gate's fp32 rows (64-row tiles) are read before the down pass writes y
+    L.g_off = L.y_off = o;
+    const size_t g = (size_t)L.entries * inter * 4, y = (size_t)L.entries * hidden * 2;
+    o = align256(o + (g > y ? g : y));
     L.total = o;
     return L;
 }
