@@ -255,6 +255,7 @@ def test_mgemm_two(rows, n0, n1, K0, K1, cb0, cb1, second):
     (14, (384, 128), 3, 2, torch.bfloat16, torch.bfloat16, {"EXL3_FAT_TALL": "0"}),
     (14, (384, 128), 3, 2, torch.bfloat16, torch.bfloat16, {"EXL3_FAT_TALL": "0", "EXL3_FAT_SPLIT_OUT": "0"}),
     (16, (256, 128), 5, 2, torch.float16, torch.bfloat16, {"EXL3_FAT_TALL": "0", "EXL3_FAT_HANDOFF": "0"}),
+    (16, (256,), 3, 1, torch.float16, torch.bfloat16, {"EXL3_FAT_TALL": "0", "EXL3_FAT_HANDOFF": "0"}),  # fp32 sums, then bf16
     (13, (4096, 128, 256), 4, 0, torch.bfloat16, torch.bfloat16, {}),  # ... by default above 4096 columns, decoded values
     (14, (384, 128), 3, 2, torch.bfloat16, torch.bfloat16, {}),       # tall tiles from 13 rows, raw entries
     (40, (128, 256), 4, 1, torch.bfloat16, torch.float16, {}),        # tall tiles, finish launch
