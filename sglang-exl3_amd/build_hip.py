@@ -109,11 +109,15 @@ def _build_ops(force: bool) -> None:
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", f'-DEXL3_TORCH_VERSION="{version}"',
            *(f"-I{i}" for i in inc), src, "-o", out + ".tmp", f"-L{os.path.join(torch_dir, 'lib')}",
            "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", f"-L{os.path.join(rocm, 'lib')}", "-lamdhip64"]
-    r = subprocess.run(cmd, capture_output=True, text=True)
+    try:
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        error = r.stderr[-6000:] if r.returncode else None
+    except OSError as e:  # no g++: hipcc brings its own compiler
+        error = str(e)
     if os.path.exists(out):
         os.remove(out)
-    if r.returncode != 0:
-        print(f"warning: the operators' native entry is not built, g++ failed for torch_ops.cpp:\n{r.stderr[-6000:]}",
+    if error is not None:
+        print(f"warning: the operators' native entry is not built, g++ failed for torch_ops.cpp:\n{error}",
               file=sys.stderr)
         return
     os.replace(out + ".tmp", out)

@@ -92,6 +92,23 @@ else:
     assert r.returncode == 0, r.stderr[-2000:]
 
 
+@pytest.mark.parametrize("fault", ["no compiler", "does not compile"])
+def test_build_without_the_native_path(fault, tmp_path, monkeypatch, capsys):
+    """Where the second library cannot be built, the build warns and leaves none behind that is out of date."""
+    monkeypatch.syspath_prepend(PKG)
+    import build_hip
+
+    old = tmp_path / build_hip.OPS_LIBNAME
+    old.write_bytes(b"an older one")
+    (tmp_path / "torch_ops.cpp").write_text("#error")
+    monkeypatch.setattr(build_hip, "LIBDIR", str(tmp_path))
+    monkeypatch.setattr(build_hip, "CSRC", str(tmp_path))
+    if fault == "no compiler":
+        monkeypatch.setenv("PATH", str(tmp_path))
+    build_hip._build_ops(force=False)
+    assert "native entry is not built" in capsys.readouterr().err and not old.exists()
+
+
 def test_cpu_tensors_are_refused():
     x = torch.zeros((1, 128), dtype=torch.float16)
     trellis = torch.zeros((8, 16, 32), dtype=torch.int16)
