@@ -343,6 +343,13 @@ def test_kv_only_has_the_bits_of_apply(outs, cb, dtype):
         got = method.apply_kv_only(layer, x)
         for g, w in zip(got, want):
             assert g.is_contiguous() and g.dtype == dtype and torch.equal(g, w)
+        # the operators themselves, from every weight on
+        args = (x.view(rows, k), *map(list, zip(*packs)), K, cb, dtype == torch.bfloat16)
+        cat = torch.ops.sglang_exl3.exl3_linear_cat(*args).split(outs, dim=1)
+        for first in range(len(outs)):
+            part = torch.ops.sglang_exl3.exl3_linear_part(*args, first).split([rows * n for n in outs[first:]])
+            for p, c in zip(part, cat[first:]):
+                assert torch.equal(p.view(rows, -1), c), (rows, first)
     assert method.apply_kv_only(layer, x[:, :0])[0].shape == (1, 0, outs[1])
 
 
